@@ -128,6 +128,7 @@ struct Plan {
   int m2l_mode = FMM2D_M2L_DENSE;   // FP64 M2L: every slot dense, or compressed as the reference
   Tree tree;
   DevBuf ops;
+  DevBuf opsm;         // FP64 M2L: the M2L blocks of each level in MFMA operand order (k_m2l_pack)
   int ops_levels = 0;
   std::vector<char> ops_set;
   DevBuf logtab;
@@ -725,12 +726,6 @@ constexpr int kM2LThreads = 256;   // threads per block and row split
 constexpr int kM2LCols = 64;
 constexpr int kM2LRowSplit = 1;   // blocks of 4 waves, each wave all PD rows of 16 boxes
 constexpr int kM2LSplitF64 = 2;   // FP64 M2L: blocks per tile when tiles are few
-// Dense FP64 M2L in narrow tiles (k_m2l_waves_f64) up to this padded
-// dimension: at PD 32 it beats the LDS-staged tiles (100K points, p 32:
-// 0.034 -> 0.028 ms); at PD 64 each wave re-reading 32 KB per slot from L2
-// costs more than the shared stage (1M points, p 60: 0.151 -> 0.189 ms).
-constexpr int kM2LWavesF64MaxPD = 32;
-
 struct M2LSetup {
   int li, c, col, kq, g, nph, rh;
   bool active;
@@ -865,7 +860,7 @@ __global__ __launch_bounds__(kM2LOrderThreads) void k_m2l_order(M2LOrderTable ot
     perm[ot.poff[li] + c * ng + q0 + i] = q0 + (int)(key[i] & 2047u);
 }
 
-// FP64 M2L.  use_svd: slots whose rank table entry is r > 0 are applied in
+// FP64 M2L in the compressed form (FMM2D_M2L_SVD): slots whose rank table entry is r > 0 are applied in
 // the reference's compressed form, M2 (M1 q) (helpers.py:37-45), in two MFMA
 // stages: T = M1 q (r rows, ceil(r/16) row blocks, K = PD), then
 // acc += M2 T with K = 4 ceil(r/4); the first stage's result registers (lane
@@ -879,8 +874,7 @@ __global__ __launch_bounds__(kM2LThreads * RS) void k_m2l_all(LevelTable lt,
                                                         const double* __restrict__ mult,
                                                         const double* __restrict__ ops,
                                                         int64_t opsz, double* __restrict__ ple,
-                                                        int64_t rstride, int64_t nstride,
-                                                        int use_svd) {
+                                                        int64_t rstride, int64_t nstride) {
   // density blockIdx.y: multipole rows rstride rows further, local rows nstride nodes further
   mult += (int64_t)blockIdx.y * rstride * PD;
   ple += (int64_t)blockIdx.y * nstride * PD;
@@ -896,7 +890,7 @@ __global__ __launch_bounds__(kM2LThreads * RS) void k_m2l_all(LevelTable lt,
   const int rb0 = S.rh * RB;   // this wave's first row block
   const double* opsL = ops + (int64_t)lt.d[S.li] * opsz;
   if (threadIdx.x < kNumM2L)
-    srank[threadIdx.x] = use_svd ? (int)opsL[ops_off_svd_rank(PD) + threadIdx.x] : -1;
+    srank[threadIdx.x] = (int)opsL[ops_off_svd_rank(PD) + threadIdx.x];
   __syncthreads();
   d4 acc[RB];
 #pragma unroll
@@ -1255,118 +1249,225 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   }
 }
 
-// FP64 M2L (dense form) in narrow tiles, as k_m2l_waves_f32: 16 boxes per
-// block, their slots dealt to 4 waves, sums added in wave order at the end.
-// The M2L blocks stay row-major: step 2 m + h of lane group kq multiplies
-// k = 8 m + 2 kq + h, so a lane's A operands for two steps are one 16-byte
-// load and the 4 lane groups of a row read 64 consecutive bytes (as for the
-// multipoles).  Row blocks run one after another, each loading its operands
-// just before its 16 steps, which keeps the kernel at 4 waves per SIMD.
-// D layout of v_mfma_f64_16x16x4f64: lane l holds D[4 v + l/16][l%16].
-template <int PD>
-__global__ __launch_bounds__(64 * kM2LWWaves) __attribute__((amdgpu_waves_per_eu(4)))
-void k_m2l_waves_f64(LevelTable lt, const int* __restrict__ flags, const int* __restrict__ m2l,
-                     const double* __restrict__ mult, const double* __restrict__ ops,
-                     int64_t opsz, double* __restrict__ ple, int64_t rstride, int64_t nstride) {
-  constexpr int RB = PD / 16, KS = PD / 4, NW = kM2LWWaves;
+// FP64 M2L, dense form.  A block takes 16 NCG target boxes of one level and
+// child position (NCG column groups of 16) and deals the slots that any of
+// its boxes uses to SG waves; every wave computes RBW row blocks of 16 rows
+// (RB / RBW blocks share a tile).  PE is p rounded up to 16 (PD is the row
+// stride): the padding past PE is never multiplied.  ODD (p mod 8 in 1..4):
+// the last pair of k-steps is one step.
+//
+// What bounds it: the FP64 matrix cores, once their operands arrive.  They
+// come straight from L2 into registers, with no LDS stage and no barrier per
+// slot: the operator from a copy in MFMA operand order (k_m2l_pack: one wave
+// load reads 1 KB in one piece; row-major blocks cost 16 pieces of 64 bytes),
+// the multipoles by 16-byte loads.  Step 2 m + h of lane group kq multiplies
+// k = 8 m + 2 kq + h, so a 16-byte load of either operand feeds two steps.
+// The loads of step pair m run kDepth pairs ahead of its MFMAs, across slot
+// boundaries.  Every operator load feeds NCG column groups: with one group
+// the operands alone take 60% of a CU's L2 bandwidth at full matrix rate.
+// Against 64-box tiles that staged the operator in LDS (kernel time, PD 64):
+// 1M uniform points 143 -> 95 us, order-8 black-box on the same points
+// 480 -> 358 us, 1M clustered points 315 -> 230 us, 50K points at Ncutoff
+// 500 (5 levels) 51 -> 14 us; at PD 32, 100K points, 25.6 -> 16.5 us.
+template <int PE, int NCG, int RBW>
+struct M2LShape {
+  // row blocks, step pairs, blocks per tile, boxes per tile
+  static constexpr int RB = PE / 16, KP = PE / 8, RG = RB / RBW, C = 16 * NCG;
+  // step pairs of operands in flight
+  static constexpr int kDepth = NCG == 1 ? KP / 2 : 2;
+};
+constexpr int kM2LF64Waves = 4;
+
+template <int PD, int PE, int NCG, int RBW, bool ODD>
+__global__ __launch_bounds__(64 * kM2LF64Waves) void k_m2l_f64(
+    LevelTable lt, const int* __restrict__ flags, const int* __restrict__ m2l,
+    const double* __restrict__ mult, const double* __restrict__ opsm, int64_t opsmsz,
+    double* __restrict__ ple, int64_t rstride, int64_t nstride) {
+  typedef M2LShape<PE, NCG, RBW> Sh;
+  constexpr int RB = Sh::RB, KP = Sh::KP, RG = Sh::RG, C = Sh::C, D = Sh::kDepth;
+  constexpr int SG = kM2LF64Waves;
+  static_assert(RG * RBW == RB && KP % D == 0 && C <= 32, "tile shape");
+  __shared__ int srcs[32][C];
+  __shared__ int pidx[32], pslot[32];
+  __shared__ unsigned int smask;
+  __shared__ double red[SG - 1][16 * RBW][17];
+  // density blockIdx.y
   mult += (int64_t)blockIdx.y * rstride * PD;
   ple += (int64_t)blockIdx.y * nstride * PD;
-  __shared__ int srcs[27][kM2LWCols];
-  __shared__ int pslot[28];
-  __shared__ unsigned int smask;
-  __shared__ double red[NW - 1][PD][kM2LWCols + 1];
-  const int bid = xcd_block(blockIdx.x, gridDim.x);
+  const int bid0 = xcd_block(blockIdx.x, gridDim.x);
+  const int rg = bid0 % RG, bid = bid0 / RG;   // the row groups of a tile are neighbours
   int li = 0;
   while (li + 1 < lt.nlev && bid >= lt.boff[li + 1]) ++li;
   const int lb = bid - lt.boff[li];
   const int c = lb & 3;
   const int tile = lb >> 2;
   const int ngroups = lt.ngroups[li];
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int l = threadIdx.x & 63, sg = threadIdx.x >> 6;
   const int col = l & 15, kq = l >> 4;
-  const int qq = tile * kM2LWCols + col;
-  const int q = (lt.perm && qq < ngroups) ? lt.perm[lt.poff[li] + c * ngroups + qq] : qq;
-  const int g = lt.g0[li] + 4 * q + c;
-  const bool active = q < ngroups && !(flags[q < ngroups ? g : lt.g0[li]] & NF_FAKE);
   const int nv = c_valid.n[c];
-  const int* lst = m2l + (int64_t)g * kNumM2L;
+  // box of column cc of the tile (a column past the level's last box: that
+  // box); live(cc, g): whether the column has a box of its own to fill
+  auto box = [&](int cc) -> int {
+    const int qq = min(tile * C + cc, ngroups - 1);
+    return lt.g0[li] + 4 * (lt.perm ? lt.perm[lt.poff[li] + c * ngroups + qq] : qq) + c;
+  };
+  auto live = [&](int cc, int g) -> bool {
+    return tile * C + cc < ngroups && !(flags[g] & NF_FAKE);
+  };
   if (threadIdx.x == 0) smask = 0u;
   __syncthreads();
   unsigned int used = 0u;
+  {
+    const int cc = threadIdx.x & (C - 1);
+    const int g = box(cc);
+    const bool act = live(cc, g);
+    const int* lst = m2l + (int64_t)g * kNumM2L;
+    constexpr int NE = 32 * C / (64 * SG);
+    int e[NE];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int i = 4 * w + kq + 16 * j;
-    const int src = (active && i < nv) ? lst[c_valid.slot[c][i]] : -1;
-    if (i < nv) srcs[i][col] = src;
-    const unsigned long long b = __ballot(src >= 0);
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if ((b >> (16 * k)) & 0xffffull) used |= 1u << (4 * w + k + 16 * j);
-  }
-  if (l == 0 && used) atomicOr(&smask, used);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned int m = smask;
-    int k = 0;
-    while (m) {
-      pslot[k++] = __builtin_ctz(m);
-      m &= m - 1u;
+    for (int j = 0; j < NE; ++j) {
+      const int i = (threadIdx.x + 64 * SG * j) / C;
+      e[j] = lst[c_valid.slot[c][i < nv ? i : 0]];   // loaded with the flags
     }
-    pslot[27] = k;
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      const int i = (threadIdx.x + 64 * SG * j) / C;
+      const int src = act && i < nv ? e[j] : -1;
+      srcs[i][cc] = src;
+      const unsigned long long b = __ballot(src >= 0) >> (l & ~(C - 1));
+      if ((l & (C - 1)) == 0 && (b & ((1ull << C) - 1ull))) used |= 1u << i;
+    }
+  }
+  if (used) atomicOr(&smask, used);
+  __syncthreads();
+  const unsigned int mask = smask;
+  const int nph = __popc(mask);
+  if (threadIdx.x < 32 && (mask >> threadIdx.x & 1u)) {
+    const int k = __popc(mask & ((1u << threadIdx.x) - 1u));
+    pidx[k] = threadIdx.x;
+    pslot[k] = c_valid.slot[c][threadIdx.x];
   }
   __syncthreads();
-  const int nph = pslot[27];
-  const double* opsL = ops + (int64_t)lt.d[li] * opsz;
-  d4 acc[RB];
+  const dv2* A = reinterpret_cast<const dv2*>(opsm + (int64_t)lt.d[li] * opsmsz) + l;
+  d4 acc[RBW][NCG];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) acc[rb] = d4{0.0, 0.0, 0.0, 0.0};
-  for (int k = w; k < nph; k += NW) {
-    const int i = pslot[k];
-    const int slot = c_valid.slot[c][i];
-    const int src = srcs[i][col];
-    dv2 b[KS / 2];   // source row entries 8 m + 2 kq + {0, 1}
-    if (src >= 0) {
-      const double* brow = mult + (int64_t)src * PD + 2 * kq;
+  for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
-      for (int m = 0; m < KS / 2; ++m) b[m] = *reinterpret_cast<const dv2*>(brow + 8 * m);
-    } else {
+    for (int g = 0; g < NCG; ++g) acc[rb][g] = d4{0.0, 0.0, 0.0, 0.0};
+  // this wave's slots: pslot[sg + SG j], j < nmine
+  const int nmine = sg < nph ? (nph - 1 - sg) / SG + 1 : 0;
+  if (nmine > 0) {
+    const dv2* pa;
+    const dv2* pb[NCG];
+    auto point = [&](int k, const dv2*& qa, const dv2* (&qb)[NCG]) {
+      const int slot = __builtin_amdgcn_readfirstlane(pslot[k]);
+      const int i = __builtin_amdgcn_readfirstlane(pidx[k]);
+      qa = A + ((int64_t)slot * KP * RB + rg * RBW) * 64;
 #pragma unroll
-      for (int m = 0; m < KS / 2; ++m) b[m] = dv2{0.0, 0.0};
+      for (int g = 0; g < NCG; ++g) {
+        const int src = srcs[i][g * 16 + col];
+        qb[g] = reinterpret_cast<const dv2*>(
+            (src >= 0 ? mult + (int64_t)src * PD : c_zero_row) + 2 * kq);
+      }
+    };
+    // multipole entries of step pair m; ODD: the last step's k = 8 m + kq
+    auto loadb = [&](const dv2* q, int m) -> dv2 {
+      if (ODD && m == KP - 1)
+        return dv2{*(reinterpret_cast<const double*>(q + 4 * m) - kq), 0.0};
+      return q[4 * m];
+    };
+    dv2 a[D][RBW], b[D][NCG];
+    point(sg, pa, pb);
+#pragma unroll
+    for (int m = 0; m < D; ++m) {
+#pragma unroll
+      for (int rb = 0; rb < RBW; ++rb) a[m][rb] = pa[(m * RB + rb) * 64];
+#pragma unroll
+      for (int g = 0; g < NCG; ++g) b[m][g] = loadb(pb[g], m);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    const double* arow =
-        opsL + (int64_t)(OP_M2L + slot) * PD * PD + (int64_t)col * PD + 2 * kq;
+    for (int jj = 0; jj < nmine; ++jj) {
+      // the next slot of this wave (the current one again after the last)
+      const dv2* pan;
+      const dv2* pbn[NCG];
+      point(jj + 1 < nmine ? sg + SG * (jj + 1) : sg + SG * jj, pan, pbn);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      dv2 a[KS / 2];
+      for (int m = 0; m < KP; ++m) {
+        const int r = m % D;
 #pragma unroll
-      for (int m = 0; m < KS / 2; ++m)
-        a[m] = *reinterpret_cast<const dv2*>(arow + (int64_t)rb * 16 * PD + 8 * m);
+        for (int h = 0; h < (ODD && m == KP - 1 ? 1 : 2); ++h)
 #pragma unroll
-      for (int m = 0; m < KS / 2; ++m) {
-        acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m].x, b[m].x, acc[rb], 0, 0, 0);
-        acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[m].y, b[m].y, acc[rb], 0, 0, 0);
+          for (int rb = 0; rb < RBW; ++rb)
+#pragma unroll
+            for (int g = 0; g < NCG; ++g)
+              acc[rb][g] =
+                  __builtin_amdgcn_mfma_f64_16x16x4f64(a[r][rb][h], b[r][g][h], acc[rb][g], 0, 0, 0);
+        // reload the pair just used with the one D further on
+        const int mn = m + D < KP ? m + D : m + D - KP;
+        const dv2* qa = m + D < KP ? pa : pan;
+#pragma unroll
+        for (int rb = 0; rb < RBW; ++rb) a[r][rb] = qa[(mn * RB + rb) * 64];
+#pragma unroll
+        for (int g = 0; g < NCG; ++g) b[r][g] = loadb(m + D < KP ? pb[g] : pbn[g], mn);
+        // in program order: the scheduler would otherwise move each load
+        // down to its use
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      pa = pan;
+#pragma unroll
+      for (int g = 0; g < NCG; ++g) pb[g] = pbn[g];
+      // keeps the next slot's loads ahead of the loop's back edge
+      __asm__ volatile("" ::: "memory");
+    }
+  }
+  // the wave groups' sums in a fixed order: group 0 adds the others' and
+  // stores, one column group at a time
+#pragma unroll
+  for (int g = 0; g < NCG; ++g) {
+    if (g > 0) __syncthreads();
+    if (sg > 0) {
+#pragma unroll
+      for (int rb = 0; rb < RBW; ++rb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) red[sg - 1][16 * rb + 4 * v + kq][col] = acc[rb][g][v];
+    }
+    __syncthreads();
+    if (sg == 0) {
+      const int cc = g * 16 + col;
+      const int node = box(cc);
+      if (live(cc, node)) {
+        double* rowp = ple + (int64_t)node * PD;
+#pragma unroll
+        for (int rb = 0; rb < RBW; ++rb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int row = 16 * rb + 4 * v + kq;
+            double sum = acc[rb][g][v];
+#pragma unroll
+            for (int s = 0; s < SG - 1; ++s) sum += red[s][row][col];
+            rowp[16 * rg * RBW + row] = sum;
+          }
+        if (PE < PD && rg == 0)
+          for (int row = PE + kq; row < PD; row += 4) rowp[row] = 0.0;
       }
     }
   }
-  if (w > 0) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) red[w - 1][16 * rb + 4 * v + kq][col] = acc[rb][v];
-  }
-  __syncthreads();
-  if (w == 0 && active) {
-    double* rowp = ple + (int64_t)g * PD;
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        double sum = acc[rb][v];
-#pragma unroll
-        for (int ww = 0; ww < NW - 1; ++ww) sum += red[ww][16 * rb + 4 * v + kq][col];
-        rowp[16 * rb + 4 * v + kq] = sum;
-      }
-  }
+}
+
+// Operator copy of k_m2l_f64 for one level: dv2 entry
+// ((slot KP + m) RB + rb) 64 + lane holds M[16 rb + lane % 16][8 m + 2 (lane / 16) + {0, 1}],
+// or, when the last pair is one step (odd), column 8 m + lane / 16 and 0 for m = KP - 1.
+__global__ __launch_bounds__(256) void k_m2l_pack(const double* __restrict__ ops, int PD, int PE,
+                                                  bool odd, dv2* __restrict__ out) {
+  const int RB = PE / 16, KP = PE / 8;
+  const int n = kNumM2L * KP * RB * 64;
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  const int lane = e & 63, rb = (e >> 6) % RB, m = (e >> 6) / RB % KP, slot = (e >> 6) / RB / KP;
+  const double* M = ops + (int64_t)(OP_M2L + slot) * PD * PD;
+  const double* row = M + (16 * rb + (lane & 15)) * PD + 8 * m;
+  out[e] = odd && m == KP - 1 ? dv2{row[lane >> 4], 0.0}
+                              : *reinterpret_cast<const dv2*>(row + 2 * (lane >> 4));
 }
 
 // ---------------------------------------------------------------------------
@@ -3051,6 +3152,53 @@ static bool m2l_in_fp32(const Plan& P) {
   return P.precision != PREC_FP64 && !P.cheb && !(P.kernel_id == KER_STOKES && P.have_dip);
 }
 
+// The dense FP64 M2L of the levels in lt.
+static int m2l_pe(int p) { return (int)ceil_div(p, 16) * 16; }
+static bool m2l_odd(int p) { return (p - 1) % 8 < 4; }
+static int64_t opsm_per_level(int p) { return (int64_t)kNumM2L * m2l_pe(p) * m2l_pe(p); }
+
+template <int PD, int PE, int NCG, int RBW>
+static void m2l_f64_run(Plan& P, LevelTable& lt, hipStream_t s) {
+  typedef M2LShape<PE, NCG, RBW> Sh;
+  const Tree& t = P.tree;
+  int nb = 0;
+  for (int li = 0; li < lt.nlev; ++li) {
+    lt.boff[li] = nb;
+    nb += 4 * (int)ceil_div(lt.ngroups[li], Sh::C);
+  }
+  lt.boff[lt.nlev] = nb;
+  auto kern = m2l_odd(P.p) ? k_m2l_f64<PD, PE, NCG, RBW, true> : k_m2l_f64<PD, PE, NCG, RBW, false>;
+  hipLaunchKernelGGL(kern, dim3(nb * Sh::RG, P.nd), dim3(64 * kM2LF64Waves), 0, s, lt,
+                     t.flags.as<int>(), t.m2l.as<int>(), P.mult.as<double>(),
+                     P.opsm.as<double>(), opsm_per_level(P.p), P.ple.as<double>(), t.n_rows + 1,
+                     t.n_nodes + 1);
+  FMM_LAUNCH_CHECK();
+}
+// Fewer than two 16-box tiles per CU: two blocks share a tile's rows, since a
+// CU then waits for its blocks' operands (27 blocks of 32 KB each) rather
+// than for its matrix cores (30K points, p 60: 20.7 -> 14.8 us; at 1.3 tiles
+// per CU equal).  Complete trees of at least four tiles per CU take two
+// column groups per block, which halves the operator traffic (1M points
+// 107 -> 98 us); adaptive trees do not, as the union of 32 boxes' slots there
+// multiplies more absent partners than it saves loads (100K points on a
+// curve 69 -> 93 us).
+template <int PD, int PE>
+static void m2l_f64_shape(Plan& P, LevelTable& lt, hipStream_t s) {
+  constexpr int RB = PE / 16, RH = RB == 4 ? 2 : 1;
+  int64_t tiles = 0;   // of 16 boxes
+  for (int li = 0; li < lt.nlev; ++li) tiles += 4 * ceil_div(lt.ngroups[li], 16);
+  tiles *= P.nd;
+  if (tiles < 2 * kNumCUs && RH < RB) m2l_f64_run<PD, PE, 1, RH>(P, lt, s);
+  else if (lt.perm || tiles < 4 * kNumCUs) m2l_f64_run<PD, PE, 1, RB>(P, lt, s);
+  else m2l_f64_run<PD, PE, 2, RB>(P, lt, s);
+}
+static void m2l_f64_launch(Plan& P, LevelTable& lt, hipStream_t s) {
+  if (P.p <= 16) m2l_f64_shape<32, 16>(P, lt, s);
+  else if (P.p <= 32) m2l_f64_shape<32, 32>(P, lt, s);
+  else if (P.p <= 48) m2l_f64_shape<64, 48>(P, lt, s);
+  else m2l_f64_shape<64, 64>(P, lt, s);
+}
+
 static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t s) {
   const Tree& t = P.tree;
   const int PD = P.PD;
@@ -3097,22 +3245,11 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
     FMM_LAUNCH_CHECK();
     return;
   }
-  if (P.m2l_mode == FMM2D_M2L_DENSE && PD <= kM2LWavesF64MaxPD) {
-    LevelTable lw = lt;
-    int nbw = 0;
-    for (int li = 0; li < lw.nlev; ++li) {
-      lw.boff[li] = nbw;
-      nbw += 4 * (int)ceil_div(lw.ngroups[li], kM2LWCols);
-    }
-    lw.boff[lw.nlev] = nbw;
-    lw.split = 1;
-    hipLaunchKernelGGL(k_m2l_waves_f64<32>, dim3(nbw, nd), dim3(64 * kM2LWWaves), 0, s, lw,
-                       t.flags.as<int>(),
-                       t.m2l.as<int>(), P.mult.as<double>(), P.ops.as<double>(), opsz,
-                       P.ple.as<double>(), rstride, nstride);
-    FMM_LAUNCH_CHECK();
+  if (P.m2l_mode == FMM2D_M2L_DENSE) {
+    m2l_f64_launch(P, lt, s);
     return;
   }
+  // compressed form
   // fewer than 3 tiles per CU: split the tiles' phases over several blocks
   lt.split = (int64_t)nb * nd < 3 * kNumCUs ? kM2LSplitF64 : 1;
   if (lt.split > 1) {
@@ -3124,7 +3261,7 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
   auto kern = PD == 32 ? k_m2l_all<32, RS> : k_m2l_all<64, RS>;
   hipLaunchKernelGGL(kern, dim3(nb, nd), dim3(kM2LThreads * RS), 0, s, lt, t.flags.as<int>(),
                      t.m2l.as<int>(), P.mult.as<double>(), P.ops.as<double>(), opsz,
-                     P.ple.as<double>(), rstride, nstride, P.m2l_mode == FMM2D_M2L_SVD ? 1 : 0);
+                     P.ple.as<double>(), rstride, nstride);
   FMM_LAUNCH_CHECK();
 }
 
@@ -3783,6 +3920,17 @@ int fmm2d_set_operators(void* plan, int level, const double* dev_ops, int64_t n,
   }
   FMM_HIP(hipMemcpyAsync(P->ops.as<double>() + level * opsz, dev_ops, opsz * sizeof(double),
                          hipMemcpyDeviceToDevice, s));
+  // the dense FP64 M2L's copy in operand order (scalar KIFMM plans of the
+  // mixed forms always run the FP32 M2L)
+  if (P->precision == fmm::PREC_FP64 || P->cheb || P->kernel_id == fmm::KER_STOKES) {
+    const int64_t msz = fmm::opsm_per_level(P->p);
+    P->opsm.ensure(fmm::kMaxLevels * msz * sizeof(double));
+    hipLaunchKernelGGL(fmm::k_m2l_pack, dim3(fmm::grid256(msz / 2)), dim3(256), 0, s,
+                       P->ops.as<double>() + level * opsz, P->PD, fmm::m2l_pe(P->p),
+                       fmm::m2l_odd(P->p),
+                       reinterpret_cast<fmm::dv2*>(P->opsm.as<double>() + level * msz));
+    FMM_LAUNCH_CHECK();
+  }
   P->ops_set[level] = 1;
   ABI_END
 }
