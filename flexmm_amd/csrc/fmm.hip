@@ -699,7 +699,15 @@ struct LevelTable {
   // when few tiles would leave CUs idle.  Two addends onto 0 give the same sum
   // in either order; more parts make the sum's rounding depend on the order.
   int split;
+  // tiles per XCD and turn (xcd_block)
+  int xchunk;
 };
+// Tiles of a complete tree cost the same and keep contiguous eighths (0).  On
+// adaptive trees the column order sorts a chunk's tiles by their slots, so
+// that eighths leave XCDs idle: 4 tiles at a time took the FP64 M2L of 1M
+// clustered points from 218 to 194 us and the FP32 one of 2M Stokeslets from
+// 1094 to 896 us (1 to 16 within 3%, 64 no better than eighths).
+constexpr int kTileChunk = 4;
 
 struct ValidSlots {
   int n[4];
@@ -738,7 +746,7 @@ __device__ __forceinline__ M2LSetup m2l_setup(const LevelTable& lt, const int* _
                                               int (&srcs)[27][kM2LCols], int (&pslot)[28],
                                               unsigned long long& smask) {
   M2LSetup S;
-  const int bid0 = xcd_block(blockIdx.x, gridDim.x);
+  const int bid0 = xcd_block(blockIdx.x, gridDim.x, lt.xchunk);
   const int part = bid0 % lt.split;   // the parts of a tile are neighbours
   const int bid = bid0 / lt.split;
   int li = 0;
@@ -1040,7 +1048,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   __shared__ int pslotv[27];   // the M2L slot (offset) of each used slot index
   __shared__ unsigned int smask;
   __shared__ double red[NW - 1][PD][17];
-  const int bid = xcd_block(blockIdx.x, gridDim.x);
+  const int bid = xcd_block(blockIdx.x, gridDim.x, lt.xchunk);
   int li = 0;
   while (li + 1 < lt.nlev && bid >= lt.boff[li + 1]) ++li;
   const int lb = bid - lt.boff[li];
@@ -1294,7 +1302,7 @@ __global__ __launch_bounds__(64 * kM2LF64Waves) void k_m2l_f64(
   // density blockIdx.y
   mult += (int64_t)blockIdx.y * rstride * PD;
   ple += (int64_t)blockIdx.y * nstride * PD;
-  const int bid0 = xcd_block(blockIdx.x, gridDim.x);
+  const int bid0 = xcd_block(blockIdx.x, gridDim.x, lt.xchunk);
   const int rg = bid0 % RG, bid = bid0 / RG;   // the row groups of a tile are neighbours
   int li = 0;
   while (li + 1 < lt.nlev && bid >= lt.boff[li + 1]) ++li;
@@ -1980,25 +1988,33 @@ __global__ __launch_bounds__(256) void k_make_items(const int* __restrict__ ioff
 // ---------------------------------------------------------------------------
 // L2T + P2P, one wave per (box, chunk of 64 targets); lane = target.
 // Work items of the evaluation kernels, one per wave, kEvalWaves waves per
-// block (the block shares one copy of the log table): XCD x (blocks b with
-// b % 8 == x, dispatched in order) takes the x-th contiguous eighth of the
-// items.  Items are in leaf (Morton) order, so the colleague sources that
-// neighbouring leaves share stay in one XCD's L2.  The grid holds at least
-// ceil(ni / 8) waves per XCD; surplus waves exit.  (A grid capped at 8
-// blocks per CU, waves striding over several items, measured 8-20% slower.)
+// block (the block shares one copy of the log table).  Items are in node
+// order (by level, then Morton), so the colleague sources that neighbouring
+// leaves share should stay in one XCD's L2 (blocks b with b % 8 == x run on
+// XCD x, dispatched in order).  chunk = 0: XCD x takes the x-th contiguous
+// eighth of the items; chunk > 0: chunks of that many items go to the XCDs in
+// turn.  Surplus waves exit.  (A grid capped at 8 blocks per CU, waves
+// striding over several items, measured 8-20% slower.)
 constexpr int kEvalWaves = 4;
 constexpr int kStageSources = 64;   // LDS staging of few-target items: sources per wave and chunk
-struct ItemRange {
-  int first, last, step;
-};
-__device__ __forceinline__ ItemRange xcd_items(int ni) {
+// Items of a complete tree cost about the same, and eighths keep the most
+// sources in one L2 (mixed form, 1M points: 208 us, 229 with chunks of 32).
+// Elsewhere an item's cost follows its level and cluster, so eighths leave
+// whole XCDs idle: chunks of 32 took the Stokeslet on 2M clustered points
+// from 2092 to 1636 us, the order-8 black-box form from 325 to 185 us, 1M
+// points on a clustered tree from 117 to 88 us (16 to 256 within 5%).
+constexpr int kItemChunk = 32;
+// this wave's item, or -1
+__device__ __forceinline__ int xcd_item(int ni, int chunk) {
   const int x = blockIdx.x % kNumXcd;
-  ItemRange r;
-  r.first = (int)((int64_t)ni * x / kNumXcd) +
-            (int)(blockIdx.x / kNumXcd) * kEvalWaves + (int)(threadIdx.x >> 6);
-  r.last = min(r.first + 1, (int)((int64_t)ni * (x + 1) / kNumXcd));
-  r.step = 1;
-  return r;
+  const int j = (int)(blockIdx.x / kNumXcd) * kEvalWaves + (int)(threadIdx.x >> 6);
+  int first = (int)((int64_t)ni * x / kNumXcd) + j;
+  int last = (int)((int64_t)ni * (x + 1) / kNumXcd);
+  if (chunk > 0) {
+    first = (j / chunk * kNumXcd + x) * chunk + j % chunk;
+    last = ni;
+  }
+  return first < last ? first : -1;
 }
 
 template <int KER, int NOUT, bool CHECK>
@@ -2295,96 +2311,95 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
     const double2* __restrict__ dip,
     const double* __restrict__ le, const double* __restrict__ ops, int64_t opsz, int p,
     const double2* __restrict__ logtab, double kp, int64_t nt, double* __restrict__ out,
-    int scap) {
+    int scap, int chunk) {
   __shared__ double2 tab[kLogTableSize];
   extern __shared__ double4 stage_lds[];   // scap per wave when launched with it
   double4* stage = stage_lds + (int)(threadIdx.x >> 6) * scap;
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const ItemRange R = xcd_items(ni);
-  for (int ii = R.first; ii < R.last; ii += R.step) {
-    const int4 it = items[ii];
-    // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
-    const int g = __builtin_amdgcn_readfirstlane(it.x);
-    const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
-    if (t1 - t0 <= kFewTargets) {
-      eval_few<PD, KER, NOUT, CHECK, DIP, CHEB>(g, t0, t1 - t0, tperm, tsx, tsy, nlevel, xmid,
-                                                ymid, coll, crange, bot, top, src, dip, le, ops, opsz, p,
-                                                tab, kp, nt, out, stage, scap);
-      continue;
-    }
-    const int t = t0 + (int)(threadIdx.x & 63);
-    const bool act = t < t1;
-    Target<KER, NOUT, CHECK> T;
-    T.kp = helm_consts(kp);
-    T.x = tsx[act ? t : t0];   // idle lanes: as in eval_few
-    T.y = tsy[act ? t : t0];
-    // L2T: helpers.py:219-235 (the equivalent density sits on the large circle);
-    // Chebyshev expansions: bbfmm.py:185-199
-    const int d = nlevel[g];
-    double far = 0.0;
-    if (CHEB && d >= 2) {
-      far = cheb_l2t(T.x - xmid[g], T.y - ymid[g], ops[d * opsz + ops_off_circles(PD)],
-                     le + (int64_t)g * PD, p, 0, 1);
-    } else if (d >= 2) {
-      const double* lx = ops + d * opsz + (int64_t)OP_NBLK * PD * PD;
-      const double* ly = lx + PD;
-      Target<KER, NOUT, false> L;
-      L.kp = T.kp;
-      L.x = T.x - xmid[g];
-      L.y = T.y - ymid[g];
-      const double* lg = le + (int64_t)g * PD;
-      for (int k = 0; k < p; ++k) L.pair(lx[k], ly[k], lg[k], tab);
-      T.u = L.u;
-      T.gx = L.gx;
-      T.gy = L.gy;
-    }
-    // P2P over the leaf's colleagues: helpers.py:180-217.  Only colleague 4,
-    // the target's own box, can hold a source at the target (a point and its
-    // box are found by the same midpoint tests for sources and targets), so
-    // only its pairs test for coincidence.
-    const CollLanes CL = coll_lanes(g, coll, crange);
-    auto colleague = [&](auto guard, int b, int e) {
-      constexpr bool G = decltype(guard)::value;
-      int j = b;
-      if constexpr (DIP) {
-        for (; j < e; ++j) {
-          const double4 sj = src[j];
-          const double2 q = dip[j];
-          T.template pair_dip<G>(sj.x, sj.y, sj.z, q.x, q.y, tab);
-        }
-        return;
-      }
-      for (; j + 4 <= e; j += 4) {
-        double4 s4[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) s4[u] = src[j + u];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) T.template pair<G>(s4[u].x, s4[u].y, s4[u].z, tab);
-      }
+  const int ii = xcd_item(ni, chunk);
+  if (ii < 0) return;   // wave-uniform
+  const int4 it = items[ii];
+  // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
+  const int g = __builtin_amdgcn_readfirstlane(it.x);
+  const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
+  if (t1 - t0 <= kFewTargets) {
+    eval_few<PD, KER, NOUT, CHECK, DIP, CHEB>(g, t0, t1 - t0, tperm, tsx, tsy, nlevel, xmid,
+                                              ymid, coll, crange, bot, top, src, dip, le, ops, opsz, p,
+                                              tab, kp, nt, out, stage, scap);
+    return;
+  }
+  const int t = t0 + (int)(threadIdx.x & 63);
+  const bool act = t < t1;
+  Target<KER, NOUT, CHECK> T;
+  T.kp = helm_consts(kp);
+  T.x = tsx[act ? t : t0];   // idle lanes: as in eval_few
+  T.y = tsy[act ? t : t0];
+  // L2T: helpers.py:219-235 (the equivalent density sits on the large circle);
+  // Chebyshev expansions: bbfmm.py:185-199
+  const int d = nlevel[g];
+  double far = 0.0;
+  if (CHEB && d >= 2) {
+    far = cheb_l2t(T.x - xmid[g], T.y - ymid[g], ops[d * opsz + ops_off_circles(PD)],
+                   le + (int64_t)g * PD, p, 0, 1);
+  } else if (d >= 2) {
+    const double* lx = ops + d * opsz + (int64_t)OP_NBLK * PD * PD;
+    const double* ly = lx + PD;
+    Target<KER, NOUT, false> L;
+    L.kp = T.kp;
+    L.x = T.x - xmid[g];
+    L.y = T.y - ymid[g];
+    const double* lg = le + (int64_t)g * PD;
+    for (int k = 0; k < p; ++k) L.pair(lx[k], ly[k], lg[k], tab);
+    T.u = L.u;
+    T.gx = L.gx;
+    T.gy = L.gy;
+  }
+  // P2P over the leaf's colleagues: helpers.py:180-217.  Only colleague 4,
+  // the target's own box, can hold a source at the target (a point and its
+  // box are found by the same midpoint tests for sources and targets), so
+  // only its pairs test for coincidence.
+  const CollLanes CL = coll_lanes(g, coll, crange);
+  auto colleague = [&](auto guard, int b, int e) {
+    constexpr bool G = decltype(guard)::value;
+    int j = b;
+    if constexpr (DIP) {
       for (; j < e; ++j) {
         const double4 sj = src[j];
-        T.template pair<G>(sj.x, sj.y, sj.z, tab);
+        const double2 q = dip[j];
+        T.template pair_dip<G>(sj.x, sj.y, sj.z, q.x, q.y, tab);
       }
-    };
-    for (int qn = 0; qn < 9; ++qn) {
-      const int b = __builtin_amdgcn_readlane(CL.b, qn);
-      const int e = __builtin_amdgcn_readlane(CL.e, qn);
-      if (e <= b) continue;
-      if (qn == 4) colleague(std::true_type{}, b, e);
-      else colleague(std::false_type{}, b, e);
+      return;
     }
-    if (act) {
-      const int64_t o = tperm[t];
-      double u = DIP ? __builtin_fma(kInv2Pi, T.dip, T.u.result()) : T.u.result() + far;
-      // log(0): the reference's -log(0) = +inf; with a dipole also 0/0
-      if (!CHECK && T.zhit()) u = DIP ? __builtin_nan("") : __builtin_inf();
-      out[o] = u;
-      if (NOUT == 3) {
-        out[nt + o] = T.gscale() * T.gx;
-        out[2 * nt + o] = T.gscale() * T.gy;
-      }
+    for (; j + 4 <= e; j += 4) {
+      double4 s4[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s4[u] = src[j + u];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) T.template pair<G>(s4[u].x, s4[u].y, s4[u].z, tab);
+    }
+    for (; j < e; ++j) {
+      const double4 sj = src[j];
+      T.template pair<G>(sj.x, sj.y, sj.z, tab);
+    }
+  };
+  for (int qn = 0; qn < 9; ++qn) {
+    const int b = __builtin_amdgcn_readlane(CL.b, qn);
+    const int e = __builtin_amdgcn_readlane(CL.e, qn);
+    if (e <= b) continue;
+    if (qn == 4) colleague(std::true_type{}, b, e);
+    else colleague(std::false_type{}, b, e);
+  }
+  if (act) {
+    const int64_t o = tperm[t];
+    double u = DIP ? __builtin_fma(kInv2Pi, T.dip, T.u.result()) : T.u.result() + far;
+    // log(0): the reference's -log(0) = +inf; with a dipole also 0/0
+    if (!CHECK && T.zhit()) u = DIP ? __builtin_nan("") : __builtin_inf();
+    out[o] = u;
+    if (NOUT == 3) {
+      out[nt + o] = T.gscale() * T.gx;
+      out[2 * nt + o] = T.gscale() * T.gy;
     }
   }
 }
@@ -2548,124 +2563,123 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
     const double4* __restrict__ src, const f4* __restrict__ srcf,
     const double* __restrict__ tsum, LevelConsts lc, const double* __restrict__ le,
     const double* __restrict__ ops, int64_t opsz, int p, const double2* __restrict__ logtab,
-    double* __restrict__ out) {
+    double* __restrict__ out, int chunk) {
   __shared__ double2 tab[kLogTableSize];
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const ItemRange R = xcd_items(ni);
-  for (int ii = R.first; ii < R.last; ii += R.step) {
-    const int4 it = items[ii];
-    // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
-    const int g = __builtin_amdgcn_readfirstlane(it.x);
-    const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
-    if (t1 - t0 <= kFewTargets) {
-      eval_few_mixed<PD, CHECK, CHEB>(g, t0, t1 - t0, tperm, tsx, tsy, nlevel, flags, xmid,
-                                      ymid, coll, crange, bot, top, src, srcf, tsum, lc, le, ops, opsz,
-                                      p, tab, out);
-      continue;
-    }
-    const int t = t0 + (int)(threadIdx.x & 63);
-    const bool act = t < t1;
-    Target<KER_LAPLACE, 1, CHECK> T;
-    T.kp = HelmConsts{};
-    // idle lanes repeat the item's first target: they then take the same
-    // branches as a real lane (no near-pair path of their own)
-    T.x = tsx[act ? t : t0];
-    T.y = tsy[act ? t : t0];
-    const int d = nlevel[g];
-    double far = 0.0;   // Chebyshev L2T
-    if (CHEB && d >= 2) {
-      far = cheb_l2t(T.x - xmid[g], T.y - ymid[g], ops[d * opsz + ops_off_circles(PD)],
-                     le + (int64_t)g * PD, p, 0, 1);
-    } else if (d >= 2) {   // L2T in FP64 (the local densities carry large cancelling modes)
-      const double* lx = ops + d * opsz + ops_off_circles(PD);
-      const double* ly = lx + PD;
-      Target<KER_LAPLACE, 1, false> L;
-      L.kp = HelmConsts{};
-      L.x = T.x - xmid[g];
-      L.y = T.y - ymid[g];
-      const double* lg = le + (int64_t)g * PD;
-      for (int k = 0; k < p; ++k) L.pair(lx[k], ly[k], lg[k], tab);
-      T.u = L.u;
-    }
-    const double iw = lc.invw[d];
-    const double lw2 = lc.logw2[d];
-    double u32 = 0.0;      // ln2-scaled part from the FP32 near field
-    const CollLanes CL = coll_lanes(g, coll, crange);
-    for (int qn = 0; qn < 9; ++qn) {
-      const int c = __builtin_amdgcn_readlane(CL.c, qn);
-      const int b = __builtin_amdgcn_readlane(CL.b, qn);
-      const int e = __builtin_amdgcn_readlane(CL.e, qn);
-      if (e <= b) continue;
-      if (flags[c] & NF_LEAF) {
-        const float xr = (float)((T.x - xmid[c]) * iw);
-        const float yr = (float)((T.y - ymid[c]) * iw);
-        float acc = 0.f;
-        double excl = 0.0;   // charges of the pairs taken in FP64
-        // pairs closer than w/64 (and coincident ones) go to FP64: the rounding
-        // of the FP32 relative coordinates costs ~1e-7 w / d in log d
-        auto near64 = [&](int jj) {
-          const double4 sd = src[jj];
-          excl += sd.z;
-          T.pair(sd.x, sd.y, sd.z, tab);
-        };
-        int j = b;
-        for (; j + 4 <= e; j += 4) {
-          f4 s4[4];
+  const int ii = xcd_item(ni, chunk);
+  if (ii < 0) return;   // wave-uniform
+  const int4 it = items[ii];
+  // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
+  const int g = __builtin_amdgcn_readfirstlane(it.x);
+  const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
+  if (t1 - t0 <= kFewTargets) {
+    eval_few_mixed<PD, CHECK, CHEB>(g, t0, t1 - t0, tperm, tsx, tsy, nlevel, flags, xmid,
+                                    ymid, coll, crange, bot, top, src, srcf, tsum, lc, le, ops, opsz,
+                                    p, tab, out);
+    return;
+  }
+  const int t = t0 + (int)(threadIdx.x & 63);
+  const bool act = t < t1;
+  Target<KER_LAPLACE, 1, CHECK> T;
+  T.kp = HelmConsts{};
+  // idle lanes repeat the item's first target: they then take the same
+  // branches as a real lane (no near-pair path of their own)
+  T.x = tsx[act ? t : t0];
+  T.y = tsy[act ? t : t0];
+  const int d = nlevel[g];
+  double far = 0.0;   // Chebyshev L2T
+  if (CHEB && d >= 2) {
+    far = cheb_l2t(T.x - xmid[g], T.y - ymid[g], ops[d * opsz + ops_off_circles(PD)],
+                   le + (int64_t)g * PD, p, 0, 1);
+  } else if (d >= 2) {   // L2T in FP64 (the local densities carry large cancelling modes)
+    const double* lx = ops + d * opsz + ops_off_circles(PD);
+    const double* ly = lx + PD;
+    Target<KER_LAPLACE, 1, false> L;
+    L.kp = HelmConsts{};
+    L.x = T.x - xmid[g];
+    L.y = T.y - ymid[g];
+    const double* lg = le + (int64_t)g * PD;
+    for (int k = 0; k < p; ++k) L.pair(lx[k], ly[k], lg[k], tab);
+    T.u = L.u;
+  }
+  const double iw = lc.invw[d];
+  const double lw2 = lc.logw2[d];
+  double u32 = 0.0;      // ln2-scaled part from the FP32 near field
+  const CollLanes CL = coll_lanes(g, coll, crange);
+  for (int qn = 0; qn < 9; ++qn) {
+    const int c = __builtin_amdgcn_readlane(CL.c, qn);
+    const int b = __builtin_amdgcn_readlane(CL.b, qn);
+    const int e = __builtin_amdgcn_readlane(CL.e, qn);
+    if (e <= b) continue;
+    if (flags[c] & NF_LEAF) {
+      const float xr = (float)((T.x - xmid[c]) * iw);
+      const float yr = (float)((T.y - ymid[c]) * iw);
+      float acc = 0.f;
+      double excl = 0.0;   // charges of the pairs taken in FP64
+      // pairs closer than w/64 (and coincident ones) go to FP64: the rounding
+      // of the FP32 relative coordinates costs ~1e-7 w / d in log d
+      auto near64 = [&](int jj) {
+        const double4 sd = src[jj];
+        excl += sd.z;
+        T.pair(sd.x, sd.y, sd.z, tab);
+      };
+      int j = b;
+      for (; j + 4 <= e; j += 4) {
+        f4 s4[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) s4[u] = srcf[j + u];
-          float d2[4];
+        for (int u = 0; u < 4; ++u) s4[u] = srcf[j + u];
+        float d2[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float dx = xr - s4[u].x, dy = yr - s4[u].y;
+          d2[u] = __builtin_fmaf(dy, dy, dx * dx);
+        }
+        const float dm = fminf(fminf(d2[0], d2[1]), fminf(d2[2], d2[3]));
+        if (__builtin_expect(__ballot(dm < kNearF32) == 0, 1)) {
+          // no near pair in the wave's four sources: no selects
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            acc = __builtin_fmaf(s4[u].z, __builtin_amdgcn_logf(d2[u]), acc);
+        } else {
+          bool nr[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const float dx = xr - s4[u].x, dy = yr - s4[u].y;
-            d2[u] = __builtin_fmaf(dy, dy, dx * dx);
+            nr[u] = d2[u] < kNearF32;
+            const float lg2 = __builtin_amdgcn_logf(nr[u] ? 1.0f : d2[u]);
+            acc = __builtin_fmaf(nr[u] ? 0.f : s4[u].z, lg2, acc);
           }
-          const float dm = fminf(fminf(d2[0], d2[1]), fminf(d2[2], d2[3]));
-          if (__builtin_expect(__ballot(dm < kNearF32) == 0, 1)) {
-            // no near pair in the wave's four sources: no selects
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-              acc = __builtin_fmaf(s4[u].z, __builtin_amdgcn_logf(d2[u]), acc);
-          } else {
-            bool nr[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              nr[u] = d2[u] < kNearF32;
-              const float lg2 = __builtin_amdgcn_logf(nr[u] ? 1.0f : d2[u]);
-              acc = __builtin_fmaf(nr[u] ? 0.f : s4[u].z, lg2, acc);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-              if (nr[u]) near64(j + u);
-          }
-        }
-        for (; j < e; ++j) {
-          const f4 sj = srcf[j];
-          const float dx = xr - sj.x, dy = yr - sj.y;
-          const float d2 = __builtin_fmaf(dy, dy, dx * dx);
-          const bool nr = d2 < kNearF32;
-          const float lg2 = __builtin_amdgcn_logf(nr ? 1.0f : d2);
-          acc = __builtin_fmaf(nr ? 0.f : sj.z, lg2, acc);
-          if (nr) near64(j);
-        }
-        u32 += (double)acc;
-        T.u.a.at = __builtin_fma(lw2, tsum[c] - excl, T.u.a.at);
-      } else {
-        // colleague with children (adaptive trees): its sources are not stored
-        // relative to it, so this range stays FP64
-        int j = b;
-        for (; j < e; ++j) {
-          const double4 sj = src[j];
-          T.pair(sj.x, sj.y, sj.z, tab);
+          for (int u = 0; u < 4; ++u)
+            if (nr[u]) near64(j + u);
         }
       }
+      for (; j < e; ++j) {
+        const f4 sj = srcf[j];
+        const float dx = xr - sj.x, dy = yr - sj.y;
+        const float d2 = __builtin_fmaf(dy, dy, dx * dx);
+        const bool nr = d2 < kNearF32;
+        const float lg2 = __builtin_amdgcn_logf(nr ? 1.0f : d2);
+        acc = __builtin_fmaf(nr ? 0.f : sj.z, lg2, acc);
+        if (nr) near64(j);
+      }
+      u32 += (double)acc;
+      T.u.a.at = __builtin_fma(lw2, tsum[c] - excl, T.u.a.at);
+    } else {
+      // colleague with children (adaptive trees): its sources are not stored
+      // relative to it, so this range stays FP64
+      int j = b;
+      for (; j < e; ++j) {
+        const double4 sj = src[j];
+        T.pair(sj.x, sj.y, sj.z, tab);
+      }
     }
-    if (act) {
-      double u = __builtin_fma(-kInv4Pi, __builtin_fma(u32, kLn2, T.u.a.value()), far);
-      if (!CHECK && T.zhit()) u = __builtin_inf();
-      out[tperm[t]] = u;
-    }
+  }
+  if (act) {
+    double u = __builtin_fma(-kInv4Pi, __builtin_fma(u32, kLn2, T.u.a.value()), far);
+    if (!CHECK && T.zhit()) u = __builtin_inf();
+    out[tperm[t]] = u;
   }
 }
 
@@ -2958,30 +2972,32 @@ void k_eval_stokes(
     const double4* __restrict__ sdip,
     const double* __restrict__ le, int64_t nstride, const double* __restrict__ ops, int64_t opsz,
     int p, const double2* __restrict__ logtab, double c0x, double c0y, int64_t nt,
-    double* __restrict__ out) {
+    double* __restrict__ out, int chunk) {
   __shared__ double2 tab[kLogTableSize];
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const ItemRange R = xcd_items(ni);
-  for (int ii = R.first; ii < R.last; ii += R.step) {
-    const int4 it = items[ii];
-    // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
-    const int g = __builtin_amdgcn_readfirstlane(it.x);
-    const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
-    if (t1 - t0 <= kFewTargets)
-      stokes_item<PD, CHECK, true, DIP>(g, t0, t1, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
-                                        bot, top, src, sdip, le, nstride, ops, opsz, p, tab, c0x,
-                                        c0y, nt, out);
-    else
-      stokes_item<PD, CHECK, false, DIP>(g, t0, t1, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
-                                         bot, top, src, sdip, le, nstride, ops, opsz, p, tab,
-                                         c0x, c0y, nt, out);
-  }
+  const int ii = xcd_item(ni, chunk);
+  if (ii < 0) return;   // wave-uniform
+  const int4 it = items[ii];
+  // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
+  const int g = __builtin_amdgcn_readfirstlane(it.x);
+  const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
+  if (t1 - t0 <= kFewTargets)
+    stokes_item<PD, CHECK, true, DIP>(g, t0, t1, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
+                                      bot, top, src, sdip, le, nstride, ops, opsz, p, tab, c0x,
+                                      c0y, nt, out);
+  else
+    stokes_item<PD, CHECK, false, DIP>(g, t0, t1, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
+                                       bot, top, src, sdip, le, nstride, ops, opsz, p, tab,
+                                       c0x, c0y, nt, out);
 }
 
-inline int eval_grid(int64_t icap) {
-  return (int)(ceil_div(ceil_div(icap, kNumXcd) + 1, kEvalWaves) * kNumXcd);
+// blocks for at most icap items in chunks of `chunk` (a multiple of kEvalWaves, or 0)
+inline int eval_grid(int64_t icap, int chunk) {
+  const int64_t per_xcd = chunk > 0 ? ceil_div(icap, (int64_t)kNumXcd * chunk) * chunk
+                                    : ceil_div(icap, kNumXcd) + 1;
+  return (int)(ceil_div(per_xcd, kEvalWaves) * kNumXcd);
 }
 
 // Selects the k_eval instance of (PD, kernel, outputs, self-exclusion).
@@ -3217,6 +3233,7 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
   }
   lt.boff[lt.nlev] = T.lt.boff[l1] - T.lt.boff[l0];
   lt.perm = T.adaptive ? P.m2lperm.as<int>() : nullptr;
+  lt.xchunk = T.adaptive ? kTileChunk : 0;
   int nb = lt.boff[lt.nlev];
   if (nb == 0) return;
   if (m2l_in_fp32(P)) {
@@ -3546,6 +3563,8 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   FMM_LAUNCH_CHECK();
   const int PD = P.PD;
   const int64_t opsz = ops_per_level(PD);
+  // few items: smaller chunks, so that every XCD gets some
+  const int chunk = t.complete ? 0 : icap < 32 * kNumXcd * kItemChunk ? kItemChunk / 4 : kItemChunk;
   if (stokes) {
     const bool dl = ev == EVAL_STOKES_DIPOLE;
     auto sk = dl ? (PD == 32 ? (check ? k_eval_stokes<32, true, true> : k_eval_stokes<32, false, true>)
@@ -3553,14 +3572,14 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
                  : (PD == 32 ? (check ? k_eval_stokes<32, true, false> : k_eval_stokes<32, false, false>)
                              : (check ? k_eval_stokes<64, true, false> : k_eval_stokes<64, false, false>));
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
-    hipLaunchKernelGGL(sk, dim3(eval_grid(icap)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
+    hipLaunchKernelGGL(sk, dim3(eval_grid(icap, chunk)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
                        t.evalnode.as<int>(), w.toff, w.tperm,
                        w.tsx, w.tsy, t.nlevel.as<int>(),
                        t.xmid.as<double>(), t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(),
                        t.bot.as<int>(), t.top.as<int>(), P.src.as<double4>(),
                        dl ? P.sdip.as<double4>() : nullptr, P.le.as<double>(),
                        t.n_nodes + 1, P.ops.as<double>(), opsz, P.p, P.logtab.as<double2>(),
-                       t.xmin + 0.5 * t.w0, t.ymin + 0.5 * t.w0, nt, out);
+                       t.xmin + 0.5 * t.w0, t.ymin + 0.5 * t.w0, nt, out, chunk);
     FMM_LAUNCH_CHECK();
     P.mark(FMM2D_PHASE_EVAL_KERNEL, true, s);
     return;
@@ -3582,14 +3601,14 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
                      : (check ? (PD == 32 ? k_eval_mixed<32, true, false> : k_eval_mixed<64, true, false>)
                               : (PD == 32 ? k_eval_mixed<32, false, false> : k_eval_mixed<64, false, false>));
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
-    hipLaunchKernelGGL(mk, dim3(eval_grid(icap)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
+    hipLaunchKernelGGL(mk, dim3(eval_grid(icap, chunk)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
                        t.evalnode.as<int>(), w.toff, w.tperm,
                        w.tsx, w.tsy, t.nlevel.as<int>(),
                        t.flags.as<int>(), t.xmid.as<double>(), t.ymid.as<double>(),
                        t.coll.as<int>(), t.crange.as<int2>(), t.bot.as<int>(), t.top.as<int>(), P.src.as<double4>(),
                        P.srcf.as<f4>(), P.tsum.as<double>(), lc, P.le.as<double>(),
                        P.ops.as<double>(), opsz, P.cheb ? P.cheb : P.p, P.logtab.as<double2>(),
-                       out);
+                       out, chunk);
     FMM_LAUNCH_CHECK();
     P.mark(FMM2D_PHASE_EVAL_KERNEL, true, s);
     return;
@@ -3603,13 +3622,13 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   // full-wave items occupancy)
   const int scap = (ev != EVAL_DIPOLE && few_targets) ? kStageSources : 0;
   const size_t dyn = (size_t)scap * kEvalWaves * sizeof(double4);
-  hipLaunchKernelGGL(kern, dim3(eval_grid(icap)), dim3(64 * kEvalWaves), dyn, s, w.items, w.ntot,
+  hipLaunchKernelGGL(kern, dim3(eval_grid(icap, chunk)), dim3(64 * kEvalWaves), dyn, s, w.items, w.ntot,
                      t.evalnode.as<int>(), w.toff, w.tperm, w.tsx,
                      w.tsy, t.nlevel.as<int>(), t.xmid.as<double>(),
                      t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(), t.bot.as<int>(), t.top.as<int>(),
                      P.src.as<double4>(), ev == EVAL_DIPOLE ? P.dip.as<double2>() : nullptr,
                      P.le.as<double>(), P.ops.as<double>(), opsz, P.cheb ? P.cheb : P.p,
-                     P.logtab.as<double2>(), P.kparam, nt, out, scap);
+                     P.logtab.as<double2>(), P.kparam, nt, out, scap, chunk);
   FMM_LAUNCH_CHECK();
   P.mark(FMM2D_PHASE_EVAL_KERNEL, true, s);
 }
