@@ -2004,10 +2004,22 @@ constexpr int kStageSources = 64;   // LDS staging of few-target items: sources 
 // from 2092 to 1636 us, the order-8 black-box form from 325 to 185 us, 1M
 // points on a clustered tree from 117 to 88 us (16 to 256 within 5%).
 constexpr int kItemChunk = 32;
-// this wave's item, or -1
-__device__ __forceinline__ int xcd_item(int ni, int chunk) {
+// Up to 16 items per SIMD, the kEvalWaves waves of a block share an item: each
+// takes a quarter of the L2T terms and of every colleague's sources, and the
+// sums are added in wave order through LDS.  One wave per item leaves such a
+// launch bound by its load and table latencies (50K points at Ncutoff 500, one
+// item per SIMD: 180 -> 81 us; 2,003 points 27 -> 11; dipoles on 100K points
+// of a curve, 12 items per SIMD, 134 -> 60; Stokeslets and stresslets on 300K
+// points, 15 per SIMD, 456 -> 382).  Past that (47 per SIMD: 84 -> 137 us), or
+// where most boxes hold few targets or none (a box per 0.5 targets: 15 -> 42
+// us), a block's start-up per item costs more than it hides.  FP32 near
+// fields keep one wave per item (their FP32 runs stay whole).
+constexpr int64_t kSplitItems = 16 * 4 * kNumCUs;
+constexpr int64_t kSplitTargets = 4;   // targets per evaluation box at least
+// this wave's item, or -1; ns waves share an item
+__device__ __forceinline__ int xcd_item(int ni, int chunk, int ns) {
   const int x = blockIdx.x % kNumXcd;
-  const int j = (int)(blockIdx.x / kNumXcd) * kEvalWaves + (int)(threadIdx.x >> 6);
+  const int j = ((int)(blockIdx.x / kNumXcd) * kEvalWaves + (int)(threadIdx.x >> 6)) / ns;
   int first = (int)((int64_t)ni * x / kNumXcd) + j;
   int last = (int)((int64_t)ni * (x + 1) / kNumXcd);
   if (chunk > 0) {
@@ -2172,17 +2184,65 @@ __device__ __forceinline__ uint32_t slot_min(uint32_t v, int lg) {
   return v;
 }
 
-template <int PD, int KER, int NOUT, bool CHECK, bool DIP, bool CHEB>
+// Sums of the NS waves that share an item, in wave order; valid in wave 0.
+template <int NS, int NV>
+__device__ __forceinline__ void item_sum(double (&v)[NV], int part) {
+  static_assert(NS == 1 || NS == kEvalWaves, "an item's waves are one wave or the block");
+  if constexpr (NS > 1) {
+    __shared__ double red[NS - 1][NV][64];
+    const int lane = threadIdx.x & 63;
+    if (part > 0) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) red[part - 1][i][lane] = v[i];
+    }
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int w = 0; w < NS - 1; ++w) v[i] += red[w][i][lane];
+    }
+  }
+}
+template <int NS>
+__device__ __forceinline__ bool item_any(bool hit, int part) {
+  if constexpr (NS > 1) {
+    __shared__ unsigned char any[NS][64];
+    const int lane = threadIdx.x & 63;
+    any[part][lane] = hit;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NS; ++w) hit |= any[w][lane] != 0;
+  }
+  return hit;
+}
+
+// The L2T terms k0, k0 + step, ... < p of one target: four terms' loads in
+// flight (lanes of different source groups read different terms), each with
+// weight 0 past the last.
+template <class F>
+__device__ __forceinline__ void l2t_terms(int k0, int step, int p, F term) {
+  for (int k = k0; k < p; k += 4 * step) {
+    int kk[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) kk[u] = min(k + u * step, p - 1);
+    term(kk, k + step < p, k + 2 * step < p, k + 3 * step < p);
+  }
+}
+
+template <int PD, int KER, int NOUT, bool CHECK, bool DIP, bool CHEB, int NS>
 __device__ __forceinline__ void eval_few(
-    int g, int t0, int na, const int* __restrict__ tperm, const double* __restrict__ tsx,
+    int g, int t0, int na, int part, const int* __restrict__ tperm, const double* __restrict__ tsx,
     const double* __restrict__ tsy, const int* __restrict__ nlevel,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
     const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
     const double4* __restrict__ src, const double2* __restrict__ dip,
     const double* __restrict__ le, const double* __restrict__ ops, int64_t opsz, int p,
     const double2* __restrict__ tab, double kp, int64_t nt, double* __restrict__ out,
-    double4* __restrict__ stage, int scap) {
+    double4* __restrict__ stage, double2* __restrict__ dstage, int scap) {
   const FewLanes F = few_lanes(na);
+  // source group among all NS waves' groups
+  const int sg = F.sg + part * F.ng, ng = NS * F.ng;
   const int t = t0 + F.slot;
   Target<KER, NOUT, CHECK> T;
   T.kp = helm_consts(kp);
@@ -2194,7 +2254,7 @@ __device__ __forceinline__ void eval_few(
   double far = 0.0;   // Chebyshev L2T
   if (CHEB && d >= 2) {
     far = cheb_l2t(T.x - xmid[g], T.y - ymid[g], ops[d * opsz + ops_off_circles(PD)],
-                   le + (int64_t)g * PD, p, F.sg, F.ng);
+                   le + (int64_t)g * PD, p, sg, ng);
   } else if (d >= 2) {
     Target<KER, NOUT, false> L;
     L.kp = T.kp;
@@ -2203,13 +2263,24 @@ __device__ __forceinline__ void eval_few(
     const double* lx = ops + d * opsz + (int64_t)OP_NBLK * PD * PD;
     const double* ly = lx + PD;
     const double* lg = le + (int64_t)g * PD;
-    for (int k = F.sg; k < p; k += F.ng) L.pair(lx[k], ly[k], lg[k], tab);
+    l2t_terms(sg, ng, p, [&](const int (&k)[4], bool h1, bool h2, bool h3) {
+      double cx[4], cy[4], cw[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        cx[u] = lx[k[u]];
+        cy[u] = ly[k[u]];
+        cw[u] = lg[k[u]];
+      }
+      const bool has[4] = {true, h1, h2, h3};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) L.pair(cx[u], cy[u], has[u] ? cw[u] : 0.0, tab);
+    });
     T.u = L.u;
     T.gx = L.gx;
     T.gy = L.gy;
   }
   const CollLanes CL = coll_lanes(g, coll, crange);
-  if (!DIP && scap > 0) {
+  if (scap > 0) {
     // The colleague sources, concatenated, pass through this wave's LDS area
     // scap at a time: every lane loads its share of a chunk at once (one
     // memory round trip per chunk instead of one per colleague), then the
@@ -2223,7 +2294,7 @@ __device__ __forceinline__ void eval_few(
       cp[q + 1] = cp[q] + (ce > cb[q] ? ce - cb[q] : 0);
     }
     const int lane = threadIdx.x & 63;
-    for (int base = 0; base < cp[9]; base += scap) {
+    for (int base = part * scap; base < cp[9]; base += NS * scap) {
       const int n = min(scap, cp[9] - base);
       for (int v = lane; v < n; v += 64) {
         const int vv = base + v;
@@ -2231,13 +2302,19 @@ __device__ __forceinline__ void eval_few(
 #pragma unroll
         for (int q = 1; q < 9; ++q) j = vv >= cp[q] ? vv - cp[q] + cb[q] : j;
         stage[v] = src[j];
+        if constexpr (DIP) dstage[v] = dip[j];
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       for (int v = F.sg; v < n; v += F.ng) {
         const double4 sj = stage[v];
-        T.pair(sj.x, sj.y, sj.z, tab);
+        if constexpr (DIP) {
+          const double2 q = dstage[v];
+          T.pair_dip(sj.x, sj.y, sj.z, q.x, q.y, tab);
+        } else {
+          T.pair(sj.x, sj.y, sj.z, tab);
+        }
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -2249,19 +2326,19 @@ __device__ __forceinline__ void eval_few(
   // midpoint tests for sources and targets)
   auto colleague = [&](auto guard, int b, int e) {
     constexpr bool G = decltype(guard)::value;
-    int j = b + F.sg;
+    int j = b + sg;
     if constexpr (!DIP) {
       // four sources per lane in flight: the loads are per lane here (lanes
       // of different source groups read different sources)
-      for (; j + 3 * F.ng < e; j += 4 * F.ng) {
+      for (; j + 3 * ng < e; j += 4 * ng) {
         double4 s4[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) s4[u] = src[j + u * F.ng];
+        for (int u = 0; u < 4; ++u) s4[u] = src[j + u * ng];
 #pragma unroll
         for (int u = 0; u < 4; ++u) T.template pair<G>(s4[u].x, s4[u].y, s4[u].z, tab);
       }
     }
-    for (; j < e; j += F.ng) {
+    for (; j < e; j += ng) {
       const double4 sj = src[j];
       if constexpr (DIP) {
         const double2 q = dip[j];
@@ -2271,35 +2348,36 @@ __device__ __forceinline__ void eval_few(
       }
     }
   };
-  for (int qn = 0; qn < 9 && (DIP || scap == 0); ++qn) {
+  for (int qn = 0; qn < 9 && scap == 0; ++qn) {
     const int b = __builtin_amdgcn_readlane(CL.b, qn);
     const int e = __builtin_amdgcn_readlane(CL.e, qn);
     if (e <= b) continue;
     if (qn == 4) colleague(std::true_type{}, b, e);
     else colleague(std::false_type{}, b, e);
   }
-  double u = slot_sum(DIP ? __builtin_fma(kInv2Pi, T.dip, T.u.result()) : T.u.result() + far,
-                      F.lg);
-  double gx = 0.0, gy = 0.0;
-  if (NOUT == 3) {
-    gx = slot_sum(T.gx, F.lg);
-    gy = slot_sum(T.gy, F.lg);
+  double sum[NOUT];
+  sum[0] = slot_sum(DIP ? __builtin_fma(kInv2Pi, T.dip, T.u.result()) : T.u.result() + far, F.lg);
+  if constexpr (NOUT == 3) {
+    sum[1] = slot_sum(T.gx, F.lg);
+    sum[2] = slot_sum(T.gy, F.lg);
   }
-  const bool zh = CHECK ? false : slot_min(T.dmin, F.lg) == 0u;
-  if (F.act && F.sg == 0) {
+  item_sum<NS>(sum, part);
+  const bool zh =
+      CHECK ? false : item_any<NS>(slot_min(T.dmin, F.lg) == 0u, part);
+  if (F.act && F.sg == 0 && part == 0) {
     const int64_t o = tperm[t];
-    if (zh) u = DIP ? __builtin_nan("") : __builtin_inf();
-    out[o] = u;
-    if (NOUT == 3) {
-      out[nt + o] = T.gscale() * gx;
-      out[2 * nt + o] = T.gscale() * gy;
+    if (zh) sum[0] = DIP ? __builtin_nan("") : __builtin_inf();
+    out[o] = sum[0];
+    if constexpr (NOUT == 3) {
+      out[nt + o] = T.gscale() * sum[1];
+      out[2 * nt + o] = T.gscale() * sum[2];
     }
   }
 }
 
 // The Helmholtz gradient instance is held to 3 waves per SIMD (168 VGPRs;
 // it needs 169 unconstrained, which leaves 2).
-template <int PD, int KER, int NOUT, bool CHECK, bool DIP, bool CHEB>
+template <int PD, int KER, int NOUT, bool CHECK, bool DIP, bool CHEB, int NS>
 __global__ __launch_bounds__(64 * kEvalWaves)
 __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) void k_eval(
     const int4* __restrict__ items, const int* __restrict__ nitems,
@@ -2315,19 +2393,23 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
   __shared__ double2 tab[kLogTableSize];
   extern __shared__ double4 stage_lds[];   // scap per wave when launched with it
   double4* stage = stage_lds + (int)(threadIdx.x >> 6) * scap;
+  double2* dstage = reinterpret_cast<double2*>(stage_lds + kEvalWaves * scap) +
+                    (int)(threadIdx.x >> 6) * scap;
+  // this wave's share of its item
+  const int part = NS > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % NS : 0;
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const int ii = xcd_item(ni, chunk);
-  if (ii < 0) return;   // wave-uniform
+  const int ii = xcd_item(ni, chunk, NS);
+  if (ii < 0) return;   // uniform among the waves of an item
   const int4 it = items[ii];
   // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
   const int g = __builtin_amdgcn_readfirstlane(it.x);
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets) {
-    eval_few<PD, KER, NOUT, CHECK, DIP, CHEB>(g, t0, t1 - t0, tperm, tsx, tsy, nlevel, xmid,
+    eval_few<PD, KER, NOUT, CHECK, DIP, CHEB, NS>(g, t0, t1 - t0, part, tperm, tsx, tsy, nlevel, xmid,
                                               ymid, coll, crange, bot, top, src, dip, le, ops, opsz, p,
-                                              tab, kp, nt, out, stage, scap);
+                                              tab, kp, nt, out, stage, dstage, scap);
     return;
   }
   const int t = t0 + (int)(threadIdx.x & 63);
@@ -2342,7 +2424,7 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
   double far = 0.0;
   if (CHEB && d >= 2) {
     far = cheb_l2t(T.x - xmid[g], T.y - ymid[g], ops[d * opsz + ops_off_circles(PD)],
-                   le + (int64_t)g * PD, p, 0, 1);
+                   le + (int64_t)g * PD, p, part, NS);
   } else if (d >= 2) {
     const double* lx = ops + d * opsz + (int64_t)OP_NBLK * PD * PD;
     const double* ly = lx + PD;
@@ -2351,7 +2433,8 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
     L.x = T.x - xmid[g];
     L.y = T.y - ymid[g];
     const double* lg = le + (int64_t)g * PD;
-    for (int k = 0; k < p; ++k) L.pair(lx[k], ly[k], lg[k], tab);
+    const int k1 = p * (part + 1) / NS;
+    for (int k = p * part / NS; k < k1; ++k) L.pair(lx[k], ly[k], lg[k], tab);
     T.u = L.u;
     T.gx = L.gx;
     T.gy = L.gy;
@@ -2385,21 +2468,33 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
     }
   };
   for (int qn = 0; qn < 9; ++qn) {
-    const int b = __builtin_amdgcn_readlane(CL.b, qn);
-    const int e = __builtin_amdgcn_readlane(CL.e, qn);
+    int b = __builtin_amdgcn_readlane(CL.b, qn);
+    int e = __builtin_amdgcn_readlane(CL.e, qn);
+    if constexpr (NS > 1) {   // this wave's share of the colleague's sources
+      const int n = max(e - b, 0);
+      e = b + n * (part + 1) / NS;
+      b = b + n * part / NS;
+    }
     if (e <= b) continue;
     if (qn == 4) colleague(std::true_type{}, b, e);
     else colleague(std::false_type{}, b, e);
   }
-  if (act) {
+  double sum[NOUT];
+  sum[0] = DIP ? __builtin_fma(kInv2Pi, T.dip, T.u.result()) : T.u.result() + far;
+  if constexpr (NOUT == 3) {
+    sum[1] = T.gx;
+    sum[2] = T.gy;
+  }
+  item_sum<NS>(sum, part);
+  const bool zh = CHECK ? false : item_any<NS>(T.zhit(), part);
+  if (act && part == 0) {
     const int64_t o = tperm[t];
-    double u = DIP ? __builtin_fma(kInv2Pi, T.dip, T.u.result()) : T.u.result() + far;
     // log(0): the reference's -log(0) = +inf; with a dipole also 0/0
-    if (!CHECK && T.zhit()) u = DIP ? __builtin_nan("") : __builtin_inf();
-    out[o] = u;
-    if (NOUT == 3) {
-      out[nt + o] = T.gscale() * T.gx;
-      out[2 * nt + o] = T.gscale() * T.gy;
+    if (zh) sum[0] = DIP ? __builtin_nan("") : __builtin_inf();
+    out[o] = sum[0];
+    if constexpr (NOUT == 3) {
+      out[nt + o] = T.gscale() * sum[1];
+      out[2 * nt + o] = T.gscale() * sum[2];
     }
   }
 }
@@ -2568,7 +2663,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const int ii = xcd_item(ni, chunk);
+  const int ii = xcd_item(ni, chunk, 1);
   if (ii < 0) return;   // wave-uniform
   const int4 it = items[ii];
   // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
@@ -2813,9 +2908,9 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m_stokes(int nup,
 // One item of k_eval_stokes: L2T of the three local fields + Stokeslet P2P,
 // outputs (u, v, p).  FEW selects the (target slot, source group) lane layout
 // of eval_few; otherwise lane = target and the source loop index is uniform.
-template <int PD, bool CHECK, bool FEW, bool DIP>
+template <int PD, bool CHECK, bool FEW, bool DIP, int NS>
 __device__ __forceinline__ void stokes_item(
-    int g, int t0, int t1, const int* __restrict__ tperm, const double* __restrict__ tsx,
+    int g, int t0, int t1, int part, const int* __restrict__ tperm, const double* __restrict__ tsx,
     const double* __restrict__ tsy, const int* __restrict__ nlevel,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
     const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
@@ -2833,6 +2928,8 @@ __device__ __forceinline__ void stokes_item(
     F.sg = 0;
     F.act = t0 + F.slot < t1;
   }
+  // source group among all NS waves' groups
+  const int sg = F.sg + part * F.ng, ng = NS * F.ng;
   const int t = t0 + F.slot;
   const bool act = F.act;
   const double x = act ? tsx[t] : 0.0;
@@ -2847,16 +2944,37 @@ __device__ __forceinline__ void stokes_item(
     // the three fields are the potentials -log(d^2)/(4 pi) of their local
     // equivalent densities: one log per equivalent point serves all three
     double l0 = 0.0, l1 = 0.0, l2 = 0.0;
-    for (int k = F.sg; k < p; k += F.ng) {
-      const double dx = xr - lx[k], dy = yr - ly[k];
+    auto term = [&](double cx, double cy, double a0, double a1, double a2) {
+      const double dx = xr - cx, dy = yr - cy;
       const double d2 = __builtin_fma(dy, dy, dx * dx);
-      const double a0 = a[k], a1 = a[nstride * PD + k], a2 = a[2 * nstride * PD + k];
       double e, lt;
       log_split(d2, tab, e, lt);
       const double lg = __builtin_fma(e, kLn2, lt);
       l0 = __builtin_fma(a0, lg, l0);
       l1 = __builtin_fma(a1, lg, l1);
       l2 = __builtin_fma(a2, lg, l2);
+    };
+    const double *a1 = a + nstride * PD, *a2 = a + 2 * nstride * PD;
+    if constexpr (FEW) {
+      l2t_terms(sg, ng, p, [&](const int (&k)[4], bool h1, bool h2, bool h3) {
+        double c[4][5];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          c[u][0] = lx[k[u]];
+          c[u][1] = ly[k[u]];
+          c[u][2] = a[k[u]];
+          c[u][3] = a1[k[u]];
+          c[u][4] = a2[k[u]];
+        }
+        const bool has[4] = {true, h1, h2, h3};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          term(c[u][0], c[u][1], has[u] ? c[u][2] : 0.0, has[u] ? c[u][3] : 0.0,
+               has[u] ? c[u][4] : 0.0);
+      });
+    } else {
+      const int k1 = p * (part + 1) / NS;
+      for (int k = p * part / NS; k < k1; ++k) term(lx[k], ly[k], a[k], a1[k], a2[k]);
     }
     const double Dx = -kInv4Pi * l0, Dy = -kInv4Pi * l1, D2 = -kInv4Pi * l2;
     const double X = x - c0x, Y = y - c0y;
@@ -2871,8 +2989,13 @@ __device__ __forceinline__ void stokes_item(
   double dmin = 1.0;
   const CollLanes CL = coll_lanes(g, coll, crange);
   for (int qn = 0; qn < 9; ++qn) {
-    const int b = __builtin_amdgcn_readlane(CL.b, qn);
-    const int e = __builtin_amdgcn_readlane(CL.e, qn);
+    int b = __builtin_amdgcn_readlane(CL.b, qn);
+    int e = __builtin_amdgcn_readlane(CL.e, qn);
+    if constexpr (!FEW && NS > 1) {   // this wave's share of the colleague's sources
+      const int n = max(e - b, 0);
+      e = b + n * (part + 1) / NS;
+      b = b + n * part / NS;
+    }
     if (e <= b) continue;
     // A coincident pair (d2 = 0, so dx = dy = 0) continues with d2 = 1: every
     // term with a factor dx or dy then vanishes exactly, the stresslet
@@ -2916,17 +3039,27 @@ __device__ __forceinline__ void stokes_item(
       }
     };
     auto colleague = [&](auto guard) {
-      int j = b + F.sg;
       if constexpr (FEW) {   // four per-lane loads in flight
-        for (; j + 3 * F.ng < e; j += 4 * F.ng) {
+        int j = b + sg;
+        for (; j + 3 * ng < e; j += 4 * ng) {
           double4 s4[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) s4[u] = src[j + u * F.ng];
+          for (int u = 0; u < 4; ++u) s4[u] = src[j + u * ng];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) pairS(guard, s4[u], j + u * F.ng);
+          for (int u = 0; u < 4; ++u) pairS(guard, s4[u], j + u * ng);
         }
+        for (; j < e; j += ng) pairS(guard, src[j], j);
+      } else {
+        int j = b;
+        for (; j + 2 <= e; j += 2) {
+          double4 s2[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) s2[u] = src[j + u];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) pairS(guard, s2[u], j + u);
+        }
+        for (; j < e; ++j) pairS(guard, src[j], j);
       }
-      for (; j < e; j += F.ng) pairS(guard, src[j], j);
     };
     if (qn == 4) colleague(std::true_type{});
     else colleague(std::false_type{});
@@ -2939,20 +3072,21 @@ __device__ __forceinline__ void stokes_item(
     v += kInv2Pi * dv;
     pr += 2.0 * kInv2Pi * dp;
   }
+  bool hit = !CHECK && dmin == 0.0;
+  double sum[3] = {u, v, pr};
   if constexpr (FEW) {
-    u = slot_sum(u, F.lg);
-    v = slot_sum(v, F.lg);
-    pr = slot_sum(pr, F.lg);
-    if (!CHECK)
-      for (int off = 1 << F.lg; off < 64; off <<= 1)
-        dmin = __builtin_fmin(dmin, __shfl_xor(dmin, off, 64));
+#pragma unroll
+    for (int i = 0; i < 3; ++i) sum[i] = slot_sum(sum[i], F.lg);
+    if constexpr (!CHECK) hit = slot_min(hit ? 0u : 1u, F.lg) == 0u;
   }
-  if (act && F.sg == 0) {
+  item_sum<NS>(sum, part);
+  if constexpr (!CHECK) hit = item_any<NS>(hit, part);
+  if (act && F.sg == 0 && part == 0) {
     const int64_t o = tperm[t];
-    if (!CHECK && dmin == 0.0) u = v = pr = __builtin_nan("");
-    out[o] = u;
-    out[nt + o] = v;
-    out[2 * nt + o] = pr;
+    if (hit) sum[0] = sum[1] = sum[2] = __builtin_nan("");
+    out[o] = sum[0];
+    out[nt + o] = sum[1];
+    out[2 * nt + o] = sum[2];
   }
 }
 
@@ -2960,7 +3094,7 @@ __device__ __forceinline__ void stokes_item(
 // The Stokeslet-only instance is held to 96 VGPRs (5 waves per SIMD instead of
 // 4, no spills; 2% faster on 2M clustered points); with stresslets the same
 // bound would spill, so that instance is left unconstrained.
-template <int PD, bool CHECK, bool DIP>
+template <int PD, bool CHECK, bool DIP, int NS>
 __global__ __launch_bounds__(64 * kEvalWaves) __attribute__((amdgpu_waves_per_eu(DIP ? 1 : 5)))
 void k_eval_stokes(
     const int4* __restrict__ items, const int* __restrict__ nitems,
@@ -2977,63 +3111,64 @@ void k_eval_stokes(
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const int ii = xcd_item(ni, chunk);
-  if (ii < 0) return;   // wave-uniform
+  const int ii = xcd_item(ni, chunk, NS);
+  if (ii < 0) return;   // uniform among the waves of an item
+  const int part = NS > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % NS : 0;
   const int4 it = items[ii];
   // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
   const int g = __builtin_amdgcn_readfirstlane(it.x);
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets)
-    stokes_item<PD, CHECK, true, DIP>(g, t0, t1, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
+    stokes_item<PD, CHECK, true, DIP, NS>(g, t0, t1, part, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
                                       bot, top, src, sdip, le, nstride, ops, opsz, p, tab, c0x,
                                       c0y, nt, out);
   else
-    stokes_item<PD, CHECK, false, DIP>(g, t0, t1, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
+    stokes_item<PD, CHECK, false, DIP, NS>(g, t0, t1, part, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
                                        bot, top, src, sdip, le, nstride, ops, opsz, p, tab,
                                        c0x, c0y, nt, out);
 }
 
-// blocks for at most icap items in chunks of `chunk` (a multiple of kEvalWaves, or 0)
-inline int eval_grid(int64_t icap, int chunk) {
-  const int64_t per_xcd = chunk > 0 ? ceil_div(icap, (int64_t)kNumXcd * chunk) * chunk
-                                    : ceil_div(icap, kNumXcd) + 1;
-  return (int)(ceil_div(per_xcd, kEvalWaves) * kNumXcd);
+typedef decltype(&k_eval_stokes<32, true, true, 1>) EvalStokesFn;
+template <int PD>
+EvalStokesFn eval_stokes_pd(bool dl, bool check, int ns) {
+  if (ns == 1)
+    return dl ? (check ? k_eval_stokes<PD, true, true, 1> : k_eval_stokes<PD, false, true, 1>)
+              : (check ? k_eval_stokes<PD, true, false, 1> : k_eval_stokes<PD, false, false, 1>);
+  constexpr int NS = kEvalWaves;
+  return dl ? (check ? k_eval_stokes<PD, true, true, NS> : k_eval_stokes<PD, false, true, NS>)
+            : (check ? k_eval_stokes<PD, true, false, NS> : k_eval_stokes<PD, false, false, NS>);
 }
 
-// Selects the k_eval instance of (PD, kernel, outputs, self-exclusion).
-typedef decltype(&k_eval<32, KER_LAPLACE, 1, false, false, false>) EvalKernelFn;
-template <int PD, int KER>
-EvalKernelFn eval_kernel_k(int nout, bool check) {
-  if (nout == 1)
-    return check ? k_eval<PD, KER, 1, true, false, false> : k_eval<PD, KER, 1, false, false, false>;
-  return check ? k_eval<PD, KER, 3, true, false, false> : k_eval<PD, KER, 3, false, false, false>;
+// blocks for at most icap items in chunks of `chunk` (a multiple of kEvalWaves,
+// or 0), ns waves per item
+inline int eval_grid(int64_t icap, int chunk, int ns) {
+  const int64_t per_xcd = chunk > 0 ? ceil_div(icap, (int64_t)kNumXcd * chunk) * chunk
+                                    : ceil_div(icap, kNumXcd) + 1;
+  return (int)(ceil_div(per_xcd * ns, kEvalWaves) * kNumXcd);
 }
-// Laplace single + double layer sources
-EvalKernelFn eval_kernel_dipole(int PD, bool check) {
-  if (PD == 32)
-    return check ? k_eval<32, KER_LAPLACE, 1, true, true, false>
-                 : k_eval<32, KER_LAPLACE, 1, false, true, false>;
-  return check ? k_eval<64, KER_LAPLACE, 1, true, true, false>
-               : k_eval<64, KER_LAPLACE, 1, false, true, false>;
+
+// Selects the k_eval instance of (PD, kernel, outputs, self-exclusion, waves per item).
+typedef decltype(&k_eval<32, KER_LAPLACE, 1, false, false, false, 1>) EvalKernelFn;
+template <int PD, int KER, int NOUT, bool DIP, bool CHEB>
+EvalKernelFn eval_kernel_of(bool check, int ns) {
+  if (ns == 1)
+    return check ? k_eval<PD, KER, NOUT, true, DIP, CHEB, 1>
+                 : k_eval<PD, KER, NOUT, false, DIP, CHEB, 1>;
+  return check ? k_eval<PD, KER, NOUT, true, DIP, CHEB, kEvalWaves>
+               : k_eval<PD, KER, NOUT, false, DIP, CHEB, kEvalWaves>;
 }
-// Chebyshev (black-box) expansions: potential only
 template <int PD>
-EvalKernelFn eval_kernel_cheb_pd(int ker, bool check) {
+EvalKernelFn eval_kernel_pd(int ker, int ev, bool cheb, bool check, int ns) {
+  if (cheb)   // Chebyshev (black-box) expansions: potential only
+    return ker == KER_LAPLACE ? eval_kernel_of<PD, KER_LAPLACE, 1, false, true>(check, ns)
+                              : eval_kernel_of<PD, KER_MODHELM, 1, false, true>(check, ns);
+  if (ev == EVAL_DIPOLE)   // Laplace single + double layer sources
+    return eval_kernel_of<PD, KER_LAPLACE, 1, true, false>(check, ns);
   if (ker == KER_LAPLACE)
-    return check ? k_eval<PD, KER_LAPLACE, 1, true, false, true>
-                 : k_eval<PD, KER_LAPLACE, 1, false, false, true>;
-  return check ? k_eval<PD, KER_MODHELM, 1, true, false, true>
-               : k_eval<PD, KER_MODHELM, 1, false, false, true>;
-}
-EvalKernelFn eval_kernel_cheb(int PD, int ker, bool check) {
-  return PD == 32 ? eval_kernel_cheb_pd<32>(ker, check) : eval_kernel_cheb_pd<64>(ker, check);
-}
-EvalKernelFn eval_kernel(int PD, int ker, int nout, bool check) {
-  if (ker == KER_LAPLACE)
-    return PD == 32 ? eval_kernel_k<32, KER_LAPLACE>(nout, check)
-                    : eval_kernel_k<64, KER_LAPLACE>(nout, check);
-  return PD == 32 ? eval_kernel_k<32, KER_MODHELM>(nout, check)
-                  : eval_kernel_k<64, KER_MODHELM>(nout, check);
+    return ev == EVAL_POT ? eval_kernel_of<PD, KER_LAPLACE, 1, false, false>(check, ns)
+                          : eval_kernel_of<PD, KER_LAPLACE, 3, false, false>(check, ns);
+  return ev == EVAL_POT ? eval_kernel_of<PD, KER_MODHELM, 1, false, false>(check, ns)
+                        : eval_kernel_of<PD, KER_MODHELM, 3, false, false>(check, ns);
 }
 
 // Algorithmic work counts (for the roofline accounting).
@@ -3565,14 +3700,12 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   const int64_t opsz = ops_per_level(PD);
   // few items: smaller chunks, so that every XCD gets some
   const int chunk = t.complete ? 0 : icap < 32 * kNumXcd * kItemChunk ? kItemChunk / 4 : kItemChunk;
+  const int ns = icap <= kSplitItems && nt >= kSplitTargets * ne ? kEvalWaves : 1;
   if (stokes) {
     const bool dl = ev == EVAL_STOKES_DIPOLE;
-    auto sk = dl ? (PD == 32 ? (check ? k_eval_stokes<32, true, true> : k_eval_stokes<32, false, true>)
-                             : (check ? k_eval_stokes<64, true, true> : k_eval_stokes<64, false, true>))
-                 : (PD == 32 ? (check ? k_eval_stokes<32, true, false> : k_eval_stokes<32, false, false>)
-                             : (check ? k_eval_stokes<64, true, false> : k_eval_stokes<64, false, false>));
+    auto sk = PD == 32 ? eval_stokes_pd<32>(dl, check, ns) : eval_stokes_pd<64>(dl, check, ns);
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
-    hipLaunchKernelGGL(sk, dim3(eval_grid(icap, chunk)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
+    hipLaunchKernelGGL(sk, dim3(eval_grid(icap, chunk, ns)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
                        t.evalnode.as<int>(), w.toff, w.tperm,
                        w.tsx, w.tsy, t.nlevel.as<int>(),
                        t.xmid.as<double>(), t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(),
@@ -3601,7 +3734,7 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
                      : (check ? (PD == 32 ? k_eval_mixed<32, true, false> : k_eval_mixed<64, true, false>)
                               : (PD == 32 ? k_eval_mixed<32, false, false> : k_eval_mixed<64, false, false>));
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
-    hipLaunchKernelGGL(mk, dim3(eval_grid(icap, chunk)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
+    hipLaunchKernelGGL(mk, dim3(eval_grid(icap, chunk, 1)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
                        t.evalnode.as<int>(), w.toff, w.tperm,
                        w.tsx, w.tsy, t.nlevel.as<int>(),
                        t.flags.as<int>(), t.xmid.as<double>(), t.ymid.as<double>(),
@@ -3613,16 +3746,16 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
     P.mark(FMM2D_PHASE_EVAL_KERNEL, true, s);
     return;
   }
-  auto kern = P.cheb ? eval_kernel_cheb(PD, P.kernel_id, check)
-              : ev == EVAL_DIPOLE ? eval_kernel_dipole(PD, check)
-                                  : eval_kernel(PD, P.kernel_id, ev == EVAL_POT ? 1 : 3, check);
+  auto kern = PD == 32 ? eval_kernel_pd<32>(P.kernel_id, ev, P.cheb > 0, check, ns)
+                       : eval_kernel_pd<64>(P.kernel_id, ev, P.cheb > 0, check, ns);
   P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
   // few targets per evaluation box on average: the few-target items stage
   // their colleague sources through LDS (the extra LDS would only cost the
   // full-wave items occupancy)
-  const int scap = (ev != EVAL_DIPOLE && few_targets) ? kStageSources : 0;
-  const size_t dyn = (size_t)scap * kEvalWaves * sizeof(double4);
-  hipLaunchKernelGGL(kern, dim3(eval_grid(icap, chunk)), dim3(64 * kEvalWaves), dyn, s, w.items, w.ntot,
+  const int scap = few_targets ? kStageSources : 0;
+  const size_t dyn = (size_t)scap * kEvalWaves *
+                     (sizeof(double4) + (ev == EVAL_DIPOLE ? sizeof(double2) : 0));
+  hipLaunchKernelGGL(kern, dim3(eval_grid(icap, chunk, ns)), dim3(64 * kEvalWaves), dyn, s, w.items, w.ntot,
                      t.evalnode.as<int>(), w.toff, w.tperm, w.tsx,
                      w.tsy, t.nlevel.as<int>(), t.xmid.as<double>(),
                      t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(), t.bot.as<int>(), t.top.as<int>(),
