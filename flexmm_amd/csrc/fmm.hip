@@ -145,7 +145,7 @@ struct Plan {
   bool have_exp = false;
   bool up_done = false;
   // targets
-  DevBuf tnode, tcnt, toff, tcur, tperm, tsx, tsy, icnt, ioff, items, ntot;
+  DevBuf tnode, tcnt, toff, tcur, tperm, tcx, tcy, bsum, items, ntot;
   PrimWork pw;
   HostBuf hbuf;
   int device = 0;
@@ -1535,7 +1535,8 @@ __global__ __launch_bounds__(256) void k_local_level(int g0, int ngroups, int do
     return Phase{opsL + (int64_t)(OP_PINV1 + (k - nl)) * PD * PD, nullptr, true};
   };
   run_phases<PD>(nl + 2, acc, buf[0], buf[1], next);
-  if (active) store_acc<PD>(acc, le + (int64_t)g * PD);
+  // zeros for the fake nodes (their columns are zero)
+  if (q < ngroups) store_acc<PD>(acc, le + (int64_t)g * PD);
 }
 
 // ---------------------------------------------------------------------------
@@ -1724,7 +1725,10 @@ __device__ __forceinline__ void local_small_unit(
   __shared__ __attribute__((aligned(16))) double btile[1][16][PD + kSmallPad];
   __shared__ int srow[16];
   run_small<PD, 1>(nl + 2, nl, opA, le, pg, acc, bbuf, btile, srow);
-  if (active) {
+  // the nodes above level 2 have no local expansion: zeros, as for fake nodes
+  if (!do_l2l && bx == 0)
+    for (int e = threadIdx.x; e < g0 * PD; e += 64 * (PD / 16)) le[e] = 0.0;
+  if (q < ngroups) {
     double* dst = le + (int64_t)g * PD;
 #pragma unroll
     for (int v = 0; v < 4; ++v) dst[16 * w + 4 * v + kq] = acc[v];
@@ -1792,7 +1796,8 @@ __global__ __launch_bounds__(256) void k_locate_count(const double* __restrict__
                                                      const double* __restrict__ ymid,
                                                      const int* __restrict__ evalid,
                                                      int* __restrict__ tbox, int* __restrict__ trank,
-                                                     int* __restrict__ tcnt) {
+                                                     int* __restrict__ tcnt, int ne, int ncopy) {
+  tcnt += (int64_t)(blockIdx.x % ncopy) * ne;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const bool act = i < nt;
   int e = -1;
@@ -1856,15 +1861,19 @@ __global__ __launch_bounds__(256) void k_locate_count(const double* __restrict__
     }
     e = evalid[g];
   }
-  // Group the wave's lanes by box with ballots first (no memory traffic),
-  // then let every group's lowest lane add the group size with one atomic
-  // instruction for all groups, so that targets spread over many boxes (in
-  // random input order) cost one atomic round trip instead of one per box.
+  // Targets in a coherent order: group the wave's lanes by box with ballots
+  // (no memory traffic), then let every group's lowest lane add the group
+  // size, with one atomic instruction for all groups.  Targets in random order
+  // (more runs of equal boxes than kMaxRuns) take one atomic per lane: the
+  // ballot loop would run up to 64 times for groups of one.
+  constexpr int kMaxRuns = 16;
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
   unsigned long long pending = __ballot(act);
-  int leader = lane, inrank = 0, gsize = 0;
-  while (pending) {
+  int leader = lane, inrank = 0, gsize = 1;
+  const int eprev = __shfl_up(e, 1, 64);
+  const int runs = __popcll(__ballot(act && (lane == 0 || e != eprev)));
+  while (runs <= kMaxRuns && pending) {
     const int ld = __builtin_ctzll(pending);
     const int key = __builtin_amdgcn_readlane(e, ld);
     const unsigned long long same = __ballot(act && e == key) & pending;
@@ -1884,105 +1893,153 @@ __global__ __launch_bounds__(256) void k_locate_count(const double* __restrict__
   }
 }
 
-__global__ __launch_bounds__(256) void k_target_scatter(const double* __restrict__ tx,
-                                                       const double* __restrict__ ty, int64_t nt,
-                                                       const int* __restrict__ tbox,
+// The targets' input positions in box order (the evaluation kernels read the
+// coordinates through them).  Blocks and counter copies as in k_locate_count.
+__global__ __launch_bounds__(256) void k_target_scatter(int64_t nt, const int* __restrict__ tbox,
                                                        const int* __restrict__ trank,
                                                        const int* __restrict__ toff,
-                                                       int* __restrict__ tperm,
-                                                       double* __restrict__ tsx,
-                                                       double* __restrict__ tsy) {
+                                                       int* __restrict__ tperm, int ne,
+                                                       int ncopy) {
   int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= nt) return;
-  const int pos = toff[tbox[i]] + trank[i];
-  tperm[pos] = (int)i;
-  tsx[pos] = tx[i];
-  tsy[pos] = ty[i];
+  toff += (int64_t)(blockIdx.x % ncopy) * ne;
+  tperm[toff[tbox[i]] + trank[i]] = (int)i;
+}
+
+__global__ __launch_bounds__(256) void k_copy_targets(const double* __restrict__ tx,
+                                                     const double* __restrict__ ty, int64_t nt,
+                                                     double* __restrict__ cx,
+                                                     double* __restrict__ cy) {
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= nt) return;
+  cx[i] = tx[i];
+  cy[i] = ty[i];
 }
 
 constexpr int kTgtChunk = 64;
+// Target counters: with few boxes, many waves add to each counter, and adds to
+// one address from several XCDs take turns (50K targets in random order over
+// 256 boxes: 21 us in k_locate_count).  Trees of up to kCopyBoxes boxes
+// therefore keep one set of counters per XCD (blocks b with b % 8 == x), which
+// the offset kernel adds up.
+constexpr int kBoxTile = 4096;   // boxes per block of the offset kernels
+constexpr int kCopyBoxes = kBoxTile;
+constexpr int box_copies(int64_t ne) { return ne <= kCopyBoxes ? kNumXcd : 1; }
 
-__global__ __launch_bounds__(256) void k_item_counts(const int* __restrict__ tcnt, int ne,
-                                                    int* __restrict__ icnt) {
-  int b = blockIdx.x * 256 + threadIdx.x;
-  if (b < ne) icnt[b] = (tcnt[b] + kTgtChunk - 1) / kTgtChunk;
-}
-
-// Box offsets of a tree of at most kBoxOffsetsMax evaluation boxes, in one
-// block: toff = exclusive scan of tcnt[0 .. ne] (tcnt[ne] = 0, so toff[ne] =
-// nt) and ioff = exclusive scan of the boxes' item counts ceil(tcnt /
-// kTgtChunk), with their total in *ntot: one pass over the counts for both
-// (two scans and a count kernel otherwise).  Element j 1024 + t is thread t's
-// (coalesced); tiles are scanned by wave scans and combined through LDS.
-constexpr int kBoxTiles = 32;
-constexpr int kBoxOffsetsMax = kBoxTiles * 1024 - 1;
-__global__ __launch_bounds__(1024) void k_box_offsets(const int* __restrict__ tcnt, int ne,
-                                                      int* __restrict__ toff,
-                                                      int* __restrict__ ioff,
-                                                      int* __restrict__ ntot) {
-  __shared__ int wsum[2][kBoxTiles][16];
-  __shared__ int woff[2][kBoxTiles][16];
+// Sums of (targets, items) over each tile of kBoxTile boxes.
+__global__ __launch_bounds__(1024) void k_box_sums(const int* __restrict__ tcnt, int ne,
+                                                   int2* __restrict__ partial) {
+  __shared__ int ws[2][16];
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-  const int n = ne + 1;
-  const int J = (n + 1023) >> 10;
-  int exv[kBoxTiles], exu[kBoxTiles];   // in-wave exclusive prefixes (loaded counts first)
+  int v = 0, u = 0;
 #pragma unroll
-  for (int j = 0; j < kBoxTiles; ++j) {
-    const int idx = j * 1024 + t;
-    exv[j] = (j < J && idx < ne) ? tcnt[idx] : 0;
+  for (int j = 0; j < kBoxTile / 1024; ++j) {
+    const int b = blockIdx.x * kBoxTile + j * 1024 + t;
+    const int n = b < ne ? tcnt[b] : 0;
+    v += n;
+    u += (n + kTgtChunk - 1) / kTgtChunk;
   }
-#pragma unroll
-  for (int j = 0; j < kBoxTiles; ++j) {
-    if (j < J) {
-      const int v = exv[j], u = (v + kTgtChunk - 1) / kTgtChunk;
-      const int iv = wave_inclusive_scan(v), iu = wave_inclusive_scan(u);
-      if (lane == 63) {
-        wsum[0][j][wid] = iv;
-        wsum[1][j][wid] = iu;
-      }
-      exv[j] = iv - v;
-      exu[j] = iu - u;
-    }
+  v = wave_inclusive_scan(v);
+  u = wave_inclusive_scan(u);
+  if (lane == 63) {
+    ws[0][wid] = v;
+    ws[1][wid] = u;
   }
   __syncthreads();
-  if (wid < 2) {   // wave a: offsets of array a (tile prefix, then the 16 waves of each tile)
-    const int a = wid;
-    int tile_tot = 0;
-    if (lane < J)
-      for (int w = 0; w < 16; ++w) tile_tot += wsum[a][lane][w];
-    const int tile_off = wave_inclusive_scan(lane < J ? tile_tot : 0) - (lane < J ? tile_tot : 0);
-    if (lane < J) {
-      int run = tile_off;
-      for (int w = 0; w < 16; ++w) {
-        woff[a][lane][w] = run;
-        run += wsum[a][lane][w];
-      }
-      if (a == 1 && lane == J - 1) *ntot = run;
+  if (t == 0) {
+    int2 s = make_int2(0, 0);
+    for (int w = 0; w < 16; ++w) {
+      s.x += ws[0][w];
+      s.y += ws[1][w];
     }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < kBoxTiles; ++j) {
-    const int idx = j * 1024 + t;
-    if (j < J && idx < n) {
-      toff[idx] = woff[0][j][wid] + exv[j];
-      ioff[idx] = woff[1][j][wid] + exu[j];
-    }
+    partial[blockIdx.x] = s;
   }
 }
 
-// Item = (evaluation node, first target, end target) of one chunk of at most
-// kTgtChunk targets, in sorted-target positions.
-__global__ __launch_bounds__(256) void k_make_items(const int* __restrict__ ioff, int ne,
-                                                   const int* __restrict__ evalnode,
-                                                   const int* __restrict__ toff,
-                                                   int4* __restrict__ items) {
-  int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= ne) return;
-  const int o = ioff[b];
-  const int g = evalnode[b], t0 = toff[b], t1 = toff[b + 1];
-  for (int k = 0; t0 + k * kTgtChunk < t1; ++k)
-    items[o + k] = make_int4(g, t0 + k * kTgtChunk, min(t1, t0 + (k + 1) * kTgtChunk), 0);
+// Box offsets and work items of a tile of kBoxTile boxes per block: toff[c ne
+// + b] = position in box order of the first target that counter copy c holds
+// for box b; item = (evaluation node, first target, end target) of one chunk
+// of at most kTgtChunk targets, in box-order positions; their number in *ntot.
+// tcnt[b] becomes the box's total (NC > 1).  Tiles after the first add up the
+// partial sums of the tiles before them.  Element j 1024 + t is thread t's;
+// its rows are scanned by wave scans and combined through LDS.  (Against two
+// device scans, a count and an item kernel: 7 launches, 22 us at 39K boxes.)
+template <int NC>
+__global__ __launch_bounds__(1024) void k_box_items(int* __restrict__ tcnt, int ne,
+                                                    const int2* __restrict__ partial,
+                                                    const int* __restrict__ evalnode,
+                                                    int* __restrict__ toff,
+                                                    int4* __restrict__ items,
+                                                    int* __restrict__ ntot) {
+  constexpr int J = kBoxTile / 1024;
+  __shared__ int wsum[2][J][16];
+  __shared__ int wpre[2][16];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  int c[J][NC];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int b = blockIdx.x * kBoxTile + j * 1024 + t;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) c[j][k] = b < ne ? tcnt[(int64_t)k * ne + b] : 0;
+  }
+  int pv = 0, pu = 0;   // targets and items of the tiles before this one
+  for (int i = t; i < (int)blockIdx.x; i += 1024) {
+    const int2 p = partial[i];
+    pv += p.x;
+    pu += p.y;
+  }
+  pv = wave_inclusive_scan(pv);
+  pu = wave_inclusive_scan(pu);
+  if (lane == 63) {
+    wpre[0][wid] = pv;
+    wpre[1][wid] = pu;
+  }
+  int v[J], u[J], iv[J], iu[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    v[j] = 0;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) v[j] += c[j][k];
+    u[j] = (v[j] + kTgtChunk - 1) / kTgtChunk;
+    iv[j] = wave_inclusive_scan(v[j]);
+    iu[j] = wave_inclusive_scan(u[j]);
+    if (lane == 63) {
+      wsum[0][j][wid] = iv[j];
+      wsum[1][j][wid] = iu[j];
+    }
+  }
+  __syncthreads();
+  // the 16 J wave sums in order (wave w of row j: entry 16 j + w), scanned by
+  // every wave for itself
+  static_assert(16 * J == 64, "one entry per lane");
+  int p0 = 0, p1 = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    p0 += wpre[0][w];
+    p1 += wpre[1][w];
+  }
+  const int s0 = wsum[0][lane >> 4][lane & 15], s1 = wsum[1][lane >> 4][lane & 15];
+  const int e0 = p0 + wave_inclusive_scan(s0) - s0, e1 = p1 + wave_inclusive_scan(s1) - s1;
+  if (blockIdx.x == gridDim.x - 1 && t == 63) *ntot = e1 + s1;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int b = blockIdx.x * kBoxTile + j * 1024 + t;
+    const int t0 = __shfl(e0, 16 * j + wid, 64) + iv[j] - v[j];
+    const int o = __shfl(e1, 16 * j + wid, 64) + iu[j] - u[j];
+    if (b < ne) {
+      int off = t0;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        toff[(int64_t)k * ne + b] = off;
+        off += c[j][k];
+      }
+      if (NC > 1) tcnt[b] = v[j];
+      const int g = evalnode[b];
+      for (int k = 0; k < u[j]; ++k)
+        items[o + k] =
+            make_int4(g, t0 + k * kTgtChunk, min(t0 + v[j], t0 + (k + 1) * kTgtChunk), 0);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2232,8 +2289,8 @@ __device__ __forceinline__ void l2t_terms(int k0, int step, int p, F term) {
 
 template <int PD, int KER, int NOUT, bool CHECK, bool DIP, bool CHEB, int NS>
 __device__ __forceinline__ void eval_few(
-    int g, int t0, int na, int part, const int* __restrict__ tperm, const double* __restrict__ tsx,
-    const double* __restrict__ tsy, const int* __restrict__ nlevel,
+    int g, int t0, int na, int part, const int* __restrict__ tperm, const double* __restrict__ tx,
+    const double* __restrict__ ty, const int* __restrict__ nlevel,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
     const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
     const double4* __restrict__ src, const double2* __restrict__ dip,
@@ -2248,8 +2305,11 @@ __device__ __forceinline__ void eval_few(
   T.kp = helm_consts(kp);
   // idle slots repeat the item's first target (results not stored), so that
   // they take the same branch of the kernel evaluation as the active ones
-  T.x = tsx[F.act ? t : t0];
-  T.y = tsy[F.act ? t : t0];
+  {
+    const int o = tperm[F.act ? t : t0];
+    T.x = tx[o];
+    T.y = ty[o];
+  }
   const int d = nlevel[g];
   double far = 0.0;   // Chebyshev L2T
   if (CHEB && d >= 2) {
@@ -2365,7 +2425,7 @@ __device__ __forceinline__ void eval_few(
   const bool zh =
       CHECK ? false : item_any<NS>(slot_min(T.dmin, F.lg) == 0u, part);
   if (F.act && F.sg == 0 && part == 0) {
-    const int64_t o = tperm[t];
+    const int64_t o = tperm[t];   // again: kept across the loops it costs a register
     if (zh) sum[0] = DIP ? __builtin_nan("") : __builtin_inf();
     out[o] = sum[0];
     if constexpr (NOUT == 3) {
@@ -2382,7 +2442,7 @@ __global__ __launch_bounds__(64 * kEvalWaves)
 __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) void k_eval(
     const int4* __restrict__ items, const int* __restrict__ nitems,
     const int* __restrict__ evalnode, const int* __restrict__ toff,
-    const int* __restrict__ tperm, const double* __restrict__ tsx, const double* __restrict__ tsy,
+    const int* __restrict__ tperm, const double* __restrict__ tx, const double* __restrict__ ty,
     const int* __restrict__ nlevel, const double* __restrict__ xmid,
     const double* __restrict__ ymid, const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot,
     const int* __restrict__ top, const double4* __restrict__ src,
@@ -2407,7 +2467,7 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
   const int g = __builtin_amdgcn_readfirstlane(it.x);
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets) {
-    eval_few<PD, KER, NOUT, CHECK, DIP, CHEB, NS>(g, t0, t1 - t0, part, tperm, tsx, tsy, nlevel, xmid,
+    eval_few<PD, KER, NOUT, CHECK, DIP, CHEB, NS>(g, t0, t1 - t0, part, tperm, tx, ty, nlevel, xmid,
                                               ymid, coll, crange, bot, top, src, dip, le, ops, opsz, p,
                                               tab, kp, nt, out, stage, dstage, scap);
     return;
@@ -2416,8 +2476,11 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
   const bool act = t < t1;
   Target<KER, NOUT, CHECK> T;
   T.kp = helm_consts(kp);
-  T.x = tsx[act ? t : t0];   // idle lanes: as in eval_few
-  T.y = tsy[act ? t : t0];
+  {
+    const int o = tperm[act ? t : t0];   // idle lanes: as in eval_few
+    T.x = tx[o];
+    T.y = ty[o];
+  }
   // L2T: helpers.py:219-235 (the equivalent density sits on the large circle);
   // Chebyshev expansions: bbfmm.py:185-199
   const int d = nlevel[g];
@@ -2547,8 +2610,8 @@ __global__ __launch_bounds__(64) void k_prep_mixed(const int* __restrict__ evaln
 // the lanes of source group 0; every lane removes the charges it took in FP64.
 template <int PD, bool CHECK, bool CHEB>
 __device__ __forceinline__ void eval_few_mixed(
-    int g, int t0, int na, const int* __restrict__ tperm, const double* __restrict__ tsx,
-    const double* __restrict__ tsy, const int* __restrict__ nlevel, const int* __restrict__ flags,
+    int g, int t0, int na, const int* __restrict__ tperm, const double* __restrict__ tx,
+    const double* __restrict__ ty, const int* __restrict__ nlevel, const int* __restrict__ flags,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
     const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
     const double4* __restrict__ src, const f4* __restrict__ srcf, const double* __restrict__ tsum,
@@ -2559,8 +2622,11 @@ __device__ __forceinline__ void eval_few_mixed(
   Target<KER_LAPLACE, 1, CHECK> T;
   T.kp = HelmConsts{};
   // idle lanes repeat the item's first target (same branches as a real lane)
-  T.x = tsx[F.act ? t : t0];
-  T.y = tsy[F.act ? t : t0];
+  {
+    const int o = tperm[F.act ? t : t0];
+    T.x = tx[o];
+    T.y = ty[o];
+  }
   const int d = nlevel[g];
   double far = 0.0;   // Chebyshev L2T
   if (CHEB && d >= 2) {
@@ -2651,7 +2717,7 @@ template <int PD, bool CHECK, bool CHEB>
 __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
     const int4* __restrict__ items, const int* __restrict__ nitems,
     const int* __restrict__ evalnode, const int* __restrict__ toff,
-    const int* __restrict__ tperm, const double* __restrict__ tsx, const double* __restrict__ tsy,
+    const int* __restrict__ tperm, const double* __restrict__ tx, const double* __restrict__ ty,
     const int* __restrict__ nlevel, const int* __restrict__ flags,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
     const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
@@ -2670,7 +2736,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
   const int g = __builtin_amdgcn_readfirstlane(it.x);
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets) {
-    eval_few_mixed<PD, CHECK, CHEB>(g, t0, t1 - t0, tperm, tsx, tsy, nlevel, flags, xmid,
+    eval_few_mixed<PD, CHECK, CHEB>(g, t0, t1 - t0, tperm, tx, ty, nlevel, flags, xmid,
                                     ymid, coll, crange, bot, top, src, srcf, tsum, lc, le, ops, opsz,
                                     p, tab, out);
     return;
@@ -2681,8 +2747,11 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
   T.kp = HelmConsts{};
   // idle lanes repeat the item's first target: they then take the same
   // branches as a real lane (no near-pair path of their own)
-  T.x = tsx[act ? t : t0];
-  T.y = tsy[act ? t : t0];
+  {
+    const int o = tperm[act ? t : t0];
+    T.x = tx[o];
+    T.y = ty[o];
+  }
   const int d = nlevel[g];
   double far = 0.0;   // Chebyshev L2T
   if (CHEB && d >= 2) {
@@ -2910,8 +2979,8 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m_stokes(int nup,
 // of eval_few; otherwise lane = target and the source loop index is uniform.
 template <int PD, bool CHECK, bool FEW, bool DIP, int NS>
 __device__ __forceinline__ void stokes_item(
-    int g, int t0, int t1, int part, const int* __restrict__ tperm, const double* __restrict__ tsx,
-    const double* __restrict__ tsy, const int* __restrict__ nlevel,
+    int g, int t0, int t1, int part, const int* __restrict__ tperm, const double* __restrict__ tx,
+    const double* __restrict__ ty, const int* __restrict__ nlevel,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
     const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
     const double4* __restrict__ src, const double4* __restrict__ sdip,
@@ -2932,8 +3001,8 @@ __device__ __forceinline__ void stokes_item(
   const int sg = F.sg + part * F.ng, ng = NS * F.ng;
   const int t = t0 + F.slot;
   const bool act = F.act;
-  const double x = act ? tsx[t] : 0.0;
-  const double y = act ? tsy[t] : 0.0;
+  const int o0 = tperm[act ? t : t0];   // idle lanes repeat the first target
+  const double x = tx[o0], y = ty[o0];
   double u = 0.0, v = 0.0, pr = 0.0;
   const int d = nlevel[g];
   if (d >= 2) {
@@ -3099,7 +3168,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) __attribute__((amdgpu_waves_per_eu
 void k_eval_stokes(
     const int4* __restrict__ items, const int* __restrict__ nitems,
     const int* __restrict__ evalnode, const int* __restrict__ toff,
-    const int* __restrict__ tperm, const double* __restrict__ tsx, const double* __restrict__ tsy,
+    const int* __restrict__ tperm, const double* __restrict__ tx, const double* __restrict__ ty,
     const int* __restrict__ nlevel, const double* __restrict__ xmid,
     const double* __restrict__ ymid, const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot,
     const int* __restrict__ top, const double4* __restrict__ src,
@@ -3119,11 +3188,11 @@ void k_eval_stokes(
   const int g = __builtin_amdgcn_readfirstlane(it.x);
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets)
-    stokes_item<PD, CHECK, true, DIP, NS>(g, t0, t1, part, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
+    stokes_item<PD, CHECK, true, DIP, NS>(g, t0, t1, part, tperm, tx, ty, nlevel, xmid, ymid, coll, crange,
                                       bot, top, src, sdip, le, nstride, ops, opsz, p, tab, c0x,
                                       c0y, nt, out);
   else
-    stokes_item<PD, CHECK, false, DIP, NS>(g, t0, t1, part, tperm, tsx, tsy, nlevel, xmid, ymid, coll, crange,
+    stokes_item<PD, CHECK, false, DIP, NS>(g, t0, t1, part, tperm, tx, ty, nlevel, xmid, ymid, coll, crange,
                                        bot, top, src, sdip, le, nstride, ops, opsz, p, tab,
                                        c0x, c0y, nt, out);
 }
@@ -3531,8 +3600,8 @@ static void downward(Plan& P, hipStream_t s) {
   const int64_t rstride = t.n_rows + 1, nstride = t.n_nodes + 1;
   P.le.ensure(nstride * PD * nd * sizeof(double));
   P.ple.ensure(nstride * PD * nd * sizeof(double));
-  fill_i32(P.le.as<int>(), 2 * nstride * PD * nd, 0, s);   // 0.0 (no memset node)
   if (t.L <= 2) {
+    fill_i32(P.le.as<int>(), 2 * nstride * PD * nd, 0, s);   // 0.0 (no memset node)
     P.have_exp = true;
     return;
   }
@@ -3571,24 +3640,26 @@ static void downward(Plan& P, hipStream_t s) {
 // Target-side scratch of one evaluation: target boxes, per-box counts and
 // offsets, targets in leaf order and the work items.
 struct EvalScratch {
-  int *tnode, *tcnt, *toff, *tcur, *tperm, *icnt, *ioff, *ntot, *partials;
-  double *tsx, *tsy;
+  int *tnode, *tcnt, *toff, *tcur, *tperm, *ntot;
+  int2* partials;
+  double *cx, *cy;   // copy of the targets (evaluations in place)
   int4* items;
 };
 
 constexpr int64_t eval_item_cap(int64_t ne, int64_t nt) { return ne + nt / kTgtChunk + 1; }
 
 // The plan's own scratch, grown to nt targets and ne evaluation boxes.
-static EvalScratch plan_scratch(Plan& P, int64_t nt, int64_t ne) {
+static EvalScratch plan_scratch(Plan& P, int64_t nt, int64_t ne, bool in_place) {
   P.tnode.ensure(nt * sizeof(int));
-  P.tcnt.ensure((ne + 1) * sizeof(int));
-  P.toff.ensure((ne + 1) * sizeof(int));
+  P.tcnt.ensure(ne * box_copies(ne) * sizeof(int));
+  P.toff.ensure(ne * box_copies(ne) * sizeof(int));
   P.tcur.ensure((nt + 1) * sizeof(int));   // per-target rank in its box
   P.tperm.ensure(nt * sizeof(int));
-  P.tsx.ensure(nt * sizeof(double));
-  P.tsy.ensure(nt * sizeof(double));
-  P.icnt.ensure((ne + 1) * sizeof(int));
-  P.ioff.ensure((ne + 1) * sizeof(int));
+  if (in_place) {
+    P.tcx.ensure(nt * sizeof(double));
+    P.tcy.ensure(nt * sizeof(double));
+  }
+  P.bsum.ensure(ceil_div(ne, kBoxTile) * sizeof(int2));
   P.items.ensure(eval_item_cap(ne, nt) * sizeof(int4));
   P.ntot.ensure(4 * sizeof(int));
   EvalScratch w;
@@ -3597,12 +3668,10 @@ static EvalScratch plan_scratch(Plan& P, int64_t nt, int64_t ne) {
   w.toff = P.toff.as<int>();
   w.tcur = P.tcur.as<int>();
   w.tperm = P.tperm.as<int>();
-  w.icnt = P.icnt.as<int>();
-  w.ioff = P.ioff.as<int>();
   w.ntot = P.ntot.as<int>();
-  w.partials = nullptr;   // scan partials from the plan's PrimWork
-  w.tsx = P.tsx.as<double>();
-  w.tsy = P.tsy.as<double>();
+  w.partials = P.bsum.as<int2>();
+  w.cx = P.tcx.as<double>();
+  w.cy = P.tcy.as<double>();
   w.items = P.items.as<int4>();
   return w;
 }
@@ -3656,10 +3725,22 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   FMM_REQUIRE(nt >= 0 && nt < ((int64_t)1 << 31), FMM_E_LIMIT, "too many targets");
   if (nt == 0) return;
   const int64_t ne = t.n_eval;
-  const EvalScratch w = given ? *given : plan_scratch(P, nt, ne);
+  // an output that overlaps the targets (the kernels read them while they
+  // write it) is evaluated from a copy of the targets
+  const int64_t nout = ev == EVAL_POT || ev == EVAL_DIPOLE ? 1 : 3;
+  auto overlaps = [&](const double* a) { return a < out + nout * nt && out < a + nt; };
+  const bool in_place = overlaps(tx) || overlaps(ty);
+  const EvalScratch w = given ? *given : plan_scratch(P, nt, ne, in_place);
+  if (in_place) {
+    hipLaunchKernelGGL(k_copy_targets, dim3(grid256(nt)), dim3(256), 0, s, tx, ty, nt, w.cx, w.cy);
+    FMM_LAUNCH_CHECK();
+    tx = w.cx;
+    ty = w.cy;
+  }
   P.last_tcnt = w.tcnt;
   const int64_t icap = eval_item_cap(ne, nt);
-  fill_i32(w.tcnt, ne + 1, 0, s);
+  const int ncopy = box_copies(ne);
+  fill_i32(w.tcnt, ne * ncopy, 0, s);
   LocateTable lt{};
   lt.L = t.L;
   lt.full_depth = t.complete ? t.L - 1 : -1;
@@ -3675,26 +3756,18 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   hipLaunchKernelGGL(k_locate_count, dim3(grid256(nt)), dim3(256), 0, s, tx, ty, nt, lt,
                      t.flags.as<int>(), t.child.as<int>(), t.xmid.as<double>(),
                      t.ymid.as<double>(), t.evalid.as<int>(), w.tnode,
-                     w.tcur, w.tcnt);
+                     w.tcur, w.tcnt, (int)ne, ncopy);
   FMM_LAUNCH_CHECK();
-  if (ne <= kBoxOffsetsMax) {
-    hipLaunchKernelGGL(k_box_offsets, dim3(1), dim3(1024), 0, s, w.tcnt, (int)ne, w.toff, w.ioff,
-                       w.ntot);
+  const int ntile = (int)ceil_div(ne, kBoxTile);
+  if (ntile > 1) {
+    hipLaunchKernelGGL(k_box_sums, dim3(ntile), dim3(1024), 0, s, w.tcnt, (int)ne, w.partials);
     FMM_LAUNCH_CHECK();
-  } else {
-    // toff has ne + 1 entries: scanning ne + 1 counts (the last is zero) gives toff[ne] = nt.
-    exclusive_scan_i32(w.tcnt, w.toff, ne + 1, nullptr, P.pw, s, w.partials);
-    hipLaunchKernelGGL(k_item_counts, dim3(grid256(ne)), dim3(256), 0, s, w.tcnt, (int)ne,
-                       w.icnt);
-    FMM_LAUNCH_CHECK();
-    exclusive_scan_i32(w.icnt, w.ioff, ne, w.ntot, P.pw, s, w.partials);
   }
-  hipLaunchKernelGGL(k_target_scatter, dim3(grid256(nt)), dim3(256), 0, s, tx, ty, nt,
-                     w.tnode, w.tcur, w.toff, w.tperm,
-                     w.tsx, w.tsy);
+  hipLaunchKernelGGL(ncopy > 1 ? k_box_items<kNumXcd> : k_box_items<1>, dim3(ntile), dim3(1024), 0,
+                     s, w.tcnt, (int)ne, w.partials, t.evalnode.as<int>(), w.toff, w.items, w.ntot);
   FMM_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_make_items, dim3(grid256(ne)), dim3(256), 0, s, w.ioff, (int)ne,
-                     t.evalnode.as<int>(), w.toff, w.items);
+  hipLaunchKernelGGL(k_target_scatter, dim3(grid256(nt)), dim3(256), 0, s, nt, w.tnode, w.tcur,
+                     w.toff, w.tperm, (int)ne, ncopy);
   FMM_LAUNCH_CHECK();
   const int PD = P.PD;
   const int64_t opsz = ops_per_level(PD);
@@ -3707,7 +3780,7 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
     hipLaunchKernelGGL(sk, dim3(eval_grid(icap, chunk, ns)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
                        t.evalnode.as<int>(), w.toff, w.tperm,
-                       w.tsx, w.tsy, t.nlevel.as<int>(),
+                       tx, ty, t.nlevel.as<int>(),
                        t.xmid.as<double>(), t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(),
                        t.bot.as<int>(), t.top.as<int>(), P.src.as<double4>(),
                        dl ? P.sdip.as<double4>() : nullptr, P.le.as<double>(),
@@ -3736,7 +3809,7 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
     hipLaunchKernelGGL(mk, dim3(eval_grid(icap, chunk, 1)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
                        t.evalnode.as<int>(), w.toff, w.tperm,
-                       w.tsx, w.tsy, t.nlevel.as<int>(),
+                       tx, ty, t.nlevel.as<int>(),
                        t.flags.as<int>(), t.xmid.as<double>(), t.ymid.as<double>(),
                        t.coll.as<int>(), t.crange.as<int2>(), t.bot.as<int>(), t.top.as<int>(), P.src.as<double4>(),
                        P.srcf.as<f4>(), P.tsum.as<double>(), lc, P.le.as<double>(),
@@ -3756,8 +3829,8 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   const size_t dyn = (size_t)scap * kEvalWaves *
                      (sizeof(double4) + (ev == EVAL_DIPOLE ? sizeof(double2) : 0));
   hipLaunchKernelGGL(kern, dim3(eval_grid(icap, chunk, ns)), dim3(64 * kEvalWaves), dyn, s, w.items, w.ntot,
-                     t.evalnode.as<int>(), w.toff, w.tperm, w.tsx,
-                     w.tsy, t.nlevel.as<int>(), t.xmid.as<double>(),
+                     t.evalnode.as<int>(), w.toff, w.tperm, tx,
+                     ty, t.nlevel.as<int>(), t.xmid.as<double>(),
                      t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(), t.bot.as<int>(), t.top.as<int>(),
                      P.src.as<double4>(), ev == EVAL_DIPOLE ? P.dip.as<double2>() : nullptr,
                      P.le.as<double>(), P.ops.as<double>(), opsz, P.cheb ? P.cheb : P.p,
@@ -3774,13 +3847,15 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
 // copy, so calls that overlap on one GPU race.
 constexpr int64_t kNoAllocMaxTargets = (int64_t)1 << 20;
 constexpr int64_t kNoAllocMaxBoxes = (int64_t)1 << 18;
-constexpr int64_t kNoAllocMaxPartials = 1024;   // scan partials of kNoAllocMaxBoxes + 1 counts
+constexpr int64_t kNoAllocMaxTiles = kNoAllocMaxBoxes / kBoxTile;
+static_assert(kNoAllocMaxBoxes % kBoxTile == 0 && kNoAllocMaxBoxes >= kNumXcd * kCopyBoxes,
+              "the counter copies of small trees fit the box slices");
 
 constexpr int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 
 // Byte offsets of the slices, in the order of EvalScratch's members.
 struct NoAllocLayout {
-  int64_t tnode, tcnt, toff, tcur, tperm, icnt, ioff, ntot, partials, tsx, tsy, items, total;
+  int64_t tnode, tcnt, toff, tcur, tperm, ntot, partials, cx, cy, items, total;
 };
 constexpr NoAllocLayout noalloc_layout() {
   NoAllocLayout l{};
@@ -3790,12 +3865,10 @@ constexpr NoAllocLayout noalloc_layout() {
   l.toff = o; o += align256((kNoAllocMaxBoxes + 1) * 4);
   l.tcur = o; o += align256((kNoAllocMaxTargets + 1) * 4);
   l.tperm = o; o += align256(kNoAllocMaxTargets * 4);
-  l.icnt = o; o += align256((kNoAllocMaxBoxes + 1) * 4);
-  l.ioff = o; o += align256((kNoAllocMaxBoxes + 1) * 4);
   l.ntot = o; o += align256(4 * 4);
-  l.partials = o; o += align256(kNoAllocMaxPartials * 4);
-  l.tsx = o; o += align256(kNoAllocMaxTargets * 8);
-  l.tsy = o; o += align256(kNoAllocMaxTargets * 8);
+  l.partials = o; o += align256(kNoAllocMaxTiles * 8);
+  l.cx = o; o += align256(kNoAllocMaxTargets * 8);
+  l.cy = o; o += align256(kNoAllocMaxTargets * 8);
   l.items = o; o += align256(eval_item_cap(kNoAllocMaxBoxes, kNoAllocMaxTargets) * 16);
   l.total = o;
   return l;
@@ -3829,12 +3902,10 @@ static EvalScratch noalloc_slices(unsigned char* base) {
   w.toff = reinterpret_cast<int*>(base + kNoAlloc.toff);
   w.tcur = reinterpret_cast<int*>(base + kNoAlloc.tcur);
   w.tperm = reinterpret_cast<int*>(base + kNoAlloc.tperm);
-  w.icnt = reinterpret_cast<int*>(base + kNoAlloc.icnt);
-  w.ioff = reinterpret_cast<int*>(base + kNoAlloc.ioff);
   w.ntot = reinterpret_cast<int*>(base + kNoAlloc.ntot);
-  w.partials = reinterpret_cast<int*>(base + kNoAlloc.partials);
-  w.tsx = reinterpret_cast<double*>(base + kNoAlloc.tsx);
-  w.tsy = reinterpret_cast<double*>(base + kNoAlloc.tsy);
+  w.partials = reinterpret_cast<int2*>(base + kNoAlloc.partials);
+  w.cx = reinterpret_cast<double*>(base + kNoAlloc.cx);
+  w.cy = reinterpret_cast<double*>(base + kNoAlloc.cy);
   w.items = reinterpret_cast<int4*>(base + kNoAlloc.items);
   return w;
 }
@@ -4177,8 +4248,6 @@ int fmm2d_evaluate_noalloc(void* plan, const double* tx, const double* ty, int64
   FMM_HIP(hipGetDevice(&dev));
   FMM_REQUIRE(dev == P->device, fmm::FMM_E_ARG,
               "the plan belongs to device %d but device %d is current", P->device, dev);
-  FMM_REQUIRE(fmm::scan_partials_i32(fmm::kNoAllocMaxBoxes + 1) <= fmm::kNoAllocMaxPartials,
-              fmm::FMM_E_INTERNAL, "scan partials exceed the scratch array");
   const fmm::EvalScratch w = fmm::noalloc_slices(fmm::noalloc_scratch(dev));
   // not timed: phase timing creates its HIP events on first use
   struct NoTiming {

@@ -104,3 +104,22 @@ def test_stokes_items(many, dipole):
         ref = odirect.direct_stokes(x, y, fx, fy, tx, ty)
     for a, b in zip(got, ref):
         assert H.rel_max_err(np.asarray(a), b) < 5e-11   # the p = 64 bar of the Stokes tests
+
+
+def test_output_over_the_targets():
+    """An output buffer that overlaps the target coordinates."""
+    import torch
+    from flexmm_amd import _lib, kernels
+    from flexmm_amd.kifmm2d import FMM, the_help
+    x, y, ncut, tx, ty, rng = _problem(False)
+    the_help.clear()
+    f = FMM(x, y, kernels.laplace, ncut, 32, bbox=[0, 1, 0, 1])
+    f.build_expansions(rng.standard_normal(x.size))
+    u = f.target_evaluation(tx, ty)[0]
+    dx = torch.tensor(tx, device=f.device)
+    dy = torch.tensor(ty, device=f.device)
+    torch.cuda.synchronize()
+    s = torch.cuda.current_stream().cuda_stream
+    _lib.check(f.lib.fmm2d_evaluate(f.handle, dx.data_ptr(), dy.data_ptr(), dx.numel(),
+                                    _lib.EVAL_POTENTIAL, 0, dx.data_ptr(), s))
+    assert np.array_equal(dx.cpu().numpy(), u) or H.rel_max_err(dx.cpu().numpy(), u) < 1e-14
