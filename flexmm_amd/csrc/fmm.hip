@@ -1027,19 +1027,13 @@ constexpr int kM2LWCols = 16;
 constexpr int kM2LWWaves = 4;
 constexpr int kM2LF32Waves = 4;
 
-template <int PD, bool FRAME, int NW>
+template <int PD, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_m2l_waves_f32(
     LevelTable lt, const int* __restrict__ flags, const int* __restrict__ m2l,
-    const double* __restrict__ mult, const float* __restrict__ m32,
-    const double* __restrict__ qs, const double* __restrict__ ops, int64_t opsz,
-    double* __restrict__ ple, int64_t rstride, int64_t nstride, const double* __restrict__ xmid,
-    const double* __restrict__ ymid, double c0x, double c0y) {
+    const float* __restrict__ m32, const double* __restrict__ qs, const double* __restrict__ ops,
+    int64_t opsz, double* __restrict__ ple, int64_t rstride, int64_t nstride) {
   constexpr int RB = PD / 16, KS = PD / 4, NA = KS / 4;
   typedef float fv4 __attribute__((ext_vector_type(4)));
-  // FRAME: fields 0 and 1 take the source's field-2 row (D_2) too
-  const bool frame = FRAME && blockIdx.y < 2;
-  const int64_t to2 = (int64_t)(2 - (int)blockIdx.y) * rstride;   // rows to field 2
-  mult += (int64_t)blockIdx.y * rstride * PD;
   qs += (int64_t)blockIdx.y * rstride;
   ple += (int64_t)blockIdx.y * nstride * PD;
   __shared__ int srcs[27][16];
@@ -1061,9 +1055,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   const int q = (lt.perm && qq < ngroups) ? lt.perm[lt.poff[li] + c * ngroups + qq] : qq;
   const int g = lt.g0[li] + 4 * q + c;
   const bool active = q < ngroups && !(flags[q < ngroups ? g : lt.g0[li]] & NF_FAKE);
-  // target centre coordinate blockIdx.y in the root frame (frame fields)
-  const double ct =
-      (frame && active) ? (blockIdx.y == 0 ? xmid[g] - c0x : ymid[g] - c0y) : 0.0;
   // interaction lists: the 4 NW lane groups (w, kq) read slot indices
   // 4 w + kq + 4 NW j < 32 of their column
   constexpr int LG = 4 * NW, NJ = 32 / LG;
@@ -1080,7 +1071,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
       const int src = (active && i < nv) ? lst[c_valid.slot[c][i]] : -1;
       if (i < nv) {
         srcs[i][col] = src;
-        qsl[i][col] = src < 0 ? 0.0 : frame ? __builtin_fma(ct, qs[to2 + src], qs[src]) : qs[src];
+        qsl[i][col] = src < 0 ? 0.0 : qs[src];
       }
       const unsigned long long b = __ballot(src >= 0);
 #pragma unroll
@@ -1113,44 +1104,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // this wave's slots: pslot[w + NW j], j < nmine
   const int nmine = w < nph ? (nph - 1 - w) / NW + 1 : 0;
   if (nmine > 0) {
-    if constexpr (FRAME) {
-      // Stokeslet fields: per slot, entries 8 m + 2 kq + {0, 1} of the
-      // source rows formed in FP64 (the frame fields from two rows), then
-      // each row block's residual pieces loaded before its steps
-      for (int jj = 0; jj < nmine; ++jj) {
-        const int k = w + NW * jj;
-        const int slot = __builtin_amdgcn_readfirstlane(pslotv[k]);
-        const int src = srcs[pslot[k]][col];
-        const double* brow = src >= 0 ? mult + (int64_t)src * PD + 2 * kq : c_zero_row;
-        fv4 bu[NA];
-#pragma unroll
-        for (int m = 0; m < KS / 2; ++m) {
-          dv2 v = *reinterpret_cast<const dv2*>(brow + 8 * m);
-          if (frame && src >= 0) {
-            const dv2 v2 = *reinterpret_cast<const dv2*>(brow + to2 * PD + 8 * m);
-            v.x = __builtin_fma(ct, v2.x, v.x);
-            v.y = __builtin_fma(ct, v2.y, v.y);
-          }
-          bu[m >> 1][2 * (m & 1)] = (float)v.x;
-          bu[m >> 1][2 * (m & 1) + 1] = (float)v.y;
-        }
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          fv4 a[NA];
-#pragma unroll
-          for (int j = 0; j < NA; ++j) a[j] = afr[((int64_t)slot * RB * NA + rb * NA + j) * 64];
-#pragma unroll
-          for (int j = 0; j < NA; ++j) {
-            f4 s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][0], bu[j][0], f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            f4 s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][1], bu[j][1], f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][2], bu[j][2], s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][3], bu[j][3], s1, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc64[rb][v] += (double)(s0[v] + s1[v]);
-          }
-        }
-      }
-    } else {
+    {
       // operator pieces pc = rb NA + j of a slot (16 bytes per lane, four
       // MFMA steps each), NA of them in flight: consuming a piece issues the
       // load of the piece NA further on, across row block and slot
@@ -1254,6 +1208,191 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         for (int ww = 0; ww < NW - 1; ++ww) sum += red[ww][16 * rb + 4 * kq + v][col];
         rowp[16 * rb + 4 * kq + v] = sum;
       }
+  }
+}
+
+// FP32 M2L of the three Stokeslet fields (see k_m2l_waves_f32): the fields of
+// a tile share its slots' residual pieces, and the frame fields their D_2
+// rows, so a block takes all three: per slot and wave 24 row loads and 16
+// piece loads feed 192 MFMAs.  One field per block loaded the pieces three
+// times and five rows instead of three, which kept the texture unit busier
+// than the matrix cores (2M clustered Stokeslets 869 -> 701 us).
+template <int PD, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void k_m2l_frame_f32(
+    LevelTable lt, const int* __restrict__ flags, const int* __restrict__ m2l,
+    const double* __restrict__ mult, const double* __restrict__ qs,
+    const double* __restrict__ ops, int64_t opsz, double* __restrict__ ple, int64_t rstride,
+    int64_t nstride, const double* __restrict__ xmid, const double* __restrict__ ymid, double c0x,
+    double c0y) {
+  constexpr int RB = PD / 16, KS = PD / 4, NA = KS / 4, NP = RB * NA, NF = 3;
+  typedef float fv4 __attribute__((ext_vector_type(4)));
+  __shared__ int srcs[27][16];
+  __shared__ double qsl[NF][27][16];   // source charge sums (0: no source)
+  __shared__ int pslot[28];
+  __shared__ int pslotv[27];   // the M2L slot (offset) of each used slot index
+  __shared__ unsigned int smask;
+  __shared__ double red[NW - 1][PD][17];
+  const int bid = xcd_block(blockIdx.x, gridDim.x, lt.xchunk);
+  int li = 0;
+  while (li + 1 < lt.nlev && bid >= lt.boff[li + 1]) ++li;
+  const int lb = bid - lt.boff[li];
+  const int c = lb & 3;
+  const int tile = lb >> 2;
+  const int ngroups = lt.ngroups[li];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int col = l & 15, kq = l >> 4;
+  const int qq = tile * 16 + col;
+  const int q = (lt.perm && qq < ngroups) ? lt.perm[lt.poff[li] + c * ngroups + qq] : qq;
+  const int g = lt.g0[li] + 4 * q + c;
+  const bool active = q < ngroups && !(flags[q < ngroups ? g : lt.g0[li]] & NF_FAKE);
+  // target centre in the root frame (fields 0 and 1)
+  const double ctx = active ? xmid[g] - c0x : 0.0, cty = active ? ymid[g] - c0y : 0.0;
+  // interaction lists: the 4 NW lane groups (w, kq) read slot indices
+  // 4 w + kq + 4 NW j < 32 of their column
+  constexpr int LG = 4 * NW, NJ = 32 / LG;
+  static_assert(NJ * LG == 32, "lane groups cover the 32 slot indices");
+  const int nv = c_valid.n[c];
+  if (threadIdx.x == 0) smask = 0u;
+  __syncthreads();
+  unsigned int used = 0u;
+  {
+    const int* lst = m2l + (int64_t)g * kNumM2L;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int i = 4 * w + kq + LG * j;
+      const int src = (active && i < nv) ? lst[c_valid.slot[c][i]] : -1;
+      if (i < nv) {
+        srcs[i][col] = src;
+        const double q2 = src < 0 ? 0.0 : qs[2 * rstride + src];
+        qsl[0][i][col] = src < 0 ? 0.0 : __builtin_fma(ctx, q2, qs[src]);
+        qsl[1][i][col] = src < 0 ? 0.0 : __builtin_fma(cty, q2, qs[rstride + src]);
+        qsl[2][i][col] = q2;
+      }
+      const unsigned long long b = __ballot(src >= 0);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if ((b >> (16 * k)) & 0xffffull) used |= 1u << (4 * w + k + LG * j);
+    }
+  }
+  if (l == 0 && used) atomicOr(&smask, used);
+  __syncthreads();
+  const unsigned int mask = smask;
+  const int nph = __popc(mask);
+  if (threadIdx.x < 27 && (mask >> threadIdx.x & 1u)) {
+    const int k = __popc(mask & ((1u << threadIdx.x) - 1u));
+    pslot[k] = threadIdx.x;
+    pslotv[k] = c_valid.slot[c][threadIdx.x];
+  }
+  __syncthreads();
+  const double* opsL = ops + (int64_t)lt.d[li] * opsz;
+  const double* means = opsL + ops_off_means(PD);
+  // residual piece pc = rb NA + j of a slot: afr[(slot NP + pc) 64]
+  const fv4* afr = reinterpret_cast<const fv4*>(opsL + ops_off_r32(PD)) + l;
+  d4 acc64[NF][RB];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc64[f][rb] = d4{0.0, 0.0, 0.0, 0.0};
+  // this wave's slots: pslot[w + NW j], j < nmine
+  const int nmine = w < nph ? (nph - 1 - w) / NW + 1 : 0;
+  if (nmine > 0) {
+    int slot = __builtin_amdgcn_readfirstlane(pslotv[w]);
+    fv4 a[NA];
+#pragma unroll
+    for (int j = 0; j < NA; ++j) a[j] = afr[((int64_t)slot * NP + j) * 64];
+    for (int jj = 0; jj < nmine; ++jj) {
+      const int k = w + NW * jj;
+      const int slot_n = __builtin_amdgcn_readfirstlane(pslotv[jj + 1 < nmine ? k + NW : k]);
+      const int src = srcs[pslot[k]][col];
+      // entries 8 m + 2 kq + {0, 1} of the source rows, the frame fields
+      // formed in FP64 from two rows
+      const double* brow = src >= 0 ? mult + (int64_t)src * PD + 2 * kq : c_zero_row + 2 * kq;
+      const int64_t fs = src >= 0 ? rstride * PD : 0;
+      fv4 bu[NF][NA];
+#pragma unroll
+      for (int m = 0; m < KS / 2; ++m) {
+        const dv2 v2 = *reinterpret_cast<const dv2*>(brow + 2 * fs + 8 * m);
+        dv2 v0 = *reinterpret_cast<const dv2*>(brow + 8 * m);
+        dv2 v1 = *reinterpret_cast<const dv2*>(brow + fs + 8 * m);
+        v0.x = __builtin_fma(ctx, v2.x, v0.x);
+        v0.y = __builtin_fma(ctx, v2.y, v0.y);
+        v1.x = __builtin_fma(cty, v2.x, v1.x);
+        v1.y = __builtin_fma(cty, v2.y, v1.y);
+        bu[0][m >> 1][2 * (m & 1)] = (float)v0.x;
+        bu[0][m >> 1][2 * (m & 1) + 1] = (float)v0.y;
+        bu[1][m >> 1][2 * (m & 1)] = (float)v1.x;
+        bu[1][m >> 1][2 * (m & 1) + 1] = (float)v1.y;
+        bu[2][m >> 1][2 * (m & 1)] = (float)v2.x;
+        bu[2][m >> 1][2 * (m & 1) + 1] = (float)v2.y;
+        // half of the rows in flight at a time: all of them would spill
+        if (m == KS / 4 - 1) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int pc = 0; pc < NP; ++pc) {
+        const int rb = pc / NA, j = pc % NA;
+        f4 s[NF][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int f = 0; f < NF; ++f)
+            s[f][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][h], bu[f][j][h],
+                                                           f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int f = 0; f < NF; ++f)
+            s[f][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][2 + h], bu[f][j][2 + h], s[f][h],
+                                                           0, 0, 0);
+        // the piece just used is reloaded with the one a row block further on
+        a[j] = afr[((int64_t)(pc + NA < NP ? slot : slot_n) * NP + (pc + NA) % NP) * 64];
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc64[f][rb][v] += (double)(s[f][0][v] + s[f][1][v]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      slot = slot_n;
+    }
+    // constant mode (see k_m2l_waves_f32)
+    const int prow = 4 * (col & 3) + (col >> 2);
+    for (int k0 = w; k0 < nph; k0 += 4 * NW) {
+      const int kk = k0 + NW * kq;
+      const bool ok = kk < nph;
+      const int ks = ok ? kk : k0;
+      const double* mrow = means + (int64_t)pslotv[ks] * PD + prow;
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const double bq = ok ? qsl[f][pslot[ks]][col] : 0.0;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          acc64[f][rb] =
+              __builtin_amdgcn_mfma_f64_16x16x4f64(mrow[16 * rb], bq, acc64[f][rb], 0, 0, 0);
+      }
+    }
+  }
+  // waves 1 .. NW-1 hand their sums to wave 0, which adds them in wave order
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    if (f > 0) __syncthreads();
+    if (w > 0) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) red[w - 1][16 * rb + 4 * kq + v][col] = acc64[f][rb][v];
+    }
+    __syncthreads();
+    if (w == 0 && active) {
+      double* rowp = ple + (f * nstride + g) * PD;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          double sum = acc64[f][rb][v];
+#pragma unroll
+          for (int ww = 0; ww < NW - 1; ++ww) sum += red[ww][16 * rb + 4 * kq + v][col];
+          rowp[16 * rb + 4 * kq + v] = sum;
+        }
+    }
   }
 }
 
@@ -3450,19 +3589,22 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
     }
     lw.boff[lw.nlev] = nbw;
     lw.split = 1;
-    const bool frame = P.kernel_id == KER_STOKES;
     constexpr int NW = kM2LF32Waves;
-    auto kern = PD == 32
-                    ? (frame ? k_m2l_waves_f32<32, true, NW> : k_m2l_waves_f32<32, false, NW>)
-                    : (frame ? k_m2l_waves_f32<64, true, NW> : k_m2l_waves_f32<64, false, NW>);
-    FMM_REQUIRE(frame || P.mult32.bytes >= (size_t)(rstride * PD * nd * sizeof(float)),
-                FMM_E_INTERNAL, "FP32 multipole copy missing");
-    hipLaunchKernelGGL(kern, dim3(nbw, nd), dim3(64 * NW), 0, s, lw, t.flags.as<int>(),
-                       t.m2l.as<int>(), P.mult.as<double>(),
-                       frame ? nullptr : P.mult32.as<float>(), P.qs.as<double>(),
-                       P.ops.as<double>(), opsz, P.ple.as<double>(), rstride, nstride,
-                       t.xmid.as<double>(), t.ymid.as<double>(), t.xmin + 0.5 * t.w0,
-                       t.ymin + 0.5 * t.w0);
+    if (P.kernel_id == KER_STOKES) {
+      auto kern = PD == 32 ? k_m2l_frame_f32<32, NW> : k_m2l_frame_f32<64, NW>;
+      hipLaunchKernelGGL(kern, dim3(nbw), dim3(64 * NW), 0, s, lw, t.flags.as<int>(), t.m2l.as<int>(),
+                         P.mult.as<double>(), P.qs.as<double>(), P.ops.as<double>(), opsz,
+                         P.ple.as<double>(), rstride, nstride, t.xmid.as<double>(),
+                         t.ymid.as<double>(), t.xmin + 0.5 * t.w0, t.ymin + 0.5 * t.w0);
+      FMM_LAUNCH_CHECK();
+      return;
+    }
+    FMM_REQUIRE(P.mult32.bytes >= (size_t)(rstride * PD * nd * sizeof(float)), FMM_E_INTERNAL,
+                "FP32 multipole copy missing");
+    auto kern = PD == 32 ? k_m2l_waves_f32<32, NW> : k_m2l_waves_f32<64, NW>;
+    hipLaunchKernelGGL(kern, dim3(nbw, nd), dim3(64 * NW), 0, s, lw, t.flags.as<int>(), t.m2l.as<int>(),
+                       P.mult32.as<float>(), P.qs.as<double>(), P.ops.as<double>(), opsz,
+                       P.ple.as<double>(), rstride, nstride);
     FMM_LAUNCH_CHECK();
     return;
   }
