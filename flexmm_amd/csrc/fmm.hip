@@ -204,6 +204,40 @@ struct PlanCall {
 
 namespace {
 
+constexpr int kEvalWaves = 4;   // waves per block of the evaluation and S2M kernels
+// Sums of the NS waves that share an item, in wave order; valid in wave 0.
+template <int NS, int NV>
+__device__ __forceinline__ void item_sum(double (&v)[NV], int part) {
+  static_assert(NS == 1 || NS == kEvalWaves, "an item's waves are one wave or the block");
+  if constexpr (NS > 1) {
+    __shared__ double red[NS - 1][NV][64];
+    const int lane = threadIdx.x & 63;
+    if (part > 0) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) red[part - 1][i][lane] = v[i];
+    }
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int w = 0; w < NS - 1; ++w) v[i] += red[w][i][lane];
+    }
+  }
+}
+template <int NS>
+__device__ __forceinline__ bool item_any(bool hit, int part) {
+  if constexpr (NS > 1) {
+    __shared__ unsigned char any[NS][64];
+    const int lane = threadIdx.x & 63;
+    any[part][lane] = hit;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NS; ++w) hit |= any[w][lane] != 0;
+  }
+  return hit;
+}
+
 __device__ __forceinline__ void load_logtab(double2* tab, const double2* __restrict__ g) {
   for (int i = threadIdx.x; i < kLogTableSize; i += blockDim.x) tab[i] = g[i];
 }
@@ -354,14 +388,17 @@ struct PotAcc<KER_MODHELM> {
   __device__ __forceinline__ double result() const { return kInv2Pi * s; }
 };
 
-// S2M: one wave per leaf (kS2MWaves leaves per block share the log table),
+// S2M: one wave per leaf (kEvalWaves leaves per block share the log table),
 // lane k = check point k on the large circle (helpers.py:159-173; the source
-// is taken relative to the box centre).
-constexpr int kS2MWaves = 4;
+// is taken relative to the box centre).  NS = kEvalWaves: the waves of a block
+// share a leaf, each taking a quarter of its sources.  Up to kSplitLeaves
+// leaves (one per SIMD) a leaf's wave has its SIMD to itself and waits for its
+// own loads: 256 leaves of 195 sources 29.5 -> 9.6 us, 64 leaves of 31 sources 7.8 -> 4.6.
+constexpr int64_t kSplitLeaves = 4 * kNumCUs;
 // DIP: sources also carry a dipole moment q (the double layer of the Laplace
 // kernel, (q.d)/d^2/(2 pi) with d = check point - source).
-template <int PD, int KER, bool DIP>
-__global__ __launch_bounds__(64 * kS2MWaves) void k_s2m(int nup, const int* __restrict__ upnodes,
+template <int PD, int KER, bool DIP, int NS>
+__global__ __launch_bounds__(64 * kEvalWaves) void k_s2m(int nup, const int* __restrict__ upnodes,
                                             const int* __restrict__ nlevel,
                                             const int* __restrict__ bot, const int* __restrict__ top,
                                             const int* __restrict__ row,
@@ -375,7 +412,9 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m(int nup, const int* __re
   __shared__ double2 tab[kLogTableSize];
   load_logtab(tab, logtab);
   __syncthreads();
-  const int gi = blockIdx.x * kS2MWaves + (int)(threadIdx.x >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int part = NS > 1 ? wv : 0;
+  const int gi = NS > 1 ? (int)blockIdx.x : (int)blockIdx.x * kEvalWaves + wv;
   if (gi >= nup) return;
   const int g = upnodes[gi];
   const int d = nlevel[g];
@@ -389,8 +428,13 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m(int nup, const int* __re
   // they take the same branch of the kernel evaluation as the active lanes
   const double ax = lx[k < p ? k : 0] + xmid[g];
   const double ay = ly[k < p ? k : 0] + ymid[g];
-  const int b = __builtin_amdgcn_readfirstlane(bot[g]);
-  const int t = __builtin_amdgcn_readfirstlane(top[g]);
+  int b = __builtin_amdgcn_readfirstlane(bot[g]);
+  int t = __builtin_amdgcn_readfirstlane(top[g]);
+  if constexpr (NS > 1) {   // this wave's share
+    const int n = t - b;
+    t = b + n * (part + 1) / NS;
+    b += n * part / NS;
+  }
   PotAcc<KER> acc;
   const HelmConsts hc = helm_consts(kp);
   double dsum = 0.0;   // double layer
@@ -422,7 +466,9 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m(int nup, const int* __re
       dsum = __builtin_fma(__builtin_fma(q.x, dx, q.y * dy), rcp_nr(d2), dsum);
     }
   }
-  if (k < PD) check[(int64_t)r * PD + k] = k < p ? acc.result() + kInv2Pi * dsum : 0.0;
+  double sum[1] = {acc.result() + kInv2Pi * dsum};
+  item_sum<NS>(sum, part);
+  if (k < PD && part == 0) check[(int64_t)r * PD + k] = k < p ? sum[0] : 0.0;
 }
 
 // Chebyshev moments (source2pMs, bbfmm.py:173-184; anterpolate2 :11-24):
@@ -2191,7 +2237,6 @@ __global__ __launch_bounds__(1024) void k_box_items(int* __restrict__ tcnt, int 
 // eighth of the items; chunk > 0: chunks of that many items go to the XCDs in
 // turn.  Surplus waves exit.  (A grid capped at 8 blocks per CU, waves
 // striding over several items, measured 8-20% slower.)
-constexpr int kEvalWaves = 4;
 constexpr int kStageSources = 64;   // LDS staging of few-target items: sources per wave and chunk
 // Items of a complete tree cost about the same, and eighths keep the most
 // sources in one L2 (mixed form, 1M points: 208 us, 229 with chunks of 32).
@@ -2378,39 +2423,6 @@ __device__ __forceinline__ uint32_t slot_min(uint32_t v, int lg) {
   for (int off = 1 << lg; off < 64; off <<= 1)
     v = min(v, (uint32_t)__shfl_xor((int)v, off, 64));
   return v;
-}
-
-// Sums of the NS waves that share an item, in wave order; valid in wave 0.
-template <int NS, int NV>
-__device__ __forceinline__ void item_sum(double (&v)[NV], int part) {
-  static_assert(NS == 1 || NS == kEvalWaves, "an item's waves are one wave or the block");
-  if constexpr (NS > 1) {
-    __shared__ double red[NS - 1][NV][64];
-    const int lane = threadIdx.x & 63;
-    if (part > 0) {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) red[part - 1][i][lane] = v[i];
-    }
-    __syncthreads();
-    if (part == 0) {
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-#pragma unroll
-        for (int w = 0; w < NS - 1; ++w) v[i] += red[w][i][lane];
-    }
-  }
-}
-template <int NS>
-__device__ __forceinline__ bool item_any(bool hit, int part) {
-  if constexpr (NS > 1) {
-    __shared__ unsigned char any[NS][64];
-    const int lane = threadIdx.x & 63;
-    any[part][lane] = hit;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < NS; ++w) hit |= any[w][lane] != 0;
-  }
-  return hit;
 }
 
 // The L2T terms k0, k0 + step, ... < p of one target: four terms' loads in
@@ -3047,8 +3059,8 @@ __global__ void k_pack_stokes_dipole(const double* __restrict__ tau,
 //   D_i += -f_i log|r| - X_i(s) (f.r)/|r|^2,  D_2 += (f.r)/|r|^2,
 // DIP: D_i += 2 (g r_i/|r|^2 + X_i(s) q),  D_2 -= 2 q,
 //   q = a d_xx log|r| + b d_xy log|r| = (a (r_y^2 - r_x^2) - 2 b r_x r_y)/|r|^4.
-template <int PD, bool DIP>
-__global__ __launch_bounds__(64 * kS2MWaves) void k_s2m_stokes(int nup,
+template <int PD, bool DIP, int NS>
+__global__ __launch_bounds__(64 * kEvalWaves) void k_s2m_stokes(int nup,
                                                                const int* __restrict__ upnodes,
                                                    const int* __restrict__ nlevel,
                                                    const int* __restrict__ bot,
@@ -3065,7 +3077,9 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m_stokes(int nup,
   __shared__ double2 tab[kLogTableSize];
   load_logtab(tab, logtab);
   __syncthreads();
-  const int gi = blockIdx.x * kS2MWaves + (int)(threadIdx.x >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int part = NS > 1 ? wv : 0;
+  const int gi = NS > 1 ? (int)blockIdx.x : (int)blockIdx.x * kEvalWaves + wv;
   if (gi >= nup) return;
   const int g = upnodes[gi];
   const int d = nlevel[g];
@@ -3076,8 +3090,13 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m_stokes(int nup,
   const double* ly = lx + PD;
   const double ax = (k < p ? lx[k] : 1.0) + xmid[g];   // check point, absolute
   const double ay = (k < p ? ly[k] : 1.0) + ymid[g];
-  const int b = __builtin_amdgcn_readfirstlane(bot[g]);
-  const int t = __builtin_amdgcn_readfirstlane(top[g]);
+  int b = __builtin_amdgcn_readfirstlane(bot[g]);
+  int t = __builtin_amdgcn_readfirstlane(top[g]);
+  if constexpr (NS > 1) {   // this wave's share
+    const int n = t - b;
+    t = b + n * (part + 1) / NS;
+    b += n * part / NS;
+  }
   LogAcc lfx, lfy;                 // sum f_i log|r|^2
   double ex = 0.0, ey = 0.0, e2 = 0.0;
   for (int j = b; j < t; ++j) {
@@ -3105,11 +3124,12 @@ __global__ __launch_bounds__(64 * kS2MWaves) void k_s2m_stokes(int nup,
       e2 = __builtin_fma(-2.0, qv, e2);
     }
   }
-  if (k < PD) {
-    // -f_i log|r| = -(1/2) f_i log|r|^2
-    check[r * PD + k] = k < p ? __builtin_fma(-0.5, lfx.value(), ex) : 0.0;
-    check[(rstride + r) * PD + k] = k < p ? __builtin_fma(-0.5, lfy.value(), ey) : 0.0;
-    check[(2 * rstride + r) * PD + k] = k < p ? e2 : 0.0;
+  // -f_i log|r| = -(1/2) f_i log|r|^2
+  double sum[3] = {__builtin_fma(-0.5, lfx.value(), ex), __builtin_fma(-0.5, lfy.value(), ey), e2};
+  item_sum<NS>(sum, part);
+  if (k < PD && part == 0) {
+#pragma unroll
+    for (int f = 0; f < 3; ++f) check[(f * rstride + r) * PD + k] = k < p ? sum[f] : 0.0;
   }
 }
 
@@ -3628,6 +3648,27 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
   FMM_LAUNCH_CHECK();
 }
 
+typedef decltype(&k_s2m<32, KER_LAPLACE, false, 1>) S2MFn;
+template <int PD, int NS>
+static S2MFn s2m_kernel_of(int ker, bool dip) {
+  if (dip) return k_s2m<PD, KER_LAPLACE, true, NS>;
+  return ker == KER_LAPLACE ? k_s2m<PD, KER_LAPLACE, false, NS> : k_s2m<PD, KER_MODHELM, false, NS>;
+}
+static S2MFn s2m_kernel(int PD, int ker, bool dip, int ns) {
+  if (ns == 1) return PD == 32 ? s2m_kernel_of<32, 1>(ker, dip) : s2m_kernel_of<64, 1>(ker, dip);
+  return PD == 32 ? s2m_kernel_of<32, kEvalWaves>(ker, dip)
+                  : s2m_kernel_of<64, kEvalWaves>(ker, dip);
+}
+typedef decltype(&k_s2m_stokes<32, false, 1>) S2MStokesFn;
+template <int NS>
+static S2MStokesFn s2m_stokes_of(int PD, bool dip) {
+  if (PD == 32) return dip ? k_s2m_stokes<32, true, NS> : k_s2m_stokes<32, false, NS>;
+  return dip ? k_s2m_stokes<64, true, NS> : k_s2m_stokes<64, false, NS>;
+}
+static S2MStokesFn s2m_stokes_kernel(int PD, bool dip, int ns) {
+  return ns == 1 ? s2m_stokes_of<1>(PD, dip) : s2m_stokes_of<kEvalWaves>(PD, dip);
+}
+
 // dvec: dipole directions (x [n] then y [n]) when the sources carry single
 // and double layer densities (tau: charges [n] then dipole strengths [n]).
 static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s) {
@@ -3679,11 +3720,11 @@ static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s
     P.have_exp = true;
     return;
   }
+  const int sns = t.n_up <= kSplitLeaves ? kEvalWaves : 1;   // waves per leaf
   P.mark(FMM2D_PHASE_S2M, false, s);
   if (t.n_up > 0 && stokes) {
-    auto kern = dvec ? (PD == 32 ? k_s2m_stokes<32, true> : k_s2m_stokes<64, true>)
-                     : (PD == 32 ? k_s2m_stokes<32, false> : k_s2m_stokes<64, false>);
-    hipLaunchKernelGGL(kern, dim3(ceil_div(t.n_up, kS2MWaves)), dim3(64 * kS2MWaves), 0, s,
+    auto kern = s2m_stokes_kernel(PD, dvec != nullptr, sns);
+    hipLaunchKernelGGL(kern, dim3(ceil_div(t.n_up * sns, kEvalWaves)), dim3(64 * kEvalWaves), 0, s,
                        (int)t.n_up, t.upnodes.as<int>(), t.nlevel.as<int>(),
                        t.bot.as<int>(), t.top.as<int>(), t.row.as<int>(), t.xmid.as<double>(),
                        t.ymid.as<double>(), P.src.as<double4>(), P.ops.as<double>(), opsz, P.p,
@@ -3698,11 +3739,8 @@ static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s
                        P.ops.as<double>(), opsz, P.cheb, P.check.as<double>());
     FMM_LAUNCH_CHECK();
   } else if (t.n_up > 0) {
-    auto kern = dvec ? (PD == 32 ? k_s2m<32, KER_LAPLACE, true> : k_s2m<64, KER_LAPLACE, true>)
-                : P.kernel_id == KER_LAPLACE
-                    ? (PD == 32 ? k_s2m<32, KER_LAPLACE, false> : k_s2m<64, KER_LAPLACE, false>)
-                    : (PD == 32 ? k_s2m<32, KER_MODHELM, false> : k_s2m<64, KER_MODHELM, false>);
-    hipLaunchKernelGGL(kern, dim3(ceil_div(t.n_up, kS2MWaves)), dim3(64 * kS2MWaves), 0, s,
+    auto kern = s2m_kernel(PD, P.kernel_id, dvec != nullptr, sns);
+    hipLaunchKernelGGL(kern, dim3(ceil_div(t.n_up * sns, kEvalWaves)), dim3(64 * kEvalWaves), 0, s,
                        (int)t.n_up, t.upnodes.as<int>(), t.nlevel.as<int>(),
                        t.bot.as<int>(), t.top.as<int>(), t.row.as<int>(), t.xmid.as<double>(),
                        t.ymid.as<double>(), P.src.as<double4>(), P.ops.as<double>(), opsz, P.p,
