@@ -128,7 +128,7 @@ struct Plan {
   int m2l_mode = FMM2D_M2L_DENSE;   // FP64 M2L: every slot dense, or compressed as the reference
   Tree tree;
   DevBuf ops;
-  DevBuf opsm;         // FP64 M2L: the M2L blocks of each level in MFMA operand order (k_m2l_pack)
+  DevBuf opsm;         // each level's operators in MFMA operand order (k_ops_pack)
   int ops_levels = 0;
   std::vector<char> ops_set;
   DevBuf logtab;
@@ -573,157 +573,6 @@ struct AStage {
   }
 };
 
-// acc[rb] += A[rows of row block rb0 + rb] * B, rb < NRB
-template <int PD, int NRB = PD / 16>
-__device__ __forceinline__ void mfma_block(d4 (&acc)[NRB], const double* __restrict__ A,
-                                           const double (&b)[PD / 4], int rb0 = 0) {
-  constexpr int KS = Mfma<PD>::KS, LDA = Mfma<PD>::LDA;
-  const int l = threadIdx.x & 63;
-  const double* a0 = A + (rb0 * 16 + (l & 15)) * LDA + (l >> 4);
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-    for (int rb = 0; rb < NRB; ++rb)
-      acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[rb * 16 * LDA + ks * 4], b[ks], acc[rb], 0,
-                                                     0, 0);
-}
-
-template <int PD>
-__device__ __forceinline__ void zero_acc(d4 (&acc)[PD / 16]) {
-#pragma unroll
-  for (int rb = 0; rb < PD / 16; ++rb) acc[rb] = d4{0.0, 0.0, 0.0, 0.0};
-}
-
-// acc (D layout) from / to a row of PD doubles
-template <int PD>
-__device__ __forceinline__ void load_acc(d4 (&acc)[PD / 16], const double* __restrict__ rowp) {
-  const int kq = (threadIdx.x & 63) >> 4;
-#pragma unroll
-  for (int rb = 0; rb < PD / 16; ++rb)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[rb][v] = rowp ? rowp[16 * rb + 4 * v + kq] : 0.0;
-}
-template <int PD>
-__device__ __forceinline__ void store_acc(const d4 (&acc)[PD / 16], double* __restrict__ rowp) {
-  const int kq = (threadIdx.x & 63) >> 4;
-#pragma unroll
-  for (int rb = 0; rb < PD / 16; ++rb)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) rowp[16 * rb + 4 * v + kq] = acc[rb][v];
-}
-
-// One phase: operator block A (PD x PD, global) and either a per-lane source
-// row (B column = PD doubles, or null for zeros) or the accumulator itself
-// (chain: acc <- A * acc).
-struct Phase {
-  const double* A;
-  const double* brow;
-  bool chain;
-};
-
-// `next()` returns the phases in order (it may keep state).
-template <int PD, class Next>
-__device__ __forceinline__ void run_phases(int nph, d4 (&acc)[PD / 16], double* __restrict__ buf0,
-                                           double* __restrict__ buf1, Next& next) {
-  constexpr int KS = Mfma<PD>::KS;
-  if (nph <= 0) return;
-  const int kq = (threadIdx.x & 63) >> 4;
-  AStage<PD> st;
-  double bn[KS];
-  Phase ps = next();
-  st.load(ps.A);
-  bool chain_n = ps.chain;
-  bool any_n = ps.chain || __ballot(ps.brow != nullptr) != 0;
-  if (!ps.chain) {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) bn[ks] = ps.brow ? ps.brow[4 * ks + kq] : 0.0;
-  }
-  for (int i = 0; i < nph; ++i) {
-    double* A = (i & 1) ? buf1 : buf0;
-    st.store(A);
-    const bool chain = chain_n, any = any_n;
-    double bc[KS];
-    if (chain) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) bc[ks] = acc[ks >> 2][ks & 3];
-      zero_acc<PD>(acc);
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) bc[ks] = bn[ks];
-    }
-    __syncthreads();
-    if (i + 1 < nph) {
-      ps = next();
-      st.load(ps.A);
-      chain_n = ps.chain;
-      any_n = ps.chain || __ballot(ps.brow != nullptr) != 0;
-      if (!ps.chain) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) bn[ks] = ps.brow ? ps.brow[4 * ks + kq] : 0.0;
-      }
-    }
-    if (any) mfma_block<PD>(acc, A, bc);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Upward, one level: rows [row0, row0 + nrows); 64 rows (boxes) per block.
-// check = S2M result (leaves) or M2M of the four children (parents), then
-// multipole = pinv2 * (pinv1 * check)  (fmm.py:98-122).
-template <int PD>
-__global__ __launch_bounds__(256) void k_mult_level(int64_t row0, int nrows, int with_m2m,
-                                                   const int2* __restrict__ rowinfo,
-                                                   const double* __restrict__ check,
-                                                   const double* __restrict__ opsL,
-                                                   double* __restrict__ mult,
-                                                   double* __restrict__ qs, int64_t dstride,
-                                                   float* __restrict__ m32) {
-  __shared__ __attribute__((aligned(16))) double buf[2][PD * Mfma<PD>::LDA];
-  // density blockIdx.y: its rows sit dstride rows further in check, mult and qs
-  check += (int64_t)blockIdx.y * dstride * PD;
-  mult += (int64_t)blockIdx.y * dstride * PD;
-  qs += (int64_t)blockIdx.y * dstride;
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int rl = blockIdx.x * 64 + w * 16 + (l & 15);
-  const bool active = rl < nrows;
-  const int64_t r = row0 + rl;
-  const int2 ri = active ? rowinfo[r] : make_int2(-1, 0);
-  const int f = ri.y;
-  const int crow = ri.x;
-  d4 acc[PD / 16];
-  load_acc<PD>(acc, (active && (f & NF_UP)) ? check + r * PD : nullptr);
-  const int nm = with_m2m ? 4 : 0;
-  int i = 0;
-  auto next = [&]() -> Phase {
-    const int k = i++;
-    if (k < nm)
-      return Phase{opsL + (int64_t)(OP_M2M + k) * PD * PD,
-                   crow >= 0 ? mult + (int64_t)(crow + k) * PD : nullptr, false};
-    return Phase{opsL + (int64_t)(OP_PINV1 + (k - nm)) * PD * PD, nullptr, true};
-  };
-  run_phases<PD>(nm + 2, acc, buf[0], buf[1], next);
-  // total equivalent charge of the box (used by the mixed-precision M2L)
-  double part = 0.0;
-#pragma unroll
-  for (int rb = 0; rb < PD / 16; ++rb)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) part += acc[rb][v];
-  part += __shfl_xor(part, 16, 64);
-  part += __shfl_xor(part, 32, 64);
-  if (active) {
-    store_acc<PD>(acc, mult + r * PD);
-    if ((l >> 4) == 0) qs[r] = part;
-  }
-  if (m32) {
-    float* row32 = m32 + ((int64_t)blockIdx.y * dstride + r) * PD;
-#pragma unroll
-    for (int rb = 0; rb < PD / 16; ++rb) {
-      const double v[4] = {acc[rb][0], acc[rb][1], acc[rb][2], acc[rb][3]};
-      store_m32<PD>(row32, rb, v, active);
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // M2L of all levels in one launch (the translations only read multipoles).
 // Blocks of a level are tiled by child position c so that all columns of a
@@ -1039,13 +888,13 @@ __global__ __launch_bounds__(kM2LThreads * RS) void k_m2l_all(LevelTable lt,
 // Mixed-precision M2L: PLE = sum_s [ R_s q_src (FP32 MFMA, FP32 accumulation
 //                                                within the slot)
 //                               + c_s * qs_src  (FP64) ], slots summed in FP64.
-// FRAME (Stokeslet fields): the two fields D_i whose definition holds the
+// Stokeslet fields (k_m2l_frame_f32): the two fields D_i whose definition holds the
 // position X relative to the root centre are translated in the target box's
 // frame instead, D_i^(c) = D_i + c_i D_2 with c the target centre (formed in
 // FP64 from the source's D_i and D_2 rows before rounding), so that the FP32
-// operands carry no c_i D_2 part; the downward pass returns to the root
-// frame in FP64 (k_local_level), where that part cancels exactly against
-// X_i(t) D_2 at the targets.
+// operands carry no c_i D_2 part; the kernel's last step returns to the root
+// frame in FP64, where that part cancels exactly against X_i(t) D_2 at the
+// targets.
 // v_mfma_f32_16x16x4f32: lane l holds A[l%16][l/16], B[l/16][l%16] and
 // D[4(l/16) + v][l%16].
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -1417,9 +1266,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
   }
   // waves 1 .. NW-1 hand their sums to wave 0, which adds them in wave order
+  // and returns fields 0 and 1 to the root frame: PLE_i -= c_i PLE_2
+  d4 sum2[RB];
 #pragma unroll
-  for (int f = 0; f < NF; ++f) {
-    if (f > 0) __syncthreads();
+  for (int f = NF - 1; f >= 0; --f) {
+    if (f < NF - 1) __syncthreads();
     if (w > 0) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
@@ -1429,6 +1280,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     __syncthreads();
     if (w == 0 && active) {
       double* rowp = ple + (f * nstride + g) * PD;
+      const double ct = f == 0 ? ctx : cty;
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -1436,6 +1288,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
           double sum = acc64[f][rb][v];
 #pragma unroll
           for (int ww = 0; ww < NW - 1; ++ww) sum += red[ww][16 * rb + 4 * kq + v][col];
+          if (f == NF - 1) sum2[rb][v] = sum;
+          else sum = __builtin_fma(-ct, sum2[rb][v], sum);
           rowp[16 * rb + 4 * kq + v] = sum;
         }
     }
@@ -1451,7 +1305,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 //
 // What bounds it: the FP64 matrix cores, once their operands arrive.  They
 // come straight from L2 into registers, with no LDS stage and no barrier per
-// slot: the operator from a copy in MFMA operand order (k_m2l_pack: one wave
+// slot: the operator from a copy in MFMA operand order (k_ops_pack: one wave
 // load reads 1 KB in one piece; row-major blocks cost 16 pieces of 64 bytes),
 // the multipoles by 16-byte loads.  Step 2 m + h of lane group kq multiplies
 // k = 8 m + 2 kq + h, so a 16-byte load of either operand feeds two steps.
@@ -1647,81 +1501,221 @@ __global__ __launch_bounds__(64 * kM2LF64Waves) void k_m2l_f64(
   }
 }
 
-// Operator copy of k_m2l_f64 for one level: dv2 entry
-// ((slot KP + m) RB + rb) 64 + lane holds M[16 rb + lane % 16][8 m + 2 (lane / 16) + {0, 1}],
-// or, when the last pair is one step (odd), column 8 m + lane / 16 and 0 for m = KP - 1.
-__global__ __launch_bounds__(256) void k_m2l_pack(const double* __restrict__ ops, int PD, int PE,
+// Blocks of a level's packed operators, each PE x PE in MFMA operand order.
+enum {
+  OPP_M2L = 0,      // 40 blocks in slot order
+  OPP_PINV1 = 40,
+  OPP_PINV2 = 41,
+  OPP_M2M = 42,     // 4 blocks
+  OPP_L2L = 46,     // 4 blocks
+  OPP_NBLK = 50,
+};
+// The packed operators of one level: dv2 entry ((blk KP + m) RB + rb) 64 +
+// lane holds row 16 rb + lane % 16 of the block, columns 8 m + 2 (lane / 16) +
+// {0, 1}; of the pseudo-inverse factors (whose B operand is a product's
+// result), columns 8 m + lane / 16 + {0, 4}; of the M2L blocks when the last
+// pair of k-steps is one step (odd), column 8 m + lane / 16 and 0 for m = KP - 1.
+__global__ __launch_bounds__(256) void k_ops_pack(const double* __restrict__ ops, int PD, int PE,
                                                   bool odd, dv2* __restrict__ out) {
   const int RB = PE / 16, KP = PE / 8;
-  const int n = kNumM2L * KP * RB * 64;
+  const int n = OPP_NBLK * KP * RB * 64;
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= n) return;
-  const int lane = e & 63, rb = (e >> 6) % RB, m = (e >> 6) / RB % KP, slot = (e >> 6) / RB / KP;
-  const double* M = ops + (int64_t)(OP_M2L + slot) * PD * PD;
-  const double* row = M + (16 * rb + (lane & 15)) * PD + 8 * m;
-  out[e] = odd && m == KP - 1 ? dv2{row[lane >> 4], 0.0}
-                              : *reinterpret_cast<const dv2*>(row + 2 * (lane >> 4));
+  const int lane = e & 63, rb = (e >> 6) % RB, m = (e >> 6) / RB % KP, blk = (e >> 6) / RB / KP;
+  const int src = blk < OPP_PINV1 ? OP_M2L + blk
+                  : blk < OPP_M2M ? OP_PINV1 + blk - OPP_PINV1
+                  : blk < OPP_L2L ? OP_M2M + blk - OPP_M2M : OP_L2L + blk - OPP_L2L;
+  const double* row = ops + (int64_t)src * PD * PD + (16 * rb + (lane & 15)) * PD + 8 * m;
+  const int kq = lane >> 4;
+  if (src == OP_PINV1 || src == OP_PINV2) out[e] = dv2{row[kq], row[kq + 4]};
+  else if (odd && blk < OPP_PINV1 && m == KP - 1) out[e] = dv2{row[kq], 0.0};
+  else out[e] = *reinterpret_cast<const dv2*>(row + 2 * kq);
 }
 
 // ---------------------------------------------------------------------------
-// Downward, one level: PLE += L2L(parent LE) (parent width's L2LC,
-// fmm.py:142,162), LE = pinv2 * (pinv1 * PLE)  (fmm.py:156).  Tiled by child
-// position c like the M2L.
-// Return of the Stokeslet fields D_0, D_1 from the target-box frame of the
-// FP32 M2L to the root frame: PLE_i -= c_i PLE_2, c the box centre relative to
-// the root centre (xmid null: no change).
-struct FrameFix {
-  const double* xmid;
-  const double* ymid;
-  double c0x, c0y;
-  // centre coordinate `field` (0: x, 1: y) of node g in the root frame
-  __device__ __forceinline__ double centre(int g, int field) const {
-    return field == 0 ? xmid[g] - c0x : ymid[g] - c0y;
+// Level kernels for large levels.  A wave takes 16 boxes and all their PE
+// rows: a product's result (lane (col, kq): rows 16 rb + 4 v + kq) is the next
+// one's B operand for the k-steps 4 rb + v in natural order, so the three
+// chained products of a level stay in registers, and a wave of boxes without
+// children skips the M2M products.  The operators stream from L2 in MFMA
+// operand order (k_ops_pack) as in k_m2l_f64, a few k-step pairs ahead, across
+// the products.  Against 64 boxes per block sharing operators staged in LDS,
+// with a barrier per product (bound by those, and by M2M products that most
+// boxes of an adaptive level do not need): upward levels of 20K rows 40.5 ->
+// 31.4 us, of 65K 36.5 -> 31.4, downward ones of 30K to 59K nodes 34 .. 42 ->
+// 25 .. 36, three Stokeslet fields of 41K nodes 125 -> 103 and 86 -> 69.
+template <int PE>
+struct LevelWave {
+  static constexpr int RB = PE / 16, KP = PE / 8, D = KP / 2;
+  // dv2 entries of one operator block
+  static constexpr int kBlock = KP * RB * 64;
+  dv2 a[D][RB];
+  d4 acc[RB];
+  __device__ __forceinline__ void start(const dv2* __restrict__ pa) {
+#pragma unroll
+    for (int m = 0; m < D; ++m)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) a[m][rb] = pa[(m * RB + rb) * 64];
+  }
+  // acc += A b, A at pa; the next product's operator at pan
+  __device__ __forceinline__ void product(const dv2 (&b)[KP], const dv2* __restrict__ pa,
+                                          const dv2* __restrict__ pan) {
+#pragma unroll
+    for (int m = 0; m < KP; ++m) {
+      const int r = m % D;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r][rb][h], b[m][h], acc[rb], 0, 0, 0);
+      const dv2* q = m + D < KP ? pa : pan;
+      const int mn = (m + D) % KP;
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) a[r][rb] = q[(mn * RB + rb) * 64];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // acc <- A acc (operator in natural k order)
+  __device__ __forceinline__ void chain(const dv2* __restrict__ pa, const dv2* __restrict__ pan) {
+    dv2 b[KP];
+#pragma unroll
+    for (int m = 0; m < KP; ++m) b[m] = dv2{acc[m >> 1][2 * (m & 1)], acc[m >> 1][2 * (m & 1) + 1]};
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc[rb] = d4{0.0, 0.0, 0.0, 0.0};
+    product(b, pa, pan);
+  }
+  // entries 8 m + 2 kq + {0, 1} of a source row (M2M, L2L operators)
+  static __device__ __forceinline__ void load_b(dv2 (&b)[KP], const double* __restrict__ row) {
+    const double* q = row + 2 * ((threadIdx.x & 63) >> 4);
+#pragma unroll
+    for (int m = 0; m < KP; ++m) b[m] = *reinterpret_cast<const dv2*>(q + 8 * m);
+  }
+  template <int PD>
+  __device__ __forceinline__ void store(double* __restrict__ row) const {
+    const int kq = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) row[16 * rb + 4 * v + kq] = acc[rb][v];
+    if (PE < PD)
+      for (int k = PE + kq; k < PD; k += 4) row[k] = 0.0;
   }
 };
+constexpr int kLevelWaves = 4;   // waves per block
 
-template <int PD>
-__global__ __launch_bounds__(256) void k_local_level(int g0, int ngroups, int do_l2l,
-                                                    const int* __restrict__ flags,
-                                                    const int* __restrict__ parent,
-                                                    const double* __restrict__ ple,
-                                                    const double* __restrict__ opsL,
-                                                    const double* __restrict__ opsParent,
-                                                    double* __restrict__ le, int64_t nstride,
-                                                    FrameFix fx) {
-  const double* ple2 = ple + 2 * nstride * PD;   // field 2 (FrameFix)
+// Upward, one level: rows [row0, row0 + nrows), density blockIdx.y.  check =
+// S2M result (leaves) or M2M of the four children (parents), then multipole =
+// pinv2 * (pinv1 * check)  (fmm.py:98-122).  opsL: the level's packed
+// operators.
+template <int PD, int PE>
+__global__ __launch_bounds__(64 * kLevelWaves) void k_mult_level(
+    int64_t row0, int nrows, int with_m2m, const int2* __restrict__ rowinfo,
+    const double* __restrict__ check, const dv2* __restrict__ opsL, double* __restrict__ mult,
+    double* __restrict__ qs, int64_t dstride, float* __restrict__ m32) {
+  typedef LevelWave<PE> W;
+  check += (int64_t)blockIdx.y * dstride * PD;
+  mult += (int64_t)blockIdx.y * dstride * PD;
+  const int l = threadIdx.x & 63, col = l & 15, kq = l >> 4;
+  const int rl0 = (blockIdx.x * kLevelWaves + (int)(threadIdx.x >> 6)) * 16;
+  if (rl0 >= nrows) return;   // wave-uniform
+  const bool active = rl0 + col < nrows;
+  const int64_t r = row0 + (active ? rl0 + col : rl0);
+  const int2 ri = rowinfo[r];
+  W L;
+  double ck[W::RB][4];
+#pragma unroll
+  for (int rb = 0; rb < W::RB; ++rb)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) ck[rb][v] = check[r * PD + 16 * rb + 4 * v + kq];
+  const int crow = with_m2m ? ri.x : -1;
+  const bool up = __ballot(crow >= 0) != 0;
+  const dv2* ops = opsL + l;
+  const dv2* p1 = ops + OPP_PINV1 * W::kBlock;
+  const dv2* p2 = ops + OPP_PINV2 * W::kBlock;
+  const dv2* pm = ops + OPP_M2M * W::kBlock;
+  L.start(up ? pm : p1);
+#pragma unroll
+  for (int rb = 0; rb < W::RB; ++rb)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) L.acc[rb][v] = (ri.y & NF_UP) ? ck[rb][v] : 0.0;
+  if (up) {
+    for (int c = 0; c < 4; ++c) {
+      dv2 b[W::KP];
+      W::load_b(b, crow >= 0 ? mult + (int64_t)(crow + c) * PD : c_zero_row);
+      L.product(b, pm + c * W::kBlock, c < 3 ? pm + (c + 1) * W::kBlock : p1);
+    }
+  }
+  L.chain(p1, p2);
+  L.chain(p2, p2);
+  if (active) L.template store<PD>(mult + r * PD);
+  if (qs) {   // total equivalent charge of the box (FP32 M2L)
+    double part = 0.0;
+#pragma unroll
+    for (int rb = 0; rb < W::RB; ++rb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) part += L.acc[rb][v];
+    part += __shfl_xor(part, 16, 64);
+    part += __shfl_xor(part, 32, 64);
+    if (active && kq == 0) qs[(int64_t)blockIdx.y * dstride + r] = part;
+  }
+  if (m32) {
+    float* row32 = m32 + ((int64_t)blockIdx.y * dstride + r) * PD;
+#pragma unroll
+    for (int rb = 0; rb < PD / 16; ++rb) {
+      const d4 a = rb < W::RB ? L.acc[rb < W::RB ? rb : 0] : d4{0.0, 0.0, 0.0, 0.0};
+      const double v[4] = {a[0], a[1], a[2], a[3]};
+      store_m32<PD>(row32, rb, v, active);
+    }
+  }
+}
+
+// Downward, one level: PLE += L2L(parent LE) (parent width's L2LC,
+// fmm.py:142,162), LE = pinv2 * (pinv1 * PLE)  (fmm.py:156).  A wave takes 16
+// boxes of one child position c, density blockIdx.y.  perm: the level's M2L
+// column order on adaptive trees (k_m2l_order), which puts the fake nodes of a
+// chunk last, so that most waves of fake nodes (half of the nodes of a tree
+// over a curve) hold nothing else and only write zeros.
+template <int PD, int PE>
+__global__ __launch_bounds__(64 * kLevelWaves) void k_local_level(
+    int g0, int ngroups, const int* __restrict__ perm, const int* __restrict__ flags, const int* __restrict__ parent,
+    const double* __restrict__ ple, const dv2* __restrict__ opsL,
+    const dv2* __restrict__ opsParent, double* __restrict__ le, int64_t nstride) {
+  typedef LevelWave<PE> W;
   ple += (int64_t)blockIdx.y * nstride * PD;
   le += (int64_t)blockIdx.y * nstride * PD;
-  __shared__ __attribute__((aligned(16))) double buf[2][PD * Mfma<PD>::LDA];
-  const int c = blockIdx.x & 3, tile = blockIdx.x >> 2;
-  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int q = tile * 64 + w * 16 + (l & 15);
-  const int g = g0 + 4 * q + c;
-  const bool active = q < ngroups && !(flags[q < ngroups ? g : g0] & NF_FAKE);
-  d4 acc[PD / 16];
-  load_acc<PD>(acc, active ? ple + (int64_t)g * PD : nullptr);
-  if (fx.xmid && blockIdx.y < 2 && active) {
-    d4 acc2[PD / 16];
-    load_acc<PD>(acc2, ple2 + (int64_t)g * PD);
-    const double ct = fx.centre(g, blockIdx.y);
-#pragma unroll
-    for (int rb = 0; rb < PD / 16; ++rb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[rb][v] = __builtin_fma(-ct, acc2[rb][v], acc[rb][v]);
+  const int l = threadIdx.x & 63, col = l & 15, kq = l >> 4;
+  const int c = blockIdx.x & 3;
+  const int q0 = ((blockIdx.x >> 2) * kLevelWaves + (int)(threadIdx.x >> 6)) * 16;
+  if (q0 >= ngroups) return;   // wave-uniform
+  const bool own = q0 + col < ngroups;
+  const int qq = own ? q0 + col : q0;
+  const int g = g0 + 4 * (perm ? perm[c * ngroups + qq] : qq) + c;
+  const bool active = !(flags[g] & NF_FAKE);
+  if (__ballot(active) == 0) {   // fake nodes only: zeros
+    if (own)
+      for (int k = kq; k < PD; k += 4) le[(int64_t)g * PD + k] = 0.0;
+    return;
   }
-  const int pg = (active && do_l2l) ? parent[g] : -1;
-  const int nl = do_l2l ? 1 : 0;
-  int i = 0;
-  auto next = [&]() -> Phase {
-    const int k = i++;
-    if (k < nl)
-      return Phase{opsParent + (int64_t)(OP_L2L + c) * PD * PD,
-                   pg >= 0 ? le + (int64_t)pg * PD : nullptr, false};
-    return Phase{opsL + (int64_t)(OP_PINV1 + (k - nl)) * PD * PD, nullptr, true};
-  };
-  run_phases<PD>(nl + 2, acc, buf[0], buf[1], next);
-  // zeros for the fake nodes (their columns are zero)
-  if (q < ngroups) store_acc<PD>(acc, le + (int64_t)g * PD);
+  const int par = parent[g];
+  const dv2* pl = opsParent + l + (OPP_L2L + c) * W::kBlock;
+  const dv2* p1 = opsL + l + OPP_PINV1 * W::kBlock;
+  const dv2* p2 = opsL + l + OPP_PINV2 * W::kBlock;
+  W L;
+  L.start(pl);
+#pragma unroll
+  for (int rb = 0; rb < W::RB; ++rb)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) L.acc[rb][v] = ple[(int64_t)g * PD + 16 * rb + 4 * v + kq];
+#pragma unroll
+  for (int rb = 0; rb < W::RB; ++rb)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) L.acc[rb][v] = active ? L.acc[rb][v] : 0.0;
+  dv2 b[W::KP];
+  W::load_b(b, active ? le + (int64_t)par * PD : c_zero_row);
+  L.product(b, pl, p1);
+  L.chain(p1, p2);
+  L.chain(p2, p2);
+  if (own) L.template store<PD>(le + (int64_t)g * PD);
 }
 
 // ---------------------------------------------------------------------------
@@ -1875,9 +1869,8 @@ __device__ __forceinline__ void local_small_unit(
     int bx, int by, int g0, int ngroups, int do_l2l, const int* __restrict__ flags,
     const int* __restrict__ parent, const double* __restrict__ ple,
     const double* __restrict__ opsL, const double* __restrict__ opsParent,
-    double* __restrict__ le, int64_t nstride, const FrameFix& fx) {
+    double* __restrict__ le, int64_t nstride) {
   __shared__ __attribute__((aligned(16))) double bbuf[2][16][PD + kSmallPad];
-  const double* ple2 = ple + 2 * nstride * PD;   // field 2 (FrameFix)
   ple += (int64_t)by * nstride * PD;
   le += (int64_t)by * nstride * PD;
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1893,12 +1886,6 @@ __device__ __forceinline__ void local_small_unit(
   const double* src = ple + (int64_t)gs * PD;
 #pragma unroll
   for (int v = 0; v < 4; ++v) acc[v] = src[16 * w + 4 * v + kq];
-  if (fx.xmid && by < 2) {
-    const double* src2 = ple2 + (int64_t)gs * PD;
-    const double ct = fx.centre(gs, by);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[v] = __builtin_fma(-ct, src2[16 * w + 4 * v + kq], acc[v]);
-  }
 #pragma unroll
   for (int v = 0; v < 4; ++v) acc[v] = active ? acc[v] : 0.0;
   const int pg = (active && do_l2l) ? par : -1;
@@ -1925,9 +1912,9 @@ __global__ __launch_bounds__(64 * (PD / 16)) void k_local_level_small(
     int g0, int ngroups, int do_l2l, const int* __restrict__ flags,
     const int* __restrict__ parent, const double* __restrict__ ple,
     const double* __restrict__ opsL, const double* __restrict__ opsParent,
-    double* __restrict__ le, int64_t nstride, FrameFix fx) {
+    double* __restrict__ le, int64_t nstride) {
   local_small_unit<PD>(blockIdx.x, blockIdx.y, g0, ngroups, do_l2l, flags, parent, ple, opsL,
-                       opsParent, le, nstride, fx);
+                       opsParent, le, nstride);
 }
 
 // Levels with at most this many multipole rows (or 4 x this many boxes) use
@@ -3534,7 +3521,7 @@ static bool m2l_in_fp32(const Plan& P) {
 // The dense FP64 M2L of the levels in lt.
 static int m2l_pe(int p) { return (int)ceil_div(p, 16) * 16; }
 static bool m2l_odd(int p) { return (p - 1) % 8 < 4; }
-static int64_t opsm_per_level(int p) { return (int64_t)kNumM2L * m2l_pe(p) * m2l_pe(p); }
+static int64_t opsm_per_level(int p) { return (int64_t)OPP_NBLK * m2l_pe(p) * m2l_pe(p); }
 
 template <int PD, int PE, int NCG, int RBW>
 static void m2l_f64_run(Plan& P, LevelTable& lt, hipStream_t s) {
@@ -3646,6 +3633,10 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
                      t.m2l.as<int>(), P.mult.as<double>(), P.ops.as<double>(), opsz,
                      P.ple.as<double>(), rstride, nstride);
   FMM_LAUNCH_CHECK();
+}
+
+static const dv2* packed_ops(const Plan& P, int level) {
+  return reinterpret_cast<const dv2*>(P.opsm.as<double>() + level * opsm_per_level(P.p));
 }
 
 typedef decltype(&k_s2m<32, KER_LAPLACE, false, 1>) S2MFn;
@@ -3762,10 +3753,12 @@ static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s
       FMM_LAUNCH_CHECK();
       continue;
     }
-    auto kern = PD == 32 ? k_mult_level<32> : k_mult_level<64>;
-    hipLaunchKernelGGL(kern, dim3(ceil_div(nrows, 64), nd), dim3(256), 0, s, r0, nrows,
-                       d < t.L - 1 ? 1 : 0, t.rowinfo.as<int2>(), P.check.as<double>(), opsL,
-                       P.mult.as<double>(), P.qs.as<double>(), rstride, m32);
+    auto kern = P.p <= 16 ? k_mult_level<32, 16> : P.p <= 32 ? k_mult_level<32, 32>
+                : P.p <= 48 ? k_mult_level<64, 48> : k_mult_level<64, 64>;
+    hipLaunchKernelGGL(kern, dim3(ceil_div(nrows, 16 * kLevelWaves), nd), dim3(64 * kLevelWaves), 0,
+                       s, r0, nrows, d < t.L - 1 ? 1 : 0, t.rowinfo.as<int2>(),
+                       P.check.as<double>(), packed_ops(P, d), P.mult.as<double>(),
+                       m2l_in_fp32(P) ? P.qs.as<double>() : nullptr, rstride, m32);
     FMM_LAUNCH_CHECK();
   }
   P.have_exp = false;
@@ -3790,10 +3783,6 @@ static void downward(Plan& P, hipStream_t s) {
   P.mark(FMM2D_PHASE_M2L, false, s);
   m2l_launch(P, T, 0, T.lt.nlev, s);
   P.mark(FMM2D_PHASE_M2L, true, s);
-  FrameFix fx{nullptr, nullptr, 0.0, 0.0};
-  if (P.kernel_id == KER_STOKES && m2l_in_fp32(P))   // the FP32 M2L ran in box frames
-    fx = FrameFix{t.xmid.as<double>(), t.ymid.as<double>(), t.xmin + 0.5 * t.w0,
-                  t.ymin + 0.5 * t.w0};
   for (int d = 2; d < t.L; ++d) {
     const int ngroups = (int)(t.lev[d].n_nodes / 4);
     if (ngroups == 0) continue;
@@ -3803,15 +3792,17 @@ static void downward(Plan& P, hipStream_t s) {
       hipLaunchKernelGGL(ks, dim3(4 * ceil_div(ngroups, 16), nd), dim3(64 * (PD / 16)), 0, s,
                          (int)t.lev[d].node_off, ngroups, d >= 3 ? 1 : 0, t.flags.as<int>(),
                          t.parent.as<int>(), P.ple.as<double>(), opsL, opsL - opsz,
-                         P.le.as<double>(), nstride, fx);
+                         P.le.as<double>(), nstride);
       FMM_LAUNCH_CHECK();
       continue;
     }
-    auto kern = PD == 32 ? k_local_level<32> : k_local_level<64>;
-    hipLaunchKernelGGL(kern, dim3(4 * ceil_div(ngroups, 64), nd), dim3(256), 0, s,
-                       (int)t.lev[d].node_off, ngroups, d >= 3 ? 1 : 0, t.flags.as<int>(),
-                       t.parent.as<int>(), P.ple.as<double>(), opsL, opsL - opsz,
-                       P.le.as<double>(), nstride, fx);
+    auto kern = P.p <= 16 ? k_local_level<32, 16> : P.p <= 32 ? k_local_level<32, 32>
+                : P.p <= 48 ? k_local_level<64, 48> : k_local_level<64, 64>;
+    hipLaunchKernelGGL(kern, dim3(4 * ceil_div(ngroups, 16 * kLevelWaves), nd),
+                       dim3(64 * kLevelWaves), 0, s, (int)t.lev[d].node_off, ngroups,
+                       T.adaptive ? P.m2lperm.as<int>() + T.lt.poff[d - 2] : nullptr,
+                       t.flags.as<int>(), t.parent.as<int>(), P.ple.as<double>(),
+                       packed_ops(P, d), packed_ops(P, d - 1), P.le.as<double>(), nstride);
     FMM_LAUNCH_CHECK();
   }
   P.have_exp = true;
@@ -4323,17 +4314,14 @@ int fmm2d_set_operators(void* plan, int level, const double* dev_ops, int64_t n,
   }
   FMM_HIP(hipMemcpyAsync(P->ops.as<double>() + level * opsz, dev_ops, opsz * sizeof(double),
                          hipMemcpyDeviceToDevice, s));
-  // the dense FP64 M2L's copy in operand order (scalar KIFMM plans of the
-  // mixed forms always run the FP32 M2L)
-  if (P->precision == fmm::PREC_FP64 || P->cheb || P->kernel_id == fmm::KER_STOKES) {
-    const int64_t msz = fmm::opsm_per_level(P->p);
-    P->opsm.ensure(fmm::kMaxLevels * msz * sizeof(double));
-    hipLaunchKernelGGL(fmm::k_m2l_pack, dim3(fmm::grid256(msz / 2)), dim3(256), 0, s,
-                       P->ops.as<double>() + level * opsz, P->PD, fmm::m2l_pe(P->p),
-                       fmm::m2l_odd(P->p),
-                       reinterpret_cast<fmm::dv2*>(P->opsm.as<double>() + level * msz));
-    FMM_LAUNCH_CHECK();
-  }
+  // the copy in operand order
+  const int64_t msz = fmm::opsm_per_level(P->p);
+  P->opsm.ensure(fmm::kMaxLevels * msz * sizeof(double));
+  hipLaunchKernelGGL(fmm::k_ops_pack, dim3(fmm::grid256(msz / 2)), dim3(256), 0, s,
+                     P->ops.as<double>() + level * opsz, P->PD, fmm::m2l_pe(P->p),
+                     fmm::m2l_odd(P->p),
+                     reinterpret_cast<fmm::dv2*>(P->opsm.as<double>() + level * msz));
+  FMM_LAUNCH_CHECK();
   P->ops_set[level] = 1;
   ABI_END
 }
