@@ -391,10 +391,11 @@ struct PotAcc<KER_MODHELM> {
 // S2M: one wave per leaf (kEvalWaves leaves per block share the log table),
 // lane k = check point k on the large circle (helpers.py:159-173; the source
 // is taken relative to the box centre).  NS = kEvalWaves: the waves of a block
-// share a leaf, each taking a quarter of its sources.  Up to kSplitLeaves
-// leaves (one per SIMD) a leaf's wave has its SIMD to itself and waits for its
-// own loads: 256 leaves of 195 sources 29.5 -> 9.6 us, 64 leaves of 31 sources 7.8 -> 4.6.
-constexpr int64_t kSplitLeaves = 4 * kNumCUs;
+// share a leaf, each taking a quarter of its sources: up to kSplitLeaves
+// leaves (16 per SIMD) a leaf's single wave mostly waits for its own loads
+// (256 leaves of 195 sources 29.5 -> 9.6 us, 64 of 31 sources 7.8 -> 4.6, 7K
+// leaves of 14 dipoles 23.0 -> 12.0).
+constexpr int64_t kSplitLeaves = 64 * kNumCUs;
 // DIP: sources also carry a dipole moment q (the double layer of the Laplace
 // kernel, (q.d)/d^2/(2 pi) with d = check point - source).
 template <int PD, int KER, bool DIP, int NS>
