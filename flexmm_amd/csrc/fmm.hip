@@ -314,48 +314,63 @@ __device__ __forceinline__ double helm_lnx2(double d2, const double2* __restrict
   log_split(d2, tab, e, t);
   return __builtin_fma(0.5, __builtin_fma(e, kLn2, t), h.lnk2);
 }
+// Terms of the series that leave out less than 2^-60 of each sum: 8 for q <=
+// 1/16, 10 for q <= 1/4 (next terms q^8/(8!)^2 = 1.4e-19, q^10/(10!)^2 =
+// 7.2e-20).  Near pairs have q = (k d/2)^2 far below 1 (at most 2 (k w)^2 in
+// boxes of width w); the number is chosen per wave, so that no lane's branch
+// adds to another's: gradient evaluation of 2.5e8 pairs
+// 932 -> 714 us (K1 has a third class; K0 alone gains nothing from it).
+constexpr double kHelmQ8 = 0.0625, kHelmQ10 = 0.25;
+template <int N>
+__device__ __forceinline__ double helm_k0_series(double q, double d2,
+                                                 const double2* __restrict__ tab,
+                                                 const HelmConsts& h) {
+  const BesselSeries& c = bessel_series();
+  double i0 = c.i0[N - 1], s = c.s0[N - 1];
+#pragma unroll
+  for (int j = N - 2; j >= 0; --j) {
+    i0 = __builtin_fma(i0, q, c.i0[j]);
+    s = __builtin_fma(s, q, c.s0[j]);
+  }
+  return __builtin_fma(-(helm_lnx2(d2, tab, h) + kEulerGamma), i0, s);
+}
 __device__ __forceinline__ double helm_k0(double d2, const double2* __restrict__ tab,
                                           const HelmConsts& h) {
   const double q = h.k2q * d2;
-  if (q <= 1.0) {
-    const BesselSeries& c = bessel_series();
-    constexpr int n = kBesselSeriesTerms - 1;
-    double i0 = c.i0[n], s = c.s0[n];
-#pragma unroll
-    for (int j = n - 1; j >= 0; --j) {
-      i0 = __builtin_fma(i0, q, c.i0[j]);
-      s = __builtin_fma(s, q, c.s0[j]);
-    }
-    return __builtin_fma(-(helm_lnx2(d2, tab, h) + kEulerGamma), i0, s);
-  }
+  if (__ballot(!(q <= kHelmQ8)) == 0) return helm_k0_series<8>(q, d2, tab, h);
+  if (q <= 1.0) return helm_k0_series<kBesselSeriesTerms>(q, d2, tab, h);
   return bessel_k0_large(h.k * __builtin_sqrt(d2));
 }
 // K0 and k K1(x)/r; id2 = 1/d2
+template <int N>
+__device__ __forceinline__ void helm_k01_series(double q, double d2, double id2,
+                                                const double2* __restrict__ tab,
+                                                const HelmConsts& h, double& k0, double& gk1) {
+  // K0's two sums take their coefficients from constant memory (scalar
+  // operands), K1's are compile-time values in vector registers: fewer
+  // register moves per pair than all in registers (gradient evaluation of
+  // 2.2e8 pairs 1.33 -> 1.22 ms), and all in constant memory exceeds the
+  // scalar registers
+  const BesselSeries& c = kBesselSeries;
+  const BesselSeries& cm = bessel_series();
+  double i0 = cm.i0[N - 1], s0 = cm.s0[N - 1], i1 = c.i1[N - 1], s1 = c.s1[N - 1];
+#pragma unroll
+  for (int j = N - 2; j >= 0; --j) {
+    i0 = __builtin_fma(i0, q, cm.i0[j]);
+    s0 = __builtin_fma(s0, q, cm.s0[j]);
+    i1 = __builtin_fma(i1, q, c.i1[j]);
+    s1 = __builtin_fma(s1, q, c.s1[j]);
+  }
+  const double lg = helm_lnx2(d2, tab, h);
+  k0 = __builtin_fma(-(lg + kEulerGamma), i0, s0);
+  gk1 = __builtin_fma(h.k2q, __builtin_fma(2.0 * lg, i1, -s1), id2);
+}
 __device__ __forceinline__ void helm_k01(double d2, double id2, const double2* __restrict__ tab,
                                          const HelmConsts& h, double& k0, double& gk1) {
   const double q = h.k2q * d2;
-  if (q <= 1.0) {
-    // K0's two sums take their coefficients from constant memory (scalar
-    // operands), K1's are compile-time values in vector registers: fewer
-    // register moves per pair than all in registers (gradient evaluation of
-    // 2.2e8 pairs 1.33 -> 1.22 ms), and all in constant memory exceeds the
-    // scalar registers
-    const BesselSeries& c = kBesselSeries;
-    const BesselSeries& cm = bessel_series();
-    constexpr int n = kBesselSeriesTerms - 1;
-    double i0 = cm.i0[n], s0 = cm.s0[n], i1 = c.i1[n], s1 = c.s1[n];
-#pragma unroll
-    for (int j = n - 1; j >= 0; --j) {
-      i0 = __builtin_fma(i0, q, cm.i0[j]);
-      s0 = __builtin_fma(s0, q, cm.s0[j]);
-      i1 = __builtin_fma(i1, q, c.i1[j]);
-      s1 = __builtin_fma(s1, q, c.s1[j]);
-    }
-    const double lg = helm_lnx2(d2, tab, h);
-    k0 = __builtin_fma(-(lg + kEulerGamma), i0, s0);
-    gk1 = __builtin_fma(h.k2q, __builtin_fma(2.0 * lg, i1, -s1), id2);
-    return;
-  }
+  if (__ballot(!(q <= kHelmQ8)) == 0) return helm_k01_series<8>(q, d2, id2, tab, h, k0, gk1);
+  if (__ballot(!(q <= kHelmQ10)) == 0) return helm_k01_series<10>(q, d2, id2, tab, h, k0, gk1);
+  if (q <= 1.0) return helm_k01_series<kBesselSeriesTerms>(q, d2, id2, tab, h, k0, gk1);
   const double r = __builtin_sqrt(d2);
   double k1;
   bessel_k01_large(h.k * r, k0, k1);
