@@ -1940,8 +1940,9 @@ constexpr int kSmallLevelRows = 4096;
 // ---------------------------------------------------------------------------
 // Targets: locate, count per evaluation box, scatter into box order.
 // Node lookup by (depth, cell code) for target location: direct on a full
-// level, a dense table on the other levels where the tree build made one,
-// else a binary search in the level's sorted codes.
+// level, through the bitmap index on the others of a tree that has one; in a
+// deeper tree a dense table where the build made one, else a binary search in
+// the level's sorted codes.
 struct LocateTable {
   int L;
   int full_depth;   // a complete tree's leaf depth (evaluation box = leaf code), else -1
@@ -1950,10 +1951,12 @@ struct LocateTable {
   int64_t tab_off[kMaxLevels];
   const int* tab;
   const uint64_t* code;
+  BmIndex ix;       // pp null: no bitmap index
 };
 __device__ __forceinline__ int locate_node(const LocateTable& lt, int d, uint64_t c) {
   const int64_t nl = lt.levoff[d + 1] - lt.levoff[d];
   if (d < 16 && nl == ((int64_t)1 << (2 * d))) return lt.levoff[d] + (int)c;
+  if (lt.ix.pp) return lt.ix.node(d, c);
   if (lt.tab_off[d] >= 0) return lt.tab[lt.tab_off[d] + (int64_t)c];
   const uint64_t* a = lt.code + lt.levoff[d];
   int64_t lo = 0, hi = nl;
@@ -3940,6 +3943,7 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
     lt.tab_off[d] = d < (int)t.nidx_off.size() ? t.nidx_off[d] : -1;
   lt.tab = t.nidx.as<int>();
   lt.code = t.code.as<uint64_t>();
+  if (t.bm_index) lt.ix = t.index();
   hipLaunchKernelGGL(k_locate_count, dim3(grid256(nt)), dim3(256), 0, s, tx, ty, nt, lt,
                      t.flags.as<int>(), t.child.as<int>(), t.xmid.as<double>(),
                      t.ymid.as<double>(), t.evalid.as<int>(), w.tnode,

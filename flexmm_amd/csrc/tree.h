@@ -20,6 +20,37 @@ enum NodeFlag : int {
   NF_SOURCE = 64,    // holds at least one source
 };
 
+// Node index of trees of few levels (tree.hip): bit c of depth d's bitmap is
+// the cell with Morton code c, set when that cell's node has children.  pp
+// holds each word with the number of set bits before it in its block of
+// kBmBlock words, boff the number before each block; the children of the
+// node of rank r are the nodes 1 + 4 r .. 4 + 4 r.  Each depth starts at a
+// block: kBmBlock words up to depth 6, 4^d / 32 from depth 7.
+constexpr int kBmBlock = 256;
+__host__ __device__ constexpr int bm_wo(int d) {   // first word of depth d
+  return d <= 7 ? kBmBlock * d : 7 * kBmBlock + 512 * (((1 << (2 * (d - 7))) - 1) / 3);
+}
+struct BmIndex {
+  const uint2* pp;
+  const int* boff;
+#if defined(__HIPCC__)
+  // rank of cell c of depth d among the nodes with children, or -1
+  __device__ __forceinline__ int rank(int d, uint64_t c) const {
+    const int w = bm_wo(d) + (int)(c >> 5);
+    const uint2 v = pp[w];
+    const int b = boff[w / kBmBlock];
+    const uint32_t bit = 1u << (c & 31);
+    return (v.x & bit) ? b + (int)v.y + __popc(v.x & (bit - 1u)) : -1;
+  }
+  // node of cell c of level d, or -1
+  __device__ __forceinline__ int node(int d, uint64_t c) const {
+    if (d == 0) return 0;
+    const int r = rank(d - 1, c >> 2);
+    return r >= 0 ? 1 + 4 * r + (int)(c & 3) : -1;
+  }
+#endif
+};
+
 struct TreeLevel {
   int64_t node_off = 0;
   int64_t n_nodes = 0;
@@ -56,27 +87,27 @@ struct Tree {
   DevBuf crange;   // int2[9]: colleague q's source range [bot, top); (0, 0) when absent
   DevBuf xmid, ymid;
   DevBuf row;      // i32 multipole row (levels >= 2, sibling groups holding sources) or -1
-  DevBuf rownode;  // i32[n_rows] node of each row
   DevBuf rowinfo;  // int2[n_rows]: row of the node's first child (or -1), node flags
   std::vector<int64_t> row_off;  // first row of each level (size L+1)
   DevBuf m2l;      // i32[40] multipole rows of the M2L partners or -1 (real nodes, level >= 2)
   DevBuf evalid;   // i32 index among evaluation boxes (NF_LEAF) or -1
   DevBuf evalnode; // i32[n_eval]
   DevBuf upnodes;  // i32[n_up] nodes with NF_UP
-  DevBuf levoff;   // i32[L+1] node offsets on the device
 
   // work areas
   PrimWork pw;
-  DevBuf w_flag, w_rank, w_a, w_b, w_c, w_cnt;
+  DevBuf w_flag, w_rank, w_a, w_b, w_c, w_cnt, w_rng, w_wave;
   DevBuf w_gate;   // i32: the split counts confirm the guessed complete tree
   DevBuf w_bad;    // i32 per key block: it holds a non-finite coordinate
-  HostBuf h_cnt;
   HostBuf h_up;    // pinned staging for small host->device uploads
   std::vector<int64_t> s_off;   // host offsets of the split-cell lists per depth
   DevBuf s_all, sref_all;       // u64 split-cell codes per depth (concatenated)
   DevBuf bal_bm, bal_pc;        // balance: cell bitmaps per depth, popcount scan
   DevBuf nidx;                  // dense node index of the non-full shallow levels
   std::vector<int64_t> nidx_off; // level d's table in nidx (per cell code), or -1
+  DevBuf bm, bm_pp, bm_boff;    // split cells as bitmaps, and the index of the nodes (BmIndex)
+  bool bm_index = false;        // the last build's nodes are found through that index
+  BmIndex index() const { return {bm_pp.as<uint2>(), bm_boff.as<int>()}; }
   DevBuf xy;                    // interleaved input coordinates (input order)
   DevBuf bal_k, bal_v, bal_f;   // balance below the bitmap depths: candidates
   std::vector<DevBuf> bal_lists;

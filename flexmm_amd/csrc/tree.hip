@@ -4,15 +4,16 @@
 // midpoint recurrence (tree.py:169-176, 301-304: xmid = xmin + w/2, children
 // start at xmid - w/2 or xmid, class 2*(x > xmid) + (y > ymid), tree.py:32-34),
 // so the classification of every point at every level is the reference's
-// bit for bit.  After a segmented MSD radix sort by key, the tree is a set of
-// sorted code lists:
+// bit for bit.  After a segmented MSD radix sort by key, the tree is three sets
+// of cells:
 //   S_d   cells of depth d that are split (refinement: > ncut points,
 //         tree.py:204; plus the minimal corner 2:1 balance, tree.py:529-541);
 //   X_d   real leaves with a split same-level neighbour (tree.py:542-553,
 //         385-397), which get four fake children;
 //   P_d   = S_d u X_d, the nodes of depth d that have children.
-// Level d+1 holds the children of P_d in Morton order.  Colleagues, parents,
-// point ranges and M2L partners are binary searches in these sorted lists.
+// Level d+1 holds the children of P_d in Morton order.  The sets are one bitmap
+// per depth in trees of up to kBmLevels levels and sorted code lists in deeper
+// ones; colleagues, parents, point ranges and M2L partners are lookups in them.
 #include "tree.h"
 #include "point_key.h"
 
@@ -51,13 +52,6 @@ __device__ __forceinline__ int64_t lower_bound_u64(const uint64_t* __restrict__ 
       hi = mid;
   }
   return lo;
-}
-
-template <class T>
-__device__ __forceinline__ int find_level(const T* __restrict__ off, int L, int64_t g) {
-  int d = 0;
-  while (d + 1 < L && g >= (int64_t)off[d + 1]) ++d;
-  return d;
 }
 
 // --- points ----------------------------------------------------------------
@@ -137,8 +131,8 @@ constexpr int kSplitRows = 64;
 // copy xy through perm: one 16-byte gather per point), its loads in flight
 // with the keys'.
 __global__ __launch_bounds__(1024) void k_split_pos(const uint64_t* __restrict__ keys, int n,
-                                                    int ncut, int* __restrict__ flag,
-                                                    int2* __restrict__ sc, int* __restrict__ rows,
+                                                    int ncut, int2* __restrict__ sc,
+                                                    int* __restrict__ rows,
                                                     const uint32_t* __restrict__ perm,
                                                     const double2* __restrict__ xy,
                                                     double* __restrict__ sx,
@@ -157,7 +151,6 @@ __global__ __launch_bounds__(1024) void k_split_pos(const uint64_t* __restrict__
     sy[i] = pt.y;
     s = (i == 0) ? -1 : min(clz64(k ^ kp) >> 1, kMaxDepth);
     c = ((int64_t)i + ncut < n) ? min(clz64(k ^ kc) >> 1, kMaxDepth - 1) : -1;
-    flag[i] = s < c;
     sc[i] = make_int2(s, c);
   }
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -207,6 +200,13 @@ __global__ __launch_bounds__(64) void k_split_counts(const int* __restrict__ row
     const bool all = __ballot(!ok) == 0ull;
     if (d == 0) *gate = all ? 1 : 0;
   }
+}
+
+// 1 at the split positions (those that start a split cell), for the scan
+__global__ __launch_bounds__(BS) void k_split_flags(const int2* __restrict__ sc, int n,
+                                                    int* __restrict__ flag) {
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i < n) flag[i] = sc[i].x < sc[i].y;
 }
 
 __global__ __launch_bounds__(BS) void k_compact_pos(const int* __restrict__ flag,
@@ -508,286 +508,567 @@ __global__ __launch_bounds__(BS) void k_p_scatter(const uint64_t* __restrict__ r
   p_kind[q] = kind[r];
 }
 
-// --- final node arrays ---------------------------------------------------------
-// Node index of the level-d cell with Morton code c, or -1: direct on a full
-// level, a table lookup on the other levels up to depth kIdxDepth (one int per
-// cell of the level, -1 where no node), else a binary search in the level's
-// sorted codes.
-constexpr int kIdxDepth = 11;   // tables of at most 4^12/3 ints (22 MB)
-struct NodeIdx {
-  const int* tab;
-  int64_t off[kMaxLevels];      // level d's table in tab, or -1
-};
-__device__ __forceinline__ int node_of(const uint64_t* __restrict__ code,
-                                       const int* __restrict__ levoff, const NodeIdx& ni, int d,
-                                       uint64_t c) {
-  const int64_t nl = levoff[d + 1] - levoff[d];
-  if (d < 16 && nl == ((int64_t)1 << (2 * d))) return levoff[d] + (int)c;
-  if (ni.off[d] >= 0) return ni.tab[ni.off[d] + (int64_t)c];
-  const int64_t pos = bsearch_u64(code + levoff[d], nl, c);
-  return pos >= 0 ? levoff[d] + (int)pos : -1;
-}
-__global__ __launch_bounds__(BS) void k_node_index(const uint64_t* __restrict__ code,
-                                                   const int* __restrict__ nlev, int nn,
-                                                   NodeIdx ni, int* __restrict__ tab) {
-  const int g = blockIdx.x * BS + threadIdx.x;
-  if (g >= nn) return;
-  const int64_t o = ni.off[nlev[g]];
-  if (o >= 0) tab[o + (int64_t)code[g]] = g;
+// --- trees of at most kBmLevels levels: cells as bitmaps ------------------------
+// Split cells down to depth kBmMaxD (every tree but those of points clustered
+// to 2^-12 of the box) are one bitmap per depth: bit c of depth d is cell c
+// (its Morton code), so a word is a block of 4 x 8 cells and the 3x3
+// neighbourhoods of the 2:1 balance and of the X-list are shifts and masks of
+// nine words, a cell's children a nibble, its rank among the nodes with
+// children a popcount.  The lists below (sorted codes, binary searches, sorted
+// scans) did the same work in 45 launches, copies and fills, most of them
+// bound by their launch or by a chain of dependent loads, and two more
+// counts read by the host: 270 us after the sort for 1M clustered points (58
+// thousand nodes), the bitmaps 95.  The lists stay for the deeper trees, whose
+// bitmaps would no longer fit in L2 (4^12 cells are 2 MB per bitmap and 4 MB
+// with the index).
+// Each depth's words start at a multiple of BS, so a block of BS words lies
+// in one depth.
+constexpr int kBmMaxD = 11;
+constexpr int kBmLevels = kBmMaxD + 2;
+static_assert(BS == kBmBlock, "the bitmap kernels take a block of words each");
+__host__ __device__ constexpr int bm_words(int d) { return d <= 2 ? 1 : 1 << (2 * d - 5); }
+constexpr int kBmWords = bm_wo(kBmMaxD + 1);
+constexpr int kBmBlocks = kBmWords / BS;
+static_assert(bm_wo(8) == bm_wo(7) + bm_words(7) && kBmBlocks < 1024,
+              "k_bm_sums scans the blocks' counts in one pass of 1024 threads");
+__device__ __forceinline__ int bm_depth_of(int w, int dmax) {
+  int d = 0;
+  while (d < dmax && w >= bm_wo(d + 1)) ++d;
+  return d;
 }
 
-// Source ranges of all nodes from the sorted keys: point i starts its cells
-// of depths s(i)+1.. and ends those of depths s(i+1)+1.. (s = common depth
-// with the previous key).  Cells without points keep -1 (fixed below).  A
-// cell exists only below an existing parent, so each walk stops at the first
-// depth without one.
+// The split cells of the refinement: position i starts those of depths
+// s(i)+1 .. c(i).  Depths below kBmMaxD are left out (the lists take such a
+// tree).
+__global__ __launch_bounds__(BS) void k_bm_mark_points(const uint64_t* __restrict__ keys,
+                                                       const int2* __restrict__ sc, int n,
+                                                       uint32_t* __restrict__ bm) {
+  const int i = xcd_block(blockIdx.x, gridDim.x, 0) * BS + threadIdx.x;
+  if (i >= n) return;
+  const int2 v = sc[i];
+  if (v.x >= v.y) return;
+  const uint64_t k = keys[i];
+  for (int d = v.x + 1; d <= min(v.y, kBmMaxD); ++d)
+    bm_set(bm + bm_wo(d), d == 0 ? 0 : k >> (64 - 2 * d));
+}
+
+// nibble j of v nonzero -> bit j; and back, bit j -> nibble j all ones
+__device__ __forceinline__ uint32_t nibbles_any(uint32_t v) {
+  v |= v >> 1;
+  v = (v | v >> 2) & 0x11111111u;
+  v = (v | v >> 3) & 0x03030303u;
+  v = (v | v >> 6) & 0x000F000Fu;
+  return (v | v >> 12) & 0xFFu;
+}
+__device__ __forceinline__ uint32_t nibbles_all(uint32_t b) {
+  b = (b | b << 12) & 0x000F000Fu;
+  b = (b | b << 6) & 0x03030303u;
+  b = (b | b << 3) & 0x11111111u;
+  return b * 15u;
+}
+// The cells of word w and their neighbours above and below in y; wm and wp
+// are the words at y - 8 and y + 8.  y's bits are bits 0, 2, 4 of the cell's
+// place in its word, x's bits 1 and 3: a step in y moves a cell by 1, 3 or 11
+// places by where the carry ends, and by 21 into the next word.
+__device__ __forceinline__ uint32_t bm_dilate_y(uint32_t wm, uint32_t w, uint32_t wp) {
+  const uint32_t up = (w & 0x55555555u) << 1 | (w & 0x0A0A0A0Au) << 3 | (w & 0x0000A0A0u) << 11;
+  const uint32_t dn = (w & 0xAAAAAAAAu) >> 1 | (w & 0x50505050u) >> 3 | (w & 0x05050000u) >> 11;
+  return w | up | dn | (wm & 0xA0A00000u) >> 21 | (wp & 0x00000505u) << 21;
+}
+// Word W of the 3x3 dilation of depth d's bitmap (d >= 1), whose word V is
+// word(V): words interleave the low bit of x before that of y.
+template <class F>
+__device__ __forceinline__ uint32_t bm_dilate(int d, int W, F word) {
+  if (d <= 2) {
+    const uint32_t y0 = bm_dilate_y(0, word(0), 0);
+    const uint32_t v = y0 | (y0 & 0x33333333u) << 2 | (y0 & 0x00CC00CCu) << 6 |
+                       (y0 & 0xCCCCCCCCu) >> 2 | (y0 & 0x33003300u) >> 6;
+    return v & (d == 1 ? 0xFu : 0xFFFFu);
+  }
+  uint32_t wx, wy;
+  demorton((uint64_t)W, &wy, &wx);
+  const int nx = 1 << (d - 2), ny = 1 << (d - 3);
+  uint32_t c[3][3], y[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      const int x = (int)wx + a - 1, yy = (int)wy + b - 1;
+      const bool in = x >= 0 && yy >= 0 && x < nx && yy < ny;
+      c[a][b] = in ? word((int)morton((uint32_t)yy, (uint32_t)x)) : 0u;
+    }
+#pragma unroll
+  for (int a = 0; a < 3; ++a) y[a] = bm_dilate_y(c[a][0], c[a][1], c[a][2]);
+  const uint32_t v = y[1];
+  return v | (v & 0x33333333u) << 2 | (v & 0x00CC00CCu) << 6 | (v & 0xCCCCCCCCu) >> 2 |
+         (v & 0x33003300u) >> 6 | (y[0] & 0xCC00CC00u) >> 10 | (y[2] & 0x00330033u) << 10;
+}
+
+// 2:1 balance: S_d |= N(parents(S_{d+1})), one thread per word of depth d,
+// from the deepest depth up.  An already balanced tree keeps its cells.
+__global__ __launch_bounds__(BS) void k_bm_balance(int d, uint32_t* __restrict__ bm) {
+  const int w = blockIdx.x * BS + threadIdx.x;
+  if (w >= bm_words(d)) return;
+  const uint4* next = reinterpret_cast<const uint4*>(bm + bm_wo(d + 1));
+  bm[bm_wo(d) + w] |= bm_dilate(d, w, [&](int V) {
+    const uint4 v = next[V];
+    return nibbles_any(v.x) | nibbles_any(v.y) << 8 | nibbles_any(v.z) << 16 |
+           nibbles_any(v.w) << 24;
+  });
+}
+// The depths dtop <= kBmLowD .. 1 in one block, their words (and those of
+// depth dtop + 1) in LDS: a launch per depth cost more than its work.  Depth 7
+// is the last whose words are at most one per thread; the loads of all depths
+// are in flight together (a loop over the depths took 23 us instead of 10).
+constexpr int kBmLowD = 7;
+__host__ __device__ constexpr int bm_lo(int d) {   // first LDS word of depth d >= 1
+  return d <= 2 ? d - 1 : 2 + 2 * (((1 << (2 * (d - 3))) - 1) / 3);
+}
+__global__ __launch_bounds__(1024) void k_bm_balance_low(int dtop, uint32_t* __restrict__ bm) {
+  constexpr int kLds = bm_lo(kBmLowD + 2), kPer = (kLds + 1023) / 1024;
+  __shared__ uint32_t sh[kLds];
+  const int ntop = bm_lo(dtop + 2);
+  int src[kPer];
+  uint32_t v[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = j * 1024 + threadIdx.x;
+    int d = 1;
+#pragma unroll
+    for (int e = 2; e <= kBmLowD + 1; ++e) d += i >= bm_lo(e) ? 1 : 0;
+    src[j] = bm_wo(d) + i - bm_lo(d);
+    v[j] = i < ntop ? bm[src[j]] : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j)
+    if (j * 1024 + threadIdx.x < ntop) sh[j * 1024 + threadIdx.x] = v[j];
+  __syncthreads();
+  for (int d = dtop; d >= 1; --d) {
+    const uint32_t* next = sh + bm_lo(d + 1);
+    const int nn = bm_words(d + 1), w = threadIdx.x;
+    if (w < bm_words(d))
+      sh[bm_lo(d) + w] |= bm_dilate(d, w, [&](int V) {
+        uint32_t q = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (4 * V + j < nn) q |= nibbles_any(next[4 * V + j]) << (8 * j);
+        return q;
+      });
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = j * 1024 + threadIdx.x;
+    if (i < bm_lo(dtop + 1)) bm[src[j]] = sh[i];
+  }
+}
+
+// Nodes with children, P_d = the real cells (children of S_{d-1}) in S_d or
+// next to one of it: word and popcount prefix within the block of BS words
+// (pp), and the block's count.
+__global__ __launch_bounds__(BS) void k_bm_parents(const uint32_t* __restrict__ bm, int dmax,
+                                                   uint2* __restrict__ pp,
+                                                   int* __restrict__ bsum) {
+  __shared__ int lds[BS / 64];
+  __shared__ int tot;
+  const int i = blockIdx.x * BS + threadIdx.x;
+  const int d = bm_depth_of(blockIdx.x * BS, dmax);
+  const int w = i - bm_wo(d);
+  uint32_t v = 0;
+  if (d == 0) {
+    v = bm[i];
+  } else if (w < bm_words(d)) {
+    const uint32_t* s = bm + bm_wo(d);
+    const uint32_t up = bm[bm_wo(d - 1) + (w >> 2)];
+    v = bm_dilate(d, w, [&](int V) { return s[V]; }) & nibbles_all((up >> (8 * (w & 3))) & 0xFFu);
+  }
+  const int ex = block_exclusive_scan<BS>(__popc(v), lds, &tot);
+  pp[i] = make_uint2(v, (uint32_t)ex);
+  if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+}
+// Exclusive scan of the blocks' counts; the ranks that start the depths
+// 0 .. dmax and their end to the host (words 0 .. dmax + 1 of the mailbox).
+__global__ __launch_bounds__(1024) void k_bm_sums(int* __restrict__ bsum, int dmax,
+                                                  uint64_t* __restrict__ mbox, uint32_t seq) {
+  __shared__ int lds[1024 / 64];
+  const int t = threadIdx.x, nblk = bm_wo(dmax + 1) / BS;
+  const int ex = block_exclusive_scan<1024>(t < nblk ? bsum[t] : 0, lds, nullptr);
+  if (t < nblk) bsum[t] = ex;
+  for (int d = 0; d <= dmax + 1; ++d)
+    if (t == bm_wo(d) / BS) mailbox_put(mbox, d, seq, ex);
+}
+
+// --- final node arrays ---------------------------------------------------------
+struct LevOff {
+  int lo[kMaxLevels + 1];   // node offset of each level, and the end
+};
+__device__ __forceinline__ int level_of(const LevOff& lv, int L, int g) {
+  int d = 0;
+  for (int j = 1; j < L; ++j) d += g >= lv.lo[j] ? 1 : 0;   // uniform loads
+  return d;
+}
+
+// Neighbour cells without taking a code apart: x sits on its odd bits and y on
+// its even ones, so adding a spread offset with the other bits set carries
+// within one coordinate; a step out of the level's 4^d cells leaves bits above
+// 2 d.  (With each neighbour's code formed from its coordinates k_node_slots
+// took 23 us for 115 thousand nodes, with the steps 20.)
+constexpr uint64_t kXBits = 0xAAAAAAAAAAAAAAAAull, kYBits = 0x5555555555555555ull;
+__device__ __forceinline__ uint64_t cell_step(uint64_t c, uint64_t dx, uint64_t dy) {
+  return (((c | kYBits) + dx) & kXBits) | (((c | kXBits) + dy) & kYBits);
+}
+__device__ __forceinline__ bool on_level(uint64_t c, int d) { return (c >> (2 * d)) == 0; }
+// colleague q = 3 (dx + 1) + dy + 1 of cell c
+__device__ __forceinline__ uint64_t colleague_cell(uint64_t c, int q) {
+  return cell_step(c, morton((uint32_t)(q / 3 - 1), 0), morton(0, (uint32_t)(q % 3 - 1)));
+}
+
+// M2L partners: children of the parent's colleagues, outside the 3x3
+// (tree.py:399-435).  For child position (cx, cy) the parent's 3x3 covers
+// offsets [-2-cx, 3-cx] x [-2-cy, 3-cy].
+struct SlotOffsets {
+  int ox[kNumM2L], oy[kNumM2L];
+  uint64_t dx[kNumM2L], dy[kNumM2L];   // the same as steps of a code
+};
+__constant__ SlotOffsets c_slot_off;
+// whether slot s of cell c of level d names a cell, and that cell
+__device__ __forceinline__ bool slot_cell(uint64_t c, int d, int s, uint64_t* e) {
+  const int cx = (int)(c >> 1) & 1, cy = (int)c & 1;
+  const int ox = c_slot_off.ox[s], oy = c_slot_off.oy[s];
+  *e = cell_step(c, c_slot_off.dx[s], c_slot_off.dy[s]);
+  return ox >= -2 - cx && ox <= 3 - cx && oy >= -2 - cy && oy <= 3 - cy && on_level(*e, d);
+}
+
+// Node lookups by cell: node(d, c) is the node index of the level-d cell with
+// Morton code c or -1; kids(d, c, &xl) the first child of that node or -1, xl
+// whether it is an X-list node.
+struct BmCells {
+  BmIndex ix;
+  const uint32_t* bm;
+  __device__ __forceinline__ int node(int d, uint64_t c) const { return ix.node(d, c); }
+  __device__ __forceinline__ int kids(int d, uint64_t c, bool* xl) const {
+    const uint32_t s = bm[bm_wo(d) + (int)(c >> 5)];
+    const int r = ix.rank(d, c);
+    *xl = r >= 0 && !((s >> (c & 31)) & 1u);
+    return r >= 0 ? 1 + 4 * r : -1;
+  }
+};
+// Of the deeper trees: direct on a full level, a table lookup on the other
+// levels up to depth kIdxDepth (one int per cell of the level, -1 where no
+// node), else a binary search in the level's sorted codes.
+constexpr int kIdxDepth = 11;   // tables of at most 4^12/3 ints (22 MB)
+struct ListCells {
+  const uint64_t* code;
+  LevOff lv;
+  const int* tab;
+  int64_t off[kMaxLevels];      // level d's table in tab, or -1
+  const uint64_t* p_code;       // nodes with children and their kinds
+  const int* p_kind;
+  __device__ __forceinline__ int node(int d, uint64_t c) const {
+    const int64_t nl = lv.lo[d + 1] - lv.lo[d];
+    if (d < 16 && nl == ((int64_t)1 << (2 * d))) return lv.lo[d] + (int)c;
+    if (off[d] >= 0) return tab[off[d] + (int64_t)c];
+    const int64_t pos = bsearch_u64(code + lv.lo[d], nl, c);
+    return pos >= 0 ? lv.lo[d] + (int)pos : -1;
+  }
+  __device__ __forceinline__ int kids(int d, uint64_t c, bool* xl) const {
+    const int p0 = (lv.lo[d + 1] - 1) / 4;   // rank of the depth's first
+    const int64_t pos = bsearch_u64(p_code + p0, (lv.lo[d + 2] - lv.lo[d + 1]) / 4, c);
+    *xl = pos >= 0 && p_kind[p0 + pos] == 1;
+    return pos >= 0 ? lv.lo[d + 1] + 4 * (int)pos : -1;
+  }
+};
+
+// Codes, levels and fake flags of all nodes, their point ranges not yet set
+// (-1; the root's are).  From the bitmaps: a thread per nibble of P, which
+// writes the children of its cells; one thread also writes the root.
+__global__ __launch_bounds__(BS) void k_bm_nodes(BmCells cells, int dmax, int npts,
+                                                 uint64_t* __restrict__ code,
+                                                 int* __restrict__ nlev, int* __restrict__ flags,
+                                                 int* __restrict__ rb, int* __restrict__ rt) {
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i == 0) {
+    code[0] = 0;
+    nlev[0] = 0;
+    flags[0] = 0;
+    rb[0] = 0;
+    rt[0] = npts;
+  }
+  const int w = i >> 3, q = 4 * (i & 7);
+  if (w >= bm_wo(dmax + 1)) return;
+  const uint2 v = cells.ix.pp[w];
+  uint32_t m = (v.x >> q) & 0xFu;
+  if (!m) return;
+  const uint32_t sp = cells.bm[w] >> q;
+  const int d = bm_depth_of((int)(blockIdx.x * (BS / 8)), dmax);
+  const uint64_t c0 = (uint64_t)(w - bm_wo(d)) * 32 + (uint64_t)q;
+  int g = 1 + 4 * (cells.ix.boff[w / BS] + (int)v.y + __popc(v.x & ((1u << q) - 1u)));
+  for (; m; m &= m - 1, g += 4) {
+    const int b = __builtin_ctz(m);
+    const int f = (sp >> b) & 1u ? 0 : NF_FAKE;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      code[g + k] = ((c0 + (uint64_t)b) << 2) | (uint64_t)k;
+      nlev[g + k] = d + 1;
+      flags[g + k] = f;
+      rb[g + k] = -1;
+      rt[g + k] = -1;
+    }
+  }
+}
+// From the lists, with the entries of the level tables.
+__global__ __launch_bounds__(BS) void k_list_nodes(ListCells cells, int L, int npts,
+                                                   uint64_t* __restrict__ code,
+                                                   int* __restrict__ nlev,
+                                                   int* __restrict__ flags, int* __restrict__ rb,
+                                                   int* __restrict__ rt, int* __restrict__ tab) {
+  const int g = blockIdx.x * BS + threadIdx.x;
+  if (g >= cells.lv.lo[L]) return;
+  const int d = level_of(cells.lv, L, g);
+  uint64_t c = 0;
+  int fake = 0;
+  if (d > 0) {
+    const int pj = (g - 1) / 4;
+    c = (cells.p_code[pj] << 2) | (uint64_t)((g - 1) & 3);
+    fake = cells.p_kind[pj] == 1;
+  }
+  code[g] = c;
+  nlev[g] = d;
+  flags[g] = fake ? NF_FAKE : 0;
+  rb[g] = g == 0 ? 0 : -1;
+  rt[g] = g == 0 ? npts : -1;
+  if (cells.off[d] >= 0) tab[cells.off[d] + (int64_t)c] = g;
+}
+
+// Source ranges of the nodes with points from the sorted keys: point i starts
+// its cells of depths s(i)+1.. and ends those of depths s(i+1)+1.. (s = common
+// depth with the previous key).  A cell exists only below an existing parent,
+// so each walk stops at the first depth without one.
+template <class Cells>
 __global__ __launch_bounds__(BS) void k_cell_ranges(const uint64_t* __restrict__ keys,
                                                     const int2* __restrict__ sc, int n,
-                                                    const uint64_t* __restrict__ code,
-                                                    const int* __restrict__ levoff, int L,
-                                                    NodeIdx ni, int* __restrict__ bot,
-                                                    int* __restrict__ top) {
-  const int i = blockIdx.x * BS + threadIdx.x;
+                                                    Cells cells, int L, int* __restrict__ rb,
+                                                    int* __restrict__ rt) {
+  const int i = xcd_block(blockIdx.x, gridDim.x, 0) * BS + threadIdx.x;
   if (i >= n) return;
   const int s0 = sc[i].x;
   const int s1 = i + 1 < n ? sc[i + 1].x : -1;
   if (s0 >= L - 1 && s1 >= L - 1) return;
   const uint64_t k = keys[i];
-  for (int d = max(1, s0 + 1); d <= L - 1; ++d) {
-    const int g = node_of(code, levoff, ni, d, k >> (64 - 2 * d));
+  for (int d = max(1, min(s0, s1) + 1); d <= L - 1; ++d) {
+    const int g = cells.node(d, k >> (64 - 2 * d));
     if (g < 0) break;
-    bot[g] = i;
-  }
-  for (int d = max(1, s1 + 1); d <= L - 1; ++d) {
-    const int g = node_of(code, levoff, ni, d, k >> (64 - 2 * d));
-    if (g < 0) break;
-    top[g] = i + 1;
+    if (d > s0) rb[g] = i;
+    if (d > s1) rt[g] = i + 1;
   }
 }
 
-__global__ __launch_bounds__(BS) void k_cell_ranges_init(int nn, int npts, int* __restrict__ bot,
-                                                         int* __restrict__ top) {
-  const int g = blockIdx.x * BS + threadIdx.x;
-  if (g >= nn) return;
-  bot[g] = g == 0 ? 0 : -1;
-  top[g] = g == 0 ? npts : -1;
-}
-
-__global__ __launch_bounds__(BS) void k_nodes_a(const uint64_t* __restrict__ p_code,
-                                                const int* __restrict__ p_kind,
-                                                const int64_t* __restrict__ poff,
-                                                const int* __restrict__ levoff, int L,
-                                                uint64_t* __restrict__ code,
-                                                int* __restrict__ nlev, int* __restrict__ flags) {
-  int g = blockIdx.x * BS + threadIdx.x;
-  if (g >= levoff[L]) return;
-  int d = find_level(levoff, L, g);
-  int k = g - levoff[d];
-  uint64_t c = 0;
-  int fake = 0;
-  if (d > 0) {
-    int64_t pj = poff[d - 1] + k / 4;
-    c = (p_code[pj] << 2) | (uint64_t)(k & 3);
-    fake = p_kind[pj] == 1;
-  }
-  code[g] = c;
-  nlev[g] = d;
-  flags[g] = fake ? NF_FAKE : 0;
-}
-
-__global__ __launch_bounds__(64) void k_nodes_b(
-    const uint64_t* __restrict__ p_code, const int* __restrict__ p_kind,
-    const int64_t* __restrict__ poff, const int* __restrict__ levoff, int L,
-    const uint64_t* __restrict__ keys, int npts, double xmin0, double ymin0, double w0,
-    NodeIdx ni, const uint64_t* __restrict__ code, int* __restrict__ flags, int* __restrict__ bot,
-    int* __restrict__ top, int* __restrict__ parent, int* __restrict__ child,
-    int* __restrict__ coll, double* __restrict__ xmid, double* __restrict__ ymid) {
-  int g = blockIdx.x * 64 + threadIdx.x;
-  if (g >= levoff[L]) return;
-  const int d = find_level(levoff, L, g);
-  const uint64_t c = code[g];
-  const int fake = flags[g] & NF_FAKE;
-  // children
-  int ch = -1, xl = 0;
-  if (!fake && d <= L - 2) {
-    int64_t pos = bsearch_u64(p_code + poff[d], poff[d + 1] - poff[d], c);
-    if (pos >= 0) {
-      ch = levoff[d + 1] + 4 * (int)pos;
-      xl = p_kind[poff[d] + pos] == 1;
-    }
-  }
-  const int leaf = !fake && (ch < 0 || xl);
-  // point range of the cell (k_cell_ranges); a cell without points sits at
-  // the position where its keys would be
-  int b = bot[g], t = top[g];
-  if (b < 0) {
-    b = (int)lower_bound_u64(keys, npts, c << (64 - 2 * d));
-    t = b;
-  }
-  const int has_src = t > b;
-  int f = fake ? NF_FAKE : 0;
-  if (leaf) f |= NF_LEAF;
-  if (xl) f |= NF_XLIST;
-  if (ch >= 0) f |= NF_CHILDREN;
-  if (has_src) f |= NF_SOURCE;
-  if (((leaf && !xl) || fake) && has_src) f |= NF_UP;   // tree.py:557-560
-  if ((!leaf || xl) && !fake) f |= NF_DOWN;             // tree.py:562 (fake nodes have leaf=False)
-  flags[g] = f;
-  bot[g] = b;
-  top[g] = t;
-  child[g] = ch;
-  // centre by the reference recurrence
-  double xm0 = xmin0, ym0 = ymin0, w = w0;
-  for (int l = 1; l <= d; ++l) {
-    const double h = 0.5 * w;
-    const double xm = xm0 + h, ym = ym0 + h;
-    const int dig = (int)((c >> (2 * (d - l))) & 3);
-    xm0 = (dig & 2) ? xm : xm - h;
-    ym0 = (dig & 1) ? ym : ym - h;
-    w = h;
-  }
-  xmid[g] = xm0 + 0.5 * w;
-  ymid[g] = ym0 + 0.5 * w;
-  // colleagues and parent
-  uint32_t ix, iy;
-  demorton(c, &ix, &iy);
-  const int64_t lim = (int64_t)1 << d;
-  for (int q = 0; q < 9; ++q) {
-    int64_t nx = (int64_t)ix + q / 3 - 1, ny = (int64_t)iy + q % 3 - 1;
-    int r = -1;
-    if (nx >= 0 && ny >= 0 && nx < lim && ny < lim) {
-      r = (q == 4) ? g : node_of(code, levoff, ni, d, morton((uint32_t)nx, (uint32_t)ny));
-    }
-    coll[(int64_t)g * 9 + q] = r;
-  }
-  const int par = d > 0 ? node_of(code, levoff, ni, d - 1, c >> 2) : -1;
-  parent[g] = par;
-}
-
-// Source ranges of every node's nine colleagues, for the evaluation kernels
-// (one load per colleague instead of a colleague index and then its range).
-__global__ __launch_bounds__(BS) void k_coll_ranges(int nslots, const int* __restrict__ coll,
-                                                   const int* __restrict__ bot,
-                                                   const int* __restrict__ top,
-                                                   int2* __restrict__ crange) {
-  const int i = blockIdx.x * BS + threadIdx.x;
-  if (i >= nslots) return;
-  const int c = coll[i];
-  crange[i] = c >= 0 ? make_int2(bot[c], top[c]) : make_int2(0, 0);
-}
-
-// --- density rows: sibling groups (levels >= 2) holding a source ------------------
-__global__ __launch_bounds__(BS) void k_group_flags(const int* __restrict__ flags, int g0, int ngroups,
-                                                    const int* __restrict__ levoff, int L,
-                                                    int* __restrict__ gflag,
-                                                    int* __restrict__ lcount) {
-  __shared__ int lc[kMaxLevels];
-  if (threadIdx.x < kMaxLevels) lc[threadIdx.x] = 0;
-  __syncthreads();
-  int q = blockIdx.x * BS + threadIdx.x;
-  if (q < ngroups) {
-    int g = g0 + 4 * q;
-    int any = 0;
-    for (int j = 0; j < 4; ++j) any |= flags[g + j] & NF_SOURCE;
-    gflag[q] = any ? 1 : 0;
-    if (any) atomicAdd(&lc[find_level(levoff, L, g)], 4);
-  }
-  __syncthreads();
-  if (threadIdx.x < kMaxLevels && lc[threadIdx.x]) atomicAdd(&lcount[threadIdx.x], lc[threadIdx.x]);
-}
-
-__global__ __launch_bounds__(BS) void k_rows(const int* __restrict__ gflag,
-                                             const int* __restrict__ grank, int g0, int nnodes,
-                                             int* __restrict__ row, int* __restrict__ rownode) {
-  int g = blockIdx.x * BS + threadIdx.x;
-  if (g >= nnodes) return;
-  int r = -1;
-  if (g >= g0) {
-    int q = (g - g0) / 4;
-    if (gflag[q]) r = 4 * grank[q] + (g - g0) % 4;
-  }
-  row[g] = r;
-  if (r >= 0) rownode[r] = g;
-}
-
-// Per multipole row: the row of its node's first child (-1 without children)
-// and the node's flags, so that the upward pass reads one record per row.
-__global__ __launch_bounds__(BS) void k_row_info(const int* __restrict__ rownode, int nrows,
-                                                 const int* __restrict__ flags,
-                                                 const int* __restrict__ child,
-                                                 const int* __restrict__ row,
-                                                 int2* __restrict__ info) {
-  const int r = blockIdx.x * BS + threadIdx.x;
-  if (r >= nrows) return;
-  const int g = rownode[r];
-  const int f = flags[g];
-  info[r] = make_int2((f & NF_CHILDREN) ? row[child[g]] : -1, f);
-}
-
-// --- M2L partners: children of the parent's colleagues, outside the 3x3 --------
-// (tree.py:399-435).  For child position (cx, cy) the parent's 3x3 covers
-// offsets [-2-cx, 3-cx] x [-2-cy, 3-cy].
-struct SlotOffsets {
-  int ox[kNumM2L], oy[kNumM2L];
+// The kinds of the nodes that the lists below count, as lane masks of a wave:
+// evaluation boxes, S2M boxes (compute_upwards nodes that own a multipole
+// row), and the sibling groups (levels >= 2, from node g0) holding a source,
+// which own four multipole rows.  Lane j of wave w holds node 64 w + j - 63,
+// so a group is four lanes of one wave (the root alone fills wave 0).
+struct NodeKinds {
+  unsigned long long ev, up, grp;
 };
-__constant__ SlotOffsets c_slot_off;
+__device__ __forceinline__ int wave_node(int v) { return v - 63; }
+inline int64_t wave_slots(int64_t nn) { return nn + 63; }
+__device__ __forceinline__ NodeKinds node_kinds(int f, int g, int g0) {
+  NodeKinds k;
+  k.ev = __ballot((f & NF_LEAF) != 0);
+  k.up = __ballot((f & NF_UP) != 0 && g >= g0);
+  unsigned long long m = __ballot((f & NF_SOURCE) != 0 && g >= g0);
+  m |= m >> 1;
+  m |= m >> 2;
+  k.grp = m & 0x1111111111111111ull;
+  return k;
+}
 
-__global__ __launch_bounds__(BS) void k_m2l_lists(const uint64_t* __restrict__ code,
-                                                  const int* __restrict__ flags,
-                                                  const int* __restrict__ row,
-                                                  const int* __restrict__ levoff, int L,
-                                                  NodeIdx ni, int* __restrict__ m2l) {
-  const int64_t tid = (int64_t)blockIdx.x * BS + threadIdx.x;
-  const int g = levoff[2] + (int)(tid / kNumM2L);
-  const int s = (int)(tid % kNumM2L);
-  if (g >= levoff[L]) return;
-  int r = -1;
-  if (!(flags[g] & NF_FAKE)) {
-    const int d = find_level(levoff, L, g);
-    uint32_t ix, iy;
-    demorton(code[g], &ix, &iy);
-    const int cx = ix & 1, cy = iy & 1;
-    const int ox = c_slot_off.ox[s], oy = c_slot_off.oy[s];
-    if (ox >= -2 - cx && ox <= 3 - cx && oy >= -2 - cy && oy <= 3 - cy) {
-      const int64_t lim = (int64_t)1 << d;
-      const int64_t nx = (int64_t)ix + ox, ny = (int64_t)iy + oy;
-      if (nx >= 0 && ny >= 0 && nx < lim && ny < lim) {
-        const int q = node_of(code, levoff, ni, d, morton((uint32_t)nx, (uint32_t)ny));
-        if (q >= 0) r = row[q];
+// Everything of a node but its lists, and each wave's counts of the kinds
+// (planes of nw ints).  A cell without points sits where its keys would be:
+// behind the nearest sibling before it that has points, else at its parent's
+// start, found the same way.
+template <class Cells>
+__global__ __launch_bounds__(64) void k_nodes(
+    Cells cells, LevOff lv, int L, const int* __restrict__ rb, const int* __restrict__ rt,
+    double xmin0, double ymin0, double w0, const uint64_t* __restrict__ code,
+    int* __restrict__ flags, int* __restrict__ bot, int* __restrict__ top,
+    int* __restrict__ parent, int* __restrict__ child, int* __restrict__ coll,
+    double* __restrict__ xmid, double* __restrict__ ymid, int g0, int nw,
+    int* __restrict__ wcnt) {
+  const int g = wave_node(blockIdx.x * 64 + threadIdx.x);
+  const bool act = g >= 0 && g < lv.lo[L];
+  int f = 0;
+  if (act) {
+    const int d = level_of(lv, L, g);
+    const uint64_t c = code[g];
+    const int fake = flags[g] & NF_FAKE;
+    bool xl = false;
+    const int ch = !fake && d <= L - 2 ? cells.kids(d, c, &xl) : -1;
+    const int leaf = !fake && (ch < 0 || xl);
+    int b = rb[g], t = rt[g];
+    int cg = g, cd = d;
+    while (b < 0) {
+      const int k = (cg - 1) & 3, sib = cg - k;
+      const int t0 = rt[sib], t1 = rt[sib + 1], t2 = rt[sib + 2];
+      if (k > 0) b = t0;
+      if (k > 1 && t1 >= 0) b = t1;
+      if (k > 2 && t2 >= 0) b = t2;
+      if (b < 0) {
+        --cd;
+        cg = cells.node(cd, c >> (2 * (d - cd)));
+        b = rb[cg];
       }
+      t = b;
     }
+    const int has_src = t > b;
+    if (fake) f |= NF_FAKE;
+    if (leaf) f |= NF_LEAF;
+    if (xl) f |= NF_XLIST;
+    if (ch >= 0) f |= NF_CHILDREN;
+    if (has_src) f |= NF_SOURCE;
+    if (((leaf && !xl) || fake) && has_src) f |= NF_UP;   // tree.py:557-560
+    if ((!leaf || xl) && !fake) f |= NF_DOWN;             // tree.py:562 (fake nodes have leaf=False)
+    flags[g] = f;
+    bot[g] = b;
+    top[g] = t;
+    child[g] = ch;
+    // centre by the reference recurrence
+    double xm0 = xmin0, ym0 = ymin0, w = w0;
+    for (int l = 1; l <= d; ++l) {
+      const double h = 0.5 * w;
+      const double xm = xm0 + h, ym = ym0 + h;
+      const int dig = (int)((c >> (2 * (d - l))) & 3);
+      xm0 = (dig & 2) ? xm : xm - h;
+      ym0 = (dig & 1) ? ym : ym - h;
+      w = h;
+    }
+    xmid[g] = xm0 + 0.5 * w;
+    ymid[g] = ym0 + 0.5 * w;
+    // colleagues and parent
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+      const uint64_t e = colleague_cell(c, q);
+      coll[(int64_t)g * 9 + q] = q == 4 ? g : on_level(e, d) ? cells.node(d, e) : -1;
+    }
+    parent[g] = d > 0 ? cells.node(d - 1, c >> 2) : -1;
   }
-  m2l[(int64_t)g * kNumM2L + s] = r;
+  const NodeKinds k = node_kinds(f, g, g0);
+  if (threadIdx.x == 0) {
+    wcnt[blockIdx.x] = (int)__popcll(k.ev);
+    wcnt[nw + blockIdx.x] = (int)__popcll(k.up);
+    wcnt[2 * nw + blockIdx.x] = (int)__popcll(k.grp);
+  }
 }
 
-__global__ __launch_bounds__(BS) void k_flag_bit(const int* __restrict__ flags, int n, int bit,
-                                                 int* __restrict__ out) {
-  int g = blockIdx.x * BS + threadIdx.x;
-  if (g >= n) return;
-  out[g] = (flags[g] & bit) ? 1 : 0;
+// Evaluation boxes, S2M boxes and multipole rows from the waves' counts.  Up
+// to kSumWaves waves each block adds the counts of the waves before it itself
+// (scanned = 0; a scan of its own would cost three launches); above, wcnt
+// holds their exclusive prefixes.  The totals and the first row of each level
+// >= 2 go to the host's mailbox: boxes, S2M boxes, row groups, then the levels.
+constexpr int64_t kSumWaves = 8192;   // three 21-bit sums fit in 64 bits
+__global__ __launch_bounds__(1024) void k_node_lists(const int* __restrict__ flags, LevOff lv,
+                                                     int L, int g0, int nw,
+                                                     const int* __restrict__ wcnt, int scanned,
+                                                     int* __restrict__ evalid,
+                                                     int* __restrict__ evalnode,
+                                                     int* __restrict__ upnodes,
+                                                     int* __restrict__ row,
+                                                     uint64_t* __restrict__ mbox, uint32_t seq) {
+  __shared__ unsigned long long part[16];
+  __shared__ int wv[3][16];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const int w0 = blockIdx.x * 16;   // the block's first wave, < nw
+  const int g = wave_node(blockIdx.x * 1024 + t);
+  const bool act = g >= 0 && g < lv.lo[L];
+  const int f = act ? flags[g] : 0;
+  const NodeKinds k = node_kinds(f, g, g0);
+  if (lane == 0) {
+    wv[0][wid] = (int)__popcll(k.ev);
+    wv[1][wid] = (int)__popcll(k.up);
+    wv[2][wid] = (int)__popcll(k.grp);
+  }
+  unsigned long long acc = 0;
+  if (!scanned) {
+    for (int j = t; j < w0; j += 1024)
+      acc += (unsigned long long)wcnt[j] | (unsigned long long)wcnt[nw + j] << 21 |
+             (unsigned long long)wcnt[2 * nw + j] << 42;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if (lane == 0) part[wid] = acc;
+  }
+  __syncthreads();
+  int base[3];
+  if (scanned) {
+    for (int q = 0; q < 3; ++q) base[q] = wcnt[(int64_t)q * nw + w0];
+  } else {
+    acc = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) acc += part[w];
+    for (int q = 0; q < 3; ++q) base[q] = (int)(acc >> (21 * q)) & 0x1FFFFF;
+  }
+  for (int w = 0; w < wid; ++w)
+    for (int q = 0; q < 3; ++q) base[q] += wv[q][w];
+  if (blockIdx.x == gridDim.x - 1 && wid == 15 && lane < 3) {
+    const int b = lane == 0 ? base[0] : lane == 1 ? base[1] : base[2];
+    mailbox_put(mbox, lane, seq, b + wv[lane][15]);
+  }
+  if (!act) return;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const int e = base[0] + (int)__popcll(k.ev & below);
+  const bool ev = (k.ev >> lane) & 1ull;
+  evalid[g] = ev ? e : -1;
+  if (ev) evalnode[e] = g;
+  if ((k.up >> lane) & 1ull) upnodes[base[1] + (int)__popcll(k.up & below)] = g;
+  const int lead = lane & ~3;
+  const int r = 4 * (base[2] + (int)__popcll(k.grp & ((1ull << lead) - 1ull)));
+  row[g] = (k.grp >> lead) & 1ull ? r + (lane & 3) : -1;
+  for (int d = 2; d < L; ++d)
+    if (g == lv.lo[d]) mailbox_put(mbox, 3 + d - 2, seq, r);
 }
 
-// S2M boxes: compute_upwards nodes that own a multipole row (levels >= 2;
-// the upward pass stops at level 2, fmm.py:98).
-__global__ __launch_bounds__(BS) void k_up_flag(const int* __restrict__ flags,
-                                                const int* __restrict__ row, int n,
-                                                int* __restrict__ out) {
-  int g = blockIdx.x * BS + threadIdx.x;
-  if (g >= n) return;
-  out[g] = ((flags[g] & NF_UP) && row[g] >= 0) ? 1 : 0;
-}
-
-__global__ __launch_bounds__(BS) void k_list_scatter(const int* __restrict__ flag,
-                                                     const int* __restrict__ rank, int n,
-                                                     int* __restrict__ list,
-                                                     int* __restrict__ idx_of) {
-  int g = blockIdx.x * BS + threadIdx.x;
-  if (g >= n) return;
-  if (flag[g]) {
-    list[rank[g]] = g;
-    if (idx_of) idx_of[g] = rank[g];
-  } else if (idx_of) {
-    idx_of[g] = -1;
+// The lists that read other nodes' records: the multipole rows of the M2L
+// partners (levels >= 2), the source ranges of the nine colleagues (one load
+// per colleague for the evaluation kernels instead of its index and then its
+// range), and per multipole row the row of its node's first child (-1 without
+// children) with the node's flags, one record for the upward pass.  Sixteen
+// lanes per node, its 40 partner slots j, j + 16, j + 32 on lane j: bound by
+// the chain of dependent loads, which three slots share, and then by the
+// stores (a thread per slot took 24 us for 58 thousand nodes, this 16).
+constexpr int kSlotLanes = 16;
+template <class Cells>
+__global__ __launch_bounds__(BS) void k_node_slots(
+    Cells cells, LevOff lv, int L, const uint64_t* __restrict__ code,
+    const int* __restrict__ nlev, const int* __restrict__ flags, const int* __restrict__ row,
+    const int* __restrict__ child,
+    const int* __restrict__ coll, const int* __restrict__ bot, const int* __restrict__ top,
+    int* __restrict__ m2l, int2* __restrict__ crange, int2* __restrict__ rowinfo) {
+  const int64_t tid = (int64_t)xcd_block(blockIdx.x, gridDim.x, 0) * BS + threadIdx.x;
+  const int g = (int)(tid / kSlotLanes);
+  const int j = (int)(tid % kSlotLanes);
+  if (g >= lv.lo[L]) return;
+  const int f = flags[g], d = nlev[g];
+  const uint64_t cg = code[g];
+  if (j < 9) {
+    const int c = coll[(int64_t)g * 9 + j];
+    crange[(int64_t)g * 9 + j] = c >= 0 ? make_int2(bot[c], top[c]) : make_int2(0, 0);
+  } else if (j == 9) {
+    const int r = row[g];
+    if (r >= 0) rowinfo[r] = make_int2((f & NF_CHILDREN) ? row[child[g]] : -1, f);
+  }
+  if (L < 3 || g < lv.lo[2]) return;
+  constexpr int kPer = (kNumM2L + kSlotLanes - 1) / kSlotLanes;
+  int q[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int s = j + u * kSlotLanes;
+    uint64_t e;
+    q[u] = s < kNumM2L && !(f & NF_FAKE) && slot_cell(cg, d, s, &e) ? cells.node(d, e) : -1;
+  }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int s = j + u * kSlotLanes;
+    if (s < kNumM2L) m2l[(int64_t)g * kNumM2L + s] = q[u] >= 0 ? row[q[u]] : -1;
   }
 }
 
@@ -871,11 +1152,10 @@ __global__ __launch_bounds__(BS) void k_full_nodes(
     int2* __restrict__ crange, double* __restrict__ xmid, double* __restrict__ ymid,
     int* __restrict__ row, int* __restrict__ m2l, int* __restrict__ evalid,
     int* __restrict__ evalnode, int* __restrict__ upnodes, int2* __restrict__ rowinfo,
-    int* __restrict__ levoff, const int* __restrict__ gate) {
+    const int* __restrict__ gate) {
   if (gate && *gate == 0) return;
   const int64_t tid = (int64_t)blockIdx.x * BS + threadIdx.x;
   const int g = (int)(tid / kFullLanes), j = (int)(tid % kFullLanes);
-  if (tid <= D + 1) levoff[tid] = full_levoff((int)tid);   // levels 0 .. D and the end
   if (g >= nn) return;
   int d = 0;
   while (d < D && g >= full_levoff(d + 1)) ++d;
@@ -883,9 +1163,6 @@ __global__ __launch_bounds__(BS) void k_full_nodes(
   const uint64_t c = (uint64_t)(g - lo);
   const bool leaf = d == D;
   const int g0 = full_levoff(2);
-  uint32_t ix, iy;
-  demorton(c, &ix, &iy);
-  const int64_t lim = (int64_t)1 << d;
   if (j == 0) {
     const int b = full_pos(start, keys, npts, D, d, c), t = full_pos(start, keys, npts, D, d, c + 1);
     int f = leaf ? NF_LEAF : (NF_CHILDREN | NF_DOWN);   // tree.py:557-562
@@ -921,11 +1198,10 @@ __global__ __launch_bounds__(BS) void k_full_nodes(
     }
   }
   if (j < 9) {
-    const int64_t nx = (int64_t)ix + j / 3 - 1, ny = (int64_t)iy + j % 3 - 1;
+    const uint64_t cc = colleague_cell(c, j);
     int r = -1;
     int2 rg = make_int2(0, 0);
-    if (nx >= 0 && ny >= 0 && nx < lim && ny < lim) {
-      const uint64_t cc = morton((uint32_t)nx, (uint32_t)ny);
+    if (on_level(cc, d)) {
       r = lo + (int)cc;
       rg = make_int2(full_pos(start, keys, npts, D, d, cc),
                      full_pos(start, keys, npts, D, d, cc + 1));
@@ -933,19 +1209,11 @@ __global__ __launch_bounds__(BS) void k_full_nodes(
     coll[(int64_t)g * 9 + j] = r;
     crange[(int64_t)g * 9 + j] = rg;
   }
-  if (d >= 2) {
-    const int cx = ix & 1, cy = iy & 1;
+  if (d >= 2)
     for (int s = j; s < kNumM2L; s += kFullLanes) {
-      const int ox = c_slot_off.ox[s], oy = c_slot_off.oy[s];
-      int rr = -1;
-      if (ox >= -2 - cx && ox <= 3 - cx && oy >= -2 - cy && oy <= 3 - cy) {
-        const int64_t nx = (int64_t)ix + ox, ny = (int64_t)iy + oy;
-        if (nx >= 0 && ny >= 0 && nx < lim && ny < lim)
-          rr = lo + (int)morton((uint32_t)nx, (uint32_t)ny) - g0;
-      }
-      m2l[(int64_t)g * kNumM2L + s] = rr;
+      uint64_t e;
+      m2l[(int64_t)g * kNumM2L + s] = slot_cell(c, d, s, &e) ? lo + (int)e - g0 : -1;
     }
-  }
 }
 
 }  // namespace
@@ -959,7 +1227,6 @@ static void tree_full_buffers(Tree& t, int D) {
   const int NN = full_levoff(D + 1);
   const int64_t n_eval = (int64_t)1 << (2 * D);
   const int64_t n_rows = NN - full_levoff(2);
-  t.levoff.ensure((D + 2) * sizeof(int));   // written by k_full_nodes
   t.w_flag.ensure((n_eval + 1) * sizeof(int));
   t.code.ensure(NN * sizeof(uint64_t));
   t.nlevel.ensure(NN * sizeof(int));
@@ -995,7 +1262,7 @@ static void tree_full_kernels(Tree& t, int D, int npts, hipStream_t s, const int
                      t.parent.as<int>(), t.child.as<int>(), t.coll.as<int>(), t.crange.as<int2>(),
                      t.xmid.as<double>(), t.ymid.as<double>(), t.row.as<int>(), t.m2l.as<int>(),
                      t.evalid.as<int>(), t.evalnode.as<int>(), t.upnodes.as<int>(),
-                     t.rowinfo.as<int2>(), t.levoff.as<int>(), gate);
+                     t.rowinfo.as<int2>(), gate);
   FMM_LAUNCH_CHECK();
 }
 
@@ -1017,6 +1284,7 @@ static void tree_full_host(Tree& t, int D) {
   t.n_eval = (int64_t)1 << (2 * D);
   t.n_up = t.n_eval;
   t.nidx_off.assign(kMaxLevels, -1);
+  t.bm_index = false;
   t.complete = true;
   t.full_D = D;
   ++t.build_id;
@@ -1043,65 +1311,28 @@ static void read_counts(Tree& t, const int* dev, int n, int* host, hipStream_t s
   for (int i = 0; i < n; ++i) host[i] = (int)v[i];
 }
 
-// ---------------------------------------------------------------------------
-void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmin, double ymin,
-                double w0, int ncut, hipStream_t s) {
-  FMM_REQUIRE(n >= 1 && n < ((int64_t)1 << 31) - 1, FMM_E_LIMIT,
-              "tree: number of sources %lld outside [1, 2^31-2]", (long long)n);
-  FMM_REQUIRE(ncut >= 1, FMM_E_ARG, "tree: Ncutoff must be >= 1 (got %d)", ncut);
-  FMM_REQUIRE(w0 > 0.0 && std::isfinite(w0), FMM_E_ARG, "tree: root width must be positive");
-  t.built = false;
-  t.complete = false;
-  t.n = n;
-  t.ncut = ncut;
-  t.xmin = xmin;
-  t.ymin = ymin;
-  t.w0 = w0;
-  const int nn = (int)n;
+// Device counters of a build.
+enum { CNT_R = 0, CNT_UNIQ = 1, CNT_PC = 2, CNT_BAL = CNT_PC + kMaxLevels,
+       CNT_SPLIT = CNT_BAL + kMaxLevels, CNT_ALL = CNT_SPLIT + kSplitRows * (kMaxLevels + 1) };
 
-  // -- sorted points ----------------------------------------------------------
-  t.keys.ensure(n * sizeof(uint64_t));
-  t.perm.ensure(n * sizeof(uint32_t));
-  t.sx.ensure(n * sizeof(double));
-  t.sy.ensure(n * sizeof(double));
-  uint64_t* keys = t.keys.as<uint64_t>();
-  uint32_t* perm = t.perm.as<uint32_t>();
-  t.xy.ensure(n * sizeof(double2));
-  // -- counters (zeroed before the first kernel, which flags non-finite points)
-  enum { CNT_R = 33, CNT_PC = 34, CNT_ROWS = 66, CNT_EVAL = 67, CNT_UP = 68, CNT_UNIQ = 69,
-         CNT_LR = 72, CNT_BAL = 104, CNT_BAD = 136, CNT_N = 137,
-         CNT_SPLIT = CNT_N, CNT_ALL = CNT_SPLIT + kSplitRows * (kMaxLevels + 1) };
-  t.w_cnt.ensure(CNT_ALL * sizeof(int));
-  t.h_cnt.ensure(CNT_ALL * sizeof(int));
+// Nodes with children (p_code, p_kind, p_off) of a tree of more than kBmLevels
+// levels: sorted code lists per depth, dcount[d] of them split and np split
+// positions.
+static void tree_split_lists(Tree& t, const int64_t* dcount, int np, hipStream_t s) {
+  const int L = t.L, nn = (int)t.n;
+  const int64_t n = t.n;
+  const uint64_t* keys = t.keys.as<uint64_t>();
+  const int2* sc = t.w_a.as<int2>();
   int* cnt = t.w_cnt.as<int>();
-  int* hc = t.h_cnt.as<int>();
-  const int nkey_blk = (int)ceil_div(n, kSortChunk);
-  t.w_bad.ensure(nkey_blk * sizeof(int));
-  const int sort_T = ncut < kLocalSortMax ? ncut : kLocalSortMax;
-  const bool first_round = n > sort_T;
-  const SortFirstRound fr = first_round ? sort_first_round(t.pw, n) : SortFirstRound{};
-  hipLaunchKernelGGL(k_point_keys, dim3((unsigned)ceil_div(n, kSortChunk)), dim3(KEY_BS), 0, s, x, y,
-                     nn, xmin, ymin, w0, key_scale(xmin, ymin, w0),
-                     first_round ? fr.keys : keys, first_round ? fr.vals : perm,
-                     t.xy.as<double2>(), t.w_bad.as<int>(), cnt, (int)CNT_ALL, fr,
-                     first_round ? 1 : 0);
-  FMM_LAUNCH_CHECK();
-  // Segments of at most Ncutoff points that end in the last radix round sit
-  // at the deepest radix depth D, which no cell of the tree goes below (2:1
-  // balance splits lie at least two levels above the deepest leaf, X-list
-  // children at most at depth D): the radix order within them stands.
-  // Segments that end earlier are sorted, since balance and X-list children
-  // can split their cells further.
-  sort_pairs_u64(keys, perm, n, sort_T, t.pw, s, 64, true, first_round);
-
+  int hc[CNT_SPLIT] = {};
   // Small host->device uploads go through distinct regions of a pinned buffer
   // so that the host never rewrites memory a queued copy still reads.
   constexpr int kUpRegion = kMaxLevels + 2;
-  t.h_up.ensure(8 * kUpRegion * sizeof(int64_t));
+  t.h_up.ensure(4 * kUpRegion * sizeof(int64_t));
   int64_t* hup = t.h_up.as<int64_t>();
   int up_region = 0;
   auto upload = [&](void* dst, const void* src, size_t bytes) {
-    FMM_REQUIRE(up_region < 8 && bytes <= kUpRegion * sizeof(int64_t), FMM_E_INTERNAL,
+    FMM_REQUIRE(up_region < 4 && bytes <= kUpRegion * sizeof(int64_t), FMM_E_INTERNAL,
                 "tree: upload staging exhausted");
     int64_t* slot = hup + (int64_t)up_region * kUpRegion;
     ++up_region;
@@ -1109,69 +1340,13 @@ void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmi
     FMM_HIP(hipMemcpyAsync(dst, slot, bytes, hipMemcpyHostToDevice, s));
   };
 
-  // -- split cells of the refinement --------------------------------------------
+  // compacted split positions and the split-cell lists per depth (S_ref)
   t.w_flag.ensure(n * sizeof(int));
   t.w_rank.ensure(n * sizeof(int));
-  t.w_a.ensure(n * sizeof(int2));
   int* flag = t.w_flag.as<int>();
   int* rank = t.w_rank.as<int>();
-  int2* sc = t.w_a.as<int2>();
-  hipLaunchKernelGGL(k_split_pos, dim3((unsigned)ceil_div(n, 1024)), dim3(1024), 0, s, keys, nn,
-                     ncut, flag, sc, cnt + CNT_SPLIT, perm, t.xy.as<double2>(), t.sx.as<double>(),
-                     t.sy.as<double>());
+  hipLaunchKernelGGL(k_split_flags, dim3(grid_for(n)), dim3(BS), 0, s, sc, nn, flag);
   FMM_LAUNCH_CHECK();
-  // per depth, then the split positions; then the non-finite flag
-  int64_t dcount[kMaxLevels + 2];
-  // A complete tree of the previous build's depth is built at once, gated on
-  // the device by the split counts (its kernels then follow without waiting
-  // for the host to read them); that needs its buffers to leave the split
-  // flags in w_flag (still needed otherwise) where they are.
-  const int specD = t.full_D;
-  const bool spec = t.allow_full && specD >= 2 && specD <= kFullMaxDepth &&
-                    t.w_flag.bytes >= ((((size_t)1 << (2 * specD)) + 1) * sizeof(int));
-  {
-    HostMailbox& mb = t.pw.mbox;
-    mb.ensure();
-    const uint32_t seq = mb.next();
-    int* gate = nullptr;
-    if (spec) {
-      t.w_gate.ensure(sizeof(int));
-      gate = t.w_gate.as<int>();
-      tree_full_buffers(t, specD);
-    }
-    hipLaunchKernelGGL(k_split_counts, dim3(1), dim3(64), 0, s, cnt + CNT_SPLIT,
-                       t.w_bad.as<int>(), nkey_blk, mb.dev, seq, specD, gate);
-    FMM_LAUNCH_CHECK();
-    if (spec) tree_full_kernels(t, specD, nn, s, gate);
-    mb.take(kMaxLevels + 2, seq, s, dcount);
-  }
-  FMM_REQUIRE(dcount[kMaxLevels + 1] == 0, FMM_E_ARG,
-              "tree: the source coordinates hold a NaN or infinite value");
-  const int np = (int)dcount[kMaxLevels];
-  int maxd = -1;
-  for (int d = 0; d < kMaxLevels; ++d)
-    if (dcount[d] > 0) maxd = d;
-  const int L = maxd + 2;   // deepest split depth + children level + 1
-  t.L = L;
-  FMM_REQUIRE(L <= kMaxLevels, FMM_E_INTERNAL, "tree: %d levels exceed the depth cap", L);
-
-  // a complete tree (every cell of the depths above the deepest split cells
-  // split): closed forms of the node arrays (k_full_nodes)
-  if (t.allow_full && L >= 3 && L - 1 <= kFullMaxDepth) {
-    bool complete = true;
-    for (int d = 0; d <= L - 2 && complete; ++d) complete = dcount[d] == ((int64_t)1 << (2 * d));
-    if (complete) {
-      if (!(spec && L - 1 == specD)) {   // else built already
-        tree_full_buffers(t, L - 1);
-        tree_full_kernels(t, L - 1, nn, s, nullptr);
-      }
-      tree_full_host(t, L - 1);
-      return;
-    }
-  }
-  t.full_D = 0;
-
-  // compacted split positions and the split-cell lists per depth (S_ref)
   exclusive_scan_i32(flag, rank, n, nullptr, t.pw, s);
   t.w_c.ensure((int64_t)(n + 2) * (sizeof(int) + sizeof(int2)) + 16);
   int* ppos = t.w_c.as<int>();
@@ -1182,7 +1357,7 @@ void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmi
   t.s_off.assign(L + 1, 0);
   for (int d = 0; d < L; ++d) t.s_off[d + 1] = t.s_off[d] + (d <= L - 2 ? dcount[d] : 0);
   const int64_t ns_total = t.s_off[L];
-  t.w_b.ensure((L + 1) * sizeof(int64_t) * 3 + 64);
+  t.w_b.ensure((L + 1) * sizeof(int64_t) * 2 + 64);
   int64_t* d_soff = t.w_b.as<int64_t>();
   t.sref_all.ensure((ns_total + 1) * sizeof(uint64_t));
   if (np > 0) {
@@ -1314,7 +1489,6 @@ void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmi
       FMM_HIP(hipMemcpyAsync(sall + soff[L - 2], sref + t.s_off[L - 2],
                              sz[L - 2] * sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
   }
-  t.s_off = soff;
 
   // -- nodes with children (P_d = S_d u X_d) ----------------------------------------
   std::vector<int64_t> roff(L + 1, 0);
@@ -1323,7 +1497,6 @@ void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmi
   const int64_t nr = roff[L];
   int64_t* d_soff2 = d_soff;
   int64_t* d_roff = d_soff + (L + 1);
-  int64_t* d_poff = d_soff + 2 * (L + 1);
   upload(d_soff2, soff.data(), (L + 1) * sizeof(int64_t));
   upload(d_roff, roff.data(), (L + 1) * sizeof(int64_t));
   t.w_c.ensure(nr * (sizeof(uint64_t) + 3 * sizeof(int)) + 64);
@@ -1345,28 +1518,212 @@ void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmi
   hipLaunchKernelGGL(k_p_scatter, dim3(grid_for(nr)), dim3(BS), 0, s, rcode, hasc, kind, rrank, nr,
                      t.p_code.as<uint64_t>(), t.p_kind.as<int>());
   FMM_LAUNCH_CHECK();
-  upload(d_poff, t.p_off.data(), (L + 1) * sizeof(int64_t));
+}
+
+// The node arrays of the levels lv from the cells' lookups (codes, levels and
+// fake flags of the nodes are set): point ranges, records, lists, and the
+// host's counts, which it reads while the last kernel runs.
+template <class Cells>
+static void node_arrays(Tree& t, const Cells& cells, const LevOff& lv, int g0, int nw, int* rb,
+                        int* rt, int* wcnt, hipStream_t s) {
+  const int L = t.L, NN = (int)t.n_nodes;
+  hipLaunchKernelGGL(k_cell_ranges<Cells>, dim3(grid_for(t.n)), dim3(BS), 0, s,
+                     t.keys.as<uint64_t>(), t.w_a.as<int2>(), (int)t.n, cells, L, rb, rt);
+  FMM_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_nodes<Cells>, dim3(nw), dim3(64), 0, s, cells, lv, L, rb, rt, t.xmin, t.ymin,
+                     t.w0, t.code.as<uint64_t>(), t.flags.as<int>(), t.bot.as<int>(),
+                     t.top.as<int>(), t.parent.as<int>(), t.child.as<int>(), t.coll.as<int>(),
+                     t.xmid.as<double>(), t.ymid.as<double>(), g0, nw, wcnt);
+  FMM_LAUNCH_CHECK();
+  const bool scanned = nw > kSumWaves;
+  if (scanned)
+    for (int q = 0; q < 3; ++q)
+      exclusive_scan_i32(wcnt + (int64_t)q * nw, wcnt + (int64_t)q * nw, nw, nullptr, t.pw, s);
+  HostMailbox& mb = t.pw.mbox;
+  const uint32_t seq = mb.next();
+  hipLaunchKernelGGL(k_node_lists, dim3((unsigned)ceil_div(nw, 16)), dim3(1024), 0, s,
+                     t.flags.as<int>(), lv, L, g0, nw, wcnt, scanned ? 1 : 0, t.evalid.as<int>(),
+                     t.evalnode.as<int>(), t.upnodes.as<int>(), t.row.as<int>(), mb.dev, seq);
+  FMM_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_node_slots<Cells>, dim3(grid_for((int64_t)NN * kSlotLanes)), dim3(BS), 0, s,
+                     cells, lv, L, t.code.as<uint64_t>(), t.nlevel.as<int>(), t.flags.as<int>(),
+                     t.row.as<int>(), t.child.as<int>(), t.coll.as<int>(), t.bot.as<int>(), t.top.as<int>(),
+                     t.m2l.as<int>(), t.crange.as<int2>(), t.rowinfo.as<int2>());
+  FMM_LAUNCH_CHECK();
+  int64_t v[3 + kMaxLevels];
+  mb.take(3 + std::max(0, L - 2), seq, s, v);
+  t.n_eval = v[0];
+  t.n_up = v[1];
+  t.n_rows = 4 * v[2];
+  t.row_off.assign(L + 1, 0);
+  for (int d = 2; d < L; ++d) t.row_off[d] = v[3 + d - 2];
+  t.row_off[L] = t.n_rows;
+}
+
+// ---------------------------------------------------------------------------
+void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmin, double ymin,
+                double w0, int ncut, hipStream_t s) {
+  FMM_REQUIRE(n >= 1 && n < ((int64_t)1 << 31) - 1, FMM_E_LIMIT,
+              "tree: number of sources %lld outside [1, 2^31-2]", (long long)n);
+  FMM_REQUIRE(ncut >= 1, FMM_E_ARG, "tree: Ncutoff must be >= 1 (got %d)", ncut);
+  FMM_REQUIRE(w0 > 0.0 && std::isfinite(w0), FMM_E_ARG, "tree: root width must be positive");
+  t.built = false;
+  t.complete = false;
+  t.n = n;
+  t.ncut = ncut;
+  t.xmin = xmin;
+  t.ymin = ymin;
+  t.w0 = w0;
+  const int nn = (int)n;
+
+  // -- sorted points ----------------------------------------------------------
+  t.keys.ensure(n * sizeof(uint64_t));
+  t.perm.ensure(n * sizeof(uint32_t));
+  t.sx.ensure(n * sizeof(double));
+  t.sy.ensure(n * sizeof(double));
+  uint64_t* keys = t.keys.as<uint64_t>();
+  uint32_t* perm = t.perm.as<uint32_t>();
+  t.xy.ensure(n * sizeof(double2));
+  // -- counters (zeroed by the first kernel)
+  t.w_cnt.ensure(CNT_ALL * sizeof(int));
+  int* cnt = t.w_cnt.as<int>();
+  const int nkey_blk = (int)ceil_div(n, kSortChunk);
+  t.w_bad.ensure(nkey_blk * sizeof(int));
+  const int sort_T = ncut < kLocalSortMax ? ncut : kLocalSortMax;
+  const bool first_round = n > sort_T;
+  const SortFirstRound fr = first_round ? sort_first_round(t.pw, n) : SortFirstRound{};
+  hipLaunchKernelGGL(k_point_keys, dim3((unsigned)ceil_div(n, kSortChunk)), dim3(KEY_BS), 0, s, x, y,
+                     nn, xmin, ymin, w0, key_scale(xmin, ymin, w0),
+                     first_round ? fr.keys : keys, first_round ? fr.vals : perm,
+                     t.xy.as<double2>(), t.w_bad.as<int>(), cnt, (int)CNT_ALL, fr,
+                     first_round ? 1 : 0);
+  FMM_LAUNCH_CHECK();
+  // Segments of at most Ncutoff points that end in the last radix round sit
+  // at the deepest radix depth D, which no cell of the tree goes below (2:1
+  // balance splits lie at least two levels above the deepest leaf, X-list
+  // children at most at depth D): the radix order within them stands.
+  // Segments that end earlier are sorted, since balance and X-list children
+  // can split their cells further.
+  sort_pairs_u64(keys, perm, n, sort_T, t.pw, s, 64, true, first_round);
+
+  // -- split cells of the refinement --------------------------------------------
+  t.w_a.ensure(n * sizeof(int2));
+  int2* sc = t.w_a.as<int2>();
+  hipLaunchKernelGGL(k_split_pos, dim3((unsigned)ceil_div(n, 1024)), dim3(1024), 0, s, keys, nn,
+                     ncut, sc, cnt + CNT_SPLIT, perm, t.xy.as<double2>(), t.sx.as<double>(),
+                     t.sy.as<double>());
+  FMM_LAUNCH_CHECK();
+  // per depth, then the split positions; then the non-finite flag
+  int64_t dcount[kMaxLevels + 2];
+  // A complete tree of the previous build's depth is built at once, gated on
+  // the device by the split counts (its kernels then follow without waiting
+  // for the host to read them).  Otherwise the split cells go into the bitmaps
+  // of an adaptive tree meanwhile.
+  const int specD = t.full_D;
+  const bool spec = t.allow_full && specD >= 2 && specD <= kFullMaxDepth;
+  auto mark_split_cells = [&] {
+    t.bm.ensure(kBmWords * sizeof(uint32_t));
+    fill_i32(t.bm.as<int>(), kBmWords, 0, s);
+    hipLaunchKernelGGL(k_bm_mark_points, dim3(grid_for(n)), dim3(BS), 0, s, keys, sc, nn,
+                       t.bm.as<uint32_t>());
+    FMM_LAUNCH_CHECK();
+  };
+  {
+    HostMailbox& mb = t.pw.mbox;
+    mb.ensure();
+    const uint32_t seq = mb.next();
+    int* gate = nullptr;
+    if (spec) {
+      t.w_gate.ensure(sizeof(int));
+      gate = t.w_gate.as<int>();
+      tree_full_buffers(t, specD);
+    }
+    hipLaunchKernelGGL(k_split_counts, dim3(1), dim3(64), 0, s, cnt + CNT_SPLIT,
+                       t.w_bad.as<int>(), nkey_blk, mb.dev, seq, specD, gate);
+    FMM_LAUNCH_CHECK();
+    if (spec) tree_full_kernels(t, specD, nn, s, gate);
+    else mark_split_cells();
+    mb.take(kMaxLevels + 2, seq, s, dcount);
+  }
+  FMM_REQUIRE(dcount[kMaxLevels + 1] == 0, FMM_E_ARG,
+              "tree: the source coordinates hold a NaN or infinite value");
+  const int np = (int)dcount[kMaxLevels];
+  int maxd = -1;
+  for (int d = 0; d < kMaxLevels; ++d)
+    if (dcount[d] > 0) maxd = d;
+  const int L = maxd + 2;   // deepest split depth + children level + 1
+  t.L = L;
+  FMM_REQUIRE(L <= kMaxLevels, FMM_E_INTERNAL, "tree: %d levels exceed the depth cap", L);
+
+  // a complete tree (every cell of the depths above the deepest split cells
+  // split): closed forms of the node arrays (k_full_nodes)
+  if (t.allow_full && L >= 3 && L - 1 <= kFullMaxDepth) {
+    bool complete = true;
+    for (int d = 0; d <= L - 2 && complete; ++d) complete = dcount[d] == ((int64_t)1 << (2 * d));
+    if (complete) {
+      if (!(spec && L - 1 == specD)) {   // else built already
+        tree_full_buffers(t, L - 1);
+        tree_full_kernels(t, L - 1, nn, s, nullptr);
+      }
+      tree_full_host(t, L - 1);
+      return;
+    }
+  }
+  t.full_D = 0;
+
+  // -- nodes with children (P_d = S_d u X_d) ----------------------------------------
+  t.bm_index = L <= kBmLevels;
+  if (t.bm_index) {
+    if (spec) mark_split_cells();   // else marked already
+    t.p_off.assign(L + 1, 0);
+    t.bm_pp.ensure(kBmWords * sizeof(uint2));
+    t.bm_boff.ensure(kBmBlocks * sizeof(int));
+    uint32_t* bm = t.bm.as<uint32_t>();
+    for (int d = L - 3; d > kBmLowD; --d) {
+      hipLaunchKernelGGL(k_bm_balance, dim3(grid_for(bm_words(d))), dim3(BS), 0, s, d, bm);
+      FMM_LAUNCH_CHECK();
+    }
+    if (L >= 4) {
+      hipLaunchKernelGGL(k_bm_balance_low, dim3(1), dim3(1024), 0, s, std::min(L - 3, kBmLowD), bm);
+      FMM_LAUNCH_CHECK();
+    }
+    if (L >= 2) {
+      HostMailbox& mb = t.pw.mbox;
+      const uint32_t seq = mb.next();
+      hipLaunchKernelGGL(k_bm_parents, dim3(bm_wo(L - 1) / BS), dim3(BS), 0, s, bm, L - 2,
+                         t.bm_pp.as<uint2>(), t.bm_boff.as<int>());
+      FMM_LAUNCH_CHECK();
+      hipLaunchKernelGGL(k_bm_sums, dim3(1), dim3(1024), 0, s, t.bm_boff.as<int>(), L - 2, mb.dev,
+                         seq);
+      FMM_LAUNCH_CHECK();
+      mb.take(L, seq, s, t.p_off.data());
+      t.p_off[L] = t.p_off[L - 1];
+    }
+  } else {
+    tree_split_lists(t, dcount, np, s);
+  }
 
   // -- final node arrays ------------------------------------------------------------
   t.lev.assign(L, TreeLevel());
-  std::vector<int> levoff(L + 1, 0);
+  LevOff lv{};
   int64_t off = 0;
   for (int d = 0; d < L; ++d) {
     int64_t nd = d == 0 ? 1 : 4 * (t.p_off[d] - t.p_off[d - 1]);
     t.lev[d].node_off = off;
     t.lev[d].n_nodes = nd;
     t.lev[d].width = std::ldexp(w0, -d);
-    levoff[d] = (int)off;
+    lv.lo[d] = (int)off;
     off += nd;
+    FMM_REQUIRE(off < ((int64_t)1 << 31) / kNumM2L, FMM_E_LIMIT, "tree: too many nodes (%lld)",
+                (long long)off);
   }
-  levoff[L] = (int)off;
-  FMM_REQUIRE(off < ((int64_t)1 << 31) / kNumM2L, FMM_E_LIMIT, "tree: too many nodes (%lld)",
-              (long long)off);
-  const int NN = (int)off;
+  lv.lo[L] = (int)off;
   t.n_nodes = off;
-  t.levoff.ensure((L + 1) * sizeof(int));
-  upload(t.levoff.ptr, levoff.data(), (L + 1) * sizeof(int));
-  int* d_levoff = t.levoff.as<int>();
+  t.nidx_off.assign(kMaxLevels, -1);
+  const int NN = (int)off;
+  const int g0 = L > 2 ? lv.lo[2] : NN;
+  const int ngroups = (NN - g0) / 4;
+  const int nw = (int)ceil_div(wave_slots(NN), 64);
   t.code.ensure(off * sizeof(uint64_t));
   t.nlevel.ensure(off * sizeof(int));
   t.bot.ensure(off * sizeof(int));
@@ -1375,115 +1732,61 @@ void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmi
   t.child.ensure(off * sizeof(int));
   t.flags.ensure(off * sizeof(int));
   t.coll.ensure(off * 9 * sizeof(int));
+  t.crange.ensure((off * 9 + 1) * sizeof(int2));
   t.xmid.ensure(off * sizeof(double));
   t.ymid.ensure(off * sizeof(double));
   t.row.ensure(off * sizeof(int));
+  t.rowinfo.ensure((4 * (int64_t)ngroups + 1) * sizeof(int2));
   t.m2l.ensure(off * kNumM2L * sizeof(int));
   t.evalid.ensure(off * sizeof(int));
-  hipLaunchKernelGGL(k_nodes_a, dim3(grid_for(off)), dim3(BS), 0, s, t.p_code.as<uint64_t>(),
-                     t.p_kind.as<int>(), d_poff, d_levoff, L, t.code.as<uint64_t>(),
-                     t.nlevel.as<int>(), t.flags.as<int>());
-  FMM_LAUNCH_CHECK();
-  NodeIdx ni{};
-  int64_t ntab = 0;
-  for (int d = 0; d < kMaxLevels; ++d) ni.off[d] = -1;
-  for (int d = 1; d < L && d <= kIdxDepth; ++d) {
-    if (t.lev[d].n_nodes == ((int64_t)1 << (2 * d))) continue;   // full: direct
-    ni.off[d] = ntab;
-    ntab += (int64_t)1 << (2 * d);
-  }
-  t.nidx_off.assign(ni.off, ni.off + kMaxLevels);
-  if (ntab > 0) {
+  t.evalnode.ensure(off * sizeof(int));
+  t.upnodes.ensure(off * sizeof(int));
+  t.w_rng.ensure(2 * off * sizeof(int));
+  t.w_wave.ensure(3 * (int64_t)nw * sizeof(int));
+  int* rb = t.w_rng.as<int>();
+  int* rt = rb + off;
+  int* wcnt = t.w_wave.as<int>();
+  if (t.bm_index) {
+    const BmCells cells{t.index(), t.bm.as<uint32_t>()};
+    hipLaunchKernelGGL(k_bm_nodes, dim3(grid_for(8 * (int64_t)bm_wo(L - 1))), dim3(BS), 0, s,
+                       cells, L - 2, nn, t.code.as<uint64_t>(), t.nlevel.as<int>(),
+                       t.flags.as<int>(), rb, rt);
+    FMM_LAUNCH_CHECK();
+    node_arrays(t, cells, lv, g0, nw, rb, rt, wcnt, s);
+  } else {
+    ListCells cells{};
+    int64_t ntab = 0;
+    for (int d = 0; d < kMaxLevels; ++d) cells.off[d] = -1;
+    for (int d = 1; d < L && d <= kIdxDepth; ++d) {
+      if (t.lev[d].n_nodes == ((int64_t)1 << (2 * d))) continue;   // full: direct
+      cells.off[d] = ntab;
+      ntab += (int64_t)1 << (2 * d);
+    }
+    t.nidx_off.assign(cells.off, cells.off + kMaxLevels);
     t.nidx.ensure(ntab * sizeof(int));
-    FMM_HIP(hipMemsetAsync(t.nidx.ptr, 0xFF, ntab * sizeof(int), s));
-    ni.tab = t.nidx.as<int>();
-    hipLaunchKernelGGL(k_node_index, dim3(grid_for(off)), dim3(BS), 0, s, t.code.as<uint64_t>(),
-                       t.nlevel.as<int>(), NN, ni, t.nidx.as<int>());
+    fill_i32(t.nidx.as<int>(), ntab, -1, s);
+    cells.code = t.code.as<uint64_t>();
+    cells.lv = lv;
+    cells.tab = t.nidx.as<int>();
+    cells.p_code = t.p_code.as<uint64_t>();
+    cells.p_kind = t.p_kind.as<int>();
+    hipLaunchKernelGGL(k_list_nodes, dim3(grid_for(off)), dim3(BS), 0, s, cells, L, nn,
+                       t.code.as<uint64_t>(), t.nlevel.as<int>(), t.flags.as<int>(), rb, rt,
+                       t.nidx.as<int>());
     FMM_LAUNCH_CHECK();
+    node_arrays(t, cells, lv, g0, nw, rb, rt, wcnt, s);
   }
-  hipLaunchKernelGGL(k_cell_ranges_init, dim3(grid_for(off)), dim3(BS), 0, s, NN, nn,
-                     t.bot.as<int>(), t.top.as<int>());
-  FMM_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_cell_ranges, dim3(grid_for(n)), dim3(BS), 0, s, keys, sc, nn,
-                     t.code.as<uint64_t>(), d_levoff, L, ni, t.bot.as<int>(), t.top.as<int>());
-  FMM_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_nodes_b, dim3(ceil_div(off, 64)), dim3(64), 0, s, t.p_code.as<uint64_t>(),
-                     t.p_kind.as<int>(), d_poff, d_levoff, L, keys, nn, xmin, ymin, w0, ni,
-                     t.code.as<uint64_t>(), t.flags.as<int>(), t.bot.as<int>(), t.top.as<int>(),
-                     t.parent.as<int>(), t.child.as<int>(), t.coll.as<int>(), t.xmid.as<double>(),
-                     t.ymid.as<double>());
-  FMM_LAUNCH_CHECK();
-  t.crange.ensure(((int64_t)off * 9 + 1) * sizeof(int2));
-  hipLaunchKernelGGL(k_coll_ranges, dim3(grid_for((int64_t)off * 9)), dim3(BS), 0, s,
-                     (int)(off * 9), t.coll.as<int>(), t.bot.as<int>(), t.top.as<int>(),
-                     t.crange.as<int2>());
-  FMM_LAUNCH_CHECK();
-
-  // -- density rows ------------------------------------------------------------------
-  t.w_flag.ensure((off + 1) * sizeof(int));
-  t.w_rank.ensure((off + 1) * sizeof(int));
-  flag = t.w_flag.as<int>();
-  rank = t.w_rank.as<int>();
-  const int g0 = L > 2 ? levoff[2] : NN;
-  const int ngroups = (NN - g0) / 4;
-  if (ngroups > 0) {
-    hipLaunchKernelGGL(k_group_flags, dim3(grid_for(ngroups)), dim3(BS), 0, s, t.flags.as<int>(),
-                       g0, ngroups, d_levoff, L, flag, cnt + CNT_LR);
-    FMM_LAUNCH_CHECK();
-    exclusive_scan_i32(flag, rank, ngroups, cnt + CNT_ROWS, t.pw, s);
-  }
-  t.rownode.ensure((4 * (int64_t)ngroups + 1) * sizeof(int));
-  hipLaunchKernelGGL(k_rows, dim3(grid_for(off)), dim3(BS), 0, s, flag, rank, g0, NN,
-                     t.row.as<int>(), t.rownode.as<int>());
-  FMM_LAUNCH_CHECK();
-  if (L > 2) {
-    hipLaunchKernelGGL(k_m2l_lists, dim3(grid_for((int64_t)(NN - g0) * kNumM2L)), dim3(BS), 0, s,
-                       t.code.as<uint64_t>(), t.flags.as<int>(), t.row.as<int>(), d_levoff, L,
-                       ni, t.m2l.as<int>());
-    FMM_LAUNCH_CHECK();
-  }
-
-  // -- evaluation boxes and S2M boxes ---------------------------------------------------
-  t.w_a.ensure((off + 1) * 2 * sizeof(int));
-  int* f2 = t.w_a.as<int>();
-  int* r2 = f2 + off;
-  hipLaunchKernelGGL(k_flag_bit, dim3(grid_for(off)), dim3(BS), 0, s, t.flags.as<int>(), NN,
-                     (int)NF_LEAF, flag);
-  FMM_LAUNCH_CHECK();
-  exclusive_scan_i32(flag, rank, off, cnt + CNT_EVAL, t.pw, s);
-  hipLaunchKernelGGL(k_up_flag, dim3(grid_for(off)), dim3(BS), 0, s, t.flags.as<int>(),
-                     t.row.as<int>(), NN, f2);
-  FMM_LAUNCH_CHECK();
-  exclusive_scan_i32(f2, r2, off, cnt + CNT_UP, t.pw, s);
-  read_counts(t, cnt + CNT_ROWS, CNT_N - CNT_ROWS, hc + CNT_ROWS, s);
-  t.n_rows = ngroups > 0 ? 4 * (int64_t)hc[CNT_ROWS] : 0;
-  t.row_off.assign(L + 1, 0);
-  for (int d = 0; d < L; ++d) t.row_off[d + 1] = t.row_off[d] + hc[CNT_LR + d];
-  FMM_REQUIRE(t.row_off[L] == t.n_rows, FMM_E_INTERNAL, "tree: row count mismatch");
-  t.n_eval = hc[CNT_EVAL];
-  t.n_up = hc[CNT_UP];
-  t.rowinfo.ensure((t.n_rows + 1) * sizeof(int2));
-  if (t.n_rows > 0) {
-    hipLaunchKernelGGL(k_row_info, dim3(grid_for(t.n_rows)), dim3(BS), 0, s, t.rownode.as<int>(),
-                       (int)t.n_rows, t.flags.as<int>(), t.child.as<int>(), t.row.as<int>(),
-                       t.rowinfo.as<int2>());
-    FMM_LAUNCH_CHECK();
-  }
-  t.evalnode.ensure((t.n_eval + 1) * sizeof(int));
-  t.upnodes.ensure((t.n_up + 1) * sizeof(int));
-  hipLaunchKernelGGL(k_list_scatter, dim3(grid_for(off)), dim3(BS), 0, s, flag, rank, NN,
-                     t.evalnode.as<int>(), t.evalid.as<int>());
-  FMM_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_list_scatter, dim3(grid_for(off)), dim3(BS), 0, s, f2, r2, NN,
-                     t.upnodes.as<int>(), (int*)nullptr);
-  FMM_LAUNCH_CHECK();
   ++t.build_id;
   t.built = true;
 }
 
 void tree_init_device() {
   SlotOffsets so;
-  for (int q = 0; q < kNumM2L; ++q) m2l_slot_offset(q, &so.ox[q], &so.oy[q]);
+  for (int q = 0; q < kNumM2L; ++q) {
+    m2l_slot_offset(q, &so.ox[q], &so.oy[q]);
+    so.dx[q] = morton((uint32_t)so.ox[q], 0);
+    so.dy[q] = morton(0, (uint32_t)so.oy[q]);
+  }
   FMM_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_slot_off), &so, sizeof so));
 }
 
