@@ -1742,44 +1742,64 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_local_level(
 // previous result through a double-buffered LDS tile.
 constexpr int kMaxSmallPhases = 6;   // 4 M2M + 2 pseudo-inverse factors
 
-// Phases 0 .. nb-1 take their B column from row brow + i of `bbase`, where
-// brow is the lane's box's source row (-1: none); these rows are loaded once
-// per block, cooperatively and with 16-byte loads, into the LDS tile `btile`.
-// Later phases are chained.  `opA(i)` is the operator of phase i.  A wave
-// uses only its own 16 operator rows, so it loads them straight into
-// registers, three phases ahead, with 16-byte loads: step 2 m + h of lane
-// group kq multiplies k = 8 m + 2 kq + h.  (All six phases ahead was slower:
-// the B tile fill then waits for every operator load issued before it.)  The B tiles are box-major in LDS
-// (row padded to PD + 2), so that B arrives in the same order with one
-// 16-byte LDS read per step pair.  (Staging the operator in LDS left every
-// MFMA waiting on its own LDS read, with one block per CU to hide nothing.)
+// Phases 0 .. nb-1 take their B column from row brow + i of `bbase` of the
+// box's source row (-1: none); these rows are loaded once per block,
+// cooperatively and with 16-byte loads, into the LDS tile `btile`: a thread
+// loads pair threadIdx.x mod PD/2 of the rows of boxes small_box(0) and
+// small_box(1), brow of which it is given.  Later phases are chained.
+// `opA(i)` is the operator of phase i.  A wave uses only its own 16 operator
+// rows, so it loads them straight into registers, three phases ahead, with
+// 16-byte loads: step 2 m + h of lane group kq multiplies k = 8 m + 2 kq + h.
+// (All six phases ahead was slower: the B tile fill then waits for every
+// operator load issued before it.)  The B tiles are box-major in LDS (row
+// padded to PD + 2), so that B arrives in the same order with one 16-byte LDS
+// read per step pair.  (Staging the operator in LDS left every MFMA waiting on
+// its own LDS read, with one block per CU to hide nothing.)
+//
+// What bounds these kernels is the chain from the row records through the
+// operands to the last phase, so the loads are issued as soon as their
+// addresses are known and absent rows read zeros instead of branching around
+// their loads: with a branch per piece of the tile its loads ran one after
+// another (1M points, PD 64, per level: upward 12.3 -> 9.6 us, downward 7.6 ->
+// 7.1; 100K points, PD 32: 7.0 -> 4.7 and 4.7 -> 4.3).
 constexpr int kSmallPad = 2;
+template <int PD>
+__device__ __forceinline__ int small_box(int h) {
+  return threadIdx.x / (PD / 2) + 8 * h;   // 4 PD threads: 8 boxes per half
+}
+template <int PD>
+struct SmallOps {
+  dv2 a[3][PD / 8];   // operator rows of phases i, i + 1, i + 2 (n <= kMaxSmallPhases)
+  __device__ __forceinline__ void load(int i, const double* __restrict__ A) {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double* r = A + (16 * w + (l & 15)) * PD + 2 * (l >> 4);
+#pragma unroll
+    for (int m = 0; m < PD / 8; ++m) a[i][m] = *reinterpret_cast<const dv2*>(r + 8 * m);
+  }
+};
 template <int PD, int NB, class OpFn>
 __device__ __forceinline__ void run_small(
-    int n, int nb, OpFn opA, const double* __restrict__ bbase, int brow, d4& acc,
-    double (&bbuf)[2][16][PD + kSmallPad], double (&btile)[NB][16][PD + kSmallPad],
-    int (&srow)[16]) {
-  constexpr int KM = PD / 8, NT = 64 * (PD / 16), H = PD / 2;
+    int n, int nb, OpFn opA, SmallOps<PD>& ops, const double* __restrict__ bbase,
+    const int (&brow)[2], d4& acc, double (&bbuf)[2][16][PD + kSmallPad],
+    double (&btile)[NB][16][PD + kSmallPad]) {
+  constexpr int KM = PD / 8, H = PD / 2;
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int col = l & 15, kq = l >> 4;
-  auto load_rows = [&](dv2 (&a)[KM], const double* __restrict__ A) {
-    const double* r = A + (16 * w + col) * PD + 2 * kq;
+  const int k2 = threadIdx.x % H;
+  dv2 tile[NB][2];
+  if (nb > 0) {
 #pragma unroll
-    for (int m = 0; m < KM; ++m) a[m] = *reinterpret_cast<const dv2*>(r + 8 * m);
-  };
-  dv2 ar[3][KM];   // operator rows of phases i, i + 1, i + 2 (n <= kMaxSmallPhases)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
-    if (i < n) load_rows(ar[i], opA(i));
-  if (w == 0 && kq == 0) srow[col] = brow;
-  __syncthreads();
-  for (int e = threadIdx.x; e < NB * 16 * H; e += NT) {
-    const int i = e / (16 * H), rem = e - i * 16 * H;
-    const int box = rem / H, k2 = rem - box * H;
-    const int rr = srow[box];
-    dv2 v = dv2{0.0, 0.0};
-    if (rr >= 0 && i < nb) v = *reinterpret_cast<const dv2*>(bbase + (int64_t)(rr + i) * PD + 2 * k2);
-    *reinterpret_cast<dv2*>(&btile[i][box][2 * k2]) = v;
+      for (int h = 0; h < 2; ++h)
+        tile[i][h] = *reinterpret_cast<const dv2*>(
+            (brow[h] >= 0 ? bbase + (int64_t)(brow[h] + i) * PD : c_zero_row) + 2 * k2);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<dv2*>(&btile[i][small_box<PD>(h)][2 * k2]) = tile[i][h];
   }
 #pragma unroll
   for (int i = 0; i < kMaxSmallPhases; ++i) {
@@ -1808,10 +1828,10 @@ __device__ __forceinline__ void run_small(
     __builtin_amdgcn_sched_barrier(0);   // every B read issued before the MFMA chain
 #pragma unroll
     for (int m = 0; m < KM; ++m) {
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i % 3][m].x, b[m].x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i % 3][m].y, b[m].y, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ops.a[i % 3][m].x, b[m].x, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(ops.a[i % 3][m].y, b[m].y, acc, 0, 0, 0);
     }
-    if (i + 3 < n) load_rows(ar[i % 3], opA(i + 3));
+    if (i + 3 < n) ops.load(i % 3, opA(i + 3));
   }
 }
 
@@ -1832,20 +1852,29 @@ __device__ __forceinline__ void mult_small_unit(
   const int rl = bx * 16 + col;
   const bool active = rl < nrows;
   const int64_t r = row0 + rl;
-  const int2 ri = active ? rowinfo[r] : make_int2(-1, 0);
-  const int f = ri.y;
-  const int crow = ri.x;
-  const double* src = (active && (f & NF_UP)) ? check + r * PD : nullptr;
-  d4 acc;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) acc[v] = src ? src[16 * w + 4 * v + kq] : 0.0;
   const int nm = with_m2m ? 4 : 0;
   auto opA = [&](int k) -> const double* {
     return opsL + (int64_t)(k < nm ? OP_M2M + k : OP_PINV1 + (k - nm)) * PD * PD;
   };
+  // the records of this lane's row and of the two it loads children of (past
+  // the level's end: its last row, unused)
+  const int2 ri = rowinfo[row0 + min(rl, nrows - 1)];
+  int brow[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    brow[h] = rowinfo[row0 + min(bx * 16 + small_box<PD>(h), nrows - 1)].x;
+  __builtin_amdgcn_sched_barrier(0);
+  SmallOps<PD> ops;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (i < nm + 2) ops.load(i, opA(i));
+  __builtin_amdgcn_sched_barrier(0);
+  const double* src = active && (ri.y & NF_UP) ? check + r * PD : c_zero_row;
+  d4 acc;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) acc[v] = src[16 * w + 4 * v + kq];
   __shared__ __attribute__((aligned(16))) double btile[4][16][PD + kSmallPad];
-  __shared__ int srow[16];
-  run_small<PD, 4>(nm + 2, nm, opA, mult, crow, acc, bbuf, btile, srow);
+  run_small<PD, 4>(nm + 2, nm, opA, ops, mult, brow, acc, bbuf, btile);
   double part = acc[0] + acc[1] + acc[2] + acc[3];
   part += __shfl_xor(part, 16, 64);
   part += __shfl_xor(part, 32, 64);
@@ -1896,23 +1925,36 @@ __device__ __forceinline__ void local_small_unit(
   const int g = g0 + 4 * q + c;
   const int gs = q < ngroups ? g : g0;   // a valid node for the independent loads
   const int fl = flags[gs];
-  const int par = parent[gs];
-  const bool active = q < ngroups && !(fl & NF_FAKE);
+  int fb[2], brow[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int qb = (bx >> 2) * 16 + small_box<PD>(h);
+    const int gb = g0 + 4 * min(qb, ngroups - 1) + c;
+    fb[h] = flags[gb];
+    brow[h] = parent[gb];
+  }
   d4 acc;
   const double* src = ple + (int64_t)gs * PD;
 #pragma unroll
   for (int v = 0; v < 4; ++v) acc[v] = src[16 * w + 4 * v + kq];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) acc[v] = active ? acc[v] : 0.0;
-  const int pg = (active && do_l2l) ? par : -1;
+  __builtin_amdgcn_sched_barrier(0);
   const int nl = do_l2l ? 1 : 0;
   auto opA = [&](int k) -> const double* {
     return k < nl ? opsParent + (int64_t)(OP_L2L + c) * PD * PD
                   : opsL + (int64_t)(OP_PINV1 + (k - nl)) * PD * PD;
   };
+  SmallOps<PD> ops;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (i < nl + 2) ops.load(i, opA(i));
+  __builtin_amdgcn_sched_barrier(0);
+  const bool active = q < ngroups && !(fl & NF_FAKE);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) acc[v] = active ? acc[v] : 0.0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) brow[h] = fb[h] & NF_FAKE ? -1 : brow[h];
   __shared__ __attribute__((aligned(16))) double btile[1][16][PD + kSmallPad];
-  __shared__ int srow[16];
-  run_small<PD, 1>(nl + 2, nl, opA, le, pg, acc, bbuf, btile, srow);
+  run_small<PD, 1>(nl + 2, nl, opA, ops, le, brow, acc, bbuf, btile);
   // the nodes above level 2 have no local expansion: zeros, as for fake nodes
   if (!do_l2l && bx == 0)
     for (int e = threadIdx.x; e < g0 * PD; e += 64 * (PD / 16)) le[e] = 0.0;
