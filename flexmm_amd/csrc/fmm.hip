@@ -713,7 +713,10 @@ __device__ __forceinline__ M2LSetup m2l_setup(const LevelTable& lt, const int* _
 // sibling groups (in Morton order) of one level and child position, the
 // boxes are sorted by their set of used offsets (ties by position); boxes
 // without any (and fake nodes) go last.  One block per chunk: bitonic sort
-// of (40-bit offset mask << 11 | index) in LDS.
+// of (40-bit offset mask << 11 | index).  Few blocks run, so what each reads
+// and how long its chain is bounds the kernel: the masks come with the tree
+// (from the 160-byte partner lists, and with every step of the sort in LDS, it
+// took 30 us for 1M clustered points, now 17).
 constexpr int kM2LOrderChunk = 2048;
 struct M2LOrderTable {
   int nlev;
@@ -724,9 +727,9 @@ struct M2LOrderTable {
   int poff[kMaxLevels];
 };
 constexpr int kM2LOrderThreads = 1024;
-__global__ __launch_bounds__(kM2LOrderThreads) void k_m2l_order(M2LOrderTable ot, const int* __restrict__ flags,
-                                                   const int* __restrict__ m2l,
-                                                   int* __restrict__ perm) {
+__global__ __launch_bounds__(kM2LOrderThreads) void k_m2l_order(M2LOrderTable ot,
+                                                                const uint64_t* __restrict__ m2lmask,
+                                                                int* __restrict__ perm) {
   __shared__ uint64_t key[kM2LOrderChunk];
   const int b = blockIdx.x;
   int li = 0;
@@ -738,45 +741,61 @@ __global__ __launch_bounds__(kM2LOrderThreads) void k_m2l_order(M2LOrderTable ot
   const int q0 = chunk * kM2LOrderChunk;
   const int cnt = min(kM2LOrderChunk, ng - q0);
   static_assert(kNumM2L == 40 && kM2LOrderChunk <= 2048, "key layout: 40 + 11 bits");
-#pragma unroll 2
-  for (int i = threadIdx.x; i < kM2LOrderChunk; i += kM2LOrderThreads) {
+#pragma unroll
+  for (int j = 0; j < kM2LOrderChunk / kM2LOrderThreads; ++j) {
+    const int i = j * kM2LOrderThreads + threadIdx.x;
     uint64_t k = ~0ull;
     if (i < cnt) {
-      const int g = ot.g0[li] + 4 * (q0 + i) + c;
-      const int4* lst = reinterpret_cast<const int4*>(m2l + (int64_t)g * kNumM2L);
-      int4 e[kNumM2L / 4];
-#pragma unroll
-      for (int j = 0; j < kNumM2L / 4; ++j) e[j] = lst[j];
-      uint64_t mask = 0;
-#pragma unroll
-      for (int j = 0; j < kNumM2L / 4; ++j)
-        mask |= (uint64_t)((e[j].x >= 0) | (e[j].y >= 0) << 1 | (e[j].z >= 0) << 2 |
-                           (e[j].w >= 0) << 3)
-                << (4 * j);
-      if (flags[g] & NF_FAKE) mask = 0;
+      const uint64_t mask = m2lmask[ot.g0[li] + 4 * (q0 + i) + c];   // 0 for a fake node
       k = ((mask ? mask : (1ull << 52) - 1) << 11) | (uint64_t)i;
     }
     key[i] = k;
   }
   __syncthreads();
-  for (int size = 2; size <= kM2LOrderChunk; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int t = threadIdx.x; t < kM2LOrderChunk / 2; t += kM2LOrderThreads) {
-        // stride is a power of two: lo = 2 stride (t / stride) + t % stride
-        const int lo = ((t & ~(stride - 1)) << 1) | (t & (stride - 1));
-        const int hi = lo + stride;
-        const bool up = (lo & size) == 0;
-        const uint64_t a = key[lo], e = key[hi];
-        if ((a > e) == up) {
-          key[lo] = e;
+  // Wave w sorts elements 128 w + l and 128 w + 64 + l on lane l: strides up
+  // to 64 stay in registers, the others (10 of 66 steps) go through LDS with a
+  // barrier each.  Past the power of two that holds the boxes all keys are the
+  // highest.
+  const int l = threadIdx.x & 63;
+  const int e0 = (threadIdx.x >> 6) * 128 + l;
+  uint64_t k0 = key[e0], k1 = key[e0 + 64];
+  auto order = [&](uint64_t a, uint64_t b, bool low) { return (a < b) == low ? a : b; };
+  for (int size = 2; size <= kM2LOrderChunk && size < 2 * cnt; size <<= 1) {
+    const bool up0 = (e0 & size) == 0, up1 = ((e0 + 64) & size) == 0;
+    if (size > 128) {
+      __syncthreads();   // every wave has read its elements
+      key[e0] = k0;
+      key[e0 + 64] = k1;
+      __syncthreads();
+      for (int stride = size >> 1; stride > 64; stride >>= 1) {
+        const int t = threadIdx.x;   // one pair each
+        const int lo = ((t & ~(stride - 1)) << 1) | (t & (stride - 1)), hi = lo + stride;
+        const uint64_t a = key[lo], b = key[hi];
+        if ((a > b) == ((lo & size) == 0)) {
+          key[lo] = b;
           key[hi] = a;
         }
+        __syncthreads();
       }
-      __syncthreads();
+      k0 = key[e0];
+      k1 = key[e0 + 64];
+    }
+    if (size > 64 && (k0 > k1) == up0) {   // stride 64: both elements are this lane's
+      const uint64_t k = k0;
+      k0 = k1;
+      k1 = k;
+    }
+    for (int stride = min(size >> 1, 32); stride > 0; stride >>= 1) {
+      const uint64_t p0 = __shfl_xor((unsigned long long)k0, stride, 64);
+      const uint64_t p1 = __shfl_xor((unsigned long long)k1, stride, 64);
+      const bool lower = (l & stride) == 0;
+      k0 = order(k0, p0, lower == up0);
+      k1 = order(k1, p1, lower == up1);
     }
   }
-  for (int i = threadIdx.x; i < cnt; i += kM2LOrderThreads)
-    perm[ot.poff[li] + c * ng + q0 + i] = q0 + (int)(key[i] & 2047u);
+  const int at = ot.poff[li] + c * ng + q0;
+  if (e0 < cnt) perm[at + e0] = q0 + (int)(k0 & 2047u);
+  if (e0 + 64 < cnt) perm[at + e0 + 64] = q0 + (int)(k1 & 2047u);
 }
 
 // FP64 M2L in the compressed form (FMM2D_M2L_SVD): slots whose rank table entry is r > 0 are applied in
@@ -3562,8 +3581,7 @@ static void m2l_prepare(Plan& P, const M2LTables& T, hipStream_t s) {
   if (!T.adaptive || P.perm_tree == t.build_id) return;
   P.m2lperm.ensure((T.perm_len + 1) * sizeof(int));
   hipLaunchKernelGGL(k_m2l_order, dim3(T.order_blocks), dim3(kM2LOrderThreads), 0, s, T.ot,
-                     t.flags.as<int>(),
-                     t.m2l.as<int>(), P.m2lperm.as<int>());
+                     t.m2lmask.as<uint64_t>(), P.m2lperm.as<int>());
   FMM_LAUNCH_CHECK();
   P.perm_tree = t.build_id;
 }

@@ -90,6 +90,7 @@ struct Tree {
   DevBuf rowinfo;  // int2[n_rows]: row of the node's first child (or -1), node flags
   std::vector<int64_t> row_off;  // first row of each level (size L+1)
   DevBuf m2l;      // i32[40] multipole rows of the M2L partners or -1 (real nodes, level >= 2)
+  DevBuf m2lmask;  // u64 which of the 40 are present (trees that are not complete)
   DevBuf evalid;   // i32 index among evaluation boxes (NF_LEAF) or -1
   DevBuf evalnode; // i32[n_eval]
   DevBuf upnodes;  // i32[n_up] nodes with NF_UP

@@ -1042,7 +1042,8 @@ __global__ __launch_bounds__(BS) void k_node_slots(
     const int* __restrict__ nlev, const int* __restrict__ flags, const int* __restrict__ row,
     const int* __restrict__ child,
     const int* __restrict__ coll, const int* __restrict__ bot, const int* __restrict__ top,
-    int* __restrict__ m2l, int2* __restrict__ crange, int2* __restrict__ rowinfo) {
+    int* __restrict__ m2l, uint64_t* __restrict__ m2lmask, int2* __restrict__ crange,
+    int2* __restrict__ rowinfo) {
   const int64_t tid = (int64_t)xcd_block(blockIdx.x, gridDim.x, 0) * BS + threadIdx.x;
   const int g = (int)(tid / kSlotLanes);
   const int j = (int)(tid % kSlotLanes);
@@ -1065,11 +1066,16 @@ __global__ __launch_bounds__(BS) void k_node_slots(
     uint64_t e;
     q[u] = s < kNumM2L && !(f & NF_FAKE) && slot_cell(cg, d, s, &e) ? cells.node(d, e) : -1;
   }
+  uint64_t mask = 0;
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
     const int s = j + u * kSlotLanes;
-    if (s < kNumM2L) m2l[(int64_t)g * kNumM2L + s] = q[u] >= 0 ? row[q[u]] : -1;
+    const int r = q[u] >= 0 ? row[q[u]] : -1;
+    if (s < kNumM2L) m2l[(int64_t)g * kNumM2L + s] = r;
+    const unsigned long long b = __ballot(r >= 0) >> (threadIdx.x & (64 - kSlotLanes));
+    mask |= (uint64_t)(b & ((1u << kSlotLanes) - 1u)) << (u * kSlotLanes);
   }
+  if (j == 0) m2lmask[g] = mask;
 }
 
 __global__ __launch_bounds__(BS) void k_locate(const double* __restrict__ tx,
@@ -1548,7 +1554,8 @@ static void node_arrays(Tree& t, const Cells& cells, const LevOff& lv, int g0, i
   hipLaunchKernelGGL(k_node_slots<Cells>, dim3(grid_for((int64_t)NN * kSlotLanes)), dim3(BS), 0, s,
                      cells, lv, L, t.code.as<uint64_t>(), t.nlevel.as<int>(), t.flags.as<int>(),
                      t.row.as<int>(), t.child.as<int>(), t.coll.as<int>(), t.bot.as<int>(), t.top.as<int>(),
-                     t.m2l.as<int>(), t.crange.as<int2>(), t.rowinfo.as<int2>());
+                     t.m2l.as<int>(), t.m2lmask.as<uint64_t>(), t.crange.as<int2>(),
+                     t.rowinfo.as<int2>());
   FMM_LAUNCH_CHECK();
   int64_t v[3 + kMaxLevels];
   mb.take(3 + std::max(0, L - 2), seq, s, v);
@@ -1738,6 +1745,7 @@ void tree_build(Tree& t, const double* x, const double* y, int64_t n, double xmi
   t.row.ensure(off * sizeof(int));
   t.rowinfo.ensure((4 * (int64_t)ngroups + 1) * sizeof(int2));
   t.m2l.ensure(off * kNumM2L * sizeof(int));
+  t.m2lmask.ensure(off * sizeof(uint64_t));
   t.evalid.ensure(off * sizeof(int));
   t.evalnode.ensure(off * sizeof(int));
   t.upnodes.ensure(off * sizeof(int));
