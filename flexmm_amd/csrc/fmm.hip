@@ -2000,10 +2000,10 @@ constexpr int kSmallLevelRows = 4096;
 
 // ---------------------------------------------------------------------------
 // Targets: locate, count per evaluation box, scatter into box order.
-// Node lookup by (depth, cell code) for target location: direct on a full
-// level, through the bitmap index on the others of a tree that has one; in a
-// deeper tree a dense table where the build made one, else a binary search in
-// the level's sorted codes.
+// Node lookup by (depth, cell code) for target location in trees without the
+// bitmap index: direct on a full level, a dense table on the other levels
+// where the tree build made one, else a binary search in the level's sorted
+// codes.
 struct LocateTable {
   int L;
   int full_depth;   // a complete tree's leaf depth (evaluation box = leaf code), else -1
@@ -2012,12 +2012,12 @@ struct LocateTable {
   int64_t tab_off[kMaxLevels];
   const int* tab;
   const uint64_t* code;
-  BmIndex ix;       // pp null: no bitmap index
+  const uint32_t* bm;   // split cells as bitmaps, with the node index ix; else null
+  BmIndex ix;
 };
 __device__ __forceinline__ int locate_node(const LocateTable& lt, int d, uint64_t c) {
   const int64_t nl = lt.levoff[d + 1] - lt.levoff[d];
   if (d < 16 && nl == ((int64_t)1 << (2 * d))) return lt.levoff[d] + (int)c;
-  if (lt.ix.pp) return lt.ix.node(d, c);
   if (lt.tab_off[d] >= 0) return lt.tab[lt.tab_off[d] + (int64_t)c];
   const uint64_t* a = lt.code + lt.levoff[d];
   int64_t lo = 0, hi = nl;
@@ -2038,7 +2038,9 @@ __device__ __forceinline__ int locate_node(const LocateTable& lt, int d, uint64_
 // that land in the same box share one atomic (targets arrive spatially
 // coherent, so a wave touches few boxes).  In a complete tree the first leaf
 // on the path is at the leaf depth D and its evaluation box is its code, so
-// the recurrence alone gives the box.
+// the recurrence alone gives the box.  In a tree with bitmaps it is the first
+// cell that is not split: one word per depth, all read at once, then one node
+// lookup.
 __global__ __launch_bounds__(256) void k_locate_count(const double* __restrict__ tx,
                                                      const double* __restrict__ ty, int64_t nt,
                                                      LocateTable lt,
@@ -2067,6 +2069,31 @@ __global__ __launch_bounds__(256) void k_locate_count(const double* __restrict__
       w = h;
     }
     e = (int)c;
+  } else if (act && lt.bm) {
+    const double x = tx[i], y = ty[i];
+    double xmin = lt.xmin, ymin = lt.ymin, w = lt.w0;
+    uint32_t c = 0, split[kBmMaxD + 1];
+#pragma unroll
+    for (int d = 0; d <= kBmMaxD; ++d)
+      if (d <= lt.L - 2) {
+        split[d] = lt.bm[bm_wo(d) + (int)(c >> 5)] >> (c & 31);
+        const double h = 0.5 * w;
+        const double xm = xmin + h, ym = ymin + h;
+        const int bx = x > xm, by = y > ym;
+        c = (c << 2) | (uint32_t)(2 * bx + by);
+        xmin = bx ? xm : xm - h;
+        ymin = by ? ym : ym - h;
+        w = h;
+      }
+    int dl = 0;
+    bool in = true;
+#pragma unroll
+    for (int d = 0; d <= kBmMaxD; ++d)
+      if (d <= lt.L - 2) {
+        in = in && (split[d] & 1u);
+        dl += in ? 1 : 0;
+      }
+    e = evalid[lt.ix.node(dl, c >> (2 * (lt.L - 1 - dl)))];
   } else if (act) {
     const double x = tx[i], y = ty[i];
     int g = 0;
@@ -2113,28 +2140,36 @@ __global__ __launch_bounds__(256) void k_locate_count(const double* __restrict__
     }
     e = evalid[g];
   }
-  // Targets in a coherent order: group the wave's lanes by box with ballots
-  // (no memory traffic), then let every group's lowest lane add the group
-  // size, with one atomic instruction for all groups.  Targets in random order
-  // (more runs of equal boxes than kMaxRuns) take one atomic per lane: the
-  // ballot loop would run up to 64 times for groups of one.
+  // Targets in a coherent order: lanes of one box share an atomic by their
+  // group's lowest lane (the kernel is bound by the atomics' returns).  Few
+  // runs of equal boxes are grouped with ballots, one box at a time, which also
+  // joins runs of the same box; more take an atomic per run, down to one per
+  // lane in random order (1M targets on a grid, 4 in a row per box: 42 us with
+  // an atomic per lane there, 20 per run).
   constexpr int kMaxRuns = 16;
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
   unsigned long long pending = __ballot(act);
   int leader = lane, inrank = 0, gsize = 1;
   const int eprev = __shfl_up(e, 1, 64);
-  const int runs = __popcll(__ballot(act && (lane == 0 || e != eprev)));
-  while (runs <= kMaxRuns && pending) {
-    const int ld = __builtin_ctzll(pending);
-    const int key = __builtin_amdgcn_readlane(e, ld);
-    const unsigned long long same = __ballot(act && e == key) & pending;
-    if (same >> lane & 1ull) {
-      leader = ld;
-      inrank = __popcll(same & below);
+  const unsigned long long heads = __ballot(act && (lane == 0 || e != eprev));
+  if (__popcll(heads) <= kMaxRuns) {
+    while (pending) {
+      const int ld = __builtin_ctzll(pending);
+      const int key = __builtin_amdgcn_readlane(e, ld);
+      const unsigned long long same = __ballot(act && e == key) & pending;
+      if (same >> lane & 1ull) {
+        leader = ld;
+        inrank = __popcll(same & below);
+      }
+      if (lane == ld) gsize = __popcll(same);
+      pending &= ~same;
     }
-    if (lane == ld) gsize = __popcll(same);
-    pending &= ~same;
+  } else if (act) {   // the active lanes are the first ones
+    const unsigned long long upto = below | 1ull << lane, next = heads & ~upto;
+    leader = 63 - __builtin_clzll(heads & upto);
+    inrank = lane - leader;
+    gsize = (next ? __builtin_ctzll(next) : __popcll(pending)) - lane;
   }
   int base = 0;
   if (act && lane == leader) base = atomicAdd(&tcnt[e], gsize);
@@ -4003,7 +4038,10 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
     lt.tab_off[d] = d < (int)t.nidx_off.size() ? t.nidx_off[d] : -1;
   lt.tab = t.nidx.as<int>();
   lt.code = t.code.as<uint64_t>();
-  if (t.bm_index) lt.ix = t.index();
+  if (t.bm_index) {
+    lt.bm = t.bm.as<uint32_t>();
+    lt.ix = t.index();
+  }
   hipLaunchKernelGGL(k_locate_count, dim3(grid256(nt)), dim3(256), 0, s, tx, ty, nt, lt,
                      t.flags.as<int>(), t.child.as<int>(), t.xmid.as<double>(),
                      t.ymid.as<double>(), t.evalid.as<int>(), w.tnode,

@@ -27,6 +27,7 @@ enum NodeFlag : int {
 // node of rank r are the nodes 1 + 4 r .. 4 + 4 r.  Each depth starts at a
 // block: kBmBlock words up to depth 6, 4^d / 32 from depth 7.
 constexpr int kBmBlock = 256;
+constexpr int kBmMaxD = 11;   // deepest split cells of such a tree
 __host__ __device__ constexpr int bm_wo(int d) {   // first word of depth d
   return d <= 7 ? kBmBlock * d : 7 * kBmBlock + 512 * (((1 << (2 * (d - 7))) - 1) / 3);
 }

@@ -523,7 +523,6 @@ __global__ __launch_bounds__(BS) void k_p_scatter(const uint64_t* __restrict__ r
 // with the index).
 // Each depth's words start at a multiple of BS, so a block of BS words lies
 // in one depth.
-constexpr int kBmMaxD = 11;
 constexpr int kBmLevels = kBmMaxD + 2;
 static_assert(BS == kBmBlock, "the bitmap kernels take a block of words each");
 __host__ __device__ constexpr int bm_words(int d) { return d <= 2 ? 1 : 1 << (2 * d - 5); }
