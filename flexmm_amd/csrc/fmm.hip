@@ -9,9 +9,9 @@
 //             pseudo-inverse; fmm.py:125-166.
 //   evaluate  target location, targets grouped by leaf, L2T + P2P fused in one
 //             pass; fmm.py:182-199, helpers.py:180-235.
-// Dense contractions run on FP64 MFMA (v_mfma_f64_16x16x4f64) with the
-// operator block staged in LDS; expansions are rows of PD doubles (PD = 32 or
-// 64, p padded with zeros).
+// Dense contractions run on FP64 MFMA (v_mfma_f64_16x16x4f64), their operands
+// streamed from L2 in MFMA operand order (k_ops_pack); expansions are rows of
+// PD doubles (PD = 32 or 64, p padded with zeros).
 #include "bessel.h"
 #include "tree.h"
 

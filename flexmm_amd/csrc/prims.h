@@ -61,11 +61,9 @@ struct PrimWork {
 };
 
 // out[i] = sum_{j<i} in[i]; *total_dev (optional) = sum of all in.
-// in and out may alias.  partials (optional): caller-owned space for
-// scan_partials_i32(n) ints; without it the block partials live in w.
+// in and out may alias.
 void exclusive_scan_i32(const int* in, int* out, int64_t n, int* total_dev, PrimWork& w,
-                        hipStream_t s, int* partials = nullptr);
-int64_t scan_partials_i32(int64_t n);
+                        hipStream_t s);
 
 // p[0..n) = v with a fill kernel (no memset node, so the call can sit in a
 // captured HIP graph).

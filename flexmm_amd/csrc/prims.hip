@@ -131,10 +131,8 @@ void fill_i32(int* p, int64_t n, int v, hipStream_t s) {
   FMM_LAUNCH_CHECK();
 }
 
-int64_t scan_partials_i32(int64_t n) { return n <= kScanSmallMax ? 0 : ceil_div(n, SCAN_TILE); }
-
 void exclusive_scan_i32(const int* in, int* out, int64_t n, int* total_dev, PrimWork& w,
-                        hipStream_t s, int* partials) {
+                        hipStream_t s) {
   if (n <= 0) {
     if (total_dev) fill_i32(total_dev, 1, 0, s);
     return;
@@ -145,11 +143,8 @@ void exclusive_scan_i32(const int* in, int* out, int64_t n, int* total_dev, Prim
     return;
   }
   int64_t nb = ceil_div(n, SCAN_TILE);
-  int* sums = partials;
-  if (!sums) {
-    w.blocksums.ensure(nb * sizeof(int));
-    sums = w.blocksums.as<int>();
-  }
+  w.blocksums.ensure(nb * sizeof(int));
+  int* sums = w.blocksums.as<int>();
   hipLaunchKernelGGL(k_scan_block_sums, dim3(nb), dim3(SCAN_BS), 0, s, in, n, sums);
   FMM_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, s, sums, nb, total_dev);

@@ -1180,7 +1180,7 @@ __global__ __launch_bounds__(BS) void k_full_nodes(
     parent[g] = d > 0 ? full_levoff(d - 1) + (int)(c >> 2) : -1;
     const int ch = leaf ? -1 : full_levoff(d + 1) + 4 * (int)c;
     child[g] = ch;
-    // centre by the reference recurrence (as k_nodes_b)
+    // centre by the reference recurrence (as k_nodes)
     double xm0 = xmin0, ym0 = ymin0, w = w0;
     for (int l = 1; l <= d; ++l) {
       const double h = 0.5 * w;

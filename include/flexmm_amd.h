@@ -249,8 +249,8 @@ int fmm2d_evaluate(void* plan, const double* tx, const double* ty, int64_t nt, i
  * reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments, results and errors as fmm2d_evaluate; the target-side scratch
- * (target boxes, counts, leaf-ordered targets, work items) lives in one
- * device array of the library (about 38 MB, held on each GPU the library runs
+ * (target boxes, counts, leaf order, work items) lives in one
+ * device array of the library (about 36 MB, held on each GPU the library runs
  * on until the process ends), so:
  *   - nt <= 1048576 targets and trees of <= 262144 evaluation boxes (leaves
  *     and X-list parents), else FMM2D_E_LIMIT;
