@@ -615,7 +615,7 @@ def main():
     ek = acc.get("eval_kernel", float("nan"))
     f_eval = f_p2p + f_l2t
     achieved = f_eval / (ek / 1000.0) / 1e12
-    prof_us = profiled_avg_us("k_eval<64, 0, 1, false, false, false>")
+    prof_us = profiled_avg_us("k_eval<64, 0, 1, false, false, false, 1>")
     # tree build: algorithmic bytes = 40 B per source (read x, y; write sorted
     # x, y; keys and permutation) + one write of the node table (252 B per node)
     tree_bytes = 40.0 * N_SRC + 252.0 * r64["nodes"]
