@@ -98,8 +98,10 @@ bool sort_pairs_u64(uint64_t* keys, uint32_t* vals, int64_t n, int threshold, Pr
 namespace sort_detail {
 // C_SEGS: segments of the current round; C_*_PREV: C_ACTIVE, C_FINAL and
 // C_FINAL_BIG as they stood when the round began
-enum { C_NEXT = 0, C_FINAL = 1, C_CHUNKS = 2, C_ACTIVE = 3, C_FINAL_BIG = 4, C_SEGS = 5,
-       C_ACTIVE_PREV = 6, C_FINAL_PREV = 7, C_BIG_PREV = 8, C_COUNT = 9 };
+// C_NEXT and C_FINAL, C_ACTIVE and C_FINAL_BIG are counted in pairs (64 bits)
+enum { C_NEXT = 0, C_FINAL = 1, C_ACTIVE = 2, C_FINAL_BIG = 3, C_CHUNKS = 4, C_SEGS = 5,
+       C_ACTIVE_PREV = 6, C_FINAL_PREV = 7, C_BIG_PREV = 8, C_LONGEST = 9,
+       C_COUNT = 10 };
 }
 constexpr int kSortChunk = 4096;   // keys per chunk of a radix round
 

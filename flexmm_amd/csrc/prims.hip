@@ -162,6 +162,10 @@ constexpr int CHUNK = kSortChunk;
 constexpr int SORT_BS = 256;
 constexpr int kChunkPer = CHUNK / SORT_BS;   // keys per thread of a chunk block
 constexpr int kWaveSortMax = 64;
+// Rounds of more segments than this whose longest spans at most 16 chunks
+// take four of them per block.
+constexpr int kManySegs = 512;
+constexpr int kShortSeg = 16 * CHUNK;
 
 // nseg_host < 0: the round's segments are the C_NEXT of the round before, as
 // the device holds it (a round launched before the host read the counts).
@@ -183,6 +187,7 @@ __global__ __launch_bounds__(1024) void k_make_chunks(const int2* __restrict__ s
     counters[C_BIG_PREV] = counters[C_FINAL_BIG];
     counters[C_NEXT] = 0;
     counters[C_ACTIVE] = 0;
+    counters[C_LONGEST] = 0;
   }
   __syncthreads();
   const int nseg = s_nseg;
@@ -238,19 +243,100 @@ __global__ __launch_bounds__(SORT_BS) void k_chunk_hist(const uint64_t* __restri
   chunkHist[(int64_t)b * 256 + threadIdx.x] = hist[threadIdx.x];
 }
 
+// A block's digit segments onto the next round's and the final lists, with two
+// 64-bit atomics, a pair of counters each.
+constexpr int SEG_BS = 1024;
+__device__ __forceinline__ void append_segments(int start, int run, bool nxt, bool fsm, bool fbg,
+                                                int2* __restrict__ segNext, int2* __restrict__ fin,
+                                                int finBigOff, int* __restrict__ counters) {
+  typedef unsigned long long u64;
+  __shared__ int lds[SEG_BS / 64];
+  __shared__ int tot, tot_big, act_tot, longest;
+  __shared__ int bases[3];
+  if (threadIdx.x == 0) longest = 0;
+  const int ex = block_exclusive_scan<SEG_BS>((nxt ? 1 : 0) | (fsm ? 1 << 16 : 0), lds, &tot);
+  const int exb = block_exclusive_scan<SEG_BS>(fbg ? 1 : 0, lds, &tot_big);
+  (void)block_exclusive_scan<SEG_BS>(nxt ? run : 0, lds, &act_tot);
+  if (nxt && run > kShortSeg) atomicMax(&longest, run);   // rare
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const u64 v = tot ? atomicAdd(reinterpret_cast<u64*>(&counters[C_NEXT]),
+                                  (u64)(tot & 0xFFFF) | (u64)(tot >> 16) << 32)
+                      : 0;
+    bases[0] = (int)(uint32_t)v;
+    bases[1] = (int)(v >> 32);
+  } else if (threadIdx.x == 64) {
+    const u64 v = act_tot | tot_big ? atomicAdd(reinterpret_cast<u64*>(&counters[C_ACTIVE]),
+                                                (u64)(uint32_t)act_tot | (u64)tot_big << 32)
+                                    : 0;
+    bases[2] = (int)(v >> 32);
+    if (longest) atomicMax(&counters[C_LONGEST], longest);
+  }
+  __syncthreads();
+  if (nxt) segNext[bases[0] + (ex & 0xFFFF)] = make_int2(start, run);
+  if (fsm) fin[bases[1] + (ex >> 16)] = make_int2(start, run);
+  if (fbg) fin[finBigOff - 1 - (bases[2] + exb)] = make_int2(start, run);
+}
+
+// Rounds of many short segments (kManySegs, kShortSeg): four segments per
+// block, 256 threads each.  A block per segment there is bound by the lists'
+// counters, at which the blocks take turns (third round of 1M and 2M clustered
+// points 20 -> 10 and 40 -> 17 us).
+__global__ __launch_bounds__(SEG_BS) void k_seg_offsets_short(
+    const int2* __restrict__ seg, const int* __restrict__ segChunk0, int* __restrict__ chunkHist,
+    int threshold, int last_round, int2* __restrict__ segNext, int2* __restrict__ fin,
+    int finBigOff, int* __restrict__ counters) {
+  __shared__ int wsum[SEG_BS / 64];
+  const int d = threadIdx.x & 255, wid = threadIdx.x >> 6;
+  const int si = blockIdx.x * 4 + (threadIdx.x >> 8);
+  const bool valid = si < counters[C_SEGS];
+  const int2 sg = valid ? seg[si] : make_int2(0, 0);
+  const int c0 = valid ? segChunk0[si] : 0;
+  const int ce = c0 + (int)ceil_div(sg.y, CHUNK);
+  constexpr int B = 16;
+  int h[B];
+  int run = 0;
+  for (int c = c0; c < ce; c += B) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) h[u] = c + u < ce ? chunkHist[(int64_t)(c + u) * 256 + d] : 0;
+#pragma unroll
+    for (int u = 0; u < B; ++u) run += h[u];
+  }
+  // digit starts: scan of the totals over the segment's 256 digits
+  const int inc = wave_inclusive_scan(run);
+  if ((threadIdx.x & 63) == 63) wsum[wid] = inc;
+  __syncthreads();
+  int start = sg.x + inc - run;
+  for (int w = wid & ~3; w < wid; ++w) start += wsum[w];
+  int pos = start;
+  const int cont = (run > threshold && !last_round) ? (int)0x80000000u : 0;
+  for (int c = c0; c < ce; c += B) {
+    if (ce - c0 > B) {
+#pragma unroll
+      for (int u = 0; u < B; ++u) h[u] = c + u < ce ? chunkHist[(int64_t)(c + u) * 256 + d] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      if (c + u < ce) chunkHist[(int64_t)(c + u) * 256 + d] = pos | cont;
+      pos += h[u];
+    }
+  }
+  const bool nxt = run > threshold && !last_round;
+  const bool fsm = !nxt && run >= 2 && run <= kWaveSortMax;
+  const bool fbg = !nxt && run > kWaveSortMax && run <= kLocalSortMax;
+  append_segments(start, run, nxt, fsm, fbg, segNext, fin, finBigOff, counters);
+}
+
 // One block per segment, 1024 threads: digit d = tid % 256, part = tid / 256
 // scans a quarter of the segment's chunks.  Output: chunkHist[c][d] = the
-// destination of chunk c's first element of digit d.  The digit segments of
-// the next round and the final ones are appended with one atomic per block.
-constexpr int SEG_BS = 1024;
-
+// destination of chunk c's first element of digit d, and the digit segments
+// on the lists.
 __global__ __launch_bounds__(SEG_BS) void k_seg_offsets(
     const int2* __restrict__ seg, const int* __restrict__ segChunk0, int* __restrict__ chunkHist,
     int threshold, int last_round, int2* __restrict__ segNext, int2* __restrict__ fin,
     int finBigOff, int* __restrict__ counters) {
   __shared__ int lds[SEG_BS / 64];
   __shared__ int part_sum[4][256];
-  __shared__ int bases[3];
   const int si = blockIdx.x;
   if (si >= counters[C_SEGS]) return;   // block-uniform: a grid sized by a bound
   const int d = threadIdx.x & 255, part = threadIdx.x >> 8;
@@ -323,25 +409,7 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_offsets(
   const bool nxt = part == 0 && run > threshold && !last_round;
   const bool fsm = part == 0 && !nxt && run >= 2 && run <= kWaveSortMax;
   const bool fbg = part == 0 && !nxt && run > kWaveSortMax && run <= kLocalSortMax;
-  // counts of the three kinds packed in one scan (each at most 256)
-  const int code = (nxt ? 1 : 0) | (fsm ? 1 << 10 : 0) | (fbg ? 1 << 20 : 0);
-  __shared__ int tot;
-  const int ex = block_exclusive_scan<SEG_BS>(code, lds, &tot);
-  if (threadIdx.x == 0) {
-    const int tn = tot & 1023, tf = (tot >> 10) & 1023, tb = (tot >> 20) & 1023;
-    bases[0] = tn ? atomicAdd(&counters[C_NEXT], tn) : 0;
-    bases[1] = tf ? atomicAdd(&counters[C_FINAL], tf) : 0;
-    bases[2] = tb ? atomicAdd(&counters[C_FINAL_BIG], tb) : 0;
-  }
-  int act = nxt ? run : 0;
-  __syncthreads();
-  if (nxt) segNext[bases[0] + (ex & 1023)] = make_int2(start, run);
-  if (fsm) fin[bases[1] + ((ex >> 10) & 1023)] = make_int2(start, run);
-  if (fbg) fin[finBigOff - 1 - (bases[2] + ((ex >> 20) & 1023))] = make_int2(start, run);
-  // active elements of the next round: one atomic per block
-  __shared__ int act_tot;
-  (void)block_exclusive_scan<SEG_BS>(act, lds, &act_tot);
-  if (threadIdx.x == 0 && act_tot) atomicAdd(&counters[C_ACTIVE], act_tot);
+  append_segments(start, run, nxt, fsm, fbg, segNext, fin, finBigOff, counters);
 }
 
 // Scatter of one chunk by its digit, staged through LDS: the chunk is first
@@ -599,7 +667,7 @@ bool sort_pairs_u64(uint64_t* keys, uint32_t* vals, int64_t n, int threshold, Pr
   }
 
   int nseg = 0;
-  int64_t active = 0;
+  int64_t active = 0, longest = n;
   int nfinal = 0, nbig = 0;
   int cur = 0;
   if (n > T) {
@@ -658,7 +726,10 @@ bool sort_pairs_u64(uint64_t* keys, uint32_t* vals, int64_t n, int threshold, Pr
                          w.chunks.as<int4>(), cnt, shift, w.chunkHist.as<int>());
       FMM_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(k_seg_offsets, dim3(nseg_grid), dim3(SEG_BS), 0, s, segCur,
+    const bool many = !on_device_counts && nseg > kManySegs && longest <= kShortSeg;
+    hipLaunchKernelGGL(many ? k_seg_offsets_short : k_seg_offsets,
+                       dim3(many ? (unsigned)ceil_div(nseg, 4) : (unsigned)nseg_grid),
+                       dim3(SEG_BS), 0, s, segCur,
                        w.segChunk0.as<int>(), w.chunkHist.as<int>(), T, r == rounds - 1 ? 1 : 0, segNext,
                        w.fin.as<int2>(), finBigOff, cnt);
     FMM_LAUNCH_CHECK();
@@ -676,6 +747,7 @@ bool sort_pairs_u64(uint64_t* keys, uint32_t* vals, int64_t n, int threshold, Pr
     w.mbox.take(C_COUNT, seq, s, hc);
     nseg = (int)hc[C_NEXT];
     active = hc[C_ACTIVE];
+    longest = hc[C_LONGEST];   // 0: no segment over kShortSeg
     nfinal = hc[C_FINAL];
     nbig = hc[C_FINAL_BIG];
     if (on_device_counts) {   // the first round's results, as this round began
