@@ -302,11 +302,13 @@ struct LogAcc {
 //   k K1(x)/r = 1/d2 + (k^2/4) (2 ln(x/2) I1' - S1'),
 // I1' = sum q^j/(j!(j+1)!), S1' the psi sum of bessel_k01 (x I1' / 2 = I1).
 // The x > 2 branch is bessel_k0_large / bessel_k01_large at x = k sqrt(d2).
+constexpr double kHelmQ8 = 0.0625, kHelmQ10 = 0.25;
 struct HelmConsts {
   double k, k2q, lnk2;   // k, k^2/4, ln(k/2)
+  double q8;             // helm_k0: largest q of the 8-term series
 };
-__device__ __forceinline__ HelmConsts helm_consts(double k) {
-  return HelmConsts{k, 0.25 * k * k, log(0.5 * k)};
+__device__ __forceinline__ HelmConsts helm_consts(double k, double q8 = kHelmQ8) {
+  return HelmConsts{k, 0.25 * k * k, log(0.5 * k), q8};
 }
 __device__ __forceinline__ double helm_lnx2(double d2, const double2* __restrict__ tab,
                                             const HelmConsts& h) {
@@ -320,7 +322,6 @@ __device__ __forceinline__ double helm_lnx2(double d2, const double2* __restrict
 // boxes of width w); the number is chosen per wave, so that no lane's branch
 // adds to another's: gradient evaluation of 2.5e8 pairs
 // 932 -> 714 us (K1 has a third class; K0 alone gains nothing from it).
-constexpr double kHelmQ8 = 0.0625, kHelmQ10 = 0.25;
 template <int N>
 __device__ __forceinline__ double helm_k0_series(double q, double d2,
                                                  const double2* __restrict__ tab,
@@ -337,7 +338,7 @@ __device__ __forceinline__ double helm_k0_series(double q, double d2,
 __device__ __forceinline__ double helm_k0(double d2, const double2* __restrict__ tab,
                                           const HelmConsts& h) {
   const double q = h.k2q * d2;
-  if (__ballot(!(q <= kHelmQ8)) == 0) return helm_k0_series<8>(q, d2, tab, h);
+  if (__ballot(!(q <= h.q8)) == 0) return helm_k0_series<8>(q, d2, tab, h);
   if (q <= 1.0) return helm_k0_series<kBesselSeriesTerms>(q, d2, tab, h);
   return bessel_k0_large(h.k * __builtin_sqrt(d2));
 }
@@ -410,6 +411,13 @@ struct PotAcc<KER_MODHELM> {
 // leaves (16 per SIMD) a leaf's single wave mostly waits for its own loads
 // (256 leaves of 195 sources 29.5 -> 9.6 us, 64 of 31 sources 7.8 -> 4.6, 7K
 // leaves of 14 dipoles 23.0 -> 12.0).
+// Not where the M2L rounds the multipoles to FP32: the pseudo-inverse amplifies
+// the last bits of the check potentials (to 6e-7 of a multipole at p 64), and
+// although that cancels again in FP64, the FP32 rounding in between does not:
+// another order of these sums changes mixed results by as much as their whole
+// error (1e-9 to 5e-8).  There a leaf's sums are its sources in order, by one
+// wave, with the full Helmholtz series (full_series), and the level products
+// are chains in one order (load_b_natural), whatever the size of the problem.
 constexpr int64_t kSplitLeaves = 64 * kNumCUs;
 // DIP: sources also carry a dipole moment q (the double layer of the Laplace
 // kernel, (q.d)/d^2/(2 pi) with d = check point - source).
@@ -423,6 +431,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_s2m(int nup, const int* __r
                                             const double4* __restrict__ src,
                                             const double* __restrict__ ops, int64_t opsz, int p,
                                             const double2* __restrict__ logtab, double kp,
+                                            bool full_series,
                                             const double2* __restrict__ dip,
                                             double* __restrict__ check) {
   __shared__ double2 tab[kLogTableSize];
@@ -452,7 +461,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_s2m(int nup, const int* __r
     b += n * part / NS;
   }
   PotAcc<KER> acc;
-  const HelmConsts hc = helm_consts(kp);
+  const HelmConsts hc = helm_consts(kp, full_series ? -1.0 : kHelmQ8);
   double dsum = 0.0;   // double layer
   int j = b;
   for (; j + 4 <= t; j += 4) {
@@ -1548,10 +1557,11 @@ enum {
 // The packed operators of one level: dv2 entry ((blk KP + m) RB + rb) 64 +
 // lane holds row 16 rb + lane % 16 of the block, columns 8 m + 2 (lane / 16) +
 // {0, 1}; of the pseudo-inverse factors (whose B operand is a product's
-// result), columns 8 m + lane / 16 + {0, 4}; of the M2L blocks when the last
+// result) and, if natural, the M2M blocks, columns 8 m + lane / 16 + {0, 4};
+// of the M2L blocks when the last
 // pair of k-steps is one step (odd), column 8 m + lane / 16 and 0 for m = KP - 1.
 __global__ __launch_bounds__(256) void k_ops_pack(const double* __restrict__ ops, int PD, int PE,
-                                                  bool odd, dv2* __restrict__ out) {
+                                                  bool odd, bool natural, dv2* __restrict__ out) {
   const int RB = PE / 16, KP = PE / 8;
   const int n = OPP_NBLK * KP * RB * 64;
   const int e = blockIdx.x * 256 + threadIdx.x;
@@ -1562,7 +1572,7 @@ __global__ __launch_bounds__(256) void k_ops_pack(const double* __restrict__ ops
                   : blk < OPP_L2L ? OP_M2M + blk - OPP_M2M : OP_L2L + blk - OPP_L2L;
   const double* row = ops + (int64_t)src * PD * PD + (16 * rb + (lane & 15)) * PD + 8 * m;
   const int kq = lane >> 4;
-  if (src == OP_PINV1 || src == OP_PINV2) out[e] = dv2{row[kq], row[kq + 4]};
+  if (blk >= OPP_PINV1 && blk < (natural ? OPP_L2L : OPP_M2M)) out[e] = dv2{row[kq], row[kq + 4]};
   else if (odd && blk < OPP_PINV1 && m == KP - 1) out[e] = dv2{row[kq], 0.0};
   else out[e] = *reinterpret_cast<const dv2*>(row + 2 * kq);
 }
@@ -1625,6 +1635,17 @@ struct LevelWave {
 #pragma unroll
     for (int m = 0; m < KP; ++m) b[m] = *reinterpret_cast<const dv2*>(q + 8 * m);
   }
+  // entries 8 m + kq + {0, 4}, the natural k order: the M2M products of plans
+  // whose M2L rounds the multipoles to FP32 (see kSplitLeaves).  Twice the
+  // loads: 2M clustered Stokeslets in the mixed form, forward and adjoint,
+  // 7.44 -> 7.46 ms; an FP64 plan on 1M clustered points 886 -> 895 us, so
+  // those take the wide loads.
+  static __device__ __forceinline__ void load_b_natural(dv2 (&b)[KP],
+                                                        const double* __restrict__ row) {
+    const double* q = row + ((threadIdx.x & 63) >> 4);
+#pragma unroll
+    for (int m = 0; m < KP; ++m) b[m] = dv2{q[8 * m], q[8 * m + 4]};
+  }
   template <int PD>
   __device__ __forceinline__ void store(double* __restrict__ row) const {
     const int kq = (threadIdx.x & 63) >> 4;
@@ -1641,8 +1662,8 @@ constexpr int kLevelWaves = 4;   // waves per block
 // Upward, one level: rows [row0, row0 + nrows), density blockIdx.y.  check =
 // S2M result (leaves) or M2M of the four children (parents), then multipole =
 // pinv2 * (pinv1 * check)  (fmm.py:98-122).  opsL: the level's packed
-// operators.
-template <int PD, int PE>
+// operators; NATURAL: their M2M blocks' k order.
+template <int PD, int PE, bool NATURAL>
 __global__ __launch_bounds__(64 * kLevelWaves) void k_mult_level(
     int64_t row0, int nrows, int with_m2m, const int2* __restrict__ rowinfo,
     const double* __restrict__ check, const dv2* __restrict__ opsL, double* __restrict__ mult,
@@ -1676,7 +1697,9 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_mult_level(
   if (up) {
     for (int c = 0; c < 4; ++c) {
       dv2 b[W::KP];
-      W::load_b(b, crow >= 0 ? mult + (int64_t)(crow + c) * PD : c_zero_row);
+      const double* row = crow >= 0 ? mult + (int64_t)(crow + c) * PD : c_zero_row;
+      if constexpr (NATURAL) W::load_b_natural(b, row);
+      else W::load_b(b, row);
       L.product(b, pm + c * W::kBlock, c < 3 ? pm + (c + 1) * W::kBlock : p1);
     }
   }
@@ -3749,6 +3772,14 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
   FMM_LAUNCH_CHECK();
 }
 
+// plans whose M2L can run in FP32 (m2l_in_fp32): natural k order of the M2M products
+static bool m2m_natural(const Plan& P) { return P.precision != PREC_FP64 && !P.cheb; }
+template <bool NATURAL>
+static auto mult_level_kernel(int p) {
+  return p <= 16 ? k_mult_level<32, 16, NATURAL> : p <= 32 ? k_mult_level<32, 32, NATURAL>
+         : p <= 48 ? k_mult_level<64, 48, NATURAL> : k_mult_level<64, 64, NATURAL>;
+}
+
 static const dv2* packed_ops(const Plan& P, int level) {
   return reinterpret_cast<const dv2*>(P.opsm.as<double>() + level * opsm_per_level(P.p));
 }
@@ -3825,7 +3856,8 @@ static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s
     P.have_exp = true;
     return;
   }
-  const int sns = t.n_up <= kSplitLeaves ? kEvalWaves : 1;   // waves per leaf
+  // waves per leaf; one where the M2L rounds the multipoles to FP32 (kSplitLeaves)
+  const int sns = t.n_up <= kSplitLeaves && !m2l_in_fp32(P) ? kEvalWaves : 1;
   P.mark(FMM2D_PHASE_S2M, false, s);
   if (t.n_up > 0 && stokes) {
     auto kern = s2m_stokes_kernel(PD, dvec != nullptr, sns);
@@ -3849,8 +3881,8 @@ static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s
                        (int)t.n_up, t.upnodes.as<int>(), t.nlevel.as<int>(),
                        t.bot.as<int>(), t.top.as<int>(), t.row.as<int>(), t.xmid.as<double>(),
                        t.ymid.as<double>(), P.src.as<double4>(), P.ops.as<double>(), opsz, P.p,
-                       P.logtab.as<double2>(), P.kparam, dvec ? P.dip.as<double2>() : nullptr,
-                       P.check.as<double>());
+                       P.logtab.as<double2>(), P.kparam, m2l_in_fp32(P),
+                       dvec ? P.dip.as<double2>() : nullptr, P.check.as<double>());
     FMM_LAUNCH_CHECK();
   }
   P.mark(FMM2D_PHASE_S2M, true, s);
@@ -3867,8 +3899,7 @@ static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s
       FMM_LAUNCH_CHECK();
       continue;
     }
-    auto kern = P.p <= 16 ? k_mult_level<32, 16> : P.p <= 32 ? k_mult_level<32, 32>
-                : P.p <= 48 ? k_mult_level<64, 48> : k_mult_level<64, 64>;
+    auto kern = m2m_natural(P) ? mult_level_kernel<true>(P.p) : mult_level_kernel<false>(P.p);
     hipLaunchKernelGGL(kern, dim3(ceil_div(nrows, 16 * kLevelWaves), nd), dim3(64 * kLevelWaves), 0,
                        s, r0, nrows, d < t.L - 1 ? 1 : 0, t.rowinfo.as<int2>(),
                        P.check.as<double>(), packed_ops(P, d), P.mult.as<double>(),
@@ -4437,7 +4468,7 @@ int fmm2d_set_operators(void* plan, int level, const double* dev_ops, int64_t n,
   P->opsm.ensure(fmm::kMaxLevels * msz * sizeof(double));
   hipLaunchKernelGGL(fmm::k_ops_pack, dim3(fmm::grid256(msz / 2)), dim3(256), 0, s,
                      P->ops.as<double>() + level * opsz, P->PD, fmm::m2l_pe(P->p),
-                     fmm::m2l_odd(P->p),
+                     fmm::m2l_odd(P->p), fmm::m2m_natural(*P),
                      reinterpret_cast<fmm::dv2*>(P->opsm.as<double>() + level * msz));
   FMM_LAUNCH_CHECK();
   P->ops_set[level] = 1;
