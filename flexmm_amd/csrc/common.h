@@ -10,6 +10,8 @@
 #include <string>
 #include <vector>
 
+#include "work_split.h"
+
 namespace fmm {
 
 // ---------------------------------------------------------------------------

@@ -456,9 +456,9 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_s2m(int nup, const int* __r
   int b = __builtin_amdgcn_readfirstlane(bot[g]);
   int t = __builtin_amdgcn_readfirstlane(top[g]);
   if constexpr (NS > 1) {   // this wave's share
-    const int n = t - b;
-    t = b + n * (part + 1) / NS;
-    b += n * part / NS;
+    const Span own = part_of<NS>(b, t, part);
+    b = own.b;
+    t = own.e;
   }
   PotAcc<KER> acc;
   const HelmConsts hc = helm_consts(kp, full_series ? -1.0 : kHelmQ8);
@@ -2810,9 +2810,9 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
     int b = __builtin_amdgcn_readlane(CL.b, qn);
     int e = __builtin_amdgcn_readlane(CL.e, qn);
     if constexpr (NS > 1) {   // this wave's share of the colleague's sources
-      const int n = max(e - b, 0);
-      e = b + n * (part + 1) / NS;
-      b = b + n * part / NS;
+      const Span own = part_of<NS>(b, e, part);
+      b = own.b;
+      e = own.e;
     }
     if (e <= b) continue;
     if (qn == 4) colleague(std::true_type{}, b, e);
@@ -3218,9 +3218,9 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_s2m_stokes(int nup,
   int b = __builtin_amdgcn_readfirstlane(bot[g]);
   int t = __builtin_amdgcn_readfirstlane(top[g]);
   if constexpr (NS > 1) {   // this wave's share
-    const int n = t - b;
-    t = b + n * (part + 1) / NS;
-    b += n * part / NS;
+    const Span own = part_of<NS>(b, t, part);
+    b = own.b;
+    t = own.e;
   }
   LogAcc lfx, lfy;                 // sum f_i log|r|^2
   double ex = 0.0, ey = 0.0, e2 = 0.0;
@@ -3345,9 +3345,9 @@ __device__ __forceinline__ void stokes_item(
     int b = __builtin_amdgcn_readlane(CL.b, qn);
     int e = __builtin_amdgcn_readlane(CL.e, qn);
     if constexpr (!FEW && NS > 1) {   // this wave's share of the colleague's sources
-      const int n = max(e - b, 0);
-      e = b + n * (part + 1) / NS;
-      b = b + n * part / NS;
+      const Span own = part_of<NS>(b, e, part);
+      b = own.b;
+      e = own.e;
     }
     if (e <= b) continue;
     // A coincident pair (d2 = 0, so dx = dy = 0) continues with d2 = 1: every
