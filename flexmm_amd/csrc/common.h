@@ -245,25 +245,6 @@ __device__ __forceinline__ double log_tab(double x, const double2* __restrict__ 
 #endif
 
 // ---------------------------------------------------------------------------
-// XCD-aware block order.  MI355X dispatches consecutive workgroups round-robin
-// to its 8 XCDs, each with its own L2.  These bijections of [0, n) keep
-// neighbouring logical blocks, which share source data, on one XCD (blocks b
-// with b % 8 == x): chunk = 0 gives XCD x one contiguous range, chunk > 0
-// deals chunks of that many logical blocks to the XCDs in turn (for blocks of
-// unequal cost), the remainder past a whole turn in natural order.
-constexpr int kNumXcd = 8;
-constexpr int kNumCUs = 256;   // MI355X compute units (launch-shape heuristics only)
-__device__ __forceinline__ int xcd_block(int b, int n, int chunk) {
-  const int xcd = b % kNumXcd, local = b / kNumXcd;
-  if (chunk > 0) {
-    if (b >= n / (kNumXcd * chunk) * (kNumXcd * chunk)) return b;
-    return (local / chunk * kNumXcd + xcd) * chunk + local % chunk;
-  }
-  const int per = n / kNumXcd, rem = n % kNumXcd;
-  return xcd * per + min(xcd, rem) + local;
-}
-
-// ---------------------------------------------------------------------------
 // Kernel identifiers shared with the Python registry.
 enum KernelId : int {
   KER_LAPLACE = 0,   // -log(d^2)/(4 pi)

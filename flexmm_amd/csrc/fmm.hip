@@ -204,7 +204,6 @@ struct PlanCall {
 
 namespace {
 
-constexpr int kEvalWaves = 4;   // waves per block of the evaluation and S2M kernels
 // Sums of the NS waves that share an item, in wave order; valid in wave 0.
 template <int NS, int NV>
 __device__ __forceinline__ void item_sum(double (&v)[NV], int part) {
@@ -2383,16 +2382,8 @@ constexpr int kItemChunk = 32;
 constexpr int64_t kSplitItems = 16 * 4 * kNumCUs;
 constexpr int64_t kSplitTargets = 4;   // targets per evaluation box at least
 // this wave's item, or -1; ns waves share an item
-__device__ __forceinline__ int xcd_item(int ni, int chunk, int ns) {
-  const int x = blockIdx.x % kNumXcd;
-  const int j = ((int)(blockIdx.x / kNumXcd) * kEvalWaves + (int)(threadIdx.x >> 6)) / ns;
-  int first = (int)((int64_t)ni * x / kNumXcd) + j;
-  int last = (int)((int64_t)ni * (x + 1) / kNumXcd);
-  if (chunk > 0) {
-    first = (j / chunk * kNumXcd + x) * chunk + j % chunk;
-    last = ni;
-  }
-  return first < last ? first : -1;
+__device__ __forceinline__ int own_item(int ni, int chunk, int ns) {
+  return xcd_item(blockIdx.x, (int)(threadIdx.x >> 6), ni, chunk, ns);
 }
 
 template <int KER, int NOUT, bool CHECK>
@@ -2736,7 +2727,7 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const int ii = xcd_item(ni, chunk, NS);
+  const int ii = own_item(ni, chunk, NS);
   if (ii < 0) return;   // uniform among the waves of an item
   const int4 it = items[ii];
   // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
@@ -3005,7 +2996,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const int ii = xcd_item(ni, chunk, 1);
+  const int ii = own_item(ni, chunk, 1);
   if (ii < 0) return;   // wave-uniform
   const int4 it = items[ii];
   // wave-uniform (ii is): in scalar registers, so loads indexed by them are scalar
@@ -3464,7 +3455,7 @@ void k_eval_stokes(
   const int ni = *nitems;
   load_logtab(tab, logtab);
   __syncthreads();
-  const int ii = xcd_item(ni, chunk, NS);
+  const int ii = own_item(ni, chunk, NS);
   if (ii < 0) return;   // uniform among the waves of an item
   const int part = NS > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % NS : 0;
   const int4 it = items[ii];
@@ -3490,14 +3481,6 @@ EvalStokesFn eval_stokes_pd(bool dl, bool check, int ns) {
   constexpr int NS = kEvalWaves;
   return dl ? (check ? k_eval_stokes<PD, true, true, NS> : k_eval_stokes<PD, false, true, NS>)
             : (check ? k_eval_stokes<PD, true, false, NS> : k_eval_stokes<PD, false, false, NS>);
-}
-
-// blocks for at most icap items in chunks of `chunk` (a multiple of kEvalWaves,
-// or 0), ns waves per item
-inline int eval_grid(int64_t icap, int chunk, int ns) {
-  const int64_t per_xcd = chunk > 0 ? ceil_div(icap, (int64_t)kNumXcd * chunk) * chunk
-                                    : ceil_div(icap, kNumXcd) + 1;
-  return (int)(ceil_div(per_xcd * ns, kEvalWaves) * kNumXcd);
 }
 
 // Selects the k_eval instance of (PD, kernel, outputs, self-exclusion, waves per item).

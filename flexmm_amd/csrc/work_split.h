@@ -23,4 +23,47 @@ FMM_SPLIT_HD Span part_of(int b, int e, int part) {
   return Span{b + (int)(n * part / PARTS), b + (int)(n * (part + 1) / PARTS)};
 }
 
+// XCD-aware block order.  MI355X dispatches consecutive workgroups round-robin
+// to its 8 XCDs, each with its own L2.  These bijections of [0, n) keep
+// neighbouring logical blocks, which share source data, on one XCD (blocks b
+// with b % 8 == x): chunk = 0 gives XCD x one contiguous range, chunk > 0
+// deals chunks of that many logical blocks to the XCDs in turn (for blocks of
+// unequal cost), the remainder past a whole turn in natural order.
+constexpr int kNumXcd = 8;
+constexpr int kNumCUs = 256;   // MI355X compute units (launch-shape heuristics only)
+FMM_SPLIT_HD int xcd_block(int b, int n, int chunk) {
+  const int xcd = b % kNumXcd, local = b / kNumXcd;
+  if (chunk > 0) {
+    if (b >= n / (kNumXcd * chunk) * (kNumXcd * chunk)) return b;
+    return (local / chunk * kNumXcd + xcd) * chunk + local % chunk;
+  }
+  const int per = n / kNumXcd, rem = n % kNumXcd;
+  return xcd * per + (xcd < rem ? xcd : rem) + local;
+}
+
+// Work items of the evaluation kernels: kEvalWaves waves per block, ns waves
+// (1 or kEvalWaves) per item.  chunk = 0: XCD x takes the x-th contiguous
+// eighth of the items; chunk > 0 (a multiple of kEvalWaves): chunks of that
+// many items go to the XCDs in turn.
+constexpr int kEvalWaves = 4;   // waves per block of the evaluation and S2M kernels
+// the item of wave `wave` of block `block` among ni, or -1
+FMM_SPLIT_HD int xcd_item(unsigned block, int wave, int ni, int chunk, int ns) {
+  const int x = block % kNumXcd;
+  const int j = ((int)(block / kNumXcd) * kEvalWaves + wave) / ns;
+  int first = (int)((int64_t)ni * x / kNumXcd) + j;
+  int last = (int)((int64_t)ni * (x + 1) / kNumXcd);
+  if (chunk > 0) {
+    first = (j / chunk * kNumXcd + x) * chunk + j % chunk;
+    last = ni;
+  }
+  return first < last ? first : -1;
+}
+// blocks for at most icap items
+inline int eval_grid(int64_t icap, int chunk, int ns) {
+  const int64_t per_xcd =
+      chunk > 0 ? (icap + (int64_t)kNumXcd * chunk - 1) / ((int64_t)kNumXcd * chunk) * chunk
+                : (icap + kNumXcd - 1) / kNumXcd + 1;
+  return (int)((per_xcd * ns + kEvalWaves - 1) / kEvalWaves * kNumXcd);
+}
+
 }  // namespace fmm

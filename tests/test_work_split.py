@@ -1,6 +1,7 @@
 """The index arithmetic of flexmm_amd/csrc/work_split.h, compiled by the host
 compiler: the parts of a range are consecutive, cover it and differ in length
-by at most one, up to ranges of 2^31 - 1."""
+by at most one, up to ranges of 2^31 - 1; the orders of blocks and evaluation
+items over the XCDs take every one exactly once."""
 import os
 import subprocess
 
@@ -14,6 +15,7 @@ HARNESS = r"""
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <vector>
 using namespace fmm;
 
 template <int PARTS>
@@ -36,6 +38,42 @@ int main(int argc, char** argv) {
   if (argc == 4 && !std::strcmp(argv[1], "parts")) {
     const int b = std::atoi(argv[2]), e = std::atoi(argv[3]);
     return parts<1>(b, e) | parts<4>(b, e);
+  }
+  // every logical index once, and the neighbours of a chunk on one XCD
+  if (argc == 4 && !std::strcmp(argv[1], "blocks")) {
+    const int n = std::atoi(argv[2]), chunk = std::atoi(argv[3]);
+    std::vector<int> xcd(n, -1);
+    for (int b = 0; b < n; ++b) {
+      const int l = xcd_block(b, n, chunk);
+      if (l < 0 || l >= n || xcd[l] >= 0) return 1;
+      xcd[l] = b % kNumXcd;
+    }
+    for (int l = 0; l + 1 < n; ++l) {
+      if (chunk == 0 && xcd[l + 1] < xcd[l]) return 1;
+      if (chunk > 0 && l < n / (kNumXcd * chunk) * (kNumXcd * chunk) && (l + 1) % chunk &&
+          xcd[l + 1] != xcd[l])
+        return 1;
+    }
+    return 0;
+  }
+  // every item by ns waves of one block, in any grid of at least its blocks
+  if (argc == 6 && !std::strcmp(argv[1], "items")) {
+    const int ni = std::atoi(argv[2]), icap = std::atoi(argv[3]), chunk = std::atoi(argv[4]),
+              ns = std::atoi(argv[5]);
+    std::vector<int> waves(ni, 0), block(ni, -1);
+    for (int b = 0; b < eval_grid(icap, chunk, ns); ++b)
+      for (int w = 0; w < kEvalWaves; ++w) {
+        const int i = xcd_item(b, w, ni, chunk, ns);
+        if (i < 0) continue;
+        if (i >= ni || (ns > 1 && waves[i] && block[i] != b)) return 1;
+        ++waves[i];
+        block[i] = b;
+        // a block whose waves share an item takes no other
+        if (ns == kEvalWaves && i != xcd_item(b, 0, ni, chunk, ns)) return 1;
+      }
+    for (int i = 0; i < ni; ++i)
+      if (waves[i] != ns) return 1;
+    return 0;
   }
   return 2;
 }
@@ -64,3 +102,20 @@ def test_parts_cover_the_range(harness, b, n):
 
 def test_a_range_that_ends_before_it_begins_is_empty(harness):
     assert harness("parts", 5, 3).returncode == 0
+
+
+COUNTS = [1, 7, 8, 31, 32, 33, 255, 256, 257, 1000, 4099]
+
+
+@pytest.mark.parametrize("chunk", [0, 1, 4, 8, 32])
+@pytest.mark.parametrize("n", COUNTS)
+def test_block_order_is_a_bijection(harness, n, chunk):
+    assert harness("blocks", n, chunk).returncode == 0
+
+
+@pytest.mark.parametrize("ns", [1, 4])
+@pytest.mark.parametrize("chunk", [0, 8, 32])
+@pytest.mark.parametrize("n", COUNTS)
+def test_items_are_taken_once(harness, n, chunk, ns):
+    for icap in (n, n + 1, n + 65, 3 * n):
+        assert harness("items", n, icap, chunk, ns).returncode == 0, icap
