@@ -37,7 +37,8 @@ def _chain(A, b, acc):
                                          ("mixed", 16), ("mixed_m2l", 60)])
 def test_large_level_products_are_ascending_fma_chains(precision, p):
     from flexmm_amd import kernels
-    from flexmm_amd.kifmm2d import FMM
+    from flexmm_amd.kifmm2d import FMM, the_help
+    the_help.clear()   # cached widths would snap the box
     m = 256   # one point per cell of depth 8
     rng = np.random.default_rng(3)
     g = np.stack(np.meshgrid(np.arange(m), np.arange(m), indexing="ij"), -1).reshape(-1, 2)
@@ -80,7 +81,8 @@ def _points(right):
 def test_s2m_of_mixed_plans_does_not_depend_on_the_number_of_leaves(kind, p):
     import torch
     from flexmm_amd import _lib, kernels
-    from flexmm_amd.kifmm2d import FMM, StokesFMM
+    from flexmm_amd.kifmm2d import FMM, StokesFMM, the_help
+    the_help.clear()
     rng = np.random.default_rng(5)
     dens = rng.standard_normal((4, _points(True).shape[0]))
     got = []
