@@ -962,7 +962,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 // tiles sharing an LDS stage this gives four times the waves (a 1M-point
 // tree: ~5 per SIMD instead of ~1.4).
 constexpr int kM2LWCols = 16;
-constexpr int kM2LWWaves = 4;
 constexpr int kM2LF32Waves = 4;
 
 template <int PD, int NW>
@@ -1042,73 +1041,71 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
   // this wave's slots: pslot[w + NW j], j < nmine
   const int nmine = w < nph ? (nph - 1 - w) / NW + 1 : 0;
   if (nmine > 0) {
-    {
-      // operator pieces pc = rb NA + j of a slot (16 bytes per lane, four
-      // MFMA steps each), NA of them in flight: consuming a piece issues the
-      // load of the piece NA further on, across row block and slot
-      // boundaries.  The multipole operands alternate between two buffers: a
-      // slot's first NA pieces also load the next slot's operands into the
-      // other one.  Absent sources read a zero row.
-      constexpr int NP = RB * NA;
-      const float* m32y = m32 + (int64_t)blockIdx.y * rstride * PD;
-      auto bptr = [&](int src) -> const fv4* {
-        return reinterpret_cast<const fv4*>(
-            (src >= 0 ? m32y + (int64_t)src * PD : reinterpret_cast<const float*>(c_zero_row)) +
-            kq * KS);
-      };
-      auto apiece = [&](int sl, int pc) -> const fv4* {
-        return afr + ((int64_t)sl * NP + pc) * 64;
-      };
-      int slot = __builtin_amdgcn_readfirstlane(pslotv[w]);
-      fv4 a[NA], b0[NA], b1[NA];
-      // first loads in the order the loop consumes them, so that its waits
-      // for the first pieces hold for every slot
+    // operator pieces pc = rb NA + j of a slot (16 bytes per lane, four
+    // MFMA steps each), NA of them in flight: consuming a piece issues the
+    // load of the piece NA further on, across row block and slot
+    // boundaries.  The multipole operands alternate between two buffers: a
+    // slot's first NA pieces also load the next slot's operands into the
+    // other one.  Absent sources read a zero row.
+    constexpr int NP = RB * NA;
+    const float* m32y = m32 + (int64_t)blockIdx.y * rstride * PD;
+    auto bptr = [&](int src) -> const fv4* {
+      return reinterpret_cast<const fv4*>(
+          (src >= 0 ? m32y + (int64_t)src * PD : reinterpret_cast<const float*>(c_zero_row)) +
+          kq * KS);
+    };
+    auto apiece = [&](int sl, int pc) -> const fv4* {
+      return afr + ((int64_t)sl * NP + pc) * 64;
+    };
+    int slot = __builtin_amdgcn_readfirstlane(pslotv[w]);
+    fv4 a[NA], b0[NA], b1[NA];
+    // first loads in the order the loop consumes them, so that its waits
+    // for the first pieces hold for every slot
 #pragma unroll
-      for (int h = 0; h < NA; ++h) {
-        a[h] = *apiece(slot, h);
+    for (int h = 0; h < NA; ++h) {
+      a[h] = *apiece(slot, h);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    {
+      const fv4* bp = bptr(srcs[pslot[w]][col]);
+#pragma unroll
+      for (int j = 0; j < NA; ++j) {
+        b0[j] = bp[j];
         __builtin_amdgcn_sched_barrier(0);
       }
-      {
-        const fv4* bp = bptr(srcs[pslot[w]][col]);
+    }
+    auto one_slot = [&](fv4 (&bu)[NA], fv4 (&bl)[NA], int jj) {
+      // the next slot of this wave (the current one again after the last)
+      const int kn = jj + 1 < nmine ? w + NW * (jj + 1) : w + NW * jj;
+      const int slot_n = __builtin_amdgcn_readfirstlane(pslotv[kn]);
+      const fv4* bpn = bptr(srcs[pslot[kn]][col]);
 #pragma unroll
-        for (int j = 0; j < NA; ++j) {
-          b0[j] = bp[j];
-          __builtin_amdgcn_sched_barrier(0);
-        }
+      for (int pc = 0; pc < NP; ++pc) {
+        const int rb = pc / NA, j = pc % NA;
+        // an FP32 run of four steps, added to the FP64 sums; two
+        // accumulators keep consecutive MFMAs independent
+        f4 s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][0], bu[j][0], f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        f4 s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][1], bu[j][1], f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][2], bu[j][2], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][3], bu[j][3], s1, 0, 0, 0);
+        // the piece just used is reloaded into the same registers
+        a[j] = pc + NA < NP ? *apiece(slot, pc + NA) : *apiece(slot_n, pc + NA - NP);
+        if (pc < NA) bl[pc] = bpn[pc];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc64[rb][v] += (double)(s0[v] + s1[v]);
+        // in program order: the scheduler would otherwise move each load
+        // down to its use
+        __builtin_amdgcn_sched_barrier(0);
       }
-      auto one_slot = [&](fv4 (&bu)[NA], fv4 (&bl)[NA], int jj) {
-        // the next slot of this wave (the current one again after the last)
-        const int kn = jj + 1 < nmine ? w + NW * (jj + 1) : w + NW * jj;
-        const int slot_n = __builtin_amdgcn_readfirstlane(pslotv[kn]);
-        const fv4* bpn = bptr(srcs[pslot[kn]][col]);
-#pragma unroll
-        for (int pc = 0; pc < NP; ++pc) {
-          const int rb = pc / NA, j = pc % NA;
-          // an FP32 run of four steps, added to the FP64 sums; two
-          // accumulators keep consecutive MFMAs independent
-          f4 s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][0], bu[j][0], f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          f4 s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][1], bu[j][1], f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][2], bu[j][2], s0, 0, 0, 0);
-          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][3], bu[j][3], s1, 0, 0, 0);
-          // the piece just used is reloaded into the same registers
-          a[j] = pc + NA < NP ? *apiece(slot, pc + NA) : *apiece(slot_n, pc + NA - NP);
-          if (pc < NA) bl[pc] = bpn[pc];
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc64[rb][v] += (double)(s0[v] + s1[v]);
-          // in program order: the scheduler would otherwise move each load
-          // down to its use
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        slot = slot_n;
-      };
-      for (int jj = 0; jj < nmine; jj += 2) {
-        one_slot(b0, b1, jj);
-        if (jj + 1 < nmine) one_slot(b1, b0, jj + 1);
-        // keeps the next slot's loads here, ahead of the loop's back edge
-        // (otherwise they are merged with the first slot's into one load at
-        // the top of the loop, which then waits for them at once)
-        __asm__ volatile("" ::: "memory");
-      }
+      slot = slot_n;
+    };
+    for (int jj = 0; jj < nmine; jj += 2) {
+      one_slot(b0, b1, jj);
+      if (jj + 1 < nmine) one_slot(b1, b0, jj + 1);
+      // keeps the next slot's loads here, ahead of the loop's back edge
+      // (otherwise they are merged with the first slot's into one load at
+      // the top of the loop, which then waits for them at once)
+      __asm__ volatile("" ::: "memory");
     }
     // constant mode: acc64[rb] += sum over this wave's slots of
     // means[slot][row] * qsl[slot][col], four slots per FP64 MFMA step.  Lane
@@ -2559,7 +2556,7 @@ __device__ __forceinline__ void eval_few(
     int g, int t0, int na, int part, const int* __restrict__ tperm, const double* __restrict__ tx,
     const double* __restrict__ ty, const int* __restrict__ nlevel,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
-    const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
+    const int* __restrict__ coll, const int2* __restrict__ crange,
     const double4* __restrict__ src, const double2* __restrict__ dip,
     const double* __restrict__ le, const double* __restrict__ ops, int64_t opsz, int p,
     const double2* __restrict__ tab, double kp, int64_t nt, double* __restrict__ out,
@@ -2708,11 +2705,10 @@ template <int PD, int KER, int NOUT, bool CHECK, bool DIP, bool CHEB, int NS>
 __global__ __launch_bounds__(64 * kEvalWaves)
 __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) void k_eval(
     const int4* __restrict__ items, const int* __restrict__ nitems,
-    const int* __restrict__ evalnode, const int* __restrict__ toff,
     const int* __restrict__ tperm, const double* __restrict__ tx, const double* __restrict__ ty,
     const int* __restrict__ nlevel, const double* __restrict__ xmid,
-    const double* __restrict__ ymid, const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot,
-    const int* __restrict__ top, const double4* __restrict__ src,
+    const double* __restrict__ ymid, const int* __restrict__ coll,
+    const int2* __restrict__ crange, const double4* __restrict__ src,
     const double2* __restrict__ dip,
     const double* __restrict__ le, const double* __restrict__ ops, int64_t opsz, int p,
     const double2* __restrict__ logtab, double kp, int64_t nt, double* __restrict__ out,
@@ -2735,7 +2731,7 @@ __attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) vo
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets) {
     eval_few<PD, KER, NOUT, CHECK, DIP, CHEB, NS>(g, t0, t1 - t0, part, tperm, tx, ty, nlevel, xmid,
-                                              ymid, coll, crange, bot, top, src, dip, le, ops, opsz, p,
+                                              ymid, coll, crange, src, dip, le, ops, opsz, p,
                                               tab, kp, nt, out, stage, dstage, scap);
     return;
   }
@@ -2880,7 +2876,7 @@ __device__ __forceinline__ void eval_few_mixed(
     int g, int t0, int na, const int* __restrict__ tperm, const double* __restrict__ tx,
     const double* __restrict__ ty, const int* __restrict__ nlevel, const int* __restrict__ flags,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
-    const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
+    const int* __restrict__ coll, const int2* __restrict__ crange,
     const double4* __restrict__ src, const f4* __restrict__ srcf, const double* __restrict__ tsum,
     const LevelConsts& lc, const double* __restrict__ le, const double* __restrict__ ops,
     int64_t opsz, int p, const double2* __restrict__ tab, double* __restrict__ out) {
@@ -2983,11 +2979,10 @@ __device__ __forceinline__ void eval_few_mixed(
 template <int PD, bool CHECK, bool CHEB>
 __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
     const int4* __restrict__ items, const int* __restrict__ nitems,
-    const int* __restrict__ evalnode, const int* __restrict__ toff,
     const int* __restrict__ tperm, const double* __restrict__ tx, const double* __restrict__ ty,
     const int* __restrict__ nlevel, const int* __restrict__ flags,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
-    const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
+    const int* __restrict__ coll, const int2* __restrict__ crange,
     const double4* __restrict__ src, const f4* __restrict__ srcf,
     const double* __restrict__ tsum, LevelConsts lc, const double* __restrict__ le,
     const double* __restrict__ ops, int64_t opsz, int p, const double2* __restrict__ logtab,
@@ -3004,7 +2999,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_eval_mixed(
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets) {
     eval_few_mixed<PD, CHECK, CHEB>(g, t0, t1 - t0, tperm, tx, ty, nlevel, flags, xmid,
-                                    ymid, coll, crange, bot, top, src, srcf, tsum, lc, le, ops, opsz,
+                                    ymid, coll, crange, src, srcf, tsum, lc, le, ops, opsz,
                                     p, tab, out);
     return;
   }
@@ -3257,7 +3252,7 @@ __device__ __forceinline__ void stokes_item(
     int g, int t0, int t1, int part, const int* __restrict__ tperm, const double* __restrict__ tx,
     const double* __restrict__ ty, const int* __restrict__ nlevel,
     const double* __restrict__ xmid, const double* __restrict__ ymid,
-    const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot, const int* __restrict__ top,
+    const int* __restrict__ coll, const int2* __restrict__ crange,
     const double4* __restrict__ src, const double4* __restrict__ sdip,
     const double* __restrict__ le, int64_t nstride,
     const double* __restrict__ ops, int64_t opsz, int p, const double2* __restrict__ tab,
@@ -3442,11 +3437,10 @@ template <int PD, bool CHECK, bool DIP, int NS>
 __global__ __launch_bounds__(64 * kEvalWaves) __attribute__((amdgpu_waves_per_eu(DIP ? 1 : 5)))
 void k_eval_stokes(
     const int4* __restrict__ items, const int* __restrict__ nitems,
-    const int* __restrict__ evalnode, const int* __restrict__ toff,
     const int* __restrict__ tperm, const double* __restrict__ tx, const double* __restrict__ ty,
     const int* __restrict__ nlevel, const double* __restrict__ xmid,
-    const double* __restrict__ ymid, const int* __restrict__ coll, const int2* __restrict__ crange, const int* __restrict__ bot,
-    const int* __restrict__ top, const double4* __restrict__ src,
+    const double* __restrict__ ymid, const int* __restrict__ coll,
+    const int2* __restrict__ crange, const double4* __restrict__ src,
     const double4* __restrict__ sdip,
     const double* __restrict__ le, int64_t nstride, const double* __restrict__ ops, int64_t opsz,
     int p, const double2* __restrict__ logtab, double c0x, double c0y, int64_t nt,
@@ -3464,11 +3458,11 @@ void k_eval_stokes(
   const int t0 = __builtin_amdgcn_readfirstlane(it.y), t1 = __builtin_amdgcn_readfirstlane(it.z);
   if (t1 - t0 <= kFewTargets)
     stokes_item<PD, CHECK, true, DIP, NS>(g, t0, t1, part, tperm, tx, ty, nlevel, xmid, ymid, coll, crange,
-                                      bot, top, src, sdip, le, nstride, ops, opsz, p, tab, c0x,
+                                      src, sdip, le, nstride, ops, opsz, p, tab, c0x,
                                       c0y, nt, out);
   else
     stokes_item<PD, CHECK, false, DIP, NS>(g, t0, t1, part, tperm, tx, ty, nlevel, xmid, ymid, coll, crange,
-                                       bot, top, src, sdip, le, nstride, ops, opsz, p, tab,
+                                       src, sdip, le, nstride, ops, opsz, p, tab,
                                        c0x, c0y, nt, out);
 }
 
@@ -4082,11 +4076,9 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
     auto sk = PD == 32 ? eval_stokes_pd<32>(dl, check, ns) : eval_stokes_pd<64>(dl, check, ns);
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
     hipLaunchKernelGGL(sk, dim3(eval_grid(icap, chunk, ns)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
-                       t.evalnode.as<int>(), w.toff, w.tperm,
-                       tx, ty, t.nlevel.as<int>(),
+                       w.tperm, tx, ty, t.nlevel.as<int>(),
                        t.xmid.as<double>(), t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(),
-                       t.bot.as<int>(), t.top.as<int>(), P.src.as<double4>(),
-                       dl ? P.sdip.as<double4>() : nullptr, P.le.as<double>(),
+                       P.src.as<double4>(), dl ? P.sdip.as<double4>() : nullptr, P.le.as<double>(),
                        t.n_nodes + 1, P.ops.as<double>(), opsz, P.p, P.logtab.as<double2>(),
                        t.xmin + 0.5 * t.w0, t.ymin + 0.5 * t.w0, nt, out, chunk);
     FMM_LAUNCH_CHECK();
@@ -4111,10 +4103,9 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
                               : (PD == 32 ? k_eval_mixed<32, false, false> : k_eval_mixed<64, false, false>));
     P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
     hipLaunchKernelGGL(mk, dim3(eval_grid(icap, chunk, 1)), dim3(64 * kEvalWaves), 0, s, w.items, w.ntot,
-                       t.evalnode.as<int>(), w.toff, w.tperm,
-                       tx, ty, t.nlevel.as<int>(),
+                       w.tperm, tx, ty, t.nlevel.as<int>(),
                        t.flags.as<int>(), t.xmid.as<double>(), t.ymid.as<double>(),
-                       t.coll.as<int>(), t.crange.as<int2>(), t.bot.as<int>(), t.top.as<int>(), P.src.as<double4>(),
+                       t.coll.as<int>(), t.crange.as<int2>(), P.src.as<double4>(),
                        P.srcf.as<f4>(), P.tsum.as<double>(), lc, P.le.as<double>(),
                        P.ops.as<double>(), opsz, P.cheb ? P.cheb : P.p, P.logtab.as<double2>(),
                        out, chunk);
@@ -4132,9 +4123,8 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   const size_t dyn = (size_t)scap * kEvalWaves *
                      (sizeof(double4) + (ev == EVAL_DIPOLE ? sizeof(double2) : 0));
   hipLaunchKernelGGL(kern, dim3(eval_grid(icap, chunk, ns)), dim3(64 * kEvalWaves), dyn, s, w.items, w.ntot,
-                     t.evalnode.as<int>(), w.toff, w.tperm, tx,
-                     ty, t.nlevel.as<int>(), t.xmid.as<double>(),
-                     t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(), t.bot.as<int>(), t.top.as<int>(),
+                     w.tperm, tx, ty, t.nlevel.as<int>(), t.xmid.as<double>(),
+                     t.ymid.as<double>(), t.coll.as<int>(), t.crange.as<int2>(),
                      P.src.as<double4>(), ev == EVAL_DIPOLE ? P.dip.as<double2>() : nullptr,
                      P.le.as<double>(), P.ops.as<double>(), opsz, P.cheb ? P.cheb : P.p,
                      P.logtab.as<double2>(), P.kparam, nt, out, scap, chunk);
