@@ -1365,6 +1365,8 @@ struct M2LShape {
 };
 constexpr int kM2LF64Waves = 4;
 
+// opsm: the M2L blocks of the packed operators of level 0, opsmsz doubles
+// before those of level 1
 template <int PD, int PE, int NCG, int RBW, bool ODD>
 __global__ __launch_bounds__(64 * kM2LF64Waves) void k_m2l_f64(
     LevelTable lt, const int* __restrict__ flags, const int* __restrict__ m2l,
@@ -1541,35 +1543,25 @@ __global__ __launch_bounds__(64 * kM2LF64Waves) void k_m2l_f64(
   }
 }
 
-// Blocks of a level's packed operators, each PE x PE in MFMA operand order.
-enum {
-  OPP_M2L = 0,      // 40 blocks in slot order
-  OPP_PINV1 = 40,
-  OPP_PINV2 = 41,
-  OPP_M2M = 42,     // 4 blocks
-  OPP_L2L = 46,     // 4 blocks
-  OPP_NBLK = 50,
-};
-// The packed operators of one level: dv2 entry ((blk KP + m) RB + rb) 64 +
-// lane holds row 16 rb + lane % 16 of the block, columns 8 m + 2 (lane / 16) +
-// {0, 1}; of the pseudo-inverse factors (whose B operand is a product's
-// result) and, if natural, the M2M blocks, columns 8 m + lane / 16 + {0, 4};
-// of the M2L blocks when the last
-// pair of k-steps is one step (odd), column 8 m + lane / 16 and 0 for m = KP - 1.
+// A level's packed operators: its blocks in the order of OP_*, each PE x PE in
+// MFMA operand order: dv2 entry ((blk KP + m) RB + rb) 64 + lane holds row
+// 16 rb + lane % 16 of the block, columns 8 m + 2 (lane / 16) + {0, 1}; of the
+// pseudo-inverse factors (whose B operand is a product's result) and, if
+// natural, the M2M blocks, columns 8 m + lane / 16 + {0, 4}; of the M2L blocks
+// when the last pair of k-steps is one step (odd), column 8 m + lane / 16 and 0
+// for m = KP - 1.  The first nblk blocks are packed (packed_blocks).
 __global__ __launch_bounds__(256) void k_ops_pack(const double* __restrict__ ops, int PD, int PE,
-                                                  bool odd, bool natural, dv2* __restrict__ out) {
+                                                  int nblk, bool odd, bool natural,
+                                                  dv2* __restrict__ out) {
   const int RB = PE / 16, KP = PE / 8;
-  const int n = OPP_NBLK * KP * RB * 64;
+  const int n = nblk * KP * RB * 64;
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= n) return;
   const int lane = e & 63, rb = (e >> 6) % RB, m = (e >> 6) / RB % KP, blk = (e >> 6) / RB / KP;
-  const int src = blk < OPP_PINV1 ? OP_M2L + blk
-                  : blk < OPP_M2M ? OP_PINV1 + blk - OPP_PINV1
-                  : blk < OPP_L2L ? OP_M2M + blk - OPP_M2M : OP_L2L + blk - OPP_L2L;
-  const double* row = ops + (int64_t)src * PD * PD + (16 * rb + (lane & 15)) * PD + 8 * m;
+  const double* row = ops + (int64_t)blk * PD * PD + (16 * rb + (lane & 15)) * PD + 8 * m;
   const int kq = lane >> 4;
-  if (blk >= OPP_PINV1 && blk < (natural ? OPP_L2L : OPP_M2M)) out[e] = dv2{row[kq], row[kq + 4]};
-  else if (odd && blk < OPP_PINV1 && m == KP - 1) out[e] = dv2{row[kq], 0.0};
+  if (blk < (natural ? OP_L2L : OP_M2M)) out[e] = dv2{row[kq], row[kq + 4]};
+  else if (odd && blk >= OP_M2L && m == KP - 1) out[e] = dv2{row[kq], 0.0};
   else out[e] = *reinterpret_cast<const dv2*>(row + 2 * kq);
 }
 
@@ -1682,9 +1674,9 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_mult_level(
   const int crow = with_m2m ? ri.x : -1;
   const bool up = __ballot(crow >= 0) != 0;
   const dv2* ops = opsL + l;
-  const dv2* p1 = ops + OPP_PINV1 * W::kBlock;
-  const dv2* p2 = ops + OPP_PINV2 * W::kBlock;
-  const dv2* pm = ops + OPP_M2M * W::kBlock;
+  const dv2* p1 = ops + OP_PINV1 * W::kBlock;
+  const dv2* p2 = ops + OP_PINV2 * W::kBlock;
+  const dv2* pm = ops + OP_M2M * W::kBlock;
   L.start(up ? pm : p1);
 #pragma unroll
   for (int rb = 0; rb < W::RB; ++rb)
@@ -1751,9 +1743,9 @@ __global__ __launch_bounds__(64 * kLevelWaves) void k_local_level(
     return;
   }
   const int par = parent[g];
-  const dv2* pl = opsParent + l + (OPP_L2L + c) * W::kBlock;
-  const dv2* p1 = opsL + l + OPP_PINV1 * W::kBlock;
-  const dv2* p2 = opsL + l + OPP_PINV2 * W::kBlock;
+  const dv2* pl = opsParent + l + (OP_L2L + c) * W::kBlock;
+  const dv2* p1 = opsL + l + OP_PINV1 * W::kBlock;
+  const dv2* p2 = opsL + l + OP_PINV2 * W::kBlock;
   W L;
   L.start(pl);
 #pragma unroll
@@ -3635,7 +3627,16 @@ static bool m2l_in_fp32(const Plan& P) {
 // The dense FP64 M2L of the levels in lt.
 static int m2l_pe(int p) { return (int)ceil_div(p, 16) * 16; }
 static bool m2l_odd(int p) { return (p - 1) % 8 < 4; }
-static int64_t opsm_per_level(int p) { return (int64_t)OPP_NBLK * m2l_pe(p) * m2l_pe(p); }
+// Blocks of a level that are packed: all, but for plans whose M2L always runs
+// in FP32 only those of the level kernels (10 MB instead of 52 for 32 levels
+// at p 49 to 64).
+static int packed_blocks(const Plan& P) {
+  const bool fp32 = P.precision != PREC_FP64 && !P.cheb && P.kernel_id != KER_STOKES;
+  return fp32 ? OP_M2L : OP_NBLK;
+}
+static int64_t opsm_per_level(const Plan& P) {
+  return (int64_t)packed_blocks(P) * m2l_pe(P.p) * m2l_pe(P.p);
+}
 
 template <int PD, int PE, int NCG, int RBW>
 static void m2l_f64_run(Plan& P, LevelTable& lt, hipStream_t s) {
@@ -3650,8 +3651,8 @@ static void m2l_f64_run(Plan& P, LevelTable& lt, hipStream_t s) {
   auto kern = m2l_odd(P.p) ? k_m2l_f64<PD, PE, NCG, RBW, true> : k_m2l_f64<PD, PE, NCG, RBW, false>;
   hipLaunchKernelGGL(kern, dim3(nb * Sh::RG, P.nd), dim3(64 * kM2LF64Waves), 0, s, lt,
                      t.flags.as<int>(), t.m2l.as<int>(), P.mult.as<double>(),
-                     P.opsm.as<double>(), opsm_per_level(P.p), P.ple.as<double>(), t.n_rows + 1,
-                     t.n_nodes + 1);
+                     P.opsm.as<double>() + (int64_t)OP_M2L * PE * PE, opsm_per_level(P),
+                     P.ple.as<double>(), t.n_rows + 1, t.n_nodes + 1);
   FMM_LAUNCH_CHECK();
 }
 // Fewer than two 16-box tiles per CU: two blocks share a tile's rows, since a
@@ -3758,7 +3759,7 @@ static auto mult_level_kernel(int p) {
 }
 
 static const dv2* packed_ops(const Plan& P, int level) {
-  return reinterpret_cast<const dv2*>(P.opsm.as<double>() + level * opsm_per_level(P.p));
+  return reinterpret_cast<const dv2*>(P.opsm.as<double>() + level * opsm_per_level(P));
 }
 
 typedef decltype(&k_s2m<32, KER_LAPLACE, false, 1>) S2MFn;
@@ -4437,10 +4438,11 @@ int fmm2d_set_operators(void* plan, int level, const double* dev_ops, int64_t n,
   FMM_HIP(hipMemcpyAsync(P->ops.as<double>() + level * opsz, dev_ops, opsz * sizeof(double),
                          hipMemcpyDeviceToDevice, s));
   // the copy in operand order
-  const int64_t msz = fmm::opsm_per_level(P->p);
+  const int64_t msz = fmm::opsm_per_level(*P);
   P->opsm.ensure(fmm::kMaxLevels * msz * sizeof(double));
   hipLaunchKernelGGL(fmm::k_ops_pack, dim3(fmm::grid256(msz / 2)), dim3(256), 0, s,
                      P->ops.as<double>() + level * opsz, P->PD, fmm::m2l_pe(P->p),
+                     fmm::packed_blocks(*P),
                      fmm::m2l_odd(P->p), fmm::m2m_natural(*P),
                      reinterpret_cast<fmm::dv2*>(P->opsm.as<double>() + level * msz));
   FMM_LAUNCH_CHECK();

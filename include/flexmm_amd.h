@@ -209,7 +209,13 @@ int64_t fmm2d_operator_size(int p);
  * [PD][PD] blocks, rows 0 .. PD/2-1 holding M1 = diag(s_:r) V_:r^T and rows
  * PD/2 .. PD-1 holding M2 = U_:r two rows per block row
  * (block[PD/2 + i/2][(i%2) PD/2 + j] = M2[i][j]).
- * PD = 32 for p <= 32, else 64.  Replaces Precomputation (helpers.py:250-317). */
+ * PD = 32 for p <= 32, else 64.
+ * The first call of a plan allocates room for 32 levels: these blocks, and a
+ * copy of the FP64 ones in the order its kernels read them, 50 PE^2 doubles a
+ * level with PE = p rounded up to 16 (10 PE^2 on scalar KIFMM plans of the mixed
+ * precisions, whose M2L reads the FP32 residuals).  At p 49 to 64 that is 116 MB
+ * and 52 MB (10 MB); at p <= 32, 29 MB and 13 MB (2.6 MB).
+ * Replaces Precomputation (helpers.py:250-317). */
 int fmm2d_set_operators(void* plan, int level, const double* dev_ops, int64_t n, void* stream);
 int fmm2d_clear_operators(void* plan);
 
