@@ -3661,8 +3661,10 @@ static void m2l_f64_run(Plan& P, LevelTable& lt, hipStream_t s) {
 // per CU equal).  Complete trees of at least four tiles per CU take two
 // column groups per block, which halves the operator traffic (1M points
 // 107 -> 98 us); adaptive trees do not, as the union of 32 boxes' slots there
-// multiplies more absent partners than it saves loads (100K points on a
-// curve 69 -> 93 us).
+// multiplies more absent partners than it saves loads (present columns at 16
+// and 32 boxes, and the kernel: 1M clustered points 94% and 90%, 188 -> 195 us;
+// Stokeslets and stresslets on 300K 88% and 82%, 195 -> 199; 100K points on a
+// curve 66% and 53%, 57 -> 64; 500K on a curve 81% and 70%, 229 -> 226).
 template <int PD, int PE>
 static void m2l_f64_shape(Plan& P, LevelTable& lt, hipStream_t s) {
   constexpr int RB = PE / 16, RH = RB == 4 ? 2 : 1;
