@@ -1,0 +1,59 @@
+"""Outputs that overlap the target coordinates: one and three outputs, x or y
+or both inside the output buffer or across its ends, and the evaluation that
+allocates nothing.  The same sums per target as with buffers of their own (the
+bar is that of two calls of one entry point)."""
+import numpy as np
+import pytest
+
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-13
+NT = 3001
+
+
+def _plans():
+    from flexmm_amd import _lib, kernels
+    from flexmm_amd.kifmm2d import FMM, StokesFMM, the_help
+    x, y, tau = H.uniform(9000, 81)
+    rng = np.random.default_rng(82)
+    the_help.clear()
+    f = FMM(x, y, kernels.laplace, 30, 32, bbox=[0, 1, 0, 1])
+    f.build_expansions(tau)
+    s = StokesFMM(x, y, 32, 30, bbox=[0, 1, 0, 1])
+    s.build_expansions(tau, rng.standard_normal(x.size))
+    return {"potential": (f, _lib.EVAL_POTENTIAL, 1), "gradient": (f, _lib.EVAL_GRADIENT, 3),
+            "stokes": (s, _lib.EVAL_STOKES, 3)}
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("what", ["potential", "gradient", "stokes"])
+@pytest.mark.parametrize("place", ["x_first", "y_last", "both", "across_begin", "across_end"])
+def test_output_over_the_targets(what, place, noalloc):
+    import torch
+    from flexmm_amd import _lib
+    f, ev, nout = _plans()[what]
+    call = f.lib.fmm2d_evaluate_noalloc if noalloc else f.lib.fmm2d_evaluate
+    tx, ty = (torch.from_numpy(a).cuda() for a in H.uniform(NT, 83)[:2])
+    print("in place", what, place, noalloc, flush=True)
+
+    def run(px, py, out):
+        _lib.check(call(f.handle, px.data_ptr(), py.data_ptr(), NT, ev, 0, out.data_ptr(), None))
+        torch.cuda.synchronize()
+        return out.cpu().numpy().reshape(nout, NT)
+    torch.cuda.synchronize()
+    ref = run(tx, ty, torch.empty(nout * NT, dtype=torch.float64, device="cuda"))
+    # out = buf[NT : NT + nout NT], the coordinates moved to offsets in buf
+    buf = torch.full(((nout + 2) * NT,), float("nan"), dtype=torch.float64, device="cuda")
+    out = buf[NT:NT + nout * NT]
+    at = {"x_first": (NT, None), "y_last": (None, nout * NT),
+          "both": (NT, 2 * NT), "across_begin": (NT - 700, None),
+          "across_end": (None, NT + nout * NT - 700)}[place]
+    if place == "both" and nout == 1:
+        at = (NT - 1500, NT + 1501)   # disjoint, each half inside the output
+    px, py = (c if o is None else buf[o:o + NT].copy_(c) for c, o in zip((tx, ty), at))
+    torch.cuda.synchronize()
+    got = run(px, py, out)
+    for k in range(nout):
+        assert H.rel_max_err(got[k], ref[k]) < TOL
