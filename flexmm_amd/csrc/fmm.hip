@@ -3945,16 +3945,16 @@ struct EvalScratch {
 constexpr int64_t eval_item_cap(int64_t ne, int64_t nt) { return ne + nt / kTgtChunk + 1; }
 
 // The plan's own scratch, grown to nt targets and ne evaluation boxes.
-static EvalScratch plan_scratch(Plan& P, int64_t nt, int64_t ne, bool in_place) {
+static EvalScratch plan_scratch(Plan& P, int64_t nt, int64_t ne) {
   P.tnode.ensure(nt * sizeof(int));
   P.tcnt.ensure(ne * box_copies(ne) * sizeof(int));
   P.toff.ensure(ne * box_copies(ne) * sizeof(int));
   P.tcur.ensure((nt + 1) * sizeof(int));   // per-target rank in its box
   P.tperm.ensure(nt * sizeof(int));
-  if (in_place) {
-    P.tcx.ensure(nt * sizeof(double));
-    P.tcy.ensure(nt * sizeof(double));
-  }
+  // grown whether or not this call needs the copy: a call in place may be
+  // captured into a graph after a call of the same size that was not
+  P.tcx.ensure(nt * sizeof(double));
+  P.tcy.ensure(nt * sizeof(double));
   P.bsum.ensure(ceil_div(ne, kBoxTile) * sizeof(int2));
   P.items.ensure(eval_item_cap(ne, nt) * sizeof(int4));
   P.ntot.ensure(4 * sizeof(int));
@@ -4026,7 +4026,7 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   const int64_t nout = ev == EVAL_POT || ev == EVAL_DIPOLE ? 1 : 3;
   auto overlaps = [&](const double* a) { return a < out + nout * nt && out < a + nt; };
   const bool in_place = overlaps(tx) || overlaps(ty);
-  const EvalScratch w = given ? *given : plan_scratch(P, nt, ne, in_place);
+  const EvalScratch w = given ? *given : plan_scratch(P, nt, ne);
   if (in_place) {
     hipLaunchKernelGGL(k_copy_targets, dim3(grid256(nt)), dim3(256), 0, s, tx, ty, nt, w.cx, w.cy);
     FMM_LAUNCH_CHECK();

@@ -57,3 +57,37 @@ def test_output_over_the_targets(what, place, noalloc):
     got = run(px, py, out)
     for k in range(nout):
         assert H.rel_max_err(got[k], ref[k]) < TOL
+
+
+@pytest.mark.parametrize("what", ["potential", "gradient", "stokes"])
+def test_capture_after_a_call_with_separate_buffers(what):
+    """A call that allocated for NT targets is enough for a captured call over
+    its targets; every replay gives the eager result."""
+    import torch
+    from flexmm_amd import _lib
+    f, ev, nout = _plans()[what]
+    tx, ty = (torch.from_numpy(a).cuda() for a in H.uniform(NT, 84)[:2])
+    ref = torch.empty(nout * NT, dtype=torch.float64, device="cuda")
+    buf = torch.empty(max(2, nout) * NT, dtype=torch.float64, device="cuda")
+    print("capture in place", what, flush=True)
+
+    def call(px, py, out):
+        _lib.check(f.lib.fmm2d_evaluate(f.handle, px.data_ptr(), py.data_ptr(), NT, ev, 0,
+                                        out.data_ptr(),
+                                        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    call(tx, ty, ref)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(buf[:NT], buf[NT:2 * NT], buf)
+    for _ in range(3):
+        buf[:NT].copy_(tx)
+        buf[NT:2 * NT].copy_(ty)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = buf[:nout * NT].cpu().numpy().reshape(nout, NT)
+        for k, r in enumerate(ref.cpu().numpy().reshape(nout, NT)):
+            assert H.rel_max_err(got[k], r) < TOL
+        call(tx, ty, ref)   # the program's own work between the replays
+        torch.cuda.synchronize()
