@@ -3947,8 +3947,11 @@ constexpr int64_t eval_item_cap(int64_t ne, int64_t nt) { return ne + nt / kTgtC
 // The plan's own scratch, grown to nt targets and ne evaluation boxes.
 static EvalScratch plan_scratch(Plan& P, int64_t nt, int64_t ne) {
   P.tnode.ensure(nt * sizeof(int));
-  P.tcnt.ensure(ne * box_copies(ne) * sizeof(int));
-  P.toff.ensure(ne * box_copies(ne) * sizeof(int));
+  // fewer boxes never take more: a tree of at most kCopyBoxes boxes may be
+  // evaluated under capture after a larger one
+  const int64_t counters = std::max<int64_t>(ne, (int64_t)kNumXcd * kCopyBoxes);
+  P.tcnt.ensure(counters * sizeof(int));
+  P.toff.ensure(counters * sizeof(int));
   P.tcur.ensure((nt + 1) * sizeof(int));   // per-target rank in its box
   P.tperm.ensure(nt * sizeof(int));
   // grown whether or not this call needs the copy: a call in place may be

@@ -1,7 +1,8 @@
 """Outputs that overlap the target coordinates: one and three outputs, x or y
 or both inside the output buffer or across its ends, and the evaluation that
-allocates nothing.  The same sums per target as with buffers of their own (the
-bar is that of two calls of one entry point)."""
+allocates nothing; and calls captured into graphs after eager ones.  The same sums per
+target as with buffers of their own (the bar is that of two calls of one entry
+point)."""
 import numpy as np
 import pytest
 
@@ -91,3 +92,50 @@ def test_capture_after_a_call_with_separate_buffers(what):
             assert H.rel_max_err(got[k], r) < TOL
         call(tx, ty, ref)   # the program's own work between the replays
         torch.cuda.synchronize()
+
+
+def test_capture_on_a_smaller_tree():
+    """The scratch of an evaluation on a larger tree is enough on a smaller one
+    (whose few boxes take several counters each)."""
+    import torch
+    from flexmm_amd import kernels
+    from flexmm_amd.kifmm2d import FMM, the_help
+    from flexmm_amd.kifmm2d import fmm as module
+    module._plan_pool.clear()
+    the_help.clear()
+    tx, ty = (torch.from_numpy(a).cuda() for a in H.uniform(NT, 85)[:2])
+    out = torch.empty(NT, dtype=torch.float64, device="cuda")
+    f = None
+    for n in (40000, 9000):
+        x, y, tau = (torch.from_numpy(a).cuda() for a in H.uniform(n, 86))
+        if f is not None:
+            handle = f.handle.value
+            f.close()
+        f = FMM(x, y, kernels.laplace, 6, 32, bbox=[0, 1, 0, 1])
+        f.build_expansions(tau)
+        print("boxes", f.tree.n_leaves, flush=True)
+        torch.cuda.synchronize()
+
+        def call():
+            from flexmm_amd import _lib
+            _lib.check(f.lib.fmm2d_evaluate(f.handle, tx.data_ptr(), ty.data_ptr(), NT,
+                                            _lib.EVAL_POTENTIAL, 0, out.data_ptr(),
+                                            torch.cuda.current_stream().cuda_stream))
+        if n == 40000:
+            assert f.tree.n_leaves > 4096
+            call()
+    assert f.handle.value == handle and 512 < f.tree.n_leaves <= 4096
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    got = []
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        got.append(out.cpu().numpy())
+        call()
+        torch.cuda.synchronize()
+        ref = out.cpu().numpy()
+    for g in got:
+        assert H.rel_max_err(g, ref) < TOL
