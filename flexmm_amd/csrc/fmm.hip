@@ -2354,18 +2354,6 @@ constexpr int kStageSources = 64;   // LDS staging of few-target items: sources 
 // from 2092 to 1636 us, the order-8 black-box form from 325 to 185 us, 1M
 // points on a clustered tree from 117 to 88 us (16 to 256 within 5%).
 constexpr int kItemChunk = 32;
-// Up to 16 items per SIMD, the kEvalWaves waves of a block share an item: each
-// takes a quarter of the L2T terms and of every colleague's sources, and the
-// sums are added in wave order through LDS.  One wave per item leaves such a
-// launch bound by its load and table latencies (50K points at Ncutoff 500, one
-// item per SIMD: 180 -> 81 us; 2,003 points 27 -> 11; dipoles on 100K points
-// of a curve, 12 items per SIMD, 134 -> 60; Stokeslets and stresslets on 300K
-// points, 15 per SIMD, 456 -> 382).  Past that (47 per SIMD: 84 -> 137 us), or
-// where most boxes hold few targets or none (a box per 0.5 targets: 15 -> 42
-// us), a block's start-up per item costs more than it hides.  FP32 near
-// fields keep one wave per item (their FP32 runs stay whole).
-constexpr int64_t kSplitItems = 16 * 4 * kNumCUs;
-constexpr int64_t kSplitTargets = 4;   // targets per evaluation box at least
 // this wave's item, or -1; ns waves share an item
 __device__ __forceinline__ int own_item(int ni, int chunk, int ns) {
   return xcd_item(blockIdx.x, (int)(threadIdx.x >> 6), ni, chunk, ns);
@@ -4072,7 +4060,9 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   const int64_t opsz = ops_per_level(PD);
   // few items: smaller chunks, so that every XCD gets some
   const int chunk = t.complete ? 0 : icap < 32 * kNumXcd * kItemChunk ? kItemChunk / 4 : kItemChunk;
-  const int ns = icap <= kSplitItems && nt >= kSplitTargets * ne ? kEvalWaves : 1;
+  // nearly all evaluation boxes on the deepest level
+  const bool even = t.complete || (t.L <= 16 && 10 * ne >= (int64_t)9 << (2 * (t.L - 1)));
+  const int ns = item_waves(icap, nt, ne, t.n / std::max<int64_t>(t.n_up, 1), check, even);
   if (stokes) {
     const bool dl = ev == EVAL_STOKES_DIPOLE;
     auto sk = PD == 32 ? eval_stokes_pd<32>(dl, check, ns) : eval_stokes_pd<64>(dl, check, ns);

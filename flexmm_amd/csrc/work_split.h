@@ -66,4 +66,33 @@ inline int eval_grid(int64_t icap, int chunk, int ns) {
   return (int)((per_xcd * ns + kEvalWaves - 1) / kEvalWaves * kNumXcd);
 }
 
+// Few items: the kEvalWaves waves of a block share one; each takes a quarter of
+// the L2T terms and of every colleague's sources, and the sums are added in
+// wave order through LDS.  One wave per item leaves such a launch bound by its
+// load and table latencies (50K points at Ncutoff 500, one item per SIMD: 180 ->
+// 81 us; 2,003 points 27 -> 11).  With more items that pays only where they hold
+// many sources, since a block's start-up per item (its copy of the log table)
+// then costs more than it hides; up to 16 items per SIMD, in sources per S2M
+// box (split against not): self-evaluations from kSplitSelf on (100K points of
+// a curve, 54 sources: 0.74 of the time; 100K in deep clusters, 16: 0.77; 64K
+// uniform, 4: 1.6); targets elsewhere on even trees from kSplitEven on (250K
+// uniform, 61: 0.46; 100K, 24: 1.05), on others, most of whose targets lie
+// beside no sources, from kSplitAny on (100K in clusters, 103: 0.44; 100K on a
+// curve, 54: 1.4); up to 4 items per SIMD as for self-evaluations.  Where most
+// boxes hold few targets or none (a box per 0.5 targets: 15 -> 42 us), never.
+// FP32 near fields keep one wave per item (their FP32 runs stay whole).
+constexpr int64_t kSplitItems = 16 * 4 * kNumCUs;
+constexpr int64_t kSplitTargets = 4;   // targets per evaluation box at least
+constexpr int64_t kSplitSelf = 16, kSplitEven = 32, kSplitAny = 96;
+// waves per item: icap items at most, nt targets in ne boxes, per_leaf sources
+// per S2M box; even: nearly all evaluation boxes on the deepest level
+inline int item_waves(int64_t icap, int64_t nt, int64_t ne, int64_t per_leaf, bool self,
+                      bool even) {
+  if (nt < kSplitTargets * ne || icap > kSplitItems) return 1;
+  const int64_t least = icap <= kSplitItems / 8 ? 0
+                        : self || icap <= kSplitItems / 4 ? kSplitSelf
+                        : even ? kSplitEven : kSplitAny;
+  return per_leaf >= least ? kEvalWaves : 1;
+}
+
 }  // namespace fmm

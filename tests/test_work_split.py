@@ -75,6 +75,11 @@ int main(int argc, char** argv) {
       if (waves[i] != ns) return 1;
     return 0;
   }
+  if (argc == 8 && !std::strcmp(argv[1], "waves")) {
+    const auto v = [&](int k) { return std::atoll(argv[k]); };
+    std::printf("%d", item_waves(v(2), v(3), v(4), v(5), v(6) != 0, v(7) != 0));
+    return 0;
+  }
   return 2;
 }
 """
@@ -119,3 +124,15 @@ def test_block_order_is_a_bijection(harness, n, chunk):
 def test_items_are_taken_once(harness, n, chunk, ns):
     for icap in (n, n + 1, n + 65, 3 * n):
         assert harness("items", n, icap, chunk, ns).returncode == 0, icap
+
+
+# (items, targets per box, sources per S2M box, self, even) -> waves per item
+@pytest.mark.parametrize("icap,per_box,per_leaf,own,even,waves", [
+    (1, 4, 1, 0, 0, 4), (2048, 4, 1, 0, 0, 4), (2048, 3, 500, 1, 1, 1),
+    (2049, 9, 15, 1, 1, 1), (2049, 9, 16, 0, 0, 4), (4096, 9, 16, 0, 0, 4),
+    (4097, 9, 16, 0, 1, 1), (4097, 9, 16, 1, 0, 4), (4097, 9, 31, 0, 1, 1),
+    (4097, 9, 32, 0, 1, 4), (4097, 9, 95, 0, 0, 1), (4097, 9, 96, 0, 0, 4),
+    (16384, 9, 96, 0, 0, 4), (16385, 9, 500, 1, 1, 1)])
+def test_waves_per_item(harness, icap, per_box, per_leaf, own, even, waves):
+    r = harness("waves", icap, per_box * 100, 100, per_leaf, own, even)
+    assert r.returncode == 0 and int(r.stdout) == waves
