@@ -66,6 +66,12 @@ inline int eval_grid(int64_t icap, int chunk, int ns) {
   return (int)((per_xcd * ns + kEvalWaves - 1) / kEvalWaves * kNumXcd);
 }
 
+// Whether nearly all of a tree's ne evaluation boxes are on the deepest of its
+// levels.
+inline bool even_boxes(int levels, int64_t ne) {
+  return levels <= 16 && 10 * ne >= (int64_t)9 << (2 * (levels - 1));
+}
+
 // Few items: the kEvalWaves waves of a block share one; each takes a quarter of
 // the L2T terms and of every colleague's sources, and the sums are added in
 // wave order through LDS.  One wave per item leaves such a launch bound by its
@@ -85,7 +91,7 @@ constexpr int64_t kSplitItems = 16 * 4 * kNumCUs;
 constexpr int64_t kSplitTargets = 4;   // targets per evaluation box at least
 constexpr int64_t kSplitSelf = 16, kSplitEven = 32, kSplitAny = 96;
 // waves per item: icap items at most, nt targets in ne boxes, per_leaf sources
-// per S2M box; even: nearly all evaluation boxes on the deepest level
+// per S2M box; even: even_boxes
 inline int item_waves(int64_t icap, int64_t nt, int64_t ne, int64_t per_leaf, bool self,
                       bool even) {
   if (nt < kSplitTargets * ne || icap > kSplitItems) return 1;

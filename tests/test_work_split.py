@@ -80,6 +80,10 @@ int main(int argc, char** argv) {
     std::printf("%d", item_waves(v(2), v(3), v(4), v(5), v(6) != 0, v(7) != 0));
     return 0;
   }
+  if (argc == 4 && !std::strcmp(argv[1], "even")) {
+    std::printf("%d", even_boxes(std::atoi(argv[2]), std::atoll(argv[3])));
+    return 0;
+  }
   return 2;
 }
 """
@@ -136,3 +140,11 @@ def test_items_are_taken_once(harness, n, chunk, ns):
 def test_waves_per_item(harness, icap, per_box, per_leaf, own, even, waves):
     r = harness("waves", icap, per_box * 100, 100, per_leaf, own, even)
     assert r.returncode == 0 and int(r.stdout) == waves
+
+
+@pytest.mark.parametrize("levels,ne,even", [
+    (1, 1, 1), (2, 4, 1), (2, 3, 0), (7, 4096, 1), (7, 4093, 1), (7, 3687, 1), (7, 3686, 0),
+    (7, 9067, 1), (8, 9067, 0), (16, 4 ** 15, 1), (17, 4 ** 15, 0), (31, 10 ** 6, 0)])
+def test_even_boxes(harness, levels, ne, even):
+    r = harness("even", levels, ne)
+    assert r.returncode == 0 and int(r.stdout) == even
