@@ -2516,16 +2516,28 @@ __device__ __forceinline__ uint32_t slot_min(uint32_t v, int lg) {
   return v;
 }
 
-// The L2T terms k0, k0 + step, ... < p of one target: four terms' loads in
-// flight (lanes of different source groups read different terms), each with
-// weight 0 past the last.
-template <class F>
-__device__ __forceinline__ void l2t_terms(int k0, int step, int p, F term) {
-  for (int k = k0; k < p; k += 4 * step) {
-    int kk[4];
+// The L2T terms sg, sg + ng, ... < p of one target, source group sg of F.ng in
+// each of the NS waves: the loads of four terms in flight (lanes of different
+// source groups read different terms), a lane's terms past the last one with
+// weight 0.  Terms that no lane of the wave has are left out (65K boxes of one
+// target, Laplace 52 -> 40 us, Stokeslets 138 -> 120): load(u, k) loads term k
+// as the u-th, sum(u, has) adds it.
+template <class Load, class Sum>
+__device__ __forceinline__ void l2t_terms(const FewLanes& F, int part, int ns, int p, Load load,
+                                          Sum sum) {
+  const int step = __builtin_amdgcn_readfirstlane(ns * F.ng);
+  for (int k0 = __builtin_amdgcn_readfirstlane(part * F.ng); k0 < p; k0 += 4 * step) {
+    const int k = k0 + F.sg;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) kk[u] = min(k + u * step, p - 1);
-    term(kk, k + step < p, k + 2 * step < p, k + 3 * step < p);
+    for (int u = 0; u < 4; ++u) load(u, min(k + u * step, p - 1));
+    sum(0, k < p);
+    if (k0 + step < p) {
+      sum(1, k + step < p);
+      if (k0 + 2 * step < p) {
+        sum(2, k + 2 * step < p);
+        sum(3, k + 3 * step < p);
+      }
+    }
   }
 }
 
@@ -2565,18 +2577,21 @@ __device__ __forceinline__ void eval_few(
     const double* lx = ops + d * opsz + (int64_t)OP_NBLK * PD * PD;
     const double* ly = lx + PD;
     const double* lg = le + (int64_t)g * PD;
-    l2t_terms(sg, ng, p, [&](const int (&k)[4], bool h1, bool h2, bool h3) {
+    // K0's and K1's sums are long: their loads need no more in flight, and four
+    // of them in a row only cost code size (65K boxes of one target: 185 -> 150 us)
+    if constexpr (KER == KER_MODHELM) {
+      for (int k = sg; k < p; k += ng) L.pair(lx[k], ly[k], lg[k], tab);
+    } else {
       double cx[4], cy[4], cw[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        cx[u] = lx[k[u]];
-        cy[u] = ly[k[u]];
-        cw[u] = lg[k[u]];
-      }
-      const bool has[4] = {true, h1, h2, h3};
-#pragma unroll
-      for (int u = 0; u < 4; ++u) L.pair(cx[u], cy[u], has[u] ? cw[u] : 0.0, tab);
-    });
+      l2t_terms(
+          F, part, NS, p,
+          [&](int u, int k) {
+            cx[u] = lx[k];
+            cy[u] = ly[k];
+            cw[u] = lg[k];
+          },
+          [&](int u, bool has) { L.pair(cx[u], cy[u], has ? cw[u] : 0.0, tab); });
+    }
     T.u = L.u;
     T.gx = L.gx;
     T.gy = L.gy;
@@ -3273,22 +3288,19 @@ __device__ __forceinline__ void stokes_item(
     };
     const double *a1 = a + nstride * PD, *a2 = a + 2 * nstride * PD;
     if constexpr (FEW) {
-      l2t_terms(sg, ng, p, [&](const int (&k)[4], bool h1, bool h2, bool h3) {
-        double c[4][5];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          c[u][0] = lx[k[u]];
-          c[u][1] = ly[k[u]];
-          c[u][2] = a[k[u]];
-          c[u][3] = a1[k[u]];
-          c[u][4] = a2[k[u]];
-        }
-        const bool has[4] = {true, h1, h2, h3};
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          term(c[u][0], c[u][1], has[u] ? c[u][2] : 0.0, has[u] ? c[u][3] : 0.0,
-               has[u] ? c[u][4] : 0.0);
-      });
+      double c[4][5];
+      l2t_terms(
+          F, part, NS, p,
+          [&](int u, int k) {
+            c[u][0] = lx[k];
+            c[u][1] = ly[k];
+            c[u][2] = a[k];
+            c[u][3] = a1[k];
+            c[u][4] = a2[k];
+          },
+          [&](int u, bool has) {
+            term(c[u][0], c[u][1], has ? c[u][2] : 0.0, has ? c[u][3] : 0.0, has ? c[u][4] : 0.0);
+          });
     } else {
       const int k1 = p * (part + 1) / NS;
       for (int k = p * part / NS; k < k1; ++k) term(lx[k], ly[k], a[k], a1[k], a2[k]);
