@@ -301,13 +301,11 @@ struct LogAcc {
 //   k K1(x)/r = 1/d2 + (k^2/4) (2 ln(x/2) I1' - S1'),
 // I1' = sum q^j/(j!(j+1)!), S1' the psi sum of bessel_k01 (x I1' / 2 = I1).
 // The x > 2 branch is bessel_k0_large / bessel_k01_large at x = k sqrt(d2).
-constexpr double kHelmQ8 = 0.0625, kHelmQ10 = 0.25;
 struct HelmConsts {
   double k, k2q, lnk2;   // k, k^2/4, ln(k/2)
-  double q8;             // helm_k0: largest q of the 8-term series
 };
-__device__ __forceinline__ HelmConsts helm_consts(double k, double q8 = kHelmQ8) {
-  return HelmConsts{k, 0.25 * k * k, log(0.5 * k), q8};
+__device__ __forceinline__ HelmConsts helm_consts(double k) {
+  return HelmConsts{k, 0.25 * k * k, log(0.5 * k)};
 }
 __device__ __forceinline__ double helm_lnx2(double d2, const double2* __restrict__ tab,
                                             const HelmConsts& h) {
@@ -315,12 +313,15 @@ __device__ __forceinline__ double helm_lnx2(double d2, const double2* __restrict
   log_split(d2, tab, e, t);
   return __builtin_fma(0.5, __builtin_fma(e, kLn2, t), h.lnk2);
 }
-// Terms of the series that leave out less than 2^-60 of each sum: 8 for q <=
-// 1/16, 10 for q <= 1/4 (next terms q^8/(8!)^2 = 1.4e-19, q^10/(10!)^2 =
-// 7.2e-20).  Near pairs have q = (k d/2)^2 far below 1 (at most 2 (k w)^2 in
-// boxes of width w); the number is chosen per wave, so that no lane's branch
-// adds to another's: gradient evaluation of 2.5e8 pairs
-// 932 -> 714 us (K1 has a third class; K0 alone gains nothing from it).
+// Terms of the series: 8 for q <= 1/16 and 10 for q <= 1/4 leave out less than
+// 2^-60 of K0 and of K1 (the next terms of the sums from 1 are q^8/(8!)^2 =
+// 1.4e-19 and q^10/(10!)^2 = 7.2e-20; of S0, which starts at q, 3.9e-19 and
+// 2.1e-19 are left out, against K0 > 0.9 and 0.4 there).  Near pairs have q =
+// (k d/2)^2 far below 1 (at most 2 (k w)^2 in boxes of width w); the number is
+// chosen per wave, so that no lane's branch adds to another's: gradient
+// evaluation of 2.5e8 pairs 932 -> 714 us (K1 has a third class; K0 alone gains
+// nothing from it).  FULL: always 14 terms (KER_MODHELM_FULL).
+constexpr double kHelmQ8 = 0.0625, kHelmQ10 = 0.25;
 template <int N>
 __device__ __forceinline__ double helm_k0_series(double q, double d2,
                                                  const double2* __restrict__ tab,
@@ -334,10 +335,11 @@ __device__ __forceinline__ double helm_k0_series(double q, double d2,
   }
   return __builtin_fma(-(helm_lnx2(d2, tab, h) + kEulerGamma), i0, s);
 }
+template <bool FULL>
 __device__ __forceinline__ double helm_k0(double d2, const double2* __restrict__ tab,
                                           const HelmConsts& h) {
   const double q = h.k2q * d2;
-  if (__ballot(!(q <= h.q8)) == 0) return helm_k0_series<8>(q, d2, tab, h);
+  if (!FULL && __ballot(!(q <= kHelmQ8)) == 0) return helm_k0_series<8>(q, d2, tab, h);
   if (q <= 1.0) return helm_k0_series<kBesselSeriesTerms>(q, d2, tab, h);
   return bessel_k0_large(h.k * __builtin_sqrt(d2));
 }
@@ -365,11 +367,14 @@ __device__ __forceinline__ void helm_k01_series(double q, double d2, double id2,
   k0 = __builtin_fma(-(lg + kEulerGamma), i0, s0);
   gk1 = __builtin_fma(h.k2q, __builtin_fma(2.0 * lg, i1, -s1), id2);
 }
+template <bool FULL>
 __device__ __forceinline__ void helm_k01(double d2, double id2, const double2* __restrict__ tab,
                                          const HelmConsts& h, double& k0, double& gk1) {
   const double q = h.k2q * d2;
-  if (__ballot(!(q <= kHelmQ8)) == 0) return helm_k01_series<8>(q, d2, id2, tab, h, k0, gk1);
-  if (__ballot(!(q <= kHelmQ10)) == 0) return helm_k01_series<10>(q, d2, id2, tab, h, k0, gk1);
+  if constexpr (!FULL) {
+    if (__ballot(!(q <= kHelmQ8)) == 0) return helm_k01_series<8>(q, d2, id2, tab, h, k0, gk1);
+    if (__ballot(!(q <= kHelmQ10)) == 0) return helm_k01_series<10>(q, d2, id2, tab, h, k0, gk1);
+  }
   if (q <= 1.0) return helm_k01_series<kBesselSeriesTerms>(q, d2, id2, tab, h, k0, gk1);
   const double r = __builtin_sqrt(d2);
   double k1;
@@ -381,8 +386,21 @@ __device__ __forceinline__ void helm_k01(double d2, double id2, const double2* _
 // Potential accumulators of the supported kernels: sum_j w_j K(d_j^2).
 //   Laplace           K = -log(d^2)/(4 pi)   (examples/pure_kifmm_laplace.py:24-29)
 //   modified Helmholtz K = K0(k d)/(2 pi)     (pure_kifmm_modified_helmholtz_gradient.py:36-42)
+// KER_MODHELM_FULL: the modified Helmholtz kernel by its full series, for sums
+// that must not depend on the other lanes (kSplitLeaves) and for boxes so wide
+// that whole waves hardly ever have a small q (helm_wide).
+constexpr int KER_MODHELM_FULL = 100;
 template <int KER>
-struct PotAcc;
+struct PotAcc {
+  static_assert(KER == KER_MODHELM || KER == KER_MODHELM_FULL, "kernel");
+  double s = 0.0;
+  __device__ __forceinline__ void add(double w, double d2, const double2* __restrict__ tab,
+                                      const HelmConsts& h) {
+    s = __builtin_fma(w, helm_k0<KER == KER_MODHELM_FULL>(d2, tab, h), s);
+  }
+  __device__ __forceinline__ double result() const { return kInv2Pi * s; }
+};
+
 template <>
 struct PotAcc<KER_LAPLACE> {
   LogAcc a;
@@ -391,16 +409,6 @@ struct PotAcc<KER_LAPLACE> {
     a.add(w, d2, tab);
   }
   __device__ __forceinline__ double result() const { return -kInv4Pi * a.value(); }
-};
-
-template <>
-struct PotAcc<KER_MODHELM> {
-  double s = 0.0;
-  __device__ __forceinline__ void add(double w, double d2, const double2* __restrict__ tab,
-                                      const HelmConsts& h) {
-    s = __builtin_fma(w, helm_k0(d2, tab, h), s);
-  }
-  __device__ __forceinline__ double result() const { return kInv2Pi * s; }
 };
 
 // S2M: one wave per leaf (kEvalWaves leaves per block share the log table),
@@ -415,7 +423,7 @@ struct PotAcc<KER_MODHELM> {
 // although that cancels again in FP64, the FP32 rounding in between does not:
 // another order of these sums changes mixed results by as much as their whole
 // error (1e-9 to 5e-8).  There a leaf's sums are its sources in order, by one
-// wave, with the full Helmholtz series (full_series), and the level products
+// wave, with the full Helmholtz series (KER_MODHELM_FULL), and the level products
 // are chains in one order (load_b_natural), whatever the size of the problem.
 constexpr int64_t kSplitLeaves = 64 * kNumCUs;
 // DIP: sources also carry a dipole moment q (the double layer of the Laplace
@@ -430,7 +438,6 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_s2m(int nup, const int* __r
                                             const double4* __restrict__ src,
                                             const double* __restrict__ ops, int64_t opsz, int p,
                                             const double2* __restrict__ logtab, double kp,
-                                            bool full_series,
                                             const double2* __restrict__ dip,
                                             double* __restrict__ check) {
   __shared__ double2 tab[kLogTableSize];
@@ -460,7 +467,7 @@ __global__ __launch_bounds__(64 * kEvalWaves) void k_s2m(int nup, const int* __r
     t = own.e;
   }
   PotAcc<KER> acc;
-  const HelmConsts hc = helm_consts(kp, full_series ? -1.0 : kHelmQ8);
+  const HelmConsts hc = helm_consts(kp);
   double dsum = 0.0;   // double layer
   int j = b;
   for (; j + 4 <= t; j += 4) {
@@ -2416,7 +2423,7 @@ struct Target {
         u.add(w, d2, tab, kp);
       } else {
         double k0, gk1;
-        helm_k01(d2, rcp_nr(d2), tab, kp, k0, gk1);
+        helm_k01<KER == KER_MODHELM_FULL>(d2, rcp_nr(d2), tab, kp, k0, gk1);
         u.s = __builtin_fma(w, k0, u.s);
         const double qi = z ? 0.0 : -gk1 * w;
         gx = __builtin_fma(qi, dx, gx);
@@ -2579,7 +2586,7 @@ __device__ __forceinline__ void eval_few(
     const double* lg = le + (int64_t)g * PD;
     // K0's and K1's sums are long: their loads need no more in flight, and four
     // of them in a row only cost code size (65K boxes of one target: 185 -> 150 us)
-    if constexpr (KER == KER_MODHELM) {
+    if constexpr (KER != KER_LAPLACE) {
       for (int k = sg; k < p; k += ng) L.pair(lx[k], ly[k], lg[k], tab);
     } else {
       double cx[4], cy[4], cw[4];
@@ -2696,7 +2703,7 @@ __device__ __forceinline__ void eval_few(
 // it needs 169 unconstrained, which leaves 2).
 template <int PD, int KER, int NOUT, bool CHECK, bool DIP, bool CHEB, int NS>
 __global__ __launch_bounds__(64 * kEvalWaves)
-__attribute__((amdgpu_waves_per_eu(KER == KER_MODHELM && NOUT == 3 ? 3 : 1))) void k_eval(
+__attribute__((amdgpu_waves_per_eu(KER != KER_LAPLACE && NOUT == 3 ? 3 : 1))) void k_eval(
     const int4* __restrict__ items, const int* __restrict__ nitems,
     const int* __restrict__ tperm, const double* __restrict__ tx, const double* __restrict__ ty,
     const int* __restrict__ nlevel, const double* __restrict__ xmid,
@@ -3467,6 +3474,13 @@ EvalStokesFn eval_stokes_pd(bool dl, bool check, int ns) {
             : (check ? k_eval_stokes<PD, true, false, NS> : k_eval_stokes<PD, false, false, NS>);
 }
 
+// Where the smallest boxes' width w makes k w larger than this, a wave hardly
+// ever has small q throughout, and asking costs more than it saves (one wave
+// per item, with the classes and without: potential of 250K points at k w 0.16
+// 320 and 346 us, at 0.78 789 and 760, gradient there 1323 and 1283; items
+// shared by four waves equal within 2%).
+inline bool helm_wide(double k, double w, bool gradient) { return k * w > (gradient ? 0.6 : 0.4); }
+
 // Selects the k_eval instance of (PD, kernel, outputs, self-exclusion, waves per item).
 typedef decltype(&k_eval<32, KER_LAPLACE, 1, false, false, false, 1>) EvalKernelFn;
 template <int PD, int KER, int NOUT, bool DIP, bool CHEB>
@@ -3478,7 +3492,7 @@ EvalKernelFn eval_kernel_of(bool check, int ns) {
                : k_eval<PD, KER, NOUT, false, DIP, CHEB, kEvalWaves>;
 }
 template <int PD>
-EvalKernelFn eval_kernel_pd(int ker, int ev, bool cheb, bool check, int ns) {
+EvalKernelFn eval_kernel_pd(int ker, int ev, bool cheb, bool check, int ns, bool helm_full) {
   if (cheb)   // Chebyshev (black-box) expansions: potential only
     return ker == KER_LAPLACE ? eval_kernel_of<PD, KER_LAPLACE, 1, false, true>(check, ns)
                               : eval_kernel_of<PD, KER_MODHELM, 1, false, true>(check, ns);
@@ -3487,6 +3501,11 @@ EvalKernelFn eval_kernel_pd(int ker, int ev, bool cheb, bool check, int ns) {
   if (ker == KER_LAPLACE)
     return ev == EVAL_POT ? eval_kernel_of<PD, KER_LAPLACE, 1, false, false>(check, ns)
                           : eval_kernel_of<PD, KER_LAPLACE, 3, false, false>(check, ns);
+  if (ns == 1 && helm_full)
+    return ev == EVAL_POT ? (check ? k_eval<PD, KER_MODHELM_FULL, 1, true, false, false, 1>
+                                   : k_eval<PD, KER_MODHELM_FULL, 1, false, false, false, 1>)
+                          : (check ? k_eval<PD, KER_MODHELM_FULL, 3, true, false, false, 1>
+                                   : k_eval<PD, KER_MODHELM_FULL, 3, false, false, false, 1>);
   return ev == EVAL_POT ? eval_kernel_of<PD, KER_MODHELM, 1, false, false>(check, ns)
                         : eval_kernel_of<PD, KER_MODHELM, 3, false, false>(check, ns);
 }
@@ -3766,6 +3785,8 @@ typedef decltype(&k_s2m<32, KER_LAPLACE, false, 1>) S2MFn;
 template <int PD, int NS>
 static S2MFn s2m_kernel_of(int ker, bool dip) {
   if (dip) return k_s2m<PD, KER_LAPLACE, true, NS>;
+  if constexpr (NS == 1)
+    if (ker == KER_MODHELM_FULL) return k_s2m<PD, KER_MODHELM_FULL, false, NS>;
   return ker == KER_LAPLACE ? k_s2m<PD, KER_LAPLACE, false, NS> : k_s2m<PD, KER_MODHELM, false, NS>;
 }
 static S2MFn s2m_kernel(int PD, int ker, bool dip, int ns) {
@@ -3854,12 +3875,14 @@ static void upward(Plan& P, const double* tau, const double* dvec, hipStream_t s
                        P.ops.as<double>(), opsz, P.cheb, P.check.as<double>());
     FMM_LAUNCH_CHECK();
   } else if (t.n_up > 0) {
-    auto kern = s2m_kernel(PD, P.kernel_id, dvec != nullptr, sns);
+    auto kern = s2m_kernel(
+        PD, P.kernel_id == KER_MODHELM && m2l_in_fp32(P) ? KER_MODHELM_FULL : P.kernel_id,
+        dvec != nullptr, sns);
     hipLaunchKernelGGL(kern, dim3(ceil_div(t.n_up * sns, kEvalWaves)), dim3(64 * kEvalWaves), 0, s,
                        (int)t.n_up, t.upnodes.as<int>(), t.nlevel.as<int>(),
                        t.bot.as<int>(), t.top.as<int>(), t.row.as<int>(), t.xmid.as<double>(),
                        t.ymid.as<double>(), P.src.as<double4>(), P.ops.as<double>(), opsz, P.p,
-                       P.logtab.as<double2>(), P.kparam, m2l_in_fp32(P),
+                       P.logtab.as<double2>(), P.kparam,
                        dvec ? P.dip.as<double2>() : nullptr, P.check.as<double>());
     FMM_LAUNCH_CHECK();
   }
@@ -4118,8 +4141,10 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
     P.mark(FMM2D_PHASE_EVAL_KERNEL, true, s);
     return;
   }
-  auto kern = PD == 32 ? eval_kernel_pd<32>(P.kernel_id, ev, P.cheb > 0, check, ns)
-                       : eval_kernel_pd<64>(P.kernel_id, ev, P.cheb > 0, check, ns);
+  const bool wide = P.kernel_id == KER_MODHELM &&
+                    helm_wide(P.kparam, t.lev[t.L - 1].width, ev != EVAL_POT);
+  auto kern = PD == 32 ? eval_kernel_pd<32>(P.kernel_id, ev, P.cheb > 0, check, ns, wide)
+                       : eval_kernel_pd<64>(P.kernel_id, ev, P.cheb > 0, check, ns, wide);
   P.mark(FMM2D_PHASE_EVAL_KERNEL, false, s);
   // few targets per evaluation box on average: the few-target items stage
   // their colleague sources through LDS (the extra LDS would only cost the
