@@ -1158,22 +1158,26 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
 // rows, so a block takes all three: per slot and wave 24 row loads and 16
 // piece loads feed 192 MFMAs.  One field per block loaded the pieces three
 // times and five rows instead of three, which kept the texture unit busier
-// than the matrix cores (2M clustered Stokeslets 869 -> 701 us).
-template <int PD, int NW>
+// than the matrix cores (2M clustered Stokeslets 869 -> 701 us).  With fewer
+// tiles than CUs a tile's MFMAs are the kernel's length: blocks then take RBW
+// row blocks each (p 64: 4 tiles, one field per block 32 us, all rows per block
+// 46, one row block each 25; 24 tiles 36, 51, 32; 88 tiles 43, 53, 43 with two).
+template <int PD, int NW, int RBW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void k_m2l_frame_f32(
     LevelTable lt, const int* __restrict__ flags, const int* __restrict__ m2l,
     const double* __restrict__ mult, const double* __restrict__ qs,
     const double* __restrict__ ops, int64_t opsz, double* __restrict__ ple, int64_t rstride,
     int64_t nstride, const double* __restrict__ xmid, const double* __restrict__ ymid, double c0x,
     double c0y) {
-  constexpr int RB = PD / 16, KS = PD / 4, NA = KS / 4, NP = RB * NA, NF = 3;
+  constexpr int RB = PD / 16, KS = PD / 4, NA = KS / 4, NP = RBW * NA, NF = 3;
+  const int rb0 = blockIdx.y * RBW;   // this block's first row block
   typedef float fv4 __attribute__((ext_vector_type(4)));
   __shared__ int srcs[27][16];
   __shared__ double qsl[NF][27][16];   // source charge sums (0: no source)
   __shared__ int pslot[28];
   __shared__ int pslotv[27];   // the M2L slot (offset) of each used slot index
   __shared__ unsigned int smask;
-  __shared__ double red[NW - 1][PD][17];
+  __shared__ double red[NW - 1][16 * RBW][17];
   const int bid = xcd_block(blockIdx.x, gridDim.x, lt.xchunk);
   int li = 0;
   while (li + 1 < lt.nlev && bid >= lt.boff[li + 1]) ++li;
@@ -1228,20 +1232,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   __syncthreads();
   const double* opsL = ops + (int64_t)lt.d[li] * opsz;
   const double* means = opsL + ops_off_means(PD);
-  // residual piece pc = rb NA + j of a slot: afr[(slot NP + pc) 64]
-  const fv4* afr = reinterpret_cast<const fv4*>(opsL + ops_off_r32(PD)) + l;
-  d4 acc64[NF][RB];
+  // residual piece pc = rb NA + j of a slot, from row block rb0 on: afr[(slot RB NA + pc) 64]
+  const fv4* afr = reinterpret_cast<const fv4*>(opsL + ops_off_r32(PD)) + rb0 * NA * 64 + l;
+  d4 acc64[NF][RBW];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc64[f][rb] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int rb = 0; rb < RBW; ++rb) acc64[f][rb] = d4{0.0, 0.0, 0.0, 0.0};
   // this wave's slots: pslot[w + NW j], j < nmine
   const int nmine = w < nph ? (nph - 1 - w) / NW + 1 : 0;
   if (nmine > 0) {
     int slot = __builtin_amdgcn_readfirstlane(pslotv[w]);
     fv4 a[NA];
 #pragma unroll
-    for (int j = 0; j < NA; ++j) a[j] = afr[((int64_t)slot * NP + j) * 64];
+    for (int j = 0; j < NA; ++j) a[j] = afr[((int64_t)slot * RB * NA + j) * 64];
     for (int jj = 0; jj < nmine; ++jj) {
       const int k = w + NW * jj;
       const int slot_n = __builtin_amdgcn_readfirstlane(pslotv[jj + 1 < nmine ? k + NW : k]);
@@ -1286,7 +1290,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
             s[f][h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][2 + h], bu[f][j][2 + h], s[f][h],
                                                            0, 0, 0);
         // the piece just used is reloaded with the one a row block further on
-        a[j] = afr[((int64_t)(pc + NA < NP ? slot : slot_n) * NP + (pc + NA) % NP) * 64];
+        a[j] = afr[((int64_t)(pc + NA < NP ? slot : slot_n) * RB * NA + (pc + NA) % NP) * 64];
 #pragma unroll
         for (int f = 0; f < NF; ++f)
 #pragma unroll
@@ -1301,12 +1305,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
       const int kk = k0 + NW * kq;
       const bool ok = kk < nph;
       const int ks = ok ? kk : k0;
-      const double* mrow = means + (int64_t)pslotv[ks] * PD + prow;
+      const double* mrow = means + (int64_t)pslotv[ks] * PD + 16 * rb0 + prow;
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         const double bq = ok ? qsl[f][pslot[ks]][col] : 0.0;
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+        for (int rb = 0; rb < RBW; ++rb)
           acc64[f][rb] =
               __builtin_amdgcn_mfma_f64_16x16x4f64(mrow[16 * rb], bq, acc64[f][rb], 0, 0, 0);
       }
@@ -1314,22 +1318,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   }
   // waves 1 .. NW-1 hand their sums to wave 0, which adds them in wave order
   // and returns fields 0 and 1 to the root frame: PLE_i -= c_i PLE_2
-  d4 sum2[RB];
+  d4 sum2[RBW];
 #pragma unroll
   for (int f = NF - 1; f >= 0; --f) {
     if (f < NF - 1) __syncthreads();
     if (w > 0) {
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+      for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) red[w - 1][16 * rb + 4 * kq + v][col] = acc64[f][rb][v];
     }
     __syncthreads();
     if (w == 0 && active) {
-      double* rowp = ple + (f * nstride + g) * PD;
+      double* rowp = ple + (f * nstride + g) * PD + 16 * rb0;
       const double ct = f == 0 ? ctx : cty;
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+      for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           double sum = acc64[f][rb][v];
@@ -3732,8 +3736,13 @@ static void m2l_launch(Plan& P, const M2LTables& T, int l0, int l1, hipStream_t 
     lw.split = 1;
     constexpr int NW = kM2LF32Waves;
     if (P.kernel_id == KER_STOKES) {
-      auto kern = PD == 32 ? k_m2l_frame_f32<32, NW> : k_m2l_frame_f32<64, NW>;
-      hipLaunchKernelGGL(kern, dim3(nbw), dim3(64 * NW), 0, s, lw, t.flags.as<int>(), t.m2l.as<int>(),
+      // blocks that share a tile's rows: as many as there are row blocks while
+      // every block has a CU of its own
+      const int rg = PD == 64 && 4 * nbw <= kNumCUs ? 4 : 2 * nbw <= kNumCUs ? 2 : 1;
+      auto kern = PD == 32 ? (rg == 2 ? k_m2l_frame_f32<32, NW, 1> : k_m2l_frame_f32<32, NW, 2>)
+                  : rg == 4 ? k_m2l_frame_f32<64, NW, 1>
+                  : rg == 2 ? k_m2l_frame_f32<64, NW, 2> : k_m2l_frame_f32<64, NW, 4>;
+      hipLaunchKernelGGL(kern, dim3(nbw, rg), dim3(64 * NW), 0, s, lw, t.flags.as<int>(), t.m2l.as<int>(),
                          P.mult.as<double>(), P.qs.as<double>(), P.ops.as<double>(), opsz,
                          P.ple.as<double>(), rstride, nstride, t.xmid.as<double>(),
                          t.ymid.as<double>(), t.xmin + 0.5 * t.w0, t.ymin + 0.5 * t.w0);
