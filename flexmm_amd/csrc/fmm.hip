@@ -2358,10 +2358,10 @@ __global__ __launch_bounds__(1024) void k_box_items(int* __restrict__ tcnt, int 
 // turn.  Surplus waves exit.  (A grid capped at 8 blocks per CU, waves
 // striding over several items, measured 8-20% slower.)
 constexpr int kStageSources = 64;   // LDS staging of few-target items: sources per wave and chunk
-// Items of an even tree (nearly all boxes on the deepest level) cost about the
-// same, and eighths keep the most sources in one L2 (mixed form, 1M points: 208
-// us, 229 with chunks of 32; 250K points, all but three boxes on the deepest
-// level, self: 207, 255 with chunks of 8).
+// Items of a complete or nearly complete tree (even_items) cost about the same,
+// and eighths keep the most sources in one L2 (mixed form, 1M points: 208 us, 229
+// with chunks of 32; 250K points, all but three boxes on the deepest level, self:
+// 207, 255 with chunks of 8).
 // Elsewhere an item's cost follows its level and cluster, so eighths leave
 // whole XCDs idle: chunks of 32 took the Stokeslet on 2M clustered points
 // from 2092 to 1636 us, the order-8 black-box form from 325 to 185 us, 1M
@@ -4106,7 +4106,9 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   const int64_t opsz = ops_per_level(PD);
   const bool even = even_boxes(t.L, ne);
   // few items: smaller chunks, so that every XCD gets some
-  const int chunk = even ? 0 : icap < 32 * kNumXcd * kItemChunk ? kItemChunk / 4 : kItemChunk;
+  const int chunk = even_items(t.L, ne)                  ? 0
+                    : icap < 32 * kNumXcd * kItemChunk ? kItemChunk / 4
+                                                       : kItemChunk;
   const int ns = item_waves(icap, nt, ne, t.n / std::max<int64_t>(t.n_up, 1), check, even);
   if (stokes) {
     const bool dl = ev == EVAL_STOKES_DIPOLE;

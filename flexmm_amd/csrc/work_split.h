@@ -72,6 +72,17 @@ inline bool even_boxes(int levels, int64_t ne) {
   return levels <= 16 && 10 * ne >= (int64_t)9 << (2 * (levels - 1));
 }
 
+// Whether so few boxes lie above the deepest level that a contiguous eighth of
+// the items costs about an eighth.  The boxes come level by level and those
+// above hold four times the targets, all in the first eighth: where m boxes of
+// the deepest level are missing it costs about 1 + 8m/ne of another.  Measured,
+// eighths against chunks: a 1400th missing 199 and 239 us (250K points, mixed,
+// self), a 200th 220 and 225, a 93rd 224 and 213, a 16th 335 and 220 (1M points,
+// FP64, self).
+inline bool even_items(int levels, int64_t ne) {
+  return levels <= 16 && 128 * ne >= (int64_t)127 << (2 * (levels - 1));
+}
+
 // Few items: the kEvalWaves waves of a block share one; each takes a quarter of
 // the L2T terms and of every colleague's sources, and the sums are added in
 // wave order through LDS.  One wave per item leaves such a launch bound by its

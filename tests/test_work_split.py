@@ -84,6 +84,10 @@ int main(int argc, char** argv) {
     std::printf("%d", even_boxes(std::atoi(argv[2]), std::atoll(argv[3])));
     return 0;
   }
+  if (argc == 4 && !std::strcmp(argv[1], "even_items")) {
+    std::printf("%d", even_items(std::atoi(argv[2]), std::atoll(argv[3])));
+    return 0;
+  }
   return 2;
 }
 """
@@ -147,4 +151,12 @@ def test_waves_per_item(harness, icap, per_box, per_leaf, own, even, waves):
     (7, 9067, 1), (8, 9067, 0), (16, 4 ** 15, 1), (17, 4 ** 15, 0), (31, 10 ** 6, 0)])
 def test_even_boxes(harness, levels, ne, even):
     r = harness("even", levels, ne)
+    assert r.returncode == 0 and int(r.stdout) == even
+
+
+@pytest.mark.parametrize("levels,ne,even", [
+    (1, 1, 1), (2, 4, 1), (2, 3, 0), (7, 4096, 1), (7, 4093, 1), (7, 4064, 1), (7, 4063, 0),
+    (9, 65024, 1), (9, 65023, 0), (9, 61447, 0), (16, 4 ** 15, 1), (17, 4 ** 15, 0)])
+def test_even_items(harness, levels, ne, even):
+    r = harness("even_items", levels, ne)
     assert r.returncode == 0 and int(r.stdout) == even
