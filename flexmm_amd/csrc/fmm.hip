@@ -4104,7 +4104,7 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   FMM_LAUNCH_CHECK();
   const int PD = P.PD;
   const int64_t opsz = ops_per_level(PD);
-  const bool even = even_boxes(t.L, ne);
+  const bool even = even_boxes(t.L, ne) || broad_sources(t.L, t.n_up);
   // few items: smaller chunks, so that every XCD gets some
   const int chunk = even_items(t.L, ne)                  ? 0
                     : icap < 32 * kNumXcd * kItemChunk ? kItemChunk / 4

@@ -72,6 +72,13 @@ inline bool even_boxes(int levels, int64_t ne) {
   return levels <= 16 && 10 * ne >= (int64_t)9 << (2 * (levels - 1));
 }
 
+// Whether boxes with sources (n_up of them) cover a fifth of the root box, each
+// counted as one of the deepest level: a uniform set in a root box of up to
+// twice its size.  Targets then lie beside sources as on an even tree.
+inline bool broad_sources(int levels, int64_t n_up) {
+  return levels <= 16 && 5 * n_up >= (int64_t)1 << (2 * (levels - 1));
+}
+
 // Whether so few boxes lie above the deepest level that a contiguous eighth of
 // the items costs about an eighth.  The boxes come level by level and those
 // above hold four times the targets, all in the first eighth: where m boxes of
@@ -92,17 +99,18 @@ inline bool even_items(int levels, int64_t ne) {
 // then costs more than it hides; up to 16 items per SIMD, in sources per S2M
 // box (split against not): self-evaluations from kSplitSelf on (100K points of
 // a curve, 54 sources: 0.74 of the time; 100K in deep clusters, 16: 0.77; 64K
-// uniform, 4: 1.6); targets elsewhere on even trees from kSplitEven on (250K
-// uniform, 61: 0.46; 100K, 24: 1.05), on others, most of whose targets lie
-// beside no sources, from kSplitAny on (100K in clusters, 103: 0.44; 100K on a
-// curve, 54: 1.4); up to 4 items per SIMD as for self-evaluations.  Where most
+// uniform, 4: 1.6); targets elsewhere on even trees and where sources are
+// broad from kSplitEven on (250K uniform, 61: 0.46, in a box of twice their
+// size 0.75 of the whole call; 100K, 24: 1.05), on others, most of whose
+// targets lie beside no sources, from kSplitAny on (100K in clusters, 103: 0.44;
+// 100K on a curve, 54: 1.4); up to 4 items per SIMD as for self-evaluations.  Where most
 // boxes hold few targets or none (a box per 0.5 targets: 15 -> 42 us), never.
 // FP32 near fields keep one wave per item (their FP32 runs stay whole).
 constexpr int64_t kSplitItems = 16 * 4 * kNumCUs;
 constexpr int64_t kSplitTargets = 4;   // targets per evaluation box at least
 constexpr int64_t kSplitSelf = 16, kSplitEven = 32, kSplitAny = 96;
 // waves per item: icap items at most, nt targets in ne boxes, per_leaf sources
-// per S2M box; even: even_boxes
+// per S2M box; even: even_boxes or broad_sources
 inline int item_waves(int64_t icap, int64_t nt, int64_t ne, int64_t per_leaf, bool self,
                       bool even) {
   if (nt < kSplitTargets * ne || icap > kSplitItems) return 1;

@@ -84,6 +84,10 @@ int main(int argc, char** argv) {
     std::printf("%d", even_boxes(std::atoi(argv[2]), std::atoll(argv[3])));
     return 0;
   }
+  if (argc == 4 && !std::strcmp(argv[1], "broad")) {
+    std::printf("%d", broad_sources(std::atoi(argv[2]), std::atoll(argv[3])));
+    return 0;
+  }
   if (argc == 4 && !std::strcmp(argv[1], "even_items")) {
     std::printf("%d", even_items(std::atoi(argv[2]), std::atoll(argv[3])));
     return 0;
@@ -160,3 +164,11 @@ def test_even_boxes(harness, levels, ne, even):
 def test_even_items(harness, levels, ne, even):
     r = harness("even_items", levels, ne)
     assert r.returncode == 0 and int(r.stdout) == even
+
+
+@pytest.mark.parametrize("levels,n_up,broad", [
+    (1, 1, 1), (2, 1, 1), (3, 3, 0), (3, 4, 1), (8, 4096, 1), (8, 3277, 1), (8, 3276, 0),
+    (10, 4080, 0), (16, 4 ** 14, 1), (17, 4 ** 16, 0)])
+def test_broad_sources(harness, levels, n_up, broad):
+    r = harness("broad", levels, n_up)
+    assert r.returncode == 0 and int(r.stdout) == broad
