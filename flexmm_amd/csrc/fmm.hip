@@ -4104,12 +4104,11 @@ static void evaluate(Plan& P, const double* tx, const double* ty, int64_t nt, in
   FMM_LAUNCH_CHECK();
   const int PD = P.PD;
   const int64_t opsz = ops_per_level(PD);
-  const bool even = even_boxes(t.L, ne) || broad_sources(t.L, t.n_up);
   // few items: smaller chunks, so that every XCD gets some
   const int chunk = even_items(t.L, ne)                  ? 0
                     : icap < 32 * kNumXcd * kItemChunk ? kItemChunk / 4
                                                        : kItemChunk;
-  const int ns = item_waves(icap, nt, ne, t.n / std::max<int64_t>(t.n_up, 1), check, even);
+  const int ns = item_waves(icap, nt, ne, t.n, t.n_up, t.L, check);
   if (stokes) {
     const bool dl = ev == EVAL_STOKES_DIPOLE;
     auto sk = PD == 32 ? eval_stokes_pd<32>(dl, check, ns) : eval_stokes_pd<64>(dl, check, ns);

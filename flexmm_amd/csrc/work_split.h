@@ -66,15 +66,9 @@ inline int eval_grid(int64_t icap, int chunk, int ns) {
   return (int)((per_xcd * ns + kEvalWaves - 1) / kEvalWaves * kNumXcd);
 }
 
-// Whether nearly all of a tree's ne evaluation boxes are on the deepest of its
-// levels.
-inline bool even_boxes(int levels, int64_t ne) {
-  return levels <= 16 && 10 * ne >= (int64_t)9 << (2 * (levels - 1));
-}
-
 // Whether boxes with sources (n_up of them) cover a fifth of the root box, each
 // counted as one of the deepest level: a uniform set in a root box of up to
-// twice its size.  Targets then lie beside sources as on an even tree.
+// twice its size.
 inline bool broad_sources(int levels, int64_t n_up) {
   return levels <= 16 && 5 * n_up >= (int64_t)1 << (2 * (levels - 1));
 }
@@ -94,30 +88,39 @@ inline bool even_items(int levels, int64_t ne) {
 // the L2T terms and of every colleague's sources, and the sums are added in
 // wave order through LDS.  One wave per item leaves such a launch bound by its
 // load and table latencies (50K points at Ncutoff 500, one item per SIMD: 180 ->
-// 81 us; 2,003 points 27 -> 11).  With more items that pays only where they hold
-// many sources, since a block's start-up per item (its copy of the log table)
-// then costs more than it hides; up to 16 items per SIMD, in sources per S2M
-// box (split against not): self-evaluations from kSplitSelf on (100K points of
-// a curve, 54 sources: 0.74 of the time; 100K in deep clusters, 16: 0.77; 64K
-// uniform, 4: 1.6); targets elsewhere on even trees and where sources are
-// broad from kSplitEven on (250K uniform, 61: 0.46, in a box of twice their
-// size 0.75 of the whole call; 100K, 24: 1.05), on others, most of whose
-// targets lie beside no sources, from kSplitAny on (100K in clusters, 103: 0.44;
-// 100K on a curve, 54: 1.4); up to 4 items per SIMD as for self-evaluations.  Where most
-// boxes hold few targets or none (a box per 0.5 targets: 15 -> 42 us), never.
-// FP32 near fields keep one wave per item (their FP32 runs stay whole).
+// 81 us; 2,003 points 27 -> 11).  With more items, up to 16 per SIMD, that pays
+// only where they hold many sources, since a block's start-up per item (its copy
+// of the log table) then costs more than it hides.  Lines in sources per box,
+// and shared against not (Laplace; K0, the Stokeslet and the black-box form lie
+// around it):
+//   self-evaluations kSplitSelf: 100K points of a curve, 54 sources: 0.74; 60K in
+//   clusters, 15: 0.65; 30K uniform, 7: 1.08; 64K uniform, 4: 1.6;
+//   up to 4 items per SIMD, and broad sources in boxes of several levels (a few
+//   items then hold most sources) kSplitUneven: 46K uniform, 27: 0.51; 60K, 16:
+//   0.54; 100K, 7: 1.6;
+//   where most boxes hold sources kSplitMost: 250K uniform, 61: 0.46; 200K in
+//   clusters, 44: 0.74; 100K uniform, 24: 1.0; 300K in clusters, 25: 1.2;
+//   elsewhere kSplitAny, as most targets lie beside no sources: 100K on a curve,
+//   113: 0.63; 54: 1.4.
+// Where most boxes hold few targets or none (a box per 0.5 targets: 15 -> 42
+// us), never.  FP32 near fields keep one wave per item (their FP32 runs stay
+// whole).
 constexpr int64_t kSplitItems = 16 * 4 * kNumCUs;
 constexpr int64_t kSplitTargets = 4;   // targets per evaluation box at least
-constexpr int64_t kSplitSelf = 16, kSplitEven = 32, kSplitAny = 96;
-// waves per item: icap items at most, nt targets in ne boxes, per_leaf sources
-// per S2M box; even: even_boxes or broad_sources
-inline int item_waves(int64_t icap, int64_t nt, int64_t ne, int64_t per_leaf, bool self,
-                      bool even) {
+constexpr int64_t kSplitSelf = 9, kSplitUneven = 16, kSplitMost = 32, kSplitAny = 96;
+// waves per item: icap items at most, nt targets in ne boxes, n sources in n_up
+// S2M boxes of a tree of so many levels
+inline int item_waves(int64_t icap, int64_t nt, int64_t ne, int64_t n, int64_t n_up, int levels,
+                      bool self) {
   if (nt < kSplitTargets * ne || icap > kSplitItems) return 1;
-  const int64_t least = icap <= kSplitItems / 8 ? 0
-                        : self || icap <= kSplitItems / 4 ? kSplitSelf
-                        : even ? kSplitEven : kSplitAny;
-  return per_leaf >= least ? kEvalWaves : 1;
+  int64_t least = kSplitAny;
+  if (icap <= kSplitItems / 8) least = 0;
+  else if (self) least = kSplitSelf;
+  else if (icap <= kSplitItems / 4 || (broad_sources(levels, n_up) && !even_items(levels, ne)))
+    least = kSplitUneven;
+  else if (2 * n_up >= ne) least = kSplitMost;
+  // S2M boxes can outnumber the leaves (their parts beside smaller boxes)
+  return n >= least * (n_up < ne ? n_up : ne) ? kEvalWaves : 1;
 }
 
 }  // namespace fmm

@@ -75,13 +75,9 @@ int main(int argc, char** argv) {
       if (waves[i] != ns) return 1;
     return 0;
   }
-  if (argc == 8 && !std::strcmp(argv[1], "waves")) {
+  if (argc == 9 && !std::strcmp(argv[1], "waves")) {
     const auto v = [&](int k) { return std::atoll(argv[k]); };
-    std::printf("%d", item_waves(v(2), v(3), v(4), v(5), v(6) != 0, v(7) != 0));
-    return 0;
-  }
-  if (argc == 4 && !std::strcmp(argv[1], "even")) {
-    std::printf("%d", even_boxes(std::atoi(argv[2]), std::atoll(argv[3])));
+    std::printf("%d", item_waves(v(2), v(3), v(4), v(5), v(6), (int)v(7), v(8) != 0));
     return 0;
   }
   if (argc == 4 && !std::strcmp(argv[1], "broad")) {
@@ -138,24 +134,27 @@ def test_items_are_taken_once(harness, n, chunk, ns):
         assert harness("items", n, icap, chunk, ns).returncode == 0, icap
 
 
-# (items, targets per box, sources per S2M box, self, even) -> waves per item
-@pytest.mark.parametrize("icap,per_box,per_leaf,own,even,waves", [
-    (1, 4, 1, 0, 0, 4), (2048, 4, 1, 0, 0, 4), (2048, 3, 500, 1, 1, 1),
-    (2049, 9, 15, 1, 1, 1), (2049, 9, 16, 0, 0, 4), (4096, 9, 16, 0, 0, 4),
-    (4097, 9, 16, 0, 1, 1), (4097, 9, 16, 1, 0, 4), (4097, 9, 31, 0, 1, 1),
-    (4097, 9, 32, 0, 1, 4), (4097, 9, 95, 0, 0, 1), (4097, 9, 96, 0, 0, 4),
-    (16384, 9, 96, 0, 0, 4), (16385, 9, 500, 1, 1, 1)])
-def test_waves_per_item(harness, icap, per_box, per_leaf, own, even, waves):
-    r = harness("waves", icap, per_box * 100, 100, per_leaf, own, even)
+# 1000 evaluation boxes.  (items, targets per box, sources per box, S2M boxes,
+# levels, self) -> waves per item; 1000 boxes of 6 levels: broad, not complete
+@pytest.mark.parametrize("icap,per_box,per_leaf,n_up,levels,own,waves", [
+    (1, 4, 1, 100, 20, 0, 4), (2048, 4, 0, 100, 20, 0, 4), (2048, 3, 500, 1000, 6, 1, 1),
+    (2049, 9, 8, 1000, 6, 1, 1), (2049, 9, 9, 1000, 6, 1, 4), (16384, 9, 9, 100, 20, 1, 4),
+    (2049, 9, 15, 100, 20, 0, 1), (4096, 9, 16, 100, 20, 0, 4),
+    (4097, 9, 15, 1000, 6, 0, 1), (4097, 9, 16, 1000, 6, 0, 4), (4097, 9, 16, 205, 6, 0, 4),
+    (4097, 9, 16, 204, 6, 0, 1), (4097, 9, 31, 1000, 20, 0, 1), (4097, 9, 32, 1000, 20, 0, 4),
+    (4097, 9, 32, 500, 20, 0, 4), (4097, 9, 95, 499, 20, 0, 1), (4097, 9, 96, 499, 20, 0, 4),
+    (4097, 9, 16, 2000, 20, 0, 1), (4097, 9, 32, 2000, 20, 0, 4),
+    (16384, 9, 96, 100, 20, 0, 4), (16385, 9, 500, 1000, 6, 1, 1)])
+def test_waves_per_item(harness, icap, per_box, per_leaf, n_up, levels, own, waves):
+    n = per_leaf * min(n_up, 1000)
+    r = harness("waves", icap, per_box * 1000, 1000, n, n_up, levels, own)
     assert r.returncode == 0 and int(r.stdout) == waves
 
 
-@pytest.mark.parametrize("levels,ne,even", [
-    (1, 1, 1), (2, 4, 1), (2, 3, 0), (7, 4096, 1), (7, 4093, 1), (7, 3687, 1), (7, 3686, 0),
-    (7, 9067, 1), (8, 9067, 0), (16, 4 ** 15, 1), (17, 4 ** 15, 0), (31, 10 ** 6, 0)])
-def test_even_boxes(harness, levels, ne, even):
-    r = harness("even", levels, ne)
-    assert r.returncode == 0 and int(r.stdout) == even
+@pytest.mark.parametrize("per_leaf,waves", [(31, 1), (32, 4)])
+def test_complete_trees_need_more_sources(harness, per_leaf, waves):
+    r = harness("waves", 4200, 9 * 4096, 4096, per_leaf * 4096, 4096, 7, 0)
+    assert r.returncode == 0 and int(r.stdout) == waves
 
 
 @pytest.mark.parametrize("levels,ne,even", [
